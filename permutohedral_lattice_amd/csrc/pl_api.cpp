@@ -112,6 +112,9 @@ struct pl_lattice {
     uint4 *created_entries = nullptr;      // [n_blocks * list_stride()]
     int *block_count = nullptr;            // [n_blocks]
     int *chunk_count = nullptr;            // [2][n_chunks]
+    // which of the two sets is zero: the numbering pass of a build zeroes the other set, but a
+    // build that numbers its vertices itself leaves both as they are
+    bool chunk_count_clean[2] = {false, false};
     size_t n_chunks = 0;
     size_t replay_capacity = 0;
     bool lists_wide = false;               // created_entries has room for two entries per vertex
@@ -300,6 +303,7 @@ int ensure_replay(pl_lattice *h, bool wide) {
         (h->f64 && !h->weights64))
         return PL_ENOMEM;
     PL_HIP(plk::fill_zero(reinterpret_cast<float *>(h->chunk_count), 2 * h->n_chunks, h->stream));
+    h->chunk_count_clean[0] = h->chunk_count_clean[1] = true;
     h->replay_capacity = want;
     return PL_OK;
 }
@@ -372,15 +376,6 @@ int ensure_order(pl_lattice *h) {
     h->dfree(h->point_order);
     h->dfree(h->locality_words);
     h->dfree(h->bin_rank);
-    h->dfree(h->lists_of_vertices.start);
-    h->dfree(h->lists_of_vertices.entries);
-    h->dfree(h->lists_of_vertices.count);
-    h->dfree(h->lists_of_vertices.places);
-    h->dfree(h->lists_of_vertices.block_sums);
-    h->dfree(h->lists_of_vertices.chunks.chunk_start);
-    h->dfree(h->lists_of_vertices.chunks.chunk);
-    h->dfree(h->lists_of_vertices.chunks.long_lists);
-    h->dfree(h->lists_of_vertices.chunks.partial_rows);
     h->order_capacity = 0;
     const unsigned max_bins = plk::locality_bins_for(h->N);
     const size_t words = 32 + 2 * (size_t)max_bins + 3 * (size_t)plk::locality_scan_chunks(max_bins) + 1;
@@ -486,6 +481,14 @@ int enqueue_build(pl_lattice *h, const plk::PointFeatures &features, const doubl
     const plk::VertexTables vertices{h->cell_vertex, h->vertex_keys, h->vertex_cell, h->neighbours,
                                      h->max_vertices()};
     const plk::CreatedLists lists = h->lists(h->counter_set);
+    if (!numbers_in_build) {
+        // (sums of an earlier build would shift the numbers of this one's vertices past the
+        // tables' filled rows)
+        if (!h->chunk_count_clean[h->counter_set])
+            PL_HIP(plk::fill_zero(reinterpret_cast<float *>(lists.chunk_count), h->n_chunks, h->stream));
+        h->chunk_count_clean[h->counter_set] = false;
+        h->chunk_count_clean[previous_set] = true;
+    }
     // the merging build numbers its vertices itself and reports to the host
     const plk::InBuildNumbering numbering{
         h->cell_vertex, h->vertex_keys, h->vertex_cell, h->neighbours, h->max_vertices(),
@@ -927,6 +930,15 @@ int pl_destroy(pl_handle h) {
     h->dfree(h->point_order);
     h->dfree(h->locality_words);
     h->dfree(h->bin_rank);
+    h->dfree(h->lists_of_vertices.start);
+    h->dfree(h->lists_of_vertices.entries);
+    h->dfree(h->lists_of_vertices.count);
+    h->dfree(h->lists_of_vertices.places);
+    h->dfree(h->lists_of_vertices.block_sums);
+    h->dfree(h->lists_of_vertices.chunks.chunk_start);
+    h->dfree(h->lists_of_vertices.chunks.chunk);
+    h->dfree(h->lists_of_vertices.chunks.long_lists);
+    h->dfree(h->lists_of_vertices.chunks.partial_rows);
     if (h->h_status) (void)hipHostFree(h->h_status);
     for (int i = 0; i < EV_COUNT; ++i)
         if (h->ev[i]) (void)hipEventDestroy(h->ev[i]);

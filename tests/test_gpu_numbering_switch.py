@@ -1,0 +1,58 @@
+"""One handle whose builds number their vertices in both ways by turns: in the build itself
+(``filter`` on a grid) and in the pass behind it (``build``, and ``filter`` while tiles with too many
+distinct keys keep a handle from merging them)."""
+import numpy as np
+import pytest
+
+pytestmark = pytest.mark.gpu
+
+
+def _case(side, beta, seed, blobs):
+    import torch
+    from permutohedral_lattice_amd import synth
+    img = synth.blob_image(side, side, seed) if blobs else synth.uniform_image((side, side, 3), seed)
+    pos = synth.bilateral_positions(img, 8.0, beta)
+    val = synth.uniform_image((side * side, 3), seed + 1)
+    return pos, val, torch.from_numpy(pos).cuda(), torch.from_numpy(val).cuda()
+
+
+def test_builds_and_filters_by_turns_on_one_handle():
+    import oracle
+    import torch
+    import permutohedral_lattice_amd as pla
+    side = 96
+    pos, val, d_pos, d_val = _case(side, 0.125, 5, True)
+    cpu = oracle.Lattice(5, 4, side * side)
+    want = cpu.filter(val, pos, False)
+    lat = pla.PermutohedralLattice(5, 4, side * side)
+    lat.set_point_grid((side, side))
+    out = torch.empty_like(d_val)
+    for entry in "bfbffbbfb":
+        out.zero_()
+        if entry == "b":
+            lat.build(d_pos)
+            lat.apply(out, d_val)
+        else:
+            lat.filter(out, d_val, d_pos)
+        assert lat.num_vertices == cpu.num_vertices, entry
+        assert float(np.abs(out.cpu().numpy() - want).max()) <= 1e-5
+
+
+def test_a_handle_that_returns_to_merging_again_and_again():
+    """A noise image overflows the tiles' tables: plain builds for 32 calls, another try to merge,
+    plain builds again."""
+    import oracle
+    import torch
+    import permutohedral_lattice_amd as pla
+    side = 64
+    pos, val, d_pos, d_val = _case(side, 0.05, 9, False)
+    cpu = oracle.Lattice(5, 4, side * side)
+    want = cpu.filter(val, pos, False)
+    lat = pla.PermutohedralLattice(5, 4, side * side)
+    lat.set_point_grid((side, side))
+    out = torch.empty_like(d_val)
+    for _ in range(37):
+        out.zero_()
+        lat.filter(out, d_val, d_pos)
+        assert lat.num_vertices == cpu.num_vertices
+        assert float(np.abs(out.cpu().numpy() - want).max()) <= 1e-5
