@@ -183,6 +183,8 @@ struct pl_lattice {
     int *point_order = nullptr;            // [256 * locality_tiles_for(N)]
     unsigned *locality_words = nullptr;    // the bins, range of feature 0, counts and firsts of the bins
     uint2 *bin_rank = nullptr;             // [N]
+    unsigned *bin_table = nullptr;         // histograms of the bins (plk::locality_table_rows)
+    bool list_in_order = false;            // the last list that was ordered ran from a bin to the next
     int order_capacity = 0;
     hipEvent_t ev[EV_COUNT] = {};
     bool ev_recorded[EV_COUNT] = {};
@@ -354,7 +356,8 @@ int ensure_vertex_lists(pl_lattice *h) {
 plk::LocalityScratch locality_scratch(const pl_lattice *h) {
     const unsigned max_bins = plk::locality_bins_for(h->N);
     plk::LocalityScratch scratch{};
-    // (32 words ahead of the arrays: the record of the bins, the range, the number of tiles)
+    // (32 words ahead of the arrays: the record of the bins, the range, the number of tiles, whether
+    // the list is in order)
     constexpr size_t head_words = 32;
     static_assert(plk::kLocalityBinsBytes <= 16 * sizeof(unsigned), "the record fits its place");
     scratch.bins = h->locality_words;
@@ -363,6 +366,9 @@ plk::LocalityScratch locality_scratch(const pl_lattice *h) {
     scratch.bin_count = h->locality_words + head_words;
     scratch.bin_first = h->locality_words + head_words + max_bins;
     scratch.bin_rank = h->bin_rank;
+    scratch.table = h->bin_table;
+    scratch.in_order = h->locality_words + 21;
+    scratch.expect_in_order = h->list_in_order;
     scratch.max_bins = max_bins;
     scratch.max_tiles = plk::locality_tiles_for(h->N);
     scratch.chunk_sums = h->locality_words + head_words + 2 * (size_t)max_bins;
@@ -376,13 +382,17 @@ int ensure_order(pl_lattice *h) {
     h->dfree(h->point_order);
     h->dfree(h->locality_words);
     h->dfree(h->bin_rank);
+    h->dfree(h->bin_table);
     h->order_capacity = 0;
     const unsigned max_bins = plk::locality_bins_for(h->N);
     const size_t words = 32 + 2 * (size_t)max_bins + 3 * (size_t)plk::locality_scan_chunks(max_bins) + 1;
     h->point_order = (int *)h->dmalloc(sizeof(int) * 256 * (size_t)plk::locality_tiles_for(h->N));
     h->locality_words = (unsigned *)h->dmalloc(sizeof(unsigned) * words);
     h->bin_rank = (uint2 *)h->dmalloc(sizeof(uint2) * (size_t)h->N);
-    if (!h->point_order || !h->locality_words || !h->bin_rank) return PL_ENOMEM;
+    const size_t table_words = (size_t)plk::locality_table_rows(h->N) * max_bins;
+    if (table_words) h->bin_table = (unsigned *)h->dmalloc(sizeof(unsigned) * table_words);
+    if (!h->point_order || !h->locality_words || !h->bin_rank || (table_words && !h->bin_table))
+        return PL_ENOMEM;
     // (the pass leaves its counts zero for the next call)
     PL_HIP(plk::fill_zero(reinterpret_cast<float *>(h->locality_words), words, h->stream));
     h->order_capacity = h->N;
@@ -459,7 +469,8 @@ int enqueue_build(pl_lattice *h, const plk::PointFeatures &features, const doubl
     }
     // (what this build's report will carry; never 0, which is what a fresh status holds)
     h->status_sequence = h->status_sequence + 1u ? h->status_sequence + 1u : 1u;
-    const plk::HostReport report_to{h->h_status, h->status_sequence};
+    const plk::HostReport report_to{h->h_status, h->status_sequence,
+                                    h->map.mode == 1 ? locality_scratch(h).in_order : nullptr};
     h->mark(EV_T0);
     h->stage_ran[0] = h->map.mode == 1 || !h->table_clean || cells != h->n_cells;
     h->stage_ran[1] = true;
@@ -742,6 +753,7 @@ int verify_build(pl_lattice *h, uint32_t *retry_cells) {
     }
     const int flags = status.flags;
     const int m = status.num_vertices;
+    if (h->map.mode == 1) h->list_in_order = status.list_in_order != 0;
     h->last_n_segments = status.n_segments;
     h->last_max_segment = status.max_segment;
     if (flags & plk::kFlagKeyRange) {
@@ -930,6 +942,7 @@ int pl_destroy(pl_handle h) {
     h->dfree(h->point_order);
     h->dfree(h->locality_words);
     h->dfree(h->bin_rank);
+    h->dfree(h->bin_table);
     h->dfree(h->lists_of_vertices.start);
     h->dfree(h->lists_of_vertices.entries);
     h->dfree(h->lists_of_vertices.count);
@@ -1413,7 +1426,8 @@ int pl_get_info(pl_handle h, int what, long *value) {
                 b += sizeof(int) * 256 * (size_t)plk::locality_tiles_for(h->order_capacity) +
                      sizeof(uint2) * (size_t)h->order_capacity +
                      sizeof(unsigned) * (33 + 2 * (size_t)max_bins +
-                                         3 * (size_t)plk::locality_scan_chunks(max_bins));
+                                         3 * (size_t)plk::locality_scan_chunks(max_bins) +
+                                         (size_t)plk::locality_table_rows(h->order_capacity) * max_bins);
             }
             *value = (long)b;
             return PL_OK;

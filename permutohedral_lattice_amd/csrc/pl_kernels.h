@@ -72,6 +72,7 @@ struct HostStatus {
     int max_segment;   // vertices in the fullest segment (num_vertices when there are none)
     int n_segments;
     int foreign_rows;  // CreatedLists rows of a build that numbered its vertices (an estimate)
+    int list_in_order; // LocalityScratch::in_order of the list the build ordered (0: ordered none)
     // written last, behind a system-wide fence: the number of the build the fields above belong
     // to.  The host, which holds the struct in pinned memory, polls this word instead of waiting
     // for an event behind the kernel (an event between two kernels of a stream keeps the second
@@ -82,6 +83,7 @@ struct HostStatus {
 struct HostReport {
     HostStatus *status;
     unsigned sequence;
+    const unsigned *list_in_order;   // LocalityScratch::in_order, or none
 };
 
 // Per-vertex and per-cell tables of a lattice (all sized by the hash table): vertex v has key
@@ -469,13 +471,29 @@ struct LocalityScratch {
     // for the scan of many bins by many workgroups, each a chunk of 4096 bins:
     unsigned *chunk_sums;  // [2 * locality_scan_chunks(max_bins)]
     unsigned *chunk_first; // [locality_scan_chunks(max_bins) + 1]
+    unsigned *table;       // [locality_table_rows(N) * max_bins], none where that is 0
+    unsigned *in_order;    // whether this list runs from a bin to the next (k_locality_table)
+    bool expect_in_order;  // the handle's last list did
 };
 inline unsigned locality_scan_chunks(unsigned max_bins) { return (max_bins / 4u + 1023u) / 1024u; }
+inline unsigned locality_bins_for(int N) { return ((unsigned)N / 32u + 1024u) & ~3u; }
+// The table of histograms a list of N points is counted with (k_locality_table): a row per
+// locality_table_points(N) points (one, two or four per thread of a workgroup, so that there are
+// enough workgroups and few rows), locality_table_rows(N) of them; 0: no table, ranks are drawn with
+// atomics on memory.  At most as many points as have their bins in one workgroup's LDS, and no
+// fewer than kLocalityTableFrom (a filter of a cloud
+// of 16384 points 54.3 us with atomics, 49.7 with the table; 131072: 86.3 and 60.6; a million: 237 and 173)
+constexpr unsigned kLocalityTableBins = 40960, kLocalityTableRows = 320;
+constexpr int kLocalityTableFrom = 16384;
+inline unsigned locality_table_points(int N) { return N <= (1 << 18) ? 1024u : N <= (1 << 19) ? 2048u : 4096u; }
+inline unsigned locality_table_rows(int N) {
+    const unsigned points = locality_table_points(N), rows = ((unsigned)N + points - 1u) / points;
+    return N >= kLocalityTableFrom && locality_bins_for(N) <= kLocalityTableBins && rows <= kLocalityTableRows ? rows : 0u;
+}
 inline unsigned locality_tiles_for(int N) {
     const unsigned waves = ((unsigned)N + 63u) / 64u;
     return (waves + waves / 4u + 3u) / 4u + 1u;
 }
-inline unsigned locality_bins_for(int N) { return ((unsigned)N / 32u + 1024u) & ~3u; }
 // positions or positions64 (the other null); order: 256 * scratch.max_tiles entries
 hipError_t order_by_locality(const float *positions, const double *positions64, int N, int pd,
                              const LocalityScratch &scratch, int *order, hipStream_t s);

@@ -937,6 +937,7 @@ __global__ __launch_bounds__(64) void k_number_vertices(CreatedLists lists, int 
             host_status->max_segment = (int)m;
             host_status->n_segments = 0;
             host_status->foreign_rows = 0;
+            host_status->list_in_order = host_report.list_in_order ? (int)*host_report.list_in_order : 0;
             __threadfence_system();
             __hip_atomic_store(&host_status->sequence, host_report.sequence, __ATOMIC_RELAXED,
                                __HIP_MEMORY_SCOPE_SYSTEM);
@@ -1056,6 +1057,7 @@ __global__ __launch_bounds__(kBlock) void k_neighbours(VertexTables vertices,
             host_status->max_segment = (int)fullest;
             host_status->n_segments = n_segments;
             host_status->foreign_rows = (int)(report->foreign_rows_sampled.n * kForeignSampling);
+            host_status->list_in_order = host_report.list_in_order ? (int)*host_report.list_in_order : 0;
             __threadfence_system();
             __hip_atomic_store(&host_status->sequence, host_report.sequence, __ATOMIC_RELAXED,
                                __HIP_MEMORY_SCOPE_SYSTEM);

@@ -202,9 +202,24 @@ __global__ __launch_bounds__(kScanBlock) void k_locality_bins(const T *__restric
         }
     }
     v = block_box(v, wave_part);
+    __shared__ LocalityBins shared_bins;
+    __shared__ int changes;
     if (threadIdx.x == 0) {
-        const LocalityBins bins = bins_over(v, N, pd, scratch.max_bins);
+        shared_bins = bins_over(v, N, pd, scratch.max_bins);
+        changes = 0;
+    }
+    __syncthreads();
+    const LocalityBins bins = shared_bins;
+    if (scratch.table) {
+        // how often a sample's bin is not that of the point before it in its run (64 of the runs)
+        const int bin = (int)bin_of(bins, p[0]);
+        const int changed = __builtin_popcountll(wave_ballot(threadIdx.x % kSampleRun != 0 && bin != __shfl_up(bin, 1)));
+        if ((threadIdx.x & 63) == 0) atomicAdd(&changes, changed);
+        __syncthreads();
+    }
+    if (threadIdx.x == 0) {
         *bins_record(scratch) = bins;
+        *scratch.in_order = 4 * changes < kScanBlock ? 1u : 0u;
         scratch.range0[0] = bins.lo[0];
         scratch.range0[1] = bins.hi0;
     }
@@ -269,6 +284,130 @@ __global__ __launch_bounds__(kBlock) void k_locality_count(const T *__restrict__
         first_rank[k] = __shfl(first_rank[k], leader[k]);
         if (valid[k]) scratch.bin_rank[n[k]] = make_uint2((unsigned)bin[k], first_rank[k] + index[k]);
     }
+}
+
+// The same for lists of many points, without an atomic on memory where the list has no order: a
+// workgroup of kScanBlock threads counts its points (kPerThread a thread) in a histogram of all bins in
+// LDS, two 16-bit counts to a word (the LDS atomic returns the point's rank among the workgroup's), and
+// leaves the histogram as a row of a table in memory; the next launch turns every column of the table
+// into the points of the rows above, and its sum into the bin's count.  What bounds the kernel above is
+// its returning atomics, one per point of a list in no order (8.3 G/s): half a million points of a
+// cloud 59.8 us, these two launches 6.6 + 4.6 us, the scatter 3.5 us longer.
+// A list that runs through its bins (an image row by row: a bin every 8 points) needs a fraction of the
+// atomics, and filling and reading the table would cost more than those: where the sampled runs changed
+// their bin at fewer than a quarter of their points, ranks are drawn from memory as above.  (A handle
+// whose last list was in order takes the kernel above at once: the launches here and below, which
+// then have nothing to do, and fewer workgroups cost 3 to 7 us a call; telling costs 1 us.)
+template <typename T, int kPerThread>
+__global__ __launch_bounds__(kScanBlock) void k_locality_table(const T *__restrict__ positions, int N, int pd,
+                                                                LocalityScratch scratch, int *__restrict__ order,
+                                                                size_t order_entries) {
+    __shared__ unsigned count[kLocalityTableBins / 2];
+    static_assert(kScanBlock * kPerThread < 65536, "16-bit counts");
+    const int lane = threadIdx.x & 63;
+    for (size_t i = (size_t)blockIdx.x * kScanBlock + threadIdx.x; i < order_entries;
+         i += (size_t)gridDim.x * kScanBlock)
+        order[i] = -1;
+    const LocalityBins bins = *bins_record(scratch);
+    const bool table = *scratch.in_order == 0u;
+    const unsigned n_bins = bins.n_bins < scratch.max_bins ? bins.n_bins : scratch.max_bins;
+    if (table)
+        for (unsigned i = threadIdx.x; 2u * i < n_bins; i += kScanBlock) count[i] = 0u;
+    int bin[kPerThread], leader[kPerThread];
+    unsigned size[kPerThread], index[kPerThread], rank[kPerThread];
+    bool valid[kPerThread];
+    float p[kPerThread][kBoxFeatures];
+    const size_t first_point = (size_t)blockIdx.x * (kScanBlock * kPerThread) + threadIdx.x;
+#pragma unroll
+    for (int k = 0; k < kPerThread; ++k) {
+        // (a point past the end reads the last one, so that no load waits behind a branch)
+        const size_t n = first_point + (size_t)k * kScanBlock;
+        valid[k] = n < (size_t)N;
+        first_features(positions, valid[k] ? n : (size_t)N - 1, pd, p[k]);
+    }
+    __syncthreads();
+#pragma unroll
+    for (int k = 0; k < kPerThread; ++k) {
+        bin[k] = valid[k] ? (int)bin_of(bins, p[k]) : 0;
+        // the lanes that share a bin draw together (LDS atomics on one word take turns of four
+        // cycles); not worth it in LDS once a bin has fewer than four of them
+        uint64_t todo = wave_ballot(valid[k]);
+        leader[k] = lane;
+        size[k] = 1;
+        index[k] = 0;
+        for (int turn = 0; todo != 0 && turn < 16; ++turn) {
+            const int first = __builtin_ctzll(todo);
+            const int b = __builtin_amdgcn_readlane(bin[k], first);
+            const uint64_t same = lanes_equal(bin[k], b) & todo;
+            const unsigned lanes = (unsigned)__builtin_popcountll(same);
+            if (lane_in(same)) {
+                leader[k] = first;
+                size[k] = lanes;
+                index[k] = __builtin_amdgcn_mbcnt_hi((unsigned)(same >> 32),
+                                                     __builtin_amdgcn_mbcnt_lo((unsigned)same, 0u));
+            }
+            todo &= ~same;
+            if (table && lanes < 4) break;
+        }
+    }
+#pragma unroll
+    for (int k = 0; k < kPerThread; ++k) {
+        rank[k] = 0;
+        if (valid[k] && leader[k] == lane) {
+            const unsigned shift = ((unsigned)bin[k] & 1u) * 16u;
+            rank[k] = table ? (atomicAdd(&count[(unsigned)bin[k] >> 1], size[k] << shift) >> shift) & 0xffffu
+                            : atomicAdd(&scratch.bin_count[bin[k]], size[k]);
+        }
+    }
+#pragma unroll
+    for (int k = 0; k < kPerThread; ++k) {
+        rank[k] = __shfl(rank[k], leader[k]) + index[k];
+        if (valid[k])
+            scratch.bin_rank[first_point + (size_t)k * kScanBlock] = make_uint2((unsigned)bin[k], rank[k]);
+    }
+    if (!table) return;
+    __syncthreads();
+    unsigned *__restrict__ row = scratch.table + (size_t)blockIdx.x * n_bins;
+    for (unsigned i = threadIdx.x; i < n_bins; i += kScanBlock)
+        row[i] = (count[i >> 1] >> ((i & 1u) * 16u)) & 0xffffu;
+}
+
+// Sixty-four columns per workgroup, its sixteen wavefronts a sixteenth of the rows each.
+constexpr unsigned kTableGroups = kScanBlock / 64;
+constexpr unsigned kTableHeld = (kLocalityTableRows + kTableGroups - 1) / kTableGroups;
+__global__ __launch_bounds__(kScanBlock) void k_locality_table_columns(LocalityScratch scratch, unsigned rows) {
+    __shared__ unsigned group_sum[kTableGroups][64];
+    unsigned n_bins = bins_record(scratch)->n_bins;
+    if (n_bins > scratch.max_bins) n_bins = scratch.max_bins;
+    if (blockIdx.x * 64u >= n_bins || *scratch.in_order) return;     // (the whole workgroup)
+    const unsigned lane = threadIdx.x & 63u, group = threadIdx.x >> 6;
+    const unsigned bin = blockIdx.x * 64u + lane;
+    const unsigned column = bin < n_bins ? bin : n_bins - 1u;
+    const unsigned per = (rows + kTableGroups - 1u) / kTableGroups;
+    const unsigned begin = group * per;
+    unsigned held[kTableHeld], sum = 0;
+#pragma unroll
+    for (unsigned k = 0; k < kTableHeld; ++k) {
+        const unsigned r = begin + k;
+        held[k] = scratch.table[(size_t)(k < per && r < rows ? r : 0u) * n_bins + column];
+    }
+#pragma unroll
+    for (unsigned k = 0; k < kTableHeld; ++k) {
+        if (!(k < per && begin + k < rows)) held[k] = 0u;
+        sum += held[k];
+    }
+    group_sum[group][lane] = sum;
+    __syncthreads();
+    unsigned before = 0;
+    for (unsigned g = 0; g < group; ++g) before += group_sum[g][lane];
+    if (bin >= n_bins) return;
+#pragma unroll
+    for (unsigned k = 0; k < kTableHeld; ++k) {
+        const unsigned r = begin + k;
+        if (k < per && r < rows) scratch.table[(size_t)r * n_bins + bin] = before;
+        before += held[k];
+    }
+    if (group == kTableGroups - 1u) scratch.bin_count[bin] = before;
 }
 
 // bin_first = the place of each bin's first point in the order; the counts go back to zero for
@@ -455,11 +594,16 @@ __global__ __launch_bounds__(kBlock) void k_locality_chunk_scan(LocalityScratch 
 }
 
 __global__ __launch_bounds__(kBlock) void k_locality_scatter(LocalityScratch scratch, int N,
-                                                              int *__restrict__ order) {
+                                                              unsigned points_per_row, int *__restrict__ order) {
     const size_t n = (size_t)blockIdx.x * kBlock + threadIdx.x;
     if (n >= (size_t)N) return;
     const uint2 br = scratch.bin_rank[n];
-    const unsigned place = scratch.bin_first[br.x] + br.y;
+    unsigned place = scratch.bin_first[br.x] + br.y;
+    // (a rank from the table of histograms is among the points of one row)
+    if (points_per_row && !*scratch.in_order) {
+        const unsigned n_bins = bins_record(scratch)->n_bins;
+        place += scratch.table[n / points_per_row * (n_bins < scratch.max_bins ? n_bins : scratch.max_bins) + br.x];
+    }
     // (ranks come from atomics on counts that started at zero, so the place is the point's own)
     if ((size_t)place < (size_t)scratch.max_tiles * kBlock) order[place] = (int)n;
 }
@@ -469,9 +613,19 @@ hipError_t order_points(const T *positions, int N, int pd, const LocalityScratch
                         hipStream_t s) {
     const unsigned blocks = (unsigned)(((size_t)N + kBlock - 1) / kBlock);
     hipLaunchKernelGGL((k_locality_bins<T>), dim3(1), dim3(kScanBlock), 0, s, positions, N, pd, scratch);
-    const unsigned count_blocks = (blocks + kCountPoints - 1) / kCountPoints;
-    hipLaunchKernelGGL((k_locality_count<T>), dim3(count_blocks), dim3(kBlock), 0, s, positions, N, pd, scratch,
-                       order, (size_t)scratch.max_tiles * kBlock);
+    const unsigned table_rows = scratch.table && !scratch.expect_in_order ? locality_table_rows(N) : 0u;
+    const unsigned per_thread = locality_table_points(N) / kScanBlock;
+    if (table_rows) {
+        const auto count = per_thread == 1 ? k_locality_table<T, 1> : per_thread == 2 ? k_locality_table<T, 2> : k_locality_table<T, 4>;
+        hipLaunchKernelGGL(count, dim3(table_rows), dim3(kScanBlock), 0, s, positions, N, pd, scratch, order,
+                           (size_t)scratch.max_tiles * kBlock);
+        hipLaunchKernelGGL(k_locality_table_columns, dim3((scratch.max_bins + 63u) / 64u), dim3(kScanBlock), 0, s,
+                           scratch, table_rows);
+    } else {
+        const unsigned count_blocks = (blocks + kCountPoints - 1) / kCountPoints;
+        hipLaunchKernelGGL((k_locality_count<T>), dim3(count_blocks), dim3(kBlock), 0, s, positions, N, pd, scratch,
+                           order, (size_t)scratch.max_tiles * kBlock);
+    }
     if (scratch.max_bins <= kOneWorkgroupScans) {
         hipLaunchKernelGGL(k_locality_scan, dim3(1), dim3(kScanBlock), 0, s, scratch, N);
     } else {
@@ -481,7 +635,8 @@ hipError_t order_points(const T *positions, int N, int pd, const LocalityScratch
         hipLaunchKernelGGL(k_locality_chunk_places, dim3(1), dim3(64), 0, s, scratch, N, n_chunks);
         hipLaunchKernelGGL(k_locality_chunk_scan, dim3(n_chunks), dim3(kBlock), 0, s, scratch, n_chunks);
     }
-    hipLaunchKernelGGL(k_locality_scatter, dim3(blocks), dim3(kBlock), 0, s, scratch, N, order);
+    hipLaunchKernelGGL(k_locality_scatter, dim3(blocks), dim3(kBlock), 0, s, scratch, N,
+                       table_rows ? locality_table_points(N) : 0u, order);
     return hipGetLastError();
 }
 
@@ -491,11 +646,11 @@ hipError_t order_by_locality(const float *positions, const double *positions64, 
                              const LocalityScratch &scratch, int *order, hipStream_t s) {
     if (N <= 0) return hipSuccess;
     if (!scratch.bins || !scratch.range0 || !scratch.bin_count || !scratch.bin_first ||
-        !scratch.bin_rank || !order || !scratch.n_tiles || !scratch.chunk_sums || !scratch.chunk_first ||
+        !scratch.bin_rank || !order || !scratch.n_tiles || !scratch.in_order || !scratch.chunk_sums || !scratch.chunk_first ||
         scratch.max_bins < 4u ||
         (size_t)scratch.max_tiles * kBlock < (size_t)N || scratch.max_bins % 4u != 0u ||
         (reinterpret_cast<uintptr_t>(scratch.bin_count) | reinterpret_cast<uintptr_t>(scratch.bin_first)) % 16u != 0u ||
-        pd < 1)
+        pd < 1 || (scratch.table && locality_table_rows(N) && scratch.max_bins > kLocalityTableBins))
         return hipErrorInvalidValue;
     if (positions64) return order_points<double>(positions64, N, pd, scratch, order, s);
     if (positions) return order_points<float>(positions, N, pd, scratch, order, s);

@@ -246,3 +246,32 @@ def test_lists_just_long_enough_to_be_ordered(pd, vd, n):
     assert np.abs(host(out) - want_reverse).max() <= MAX_ABS_TOL
     assert rel_l2(host(out), want_reverse) <= REL_L2_TOL
     lat.close()
+
+
+@pytest.mark.parametrize("n", [16383, 16384, 16385, (1 << 18) + 1, (1 << 19) - 1, (1 << 19) + 2047, 1277951, 1277985])
+@pytest.mark.parametrize("ordered_list", [False, True])
+def test_lists_counted_in_a_table_of_histograms(n, ordered_list):
+    """Both sides of the lengths at which the ranks of the points come from histograms in LDS (and
+    at which a workgroup takes one, two and four points per thread), lists in no order and lists that
+    run through the bins: the lattice of the list in its own order, point by point the same output."""
+    gen = torch.Generator("cuda").manual_seed(n)
+    pos = torch.rand((n, 2), device="cuda", generator=gen) * (n ** 0.5 / 6.0)
+    if ordered_list:
+        pos = pos[torch.argsort((pos[:, 0] * 1.5).floor() * 4096.0 + pos[:, 1])].contiguous()
+    val = torch.rand((n, 1), device="cuda", generator=gen)
+    outs, keys = [], []
+    for ordered in (1, 0):
+        lat = pla.PermutohedralLattice(2, 2, n)
+        lat.set_option(pla.PL_OPT_GUESS_GRID, 0)
+        lat.set_option(pla.PL_OPT_ORDER_POINTS, ordered)
+        out = torch.empty((n, 1), dtype=torch.float32, device="cuda")
+        for _ in range(2):      # (the second call runs on what the first left in the scratch arrays)
+            out.fill_(float("nan"))
+            lat.filter(out, val, pos, False)
+        torch.cuda.synchronize()
+        assert lat.info(pla.PL_INFO_BUILD_MERGED) == ordered
+        outs.append(out)
+        keys.append(sorted_keys(host(lat.debug_keys()))[0])
+        lat.close()
+    assert (keys[0] == keys[1]).all()
+    assert float((outs[0] - outs[1]).abs().max()) <= 2e-5
