@@ -353,6 +353,16 @@ int pl_lattice_filter_op_f64(const double *input, const double *reference, doubl
                              float theta_alpha, float theta_beta, float theta_gamma, int reverse,
                              pl_stream stream, const pl_alloc *alloc);
 
+/* ----------------------------------------------------------------------------------------
+ * The pointwise step of a dense CRF's mean field around two lattices (no counterpart in the
+ * reference): q[p][c] = softmax over c of logits[p][c] + (message_a[p][c] + message_b[p][c]),
+ * device arrays of n_points rows of n_classes floats, each 16-byte aligned (PL_EINVAL); q may be
+ * any of the others.  At most 128 classes (PL_EUNSUPPORTED).  Enqueued on `stream`.
+ * ---------------------------------------------------------------------------------------- */
+int pl_mean_field_update(float *q, const float *logits, const float *message_a,
+                         const float *message_b, long long n_points, int n_classes,
+                         pl_stream stream);
+
 #ifdef __cplusplus
 }
 #endif

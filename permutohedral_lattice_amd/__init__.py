@@ -44,7 +44,7 @@ EXPORTS = (
     "pl_debug_keys", "pl_debug_values", "pl_debug_replay", "pl_compute_positions", "pl_filter_image", "pl_build_image",
     "pl_filter_begin", "pl_filter_image_begin", "pl_filter_end",
     "pl_build_begin", "pl_build_image_begin", "pl_build_end", "pl_lattice_filter_op",
-    "pl_set_op_concurrency",
+    "pl_set_op_concurrency", "pl_mean_field_update",
     "pl_create_f64", "pl_filter_f64", "pl_build_f64", "pl_apply_f64", "pl_debug_simplex_f64",
     "pl_compute_positions_f64", "pl_lattice_filter_op_f64",
 )
@@ -114,6 +114,7 @@ def _load(path=LIB_PATH):
     lib.pl_build_image_begin.argtypes = [vp, vp, ci, ci, C.POINTER(ci), cf, cf]
     lib.pl_build_end.argtypes = [vp]
     lib.pl_set_op_concurrency.argtypes = [ci]
+    lib.pl_mean_field_update.argtypes = [vp, vp, vp, vp, C.c_longlong, ci, vp]
     lib.pl_lattice_filter_op.argtypes = [vp, vp, vp, ci, ci, C.POINTER(ci), ci, ci, ci, cf, cf, cf,
                                          ci, vp, vp]
     # T = double
@@ -399,6 +400,29 @@ def compute_positions(reference, spatial_dims, spatial_std, feature_std=1.0, out
     _check(call(ref_ptr, _dev(out, "positions", n * pd, dtype), n, rc, len(sd), dims,
                 float(spatial_std), float(feature_std), _stream_ptr()), "pl_compute_positions")
     return out
+
+
+def mean_field_update_supported(logits):
+    """Whether :func:`mean_field_update` may stand for torch's additions and softmax on these
+    logits: plain float32 rows of at most 128 classes on the current GPU that autograd does not
+    follow."""
+    return (type(logits) is torch.Tensor and logits.is_cuda and logits.dtype == torch.float32
+            and logits.is_contiguous() and logits.dim() >= 1 and 1 <= logits.shape[-1] <= 128
+            and logits.device.index == torch.cuda.current_device() and logits.data_ptr() % 16 == 0
+            and not (logits.requires_grad and torch.is_grad_enabled())
+            and torch.autograd.forward_ad.unpack_dual(logits).tangent is None)
+
+
+def mean_field_update(q, logits, message_a, message_b):
+    """``q = softmax(logits + (message_a + message_b))`` over the last dimension, in one pass, on
+    the current stream."""
+    n = logits.numel()
+    _check(_lib.pl_mean_field_update(_dev_f32(q, "q", n), _dev_f32(logits, "logits", n),
+                                     _dev_f32(message_a, "message_a", n),
+                                     _dev_f32(message_b, "message_b", n),
+                                     n // int(logits.shape[-1]), int(logits.shape[-1]), _stream_ptr()),
+           "pl_mean_field_update")
+    return q
 
 
 def _lattice_filter_raw(input_image, reference_image, bilateral, theta_alpha, theta_beta,

@@ -17,11 +17,12 @@ HIP stream of its own (default priority): a message-passing step waits for its i
 caller's stream, runs the applies of all lattices side by side, and the caller's stream waits for
 all of them before it adds the messages up.
 
-torch carries the tensors and does the softmax; the filters are the HIP library's.
+torch carries the tensors; the filters, and the softmax over the logits and both messages, are the
+HIP library's.
 """
 import torch
 
-from . import PermutohedralLattice
+from . import PermutohedralLattice, mean_field_update, mean_field_update_supported
 
 
 class MeanField:
@@ -88,28 +89,41 @@ class MeanField:
             done.record(s)
             caller.wait_event(done)
 
-    def messages(self, q, reverse=False):
-        """bilateral(q) + spatial(q) for ``q [B, ..., n_classes]`` (any spatial shape of N points)."""
+    def _apply_all(self, q, reverse):
+        """Both messages of every item, in the lattices' own buffers."""
         q = q.contiguous().view(self.batch, self.n, self.n_classes)
         self._side_streams_wait_for_caller()
         for b in range(self.batch):
             self.bilateral[b].apply(self._msg_bi[b], q[b], reverse)
             self.spatial[b].apply(self._msg_sp[b], q[b], reverse)
         self._caller_waits_for_side_streams()
+
+    def messages(self, q, reverse=False):
+        """bilateral(q) + spatial(q) for ``q [B, ..., n_classes]`` (any spatial shape of N points)."""
+        self._apply_all(q, reverse)
         return self._msg_bi + self._msg_sp
 
     def infer(self, logits, iterations=5):
         """-> Q after ``iterations`` mean-field updates, shaped like ``logits``."""
         flat = logits.contiguous().view(self.batch, self.n, self.n_classes)
         q = torch.softmax(flat, dim=-1)
+        if type(self).messages is not MeanField.messages or not mean_field_update_supported(flat):
+            # (messages of a class derived from this one; logits that autograd follows into the last
+            # softmax, among others)
+            for _ in range(iterations):
+                q = torch.softmax(flat + self.messages(q), dim=-1)
+            return q.view(logits.shape)
         for _ in range(iterations):
-            q = torch.softmax(flat + self.messages(q), dim=-1)
+            # (q is read by the lattices' streams, and the caller's stream, which writes it anew, has
+            # waited for them)
+            self._apply_all(q, False)
+            mean_field_update(q, flat, self._msg_bi, self._msg_sp)
         return q.view(logits.shape)
 
     def reverse(self, upstream):
         """The op's registered gradient of one message-passing step with respect to its input:
         both filters with ``reverse=True`` on ``upstream``, summed."""
-        return self.messages(upstream, reverse=True).view(upstream.shape).clone()
+        return self.messages(upstream, reverse=True).view(upstream.shape)
 
     def close(self):
         for lat in self.bilateral + self.spatial:

@@ -1556,6 +1556,22 @@ int pl_compute_positions_f64(const double *reference, double *positions, int num
 
 }  // extern "C"
 
+extern "C" int pl_mean_field_update(float *q, const float *logits, const float *message_a,
+                                    const float *message_b, long long n_points, int n_classes,
+                                    pl_stream stream) {
+    if (n_points < 0 || n_classes < 1) return PL_EINVAL;
+    if (n_classes > plk::kMeanFieldMaxClasses) return PL_EUNSUPPORTED;
+    if (n_points == 0) return PL_OK;
+    if (!q || !logits || !message_a || !message_b) return PL_EINVAL;
+    if ((reinterpret_cast<uintptr_t>(q) | reinterpret_cast<uintptr_t>(logits) |
+         reinterpret_cast<uintptr_t>(message_a) | reinterpret_cast<uintptr_t>(message_b)) % 16u != 0u)
+        return PL_EINVAL;
+    if (n_points > (1ll << 40) / n_classes) return PL_EOVERFLOW;
+    PL_HIP(plk::mean_field_update(q, logits, message_a, message_b, (size_t)n_points, n_classes,
+                                  (hipStream_t)stream));
+    return PL_OK;
+}
+
 // ------------------------------------------------------------------------------------------------
 // Op level: shape arithmetic and per-item loop of LatticeFilterOp::Compute
 // (src/LatticeFilterKernel.cpp:111-179 of the reference tree)

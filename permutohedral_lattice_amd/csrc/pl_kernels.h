@@ -502,4 +502,10 @@ hipError_t compute_positions(const float *reference, float *positions, int N, in
                              int n_spatial_dims, const SpatialDims &dims, float spatial_std,
                              float feature_std, hipStream_t s);
 
+// q = softmax(logits + (message_a + message_b)) over the classes of every point: the mean field's step.
+// All four are [n_points][classes], 16-byte aligned; q may be one of the others.
+constexpr int kMeanFieldMaxClasses = 128;
+hipError_t mean_field_update(float *q, const float *logits, const float *message_a, const float *message_b,
+                             size_t n_points, int classes, hipStream_t s);
+
 }  // namespace plk

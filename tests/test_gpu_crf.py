@@ -55,3 +55,41 @@ def test_mean_field_messages_equal_the_op_called_per_iteration():
     torch.cuda.synchronize()
     assert float((got - want).abs().max()) <= 1e-5
     mf.close()
+
+
+@pytest.mark.parametrize("classes", [1, 2, 3, 20, 21, 40, 41, 64, 127, 128])
+@pytest.mark.parametrize("n", [1, 63, 64, 255, 257, 1031])
+def test_mean_field_update_is_the_softmax_of_the_sums(classes, n):
+    import permutohedral_lattice_amd as pla
+    gen = torch.Generator("cuda").manual_seed(classes * 10000 + n)
+    logits, a, b = (3.0 * torch.randn((n, classes), device="cuda", generator=gen) for _ in range(3))
+    if n > 2 and classes > 2:
+        logits[1, 0] = float("-inf")       # (a class that is ruled out)
+        logits[2, 1] = 3.0e38
+    assert pla.mean_field_update_supported(logits)
+    q = pla.mean_field_update(torch.full_like(logits, float("nan")), logits, a, b)
+    want = torch.softmax((logits + (a + b)).double(), dim=-1)
+    # e^x and the quotient to an ulp or two each, a sum of `classes` terms
+    assert float((q.double() - want).abs().max()) <= (classes + 8) * 6e-8
+    pla.mean_field_update(logits, logits, a, b)     # in place
+    assert torch.equal(logits, q)
+
+
+def test_mean_field_update_leaves_other_calls_to_torch():
+    import permutohedral_lattice_amd as pla
+    x = torch.zeros((4, 8), device="cuda")
+    assert pla.mean_field_update_supported(x)
+    assert not pla.mean_field_update_supported(x.double())
+    assert not pla.mean_field_update_supported(x.t())
+    assert not pla.mean_field_update_supported(x.clone().requires_grad_(True))
+    assert not pla.mean_field_update_supported(x.reshape(-1)[1:25].view(3, 8))
+    assert not pla.mean_field_update_supported(torch.zeros((2, 129), device="cuda"))
+    # autograd into the last softmax, as before
+    mf = MeanField(torch.rand((1, 24, 32, 3), device="cuda") * 255.0, 4)
+    logits = torch.randn((1, 24, 32, 4), device="cuda", requires_grad=True)
+    q = mf.infer(logits, iterations=2)
+    (grad,) = torch.autograd.grad(q, logits, torch.ones_like(q))
+    assert grad.shape == logits.shape
+    with torch.no_grad():
+        assert float((mf.infer(logits, iterations=2) - q).abs().max()) <= 1e-6
+    mf.close()
