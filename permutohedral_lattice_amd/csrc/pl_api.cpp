@@ -660,11 +660,14 @@ int enqueue_apply(pl_lattice *h, void *output_any, const void *input_any, int re
         PL_HIP(plk::splat_gather(vd, h->lists_of_vertices, h->list_chunks, h->long_lists, input,
                                  in_channels, h->values[0], h->stream));
     } else if (!h->values_splatted) {
-        if (!h->values_zeroed) PL_HIP(plk::fill_zero(h->values[0], (size_t)mv * vd, h->stream));
+        // (a build that has been checked and numbered its vertices densely: their rows, not the table's)
+        const size_t filled = h->verified && h->n_segments == 0 ? (size_t)h->M : (size_t)mv;
+        if (!h->values_zeroed) PL_HIP(plk::fill_zero(h->values[0], filled * vd, h->stream));
         h->mark(EV_FILL);
-        PL_HIP(plk::splat(pd, vd, h->map, input, in_channels, h->replay,
-                          h->replay_holds_cells ? h->cell_vertex : nullptr, h->values[0],
-                          h->xcd_aware ? 1 : 0, h->stream));
+        const auto splat = h->last_build_merged && plk::splat_tile_takes(vd) ? plk::splat_tile : plk::splat;
+        PL_HIP(splat(pd, vd, h->map, input, in_channels, h->replay,
+                     h->replay_holds_cells ? h->cell_vertex : nullptr, h->values[0],
+                     h->xcd_aware ? 1 : 0, h->stream));
         h->replay_holds_cells = false;
     } else {
         h->mark(EV_FILL);
