@@ -104,7 +104,7 @@ struct pl_lattice {
     int wide_for = 0, wide_backoff = 32;
     bool may_widen = true;             // (not in the static scratch of pl_filter_static: no room)
 
-    // per-point arrays, (pd+1) rows of map.n_blocks*256 entries in thread order
+    // per-point arrays, per workgroup (pd+1) rows of 256 entries in thread order
     plk::PointMap map{};
     plk::ReplayEntry *replay = nullptr;
     // what each workgroup of the build created (see plk::CreatedLists); the chunk counts exist

@@ -42,8 +42,8 @@ __global__ __launch_bounds__(kBlock) void k_list_places(PointMap map, ReplayEntr
                                                          int max_vertices) {
     unsigned vblock;
     if (!block_of_points(map, 1, vblock)) return;
-    const size_t t = (size_t)vblock * kBlock + threadIdx.x;
-    const size_t T = (size_t)gridDim.x * kBlock;
+    const size_t t = (size_t)vblock * kBlock * D1 + threadIdx.x;
+    constexpr size_t T = kBlock;
     const int n = point_of_thread(map, vblock, threadIdx.x);
     const int lane = threadIdx.x & 63;
 
@@ -268,8 +268,8 @@ __global__ __launch_bounds__(kBlock) void k_list_fill(PointMap map,
     }
     unsigned vblock;
     if (!block_of_points(map, 1, vblock)) return;
-    const size_t t = (size_t)vblock * kBlock + threadIdx.x;
-    const size_t T = (size_t)gridDim.x * kBlock;
+    const size_t t = (size_t)vblock * kBlock * D1 + threadIdx.x;
+    constexpr size_t T = kBlock;
     const int n = point_of_thread(map, vblock, threadIdx.x);
     if (n < 0) return;
     ReplayEntry e[D1];

@@ -215,8 +215,11 @@ PointMap make_point_map(int N, int n_dims, const int *dims);
 hipError_t clear_table(uint64_t *cell_keys, uint32_t n_cells, hipStream_t s);
 
 // Stage 1+2: per point embed, enclosing simplex, barycentric weights, then insertion of the pd+1
-// vertex keys.  The replay arrays hold (pd+1) rows of T = map.n_blocks*256 entries in thread
-// order: replay[r*T+t] := hash cell of vertex r of the point of thread t (-1: no point) and its
+// vertex keys.  The replay arrays hold (pd+1) rows of 256 entries per workgroup, in thread
+// order: replay[(b*(pd+1) + r)*256 + t] := hash cell of vertex r of the point of thread t of workgroup b
+// (-1: no point; a workgroup's rows next to each other are one stretch of memory to a pass over the
+// points and constant offsets from one address; rows of all workgroups one behind the other: volume of
+// 8.4 M voxels 521.5 us a filter, this 516.2; an apply of 1024x1024 points 62.9 and 62.2) and its
 // barycentric weight.  The lane whose insertion created a vertex appends its cell and key to
 // its workgroup's list in created_lists.
 // splat_vd != 0 (allowed when build_can_splat(vd)): the kernel also splats `input`
@@ -239,7 +242,7 @@ hipError_t build(int pd, const PointFeatures &features, const PointMap &map, con
                  hipStream_t s);
 
 // The build for double values: the same kernel on points.positions with points.scale; replay[]
-// receives the cells (and the weights rounded to float), points.weights[r*T+t] the weights.
+// receives the cells (and the weights rounded to float), points.weights the weights at the same places.
 hipError_t build_f64(int pd, const Points64 &points, const PointMap &map, uint64_t *cell_keys,
                      uint32_t n_cells, Counters *counters, ReplayEntry *replay, int xcd_aware,
                      const CreatedLists &created_lists, const RegionSource &regions,

@@ -11,7 +11,7 @@
 //   vertex_keys[M]         u64  packed key of vertex v
 //   neighbours[(pd+1)*M]   int2 per blur axis a and vertex v: indices of v's two neighbours or -1
 //   values[M*vd]           f32  vertex values, two buffers (ping-pong across blur axes)
-//   replay[(pd+1)*T] {i32, f32} [r][t]: vertex r of the point of thread t (hash cell until the
+//   replay[(pd+1)*T] {i32, f32} [workgroup][r][thread]: vertex r of the thread's point (hash cell until the
 //                                first splat) and its barycentric weight
 //
 // Packed key.  Every coordinate of lattice vertex with remainder r is (pd+1)*q_i + r, so a key is
@@ -205,8 +205,8 @@ __global__ __launch_bounds__(kBlock) void k_build(PointFeatures features, PointM
     }
     __syncthreads();
     const unsigned vblock = xcd_contiguous_block(blockIdx.x, gridDim.x, xcd_aware);
-    const size_t t = (size_t)vblock * kBlock + threadIdx.x;   // slot in the replay arrays
-    const size_t n_slots = (size_t)gridDim.x * kBlock;
+    const size_t t = (size_t)vblock * kBlock * D1 + threadIdx.x;   // slot in the replay arrays
+    constexpr size_t n_slots = kBlock;
     const int n = point_of_thread(map, vblock, threadIdx.x);
     const int lane = threadIdx.x & 63;
     const bool valid = n >= 0;
@@ -483,8 +483,8 @@ __global__ __launch_bounds__(kBlock) void k_build_tile(PointFeatures features, P
         group_created = 0;
     }
 
-    const size_t t = (size_t)vblock * kBlock + tid;   // slot in the replay arrays
-    const size_t n_slots = (size_t)gridDim.x * kBlock;
+    const size_t t = (size_t)vblock * kBlock * D1 + tid;   // slot in the replay arrays
+    constexpr size_t n_slots = kBlock;
     const int n = point_of_thread(map, vblock, tid);
     const int lane = tid & 63;
     const bool valid = n >= 0;
@@ -1158,8 +1158,8 @@ __global__ __launch_bounds__(kBlock) void k_splat_dpp(PointMap map,
     constexpr int P = VD == 2 ? 2 : 4;   // lanes per vertex row in the final atomic
     unsigned vblock;
     if (!block_of_points(map, xcd_aware, vblock)) return;
-    const size_t t = (size_t)vblock * kBlock + threadIdx.x;
-    const size_t T = (size_t)gridDim.x * kBlock;
+    const size_t t = (size_t)vblock * kBlock * D1 + threadIdx.x;
+    constexpr size_t T = kBlock;
     const int n = point_of_thread(map, vblock, threadIdx.x);
     const int lane = threadIdx.x & 63;
     const int my_channel = channel_of_lane<VD>(lane);
@@ -1221,8 +1221,8 @@ __global__ __launch_bounds__(kBlock) void k_splat_dpp_blocks(int vd, PointMap ma
                                                               float *values, int xcd_aware) {
     unsigned vblock;
     if (!block_of_points(map, xcd_aware, vblock)) return;
-    const size_t t = (size_t)vblock * kBlock + threadIdx.x;
-    const size_t T = (size_t)gridDim.x * kBlock;
+    const size_t t = (size_t)vblock * kBlock * D1 + threadIdx.x;
+    constexpr size_t T = kBlock;
     const int n = point_of_thread(map, vblock, threadIdx.x);
     const int lane = threadIdx.x & 63;
     const int my_channel = channel_of_lane<4>(lane);
@@ -1296,8 +1296,8 @@ __global__ __launch_bounds__(kBlock) void k_splat_channels(int d1, int vd, Point
     constexpr int kCorners = 2;
     unsigned vblock;
     if (!block_of_points(map, xcd_aware, vblock)) return;
-    const size_t t = (size_t)vblock * kBlock + threadIdx.x;
-    const size_t T = (size_t)gridDim.x * kBlock;
+    const size_t t = (size_t)vblock * kBlock * d1 + threadIdx.x;
+    constexpr size_t T = kBlock;
     const int n = point_of_thread(map, vblock, threadIdx.x);
     const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
     float *wave_rows = rows + (size_t)wave * 64 * in_channels;
@@ -1666,8 +1666,8 @@ __global__ __launch_bounds__(kBlock) void k_slice_point(int d1, PointMap map,
     // follow the tiles) are then in its own L2 and not in all eight
     unsigned vblock;
     if (!block_of_points(map, 1, vblock)) return;
-    const size_t t = (size_t)vblock * kBlock + threadIdx.x;
-    const size_t T = (size_t)gridDim.x * kBlock;
+    const size_t t = (size_t)vblock * kBlock * (D1 > 0 ? D1 : d1) + threadIdx.x;
+    constexpr size_t T = kBlock;
     const int n = point_of_thread(map, vblock, threadIdx.x);
     if (n < 0) return;
     float acc[VD];
@@ -1718,7 +1718,7 @@ __global__ __launch_bounds__(kBlock) void k_slice_point(int d1, PointMap map,
     }
 }
 
-// The same for rows of doubles (weights64[r*T+t]: the barycentric weights as doubles; the replay
+// The same for rows of doubles (weights64, laid out as they are: the barycentric weights as doubles; the replay
 // rows give the vertices).  Arithmetic as in k_slice_point_f64.
 template <int VD, int D1>
 __global__ __launch_bounds__(kBlock) void k_slice_rows_f64(PointMap map,
@@ -1730,8 +1730,8 @@ __global__ __launch_bounds__(kBlock) void k_slice_rows_f64(PointMap map,
                                                             int normalize) {
     unsigned vblock;
     if (!block_of_points(map, 1, vblock)) return;
-    const size_t t = (size_t)vblock * kBlock + threadIdx.x;
-    const size_t T = (size_t)gridDim.x * kBlock;
+    const size_t t = (size_t)vblock * kBlock * D1 + threadIdx.x;
+    constexpr size_t T = kBlock;
     const int n = point_of_thread(map, vblock, threadIdx.x);
     if (n < 0) return;
     int v[D1];
@@ -1775,7 +1775,7 @@ __global__ __launch_bounds__(kBlock) void k_slice_rows_f64(PointMap map,
 // arithmetic and the replay loads.
 constexpr int kSliceRun = 4;   // channels per thread of k_slice_channels (8: 10 % slower)
 template <int D1>
-__global__ __launch_bounds__(kBlock) void k_slice_channels(int vd, PointMap map, size_t T,
+__global__ __launch_bounds__(kBlock) void k_slice_channels(int vd, PointMap map,
                                                             const ReplayEntry *__restrict__ replay,
                                                             const float *__restrict__ values,
                                                             float *__restrict__ output, int normalize) {
@@ -1789,7 +1789,8 @@ __global__ __launch_bounds__(kBlock) void k_slice_channels(int vd, PointMap map,
     const int j0 = kSliceRun * (int)(item - slot * runs);
     unsigned vblock;   // as in k_slice_point
     if (!block_of_points(map, 1, vblock)) return;
-    const size_t t = (size_t)vblock * kBlock + slot;
+    constexpr size_t T = kBlock;
+    const size_t t = (size_t)vblock * kBlock * D1 + slot;
     const int n = point_of_thread(map, vblock, slot);
     if (n < 0) return;
     ReplayEntry e[D1];
@@ -1844,7 +1845,7 @@ struct alignas(4) FourFloats {
 };
 constexpr int kSlicePoints = 2;   // points per group of L lanes (1: 2 % slower, 4: 4 %)
 template <int D1, int L>
-__global__ __launch_bounds__(kBlock) void k_slice_quads(int vd, PointMap map, size_t T,
+__global__ __launch_bounds__(kBlock) void k_slice_quads(int vd, PointMap map,
                                                          const ReplayEntry *__restrict__ replay,
                                                          const float *__restrict__ values,
                                                          float *__restrict__ output, int normalize) {
@@ -1862,7 +1863,8 @@ __global__ __launch_bounds__(kBlock) void k_slice_quads(int vd, PointMap map, si
 #pragma unroll
     for (int q = 0; q < P; ++q) {
         const unsigned slot = (blockIdx.y * P + q) * kGroups + threadIdx.x / L;
-        const size_t t = (size_t)vblock * kBlock + slot;
+        constexpr size_t T = kBlock;
+        const size_t t = (size_t)vblock * kBlock * D1 + slot;
         n[q] = point_of_thread(map, vblock, slot);   // (the same for all L lanes)
 #pragma unroll
         for (int u = 0; u < E; ++u) {
@@ -1987,8 +1989,8 @@ __global__ __launch_bounds__(kBlock) void k_export_replay(int d1, PointMap map,
                                                            const int *__restrict__ cell_vertex,
                                                            VertexNumbers numbers,
                                                            int *vertex, float *weight) {
-    const size_t t = (size_t)blockIdx.x * kBlock + threadIdx.x;
-    const size_t T = (size_t)gridDim.x * kBlock;
+    const size_t t = (size_t)blockIdx.x * kBlock * d1 + threadIdx.x;
+    constexpr size_t T = kBlock;
     const int n = point_of_thread(map, blockIdx.x, threadIdx.x);
     if (n < 0) return;
     for (int r = 0; r < d1; ++r) {
@@ -2399,7 +2401,6 @@ hipError_t slice(int pd, int vd, const PointMap &map, const ReplayEntry *replay,
     if (map.n_blocks == 0) return hipSuccess;
     const int d1 = pd + 1;
     const dim3 grid(map.n_blocks), block(kBlock);
-    const size_t T = (size_t)map.n_blocks * kBlock;
 #define PLK_SLICE(VD)                                                                          \
     case VD:                                                                                   \
         hipLaunchKernelGGL(k_slice_point<VD>, grid, block, 0, s, d1, map, replay,              \
@@ -2419,7 +2420,7 @@ hipError_t slice(int pd, int vd, const PointMap &map, const ReplayEntry *replay,
 #define PLK_SLICE_QUADS(L)                                                                      \
     PLK_DISPATCH_PD(pd, hipLaunchKernelGGL((k_slice_quads<PD + 1, L>),                          \
                                            dim3(map.n_blocks, L / kSlicePoints),                \
-                                           block, 0, s, vd, map, T, replay, values, output,     \
+                                           block, 0, s, vd, map, replay, values, output,     \
                                            normalize))
             if (vd <= 16) {
                 PLK_SLICE_QUADS(4);
@@ -2434,7 +2435,7 @@ hipError_t slice(int pd, int vd, const PointMap &map, const ReplayEntry *replay,
 #undef PLK_SLICE_QUADS
             PLK_DISPATCH_PD(pd, hipLaunchKernelGGL((k_slice_channels<PD + 1>),
                                                    dim3(map.n_blocks, (out_ch + kSliceRun - 1) / kSliceRun), block, 0, s,
-                                                   vd, map, T, replay, values, output, normalize));
+                                                   vd, map, replay, values, output, normalize));
         } break;
     }
 #undef PLK_SLICE

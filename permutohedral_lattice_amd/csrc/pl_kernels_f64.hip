@@ -26,7 +26,7 @@ using namespace device;
 // they leave it (points that are neighbours in the image share vertices, and what bounds a splat
 // is the number of atomic requests): for each distinct vertex of the wavefront and each channel
 // four channels at a time are summed over the members, and the first four lanes add the four
-// sums to the vertex row with one atomic instruction.  replay rows and weights are stored in thread order, [r][t],
+// sums to the vertex row with one atomic instruction.  replay rows and weights are stored in thread order,
 // like the float path's.
 template <int D1>
 __global__ __launch_bounds__(kBlock) void k_splat_f64(int vd, PointMap map,
@@ -37,8 +37,8 @@ __global__ __launch_bounds__(kBlock) void k_splat_f64(int vd, PointMap map,
                                                        double *values, int xcd_aware) {
     unsigned vblock;
     if (!block_of_points(map, xcd_aware, vblock)) return;
-    const size_t t = (size_t)vblock * kBlock + threadIdx.x;
-    const size_t n_slots = (size_t)gridDim.x * kBlock;
+    const size_t t = (size_t)vblock * kBlock * D1 + threadIdx.x;
+    constexpr size_t n_slots = kBlock;
     const int n = point_of_thread(map, vblock, threadIdx.x);
     const int lane = threadIdx.x & 63;
     // every lane stays for the sums; lanes without a point, or whose keys the build could not
@@ -104,8 +104,8 @@ __global__ __launch_bounds__(kBlock) void k_slice_point_f64(int vd, PointMap map
     // each XCD takes one contiguous range of the tiles, whose vertices' rows are then in its L2
     unsigned vblock;
     if (!block_of_points(map, 1, vblock)) return;
-    const size_t t = (size_t)vblock * kBlock + threadIdx.x;
-    const size_t n_slots = (size_t)gridDim.x * kBlock;
+    const size_t t = (size_t)vblock * kBlock * D1 + threadIdx.x;
+    constexpr size_t n_slots = kBlock;
     const int n = point_of_thread(map, vblock, threadIdx.x);
     if (n < 0) return;
     int vertex[D1];
@@ -160,8 +160,8 @@ __global__ __launch_bounds__(kBlock) void k_slice_f64(int vd, PointMap map,
     // each XCD takes one contiguous range of the tiles, whose vertices' rows are then in its L2
     unsigned vblock;
     if (!block_of_points(map, 1, vblock)) return;
-    const size_t t = (size_t)vblock * kBlock + threadIdx.x;
-    const size_t n_slots = (size_t)gridDim.x * kBlock;
+    const size_t t = (size_t)vblock * kBlock * D1 + threadIdx.x;
+    constexpr size_t n_slots = kBlock;
     const int n = point_of_thread(map, vblock, threadIdx.x);
     if (n < 0) return;
     const int j = blockIdx.y;

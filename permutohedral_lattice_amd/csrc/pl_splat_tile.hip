@@ -47,8 +47,8 @@ __global__ __launch_bounds__(kThreads) void k_splat_tile(int d1, int vd, PointMa
     float *rows = reinterpret_cast<float *>(sorted + (size_t)kBlock * d1);   // [kBlock][in_channels]
     const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
     const int point = tid % kBlock, side = tid / kBlock;   // (its corners: side, side + 2, ...)
-    const size_t t = (size_t)vblock * kBlock + point;
-    const size_t T = (size_t)gridDim.x * kBlock;
+    const size_t t = (size_t)vblock * kBlock * d1 + point;
+    constexpr size_t T = kBlock;
     const int n = point_of_thread(map, vblock, point);
     static_assert(kTileSlots == kThreads, "a slot per thread");
     slot_index[tid] = -1;
