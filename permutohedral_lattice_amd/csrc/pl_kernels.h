@@ -279,6 +279,18 @@ hipError_t neighbours(int pd, const VertexTables &vertices, const Counters *coun
 
 hipError_t fill_zero(float *p, size_t n, hipStream_t s);
 
+// Every word of each range := its word, in one launch (ranges start on 16 bytes; words == 0: none).
+constexpr int kFillRanges = 4;
+struct FillRanges {
+    struct Range {
+        uint32_t *words_at;
+        size_t words;
+        uint32_t word;
+        unsigned blocks;   // set by fill_ranges
+    } range[kFillRanges];
+};
+hipError_t fill_ranges(FillRanges ranges, hipStream_t s);
+
 // Stage 3.  in_channels is vd-1 (the homogeneous channel is the bare weight) or vd.
 // cell_vertex != nullptr: the replay rows still hold hash cells; they are translated to vertex
 // indices and written back.

@@ -1129,6 +1129,19 @@ __global__ __launch_bounds__(kBlock) void k_neighbours(VertexTables vertices,
     }
 }
 
+// Several ranges of words at once, each to a word of its own: a workgroup takes 1024 words of one.
+__global__ __launch_bounds__(kBlock) void k_fill_ranges(FillRanges ranges) {
+    unsigned block = blockIdx.x;
+    int which = 0;
+    while (which + 1 < kFillRanges && block >= ranges.range[which].blocks) block -= ranges.range[which++].blocks;
+    const FillRanges::Range r = ranges.range[which];
+    const size_t first = (size_t)block * (4 * kBlock) + 4 * threadIdx.x;
+    if (first + 4 <= r.words)
+        reinterpret_cast<uint4 *>(r.words_at)[first / 4] = make_uint4(r.word, r.word, r.word, r.word);
+    else
+        for (size_t i = first; i < r.words; ++i) r.words_at[i] = r.word;
+}
+
 __global__ __launch_bounds__(kBlock) void k_fill_zero(float *p, size_t n) {
     const size_t i = (size_t)blockIdx.x * kBlock + threadIdx.x;
     if (i < n) p[i] = 0.0f;
@@ -2218,6 +2231,18 @@ hipError_t neighbours(int pd, const VertexTables &vertices, const Counters *coun
         PLK_NEIGHBOURS(false, PLK_DISPATCH_PD);
     }
 #undef PLK_NEIGHBOURS
+    return hipGetLastError();
+}
+
+hipError_t fill_ranges(FillRanges ranges, hipStream_t s) {
+    unsigned blocks = 0;
+    for (FillRanges::Range &r : ranges.range) {
+        if (r.words && (!r.words_at || reinterpret_cast<uintptr_t>(r.words_at) % 16u != 0u)) return hipErrorInvalidValue;
+        r.blocks = blocks_for(r.words, 4 * kBlock);
+        blocks += r.blocks;
+    }
+    if (!blocks) return hipSuccess;
+    hipLaunchKernelGGL(k_fill_ranges, dim3(blocks), dim3(kBlock), 0, s, ranges);
     return hipGetLastError();
 }
 

@@ -1,5 +1,6 @@
-"""Rows of many channels splatted by tiles sorted in LDS (5 to 32 channels, merged builds): filter
-and a repeated apply against the oracle, at the edges of the channel blocks and of the tiles."""
+"""Splats whose sums meet per workgroup in LDS (merged builds; pairs sorted by vertex for 5 to 32
+channels, sums of the wavefronts added up for 2 to 4): filter and a repeated apply against the oracle, at
+the edges of the channel blocks and of the tiles."""
 import numpy as np
 import pytest
 import torch
@@ -24,7 +25,7 @@ def check(got, want):
     assert np.abs(got - want).max() <= MAX_ABS_TOL * scale and rel_l2(got, want) <= REL_L2_TOL
 
 
-@pytest.mark.parametrize("vd", [4, 5, 6, 15, 16, 17, 22, 31, 32, 33])
+@pytest.mark.parametrize("vd", [2, 3, 4, 5, 6, 15, 16, 17, 22, 31, 32, 33])
 @pytest.mark.parametrize("h,w,features", [(16, 16, 3), (17, 23, 3), (40, 33, 0), (31, 64, 6)])
 def test_many_channels_on_merged_tiles(h, w, features, vd):
     rng = np.random.default_rng(1000 * vd + h)
