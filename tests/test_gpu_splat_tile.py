@@ -1,6 +1,6 @@
-"""Splats whose sums meet per workgroup in LDS (merged builds; pairs sorted by vertex for 5 to 32
-channels, sums of the wavefronts added up for 2 to 4): filter and a repeated apply against the oracle, at
-the edges of the channel blocks and of the tiles."""
+"""Splats of a merged build whose sums meet per workgroup in LDS (pairs sorted by vertex, 5 to 32
+channels) and those of the channel counts beside them, which leave a wavefront at a time: filter and a
+repeated apply against the oracle, at the edges of the channel blocks and of the tiles."""
 import numpy as np
 import pytest
 import torch
