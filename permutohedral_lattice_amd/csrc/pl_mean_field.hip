@@ -66,12 +66,15 @@ __global__ __launch_bounds__(kRows) void k_mean_field_update(float *__restrict__
         float *own = rows + (int)threadIdx.x * pitch;
         float highest = own[0];
         for (int c = 1; c < classes; ++c) highest = fmaxf(highest, own[c]);
-        float sum = 0.0f;
+        // (a sum of doubles: one after the other in single precision the exponentials of 128 classes
+        // cost the result three times the error of a tree's sum, 1.7e-7 against 5.6e-8 of its norm)
+        double wide_sum = 0.0;
         for (int c = 0; c < classes; ++c) {
             const float e = expf(own[c] - highest);
             own[c] = e;
-            sum += e;
+            wide_sum += (double)e;
         }
+        const float sum = (float)wide_sum;
         for (int c = 0; c < classes; ++c) own[c] = own[c] / sum;
     }
     __syncthreads();
