@@ -195,9 +195,12 @@ typedef enum pl_info {
                                   too many distinct keys switched merging off for a while) */
     PL_INFO_TABLE_CELLS = 2,   /* hash cells the last build used */
     PL_INFO_SCRATCH_BYTES = 3, /* device memory the handle holds for its tables and per-point rows */
-    PL_INFO_FOREIGN_ROWS = 4   /* when the last build numbered its vertices itself: how many rows of sums
+    PL_INFO_FOREIGN_ROWS = 4,  /* when the last build numbered its vertices itself: how many rows of sums
                                   its workgroups held for vertices that other workgroups created (an
                                   estimate from every eighth workgroup); else -1 */
+    PL_INFO_LIST_COUNTED = 5   /* when the last build put a plain list in an order (PL_OPT_ORDER_POINTS):
+                                  1 if its points were counted in histograms, 0 if with atomics on memory
+                                  (short, very long and already ordered lists); else -1 */
 } pl_info;
 int pl_get_info(pl_handle h, int what, long *value);
 

@@ -186,6 +186,7 @@ struct pl_lattice {
     uint2 *bin_rank = nullptr;             // [N]
     unsigned *bin_table = nullptr;         // histograms of the bins (plk::locality_table_rows)
     bool list_in_order = false;            // the last list that was ordered ran from a bin to the next
+    int list_counted = -1;                 // PL_INFO_LIST_COUNTED (1 until the build reports: perhaps)
     int order_capacity = 0;
     hipEvent_t ev[EV_COUNT] = {};
     bool ev_recorded[EV_COUNT] = {};
@@ -478,10 +479,14 @@ int enqueue_build(pl_lattice *h, const plk::PointFeatures &features, const doubl
     h->stage_ran[1] = true;
     h->stage_ran[2] = !numbers_in_build;
     h->stage_ran[3] = true;
-    if (h->map.mode == 1)
+    h->list_counted = -1;
+    if (h->map.mode == 1) {
+        const plk::LocalityScratch scratch = locality_scratch(h);
+        h->list_counted = scratch.table && !scratch.expect_in_order ? 1 : 0;
         PL_HIP(plk::order_by_locality(h->f64 ? nullptr : features.positions,
                                       h->f64 ? positions64 : nullptr, h->N, h->pd,
-                                      locality_scratch(h), h->point_order, h->stream));
+                                      scratch, h->point_order, h->stream));
+    }
     if (!h->table_clean || cells != h->n_cells) {
         PL_HIP(plk::clear_table(h->cell_keys, wide ? 2 * cells : cells, h->stream));
     }
@@ -758,7 +763,10 @@ int verify_build(pl_lattice *h, uint32_t *retry_cells) {
     }
     const int flags = status.flags;
     const int m = status.num_vertices;
-    if (h->map.mode == 1) h->list_in_order = status.list_in_order != 0;
+    if (h->map.mode == 1) {
+        h->list_in_order = status.list_in_order != 0;
+        if (h->list_in_order) h->list_counted = 0;
+    }
     h->last_n_segments = status.n_segments;
     h->last_max_segment = status.max_segment;
     if (flags & plk::kFlagKeyRange) {
@@ -1412,6 +1420,7 @@ int pl_get_info(pl_handle h, int what, long *value) {
         case PL_INFO_BUILD_MERGED: *value = h->last_build_merged ? 1 : 0; return PL_OK;
         case PL_INFO_TABLE_CELLS: *value = (long)h->n_cells; return PL_OK;
         case PL_INFO_FOREIGN_ROWS: *value = h->foreign_rows; return PL_OK;
+        case PL_INFO_LIST_COUNTED: *value = h->list_counted; return PL_OK;
         case PL_INFO_SCRATCH_BYTES: {
             const size_t mv = plk::max_vertices_for(h->n_cells_alloc);
             size_t b = (size_t)h->n_cells_alloc * (sizeof(uint64_t) + sizeof(int)) +

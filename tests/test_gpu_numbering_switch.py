@@ -51,8 +51,11 @@ def test_a_handle_that_returns_to_merging_again_and_again():
     lat = pla.PermutohedralLattice(5, 4, side * side)
     lat.set_point_grid((side, side))
     out = torch.empty_like(d_val)
-    for _ in range(37):
+    for call in range(37):
         out.zero_()
         lat.filter(out, d_val, d_pos)
+        # (the try itself overflows and its call is repeated without merging: the second sends the
+        # handle back to plain builds for longer than the calls that are left)
+        assert lat.info(pla.PL_INFO_BUILD_MERGED) == 0, call
         assert lat.num_vertices == cpu.num_vertices
         assert float(np.abs(out.cpu().numpy() - want).max()) <= 1e-5

@@ -248,7 +248,8 @@ def test_lists_just_long_enough_to_be_ordered(pd, vd, n):
     lat.close()
 
 
-@pytest.mark.parametrize("n", [16383, 16384, 16385, (1 << 18) + 1, (1 << 19) - 1, (1 << 19) + 2047, 1277951, 1277985])
+@pytest.mark.parametrize("n", [16383, 16384, 16385, (1 << 18) + 1, (1 << 19) - 1, (1 << 19) + 2047, 1277951, 1277985,
+                               1278079, 1278080])
 @pytest.mark.parametrize("ordered_list", [False, True])
 def test_lists_counted_in_a_table_of_histograms(n, ordered_list):
     """Both sides of the lengths at which the ranks of the points come from histograms in LDS (and
@@ -270,8 +271,50 @@ def test_lists_counted_in_a_table_of_histograms(n, ordered_list):
             lat.filter(out, val, pos, False)
         torch.cuda.synchronize()
         assert lat.info(pla.PL_INFO_BUILD_MERGED) == ordered
+        table = 16384 <= n <= 1278079 and not ordered_list
+        assert lat.info(pla.PL_INFO_LIST_COUNTED) == (int(table) if ordered else -1)
         outs.append(out)
         keys.append(sorted_keys(host(lat.debug_keys()))[0])
         lat.close()
     assert (keys[0] == keys[1]).all()
     assert float((outs[0] - outs[1]).abs().max()) <= 2e-5
+
+
+@pytest.mark.parametrize("dtype", [torch.float32, torch.float64])
+@pytest.mark.parametrize("n", [16383, 16384, 21001])
+def test_one_handle_whose_lists_change_their_order(n, dtype):
+    """Lists that run through the bins and lists in no order on one handle, so that either way of
+    counting runs on what the other left in the scratch arrays; the way is that of the list (of the
+    length, below 16384 points), or atomics where the list before had another order."""
+    gen = torch.Generator("cuda").manual_seed(n)
+    pos = torch.rand((n, 2), device="cuda", generator=gen, dtype=dtype) * (n ** 0.5 / 6.0)
+    pos = pos[torch.argsort((pos[:, 0] * 1.5).floor() * 4096.0 + pos[:, 1])].contiguous()
+    val = torch.rand((n, 1), device="cuda", generator=gen, dtype=dtype)
+    shuffle = torch.randperm(n, device="cuda", generator=gen)
+    tolerance = 2e-5 if dtype == torch.float32 else 1e-12
+    out = torch.empty_like(val)
+    plain = pla.PermutohedralLattice(2, 2, n, dtype=dtype)
+    if dtype == torch.float32:
+        plain.set_option(pla.PL_OPT_GUESS_GRID, 0)
+    plain.set_option(pla.PL_OPT_ORDER_POINTS, 0)
+    plain.filter(out, val, pos)
+    want = out.clone()
+    assert plain.info(pla.PL_INFO_LIST_COUNTED) == -1
+    keys = sorted_keys(host(plain.debug_keys()))[0]
+    plain.close()
+    lat = pla.PermutohedralLattice(2, 2, n, dtype=dtype)
+    if dtype == torch.float32:
+        lat.set_option(pla.PL_OPT_GUESS_GRID, 0)
+    counted = []
+    for shuffled in (1, 1, 0, 0, 1, 1, 1, 0, 1, 0):
+        out.fill_(float("nan"))
+        if shuffled:
+            lat.filter(out, val[shuffle].contiguous(), pos[shuffle].contiguous())
+        else:
+            lat.filter(out, val, pos)
+        assert float((out - (want[shuffle] if shuffled else want)).abs().max()) <= tolerance
+        assert (sorted_keys(host(lat.debug_keys()))[0] == keys).all()
+        assert lat.info(pla.PL_INFO_BUILD_MERGED) == 1
+        counted.append(lat.info(pla.PL_INFO_LIST_COUNTED))
+    lat.close()
+    assert counted == ([1, 1, 0, 0, 0, 1, 1, 0, 0, 0] if n >= 16384 else [0] * 10)
