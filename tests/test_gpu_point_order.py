@@ -248,6 +248,16 @@ def test_lists_just_long_enough_to_be_ordered(pd, vd, n):
     lat.close()
 
 
+def clumps(n, gen, dtype=torch.float32):
+    """Points in clumps of about sixty, far smaller than their distance, clump after clump: wherever
+    the bins of the ordering pass (about sixty points each) come to lie, a tenth of them at most cut a
+    clump, and the list runs from a bin to the next."""
+    side = int((n / 60.0) ** 0.5)
+    clump = torch.randint(side * side, (n,), device="cuda", generator=gen).sort().values
+    corner = torch.stack((clump // side, clump % side), dim=1).to(dtype)
+    return (1.25 * (corner + 0.125 * torch.rand((n, 2), device="cuda", generator=gen, dtype=dtype))).contiguous()
+
+
 @pytest.mark.parametrize("n", [16383, 16384, 16385, (1 << 18) + 1, (1 << 19) - 1, (1 << 19) + 2047, 1277951, 1277985,
                                1278079, 1278080])
 @pytest.mark.parametrize("ordered_list", [False, True])
@@ -256,9 +266,7 @@ def test_lists_counted_in_a_table_of_histograms(n, ordered_list):
     at which a workgroup takes one, two and four points per thread), lists in no order and lists that
     run through the bins: the lattice of the list in its own order, point by point the same output."""
     gen = torch.Generator("cuda").manual_seed(n)
-    pos = torch.rand((n, 2), device="cuda", generator=gen) * (n ** 0.5 / 6.0)
-    if ordered_list:
-        pos = pos[torch.argsort((pos[:, 0] * 1.5).floor() * 4096.0 + pos[:, 1])].contiguous()
+    pos = clumps(n, gen) if ordered_list else torch.rand((n, 2), device="cuda", generator=gen) * (n ** 0.5 / 6.0)
     val = torch.rand((n, 1), device="cuda", generator=gen)
     outs, keys = [], []
     for ordered in (1, 0):
@@ -287,8 +295,7 @@ def test_one_handle_whose_lists_change_their_order(n, dtype):
     counting runs on what the other left in the scratch arrays; the way is that of the list (of the
     length, below 16384 points), or atomics where the list before had another order."""
     gen = torch.Generator("cuda").manual_seed(n)
-    pos = torch.rand((n, 2), device="cuda", generator=gen, dtype=dtype) * (n ** 0.5 / 6.0)
-    pos = pos[torch.argsort((pos[:, 0] * 1.5).floor() * 4096.0 + pos[:, 1])].contiguous()
+    pos = clumps(n, gen, dtype)
     val = torch.rand((n, 1), device="cuda", generator=gen, dtype=dtype)
     shuffle = torch.randperm(n, device="cuda", generator=gen)
     tolerance = 2e-5 if dtype == torch.float32 else 1e-12
