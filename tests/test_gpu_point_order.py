@@ -325,3 +325,28 @@ def test_one_handle_whose_lists_change_their_order(n, dtype):
         counted.append(lat.info(pla.PL_INFO_LIST_COUNTED))
     lat.close()
     assert counted == ([1, 1, 0, 0, 0, 1, 1, 0, 0, 0] if n >= 16384 else [0] * 10)
+
+
+@pytest.mark.parametrize("run,counted", [(5, 0), (3, 1)])
+def test_lists_near_the_line_between_the_ways_of_counting(run, counted):
+    """Runs of five points of a bin change it at 219 of 960 sampled points, fewer than the quarter from
+    which a list is counted in histograms; runs of three at a third."""
+    n, rng = 65536, np.random.default_rng(1)
+    side = int((n / 60.0) ** 0.5)
+    clump = np.sort(rng.integers(0, side * side, n))
+    pos = (1.25 * (np.stack((clump // side, clump % side), 1) + 0.03 * rng.random((n, 2)))).astype(np.float32)
+    runs = rng.permutation(-(-n // run))
+    index = (runs[:, None] * run + np.arange(run)).reshape(-1)
+    pos = pos[index[index < n]]
+    val = rng.uniform(0, 1, (n, 1)).astype(np.float32)
+    lat = pla.PermutohedralLattice(2, 2, n)
+    lat.set_option(pla.PL_OPT_GUESS_GRID, 0)
+    out = torch.empty((n, 1), dtype=torch.float32, device="cuda")
+    for _ in range(2):
+        lat.filter(out, dev(val), dev(pos), False)
+        torch.cuda.synchronize()
+        assert lat.info(pla.PL_INFO_LIST_COUNTED) == counted
+    cpu = oracle.Lattice(2, 2, n)
+    want = cpu.filter(val, pos)
+    check_against_oracle(lat, cpu, pos, out, want)
+    lat.close()
