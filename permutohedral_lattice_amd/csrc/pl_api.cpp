@@ -359,8 +359,7 @@ int ensure_vertex_lists(pl_lattice *h) {
 plk::LocalityScratch locality_scratch(const pl_lattice *h) {
     const unsigned max_bins = plk::locality_bins_for(h->N);
     plk::LocalityScratch scratch{};
-    // (32 words ahead of the arrays: the record of the bins, the range, the number of tiles, whether
-    // the list is in order)
+    // (32 words ahead of the arrays: the record of the bins, the range, the number of tiles)
     constexpr size_t head_words = 32;
     static_assert(plk::kLocalityBinsBytes <= 16 * sizeof(unsigned), "the record fits its place");
     scratch.bins = h->locality_words;
@@ -369,9 +368,6 @@ plk::LocalityScratch locality_scratch(const pl_lattice *h) {
     scratch.bin_count = h->locality_words + head_words;
     scratch.bin_first = h->locality_words + head_words + max_bins;
     scratch.bin_rank = h->bin_rank;
-    scratch.table = h->bin_table;
-    scratch.in_order = h->locality_words + 21;
-    scratch.expect_in_order = h->list_in_order;
     scratch.max_bins = max_bins;
     scratch.max_tiles = plk::locality_tiles_for(h->N);
     scratch.chunk_sums = h->locality_words + head_words + 2 * (size_t)max_bins;
@@ -472,20 +468,22 @@ int enqueue_build(pl_lattice *h, const plk::PointFeatures &features, const doubl
     }
     // (what this build's report will carry; never 0, which is what a fresh status holds)
     h->status_sequence = h->status_sequence + 1u ? h->status_sequence + 1u : 1u;
-    const plk::HostReport report_to{h->h_status, h->status_sequence,
-                                    h->map.mode == 1 ? locality_scratch(h).in_order : nullptr};
+    const plk::HostReport report_to{h->h_status, h->status_sequence};
     h->mark(EV_T0);
     h->stage_ran[0] = h->map.mode == 1 || !h->table_clean || cells != h->n_cells;
     h->stage_ran[1] = true;
     h->stage_ran[2] = !numbers_in_build;
     h->stage_ran[3] = true;
+    // the previous vertex-numbering kernel (or pl_create) left the other counter set zeroed
+    const int previous_set = h->counter_set;
+    h->counter_set = 1 - previous_set;
     h->list_counted = -1;
     if (h->map.mode == 1) {
-        const plk::LocalityScratch scratch = locality_scratch(h);
-        h->list_counted = scratch.table && !scratch.expect_in_order ? 1 : 0;
+        const plk::LocalityTable counting{h->bin_table, &h->counters()->order_tally, h->list_in_order};
+        h->list_counted = counting.table && !counting.expect_in_order ? 1 : 0;
         PL_HIP(plk::order_by_locality(h->f64 ? nullptr : features.positions,
                                       h->f64 ? positions64 : nullptr, h->N, h->pd,
-                                      scratch, h->point_order, h->stream));
+                                      locality_scratch(h), counting, h->point_order, h->stream));
     }
     if (!h->table_clean || cells != h->n_cells) {
         PL_HIP(plk::clear_table(h->cell_keys, wide ? 2 * cells : cells, h->stream));
@@ -493,9 +491,6 @@ int enqueue_build(pl_lattice *h, const plk::PointFeatures &features, const doubl
     h->table_clean = false;
     h->n_cells = cells;
     h->mark(EV_CLEAR);
-    // the previous vertex-numbering kernel (or pl_create) left the other counter set zeroed
-    const int previous_set = h->counter_set;
-    h->counter_set = 1 - previous_set;
     const plk::VertexTables vertices{h->cell_vertex, h->vertex_keys, h->vertex_cell, h->neighbours,
                                      h->max_vertices()};
     const plk::CreatedLists lists = h->lists(h->counter_set);
@@ -764,7 +759,7 @@ int verify_build(pl_lattice *h, uint32_t *retry_cells) {
     const int flags = status.flags;
     const int m = status.num_vertices;
     if (h->map.mode == 1) {
-        h->list_in_order = status.list_in_order != 0;
+        h->list_in_order = (flags & plk::kFlagListInOrder) != 0;
         if (h->list_in_order) h->list_counted = 0;
     }
     h->last_n_segments = status.n_segments;

@@ -569,6 +569,7 @@ __device__ __forceinline__ int wave_leader_of_equal(T x, bool active, int lane, 
 __device__ __forceinline__ void reset_counters(Counters *c) {
     c->vertices = 0;
     c->flags = 0;
+    c->order_tally = 0;
     for (int k = 0; k < kMaxSegments; ++k) c->segment_count[k].n = 0;   // (n_segments: set by every build)
     c->foreign_rows_sampled.n = 0;
 }

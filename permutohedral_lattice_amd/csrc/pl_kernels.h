@@ -18,6 +18,7 @@ enum : int {
     kFlagKeyRange = 2,    // a lattice coordinate does not fit its field of the key (packed key: the build
                           // is repeated with keys of two words; those: it is no short)
     kFlagTileFull = 4,    // a workgroup of the merging build has more distinct keys than its LDS table holds
+    kFlagListInOrder = 8, // in the report to the host only: locality_in_order of the list the build ordered
 };
 
 // Device-side state of one build.  Kernels after the build read the vertex counts from here, so
@@ -40,6 +41,9 @@ struct Counters {
     // again, which only have to stay valid until the build has run
     float region_lo, region_per_unit;
     int n_segments;
+    // of the list the build put in order, where there is a table of histograms (LocalityTable): points
+    // compared with the one before them << 16 | how many of them were in another bin
+    unsigned order_tally;
     // (a counter per 128 bytes: atomics on one line queue up in one memory channel, whatever
     // address in the line they name.  Each line also says how the vertices are numbered, and
     // after the numbering pass every line holds the total: a pass over the vertices learns what
@@ -68,11 +72,10 @@ inline int segments_for(uint32_t max_vertices, unsigned workgroups) {
 // What the build (or the numbering pass) writes to pinned host memory about the build.
 struct HostStatus {
     int num_vertices;
-    int flags;
+    int flags;         // (kFlagListInOrder among them: a word of its own is another write over the bus)
     int max_segment;   // vertices in the fullest segment (num_vertices when there are none)
     int n_segments;
     int foreign_rows;  // CreatedLists rows of a build that numbered its vertices (an estimate)
-    int list_in_order; // LocalityScratch::in_order of the list the build ordered (0: ordered none)
     // written last, behind a system-wide fence: the number of the build the fields above belong
     // to.  The host, which holds the struct in pinned memory, polls this word instead of waiting
     // for an event behind the kernel (an event between two kernels of a stream keeps the second
@@ -83,7 +86,6 @@ struct HostStatus {
 struct HostReport {
     HostStatus *status;
     unsigned sequence;
-    const unsigned *list_in_order;   // LocalityScratch::in_order, or none
 };
 
 // Per-vertex and per-cell tables of a lattice (all sized by the hash table): vertex v has key
@@ -493,10 +495,17 @@ struct LocalityScratch {
     // for the scan of many bins by many workgroups, each a chunk of 4096 bins:
     unsigned *chunk_sums;  // [2 * locality_scan_chunks(max_bins)]
     unsigned *chunk_first; // [locality_scan_chunks(max_bins) + 1]
-    unsigned *table;       // [locality_table_rows(N) * max_bins], none where that is 0
-    unsigned *in_order;    // whether this list runs from a bin to the next (k_locality_table)
-    bool expect_in_order;  // the handle's last list did
 };
+// The way a list is counted.  (Apart from the arrays that every list's kernels are given, and these have
+// instantiations without it: three more words in the arguments of each, and the tally taken and reported
+// where nobody asks for it, cost lists too short for a table 0.5 to 2 us of 46 to 49.)
+struct LocalityTable {
+    unsigned *table;       // [locality_table_rows(N) * max_bins], none where that is 0
+    unsigned *order_tally; // Counters::order_tally of the build, zero
+    bool expect_in_order;  // the handle's last list ran from a bin to the next
+};
+// A list that runs from a bin to the next: fewer than a quarter of the points change it (k_locality_table)
+constexpr bool locality_in_order(unsigned order_tally) { return 4u * (order_tally & 0xffffu) < order_tally >> 16; }
 inline unsigned locality_scan_chunks(unsigned max_bins) { return (max_bins / 4u + 1023u) / 1024u; }
 inline unsigned locality_bins_for(int N) { return ((unsigned)N / 32u + 1024u) & ~3u; }
 // The table of histograms a list of N points is counted with (k_locality_table): a row per
@@ -518,7 +527,8 @@ inline unsigned locality_tiles_for(int N) {
 }
 // positions or positions64 (the other null); order: 256 * scratch.max_tiles entries
 hipError_t order_by_locality(const float *positions, const double *positions64, int N, int pd,
-                             const LocalityScratch &scratch, int *order, hipStream_t s);
+                             const LocalityScratch &scratch, const LocalityTable &counting, int *order,
+                             hipStream_t s);
 
 hipError_t compute_positions(const float *reference, float *positions, int N, int n_ref_channels,
                              int n_spatial_dims, const SpatialDims &dims, float spatial_std,

@@ -865,6 +865,11 @@ __global__ __launch_bounds__(kBlock) void k_build_tile(PointFeatures features, P
     }
 }
 
+// The flags a report carries: the build's, and what was seen of the list it ordered.
+__device__ __forceinline__ int reported_flags(const Counters *counters) {
+    return counters->flags | (locality_in_order(counters->order_tally) ? kFlagListInOrder : 0);
+}
+
 // Dense vertex numbering in the order of the build's workgroups, i.e. of the image tiles: the
 // vertices a workgroup created follow those of the workgroups before it.  Vertices that are close
 // in the lattice were created by the same or a neighbouring tile, so their numbers are close, and
@@ -926,6 +931,7 @@ __global__ __launch_bounds__(64) void k_number_vertices(CreatedLists lists, int 
     if (b == gridDim.x - 1) {
         if (lane == 0) {
             const uint32_t m = (uint32_t)(before + count);
+            const int flags = reported_flags(counters);
             counters->vertices = m;
             counters->n_segments = 0;
             for (int k = 0; k < kMaxSegments; ++k) {
@@ -933,11 +939,10 @@ __global__ __launch_bounds__(64) void k_number_vertices(CreatedLists lists, int 
                 counters->segment_count[k].n_segments = 0;
             }
             host_status->num_vertices = (int)m;
-            host_status->flags = counters->flags | (m > (uint32_t)max_vertices ? kFlagTableFull : 0);
+            host_status->flags = flags | (m > (uint32_t)max_vertices ? kFlagTableFull : 0);
             host_status->max_segment = (int)m;
             host_status->n_segments = 0;
             host_status->foreign_rows = 0;
-            host_status->list_in_order = host_report.list_in_order ? (int)*host_report.list_in_order : 0;
             __threadfence_system();
             __hip_atomic_store(&host_status->sequence, host_report.sequence, __ATOMIC_RELAXED,
                                __HIP_MEMORY_SCOPE_SYSTEM);
@@ -1043,6 +1048,9 @@ __global__ __launch_bounds__(kBlock) void k_neighbours(VertexTables vertices,
         static_assert(kMaxSegments <= 64, "a lane per segment");
         const int n_segments = report->n_segments;
         const unsigned c = (int)threadIdx.x < n_segments ? report->segment_count[threadIdx.x].n : 0u;
+        // (asked for before the first word goes to the host: a load behind that waits by itself)
+        const int flags = reported_flags(report);
+        const unsigned foreign_rows = report->foreign_rows_sampled.n;
         unsigned total = c, fullest = c;
 #pragma unroll
         for (int off = 32; off >= 1; off >>= 1) {
@@ -1053,11 +1061,10 @@ __global__ __launch_bounds__(kBlock) void k_neighbours(VertexTables vertices,
         if (threadIdx.x == 0) {
             report->vertices = total;
             host_status->num_vertices = (int)total;
-            host_status->flags = report->flags;
+            host_status->flags = flags;
             host_status->max_segment = (int)fullest;
             host_status->n_segments = n_segments;
-            host_status->foreign_rows = (int)(report->foreign_rows_sampled.n * kForeignSampling);
-            host_status->list_in_order = host_report.list_in_order ? (int)*host_report.list_in_order : 0;
+            host_status->foreign_rows = (int)(foreign_rows * kForeignSampling);
             __threadfence_system();
             __hip_atomic_store(&host_status->sequence, host_report.sequence, __ATOMIC_RELAXED,
                                __HIP_MEMORY_SCOPE_SYSTEM);

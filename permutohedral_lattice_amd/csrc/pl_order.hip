@@ -172,11 +172,21 @@ __device__ __forceinline__ void first_features(const T *__restrict__ positions, 
     for (int f = 0; f < kBoxFeatures; ++f) p[f] = f < pd ? (float)row[f] : 0.0f;
 }
 
+// Counters::order_tally of a wavefront: its lanes that are a pair with the lane before them and,
+// below, how many of those are in another bin.
+__device__ __forceinline__ unsigned bin_changes(int bin, bool pair) {
+    const int before = __shfl_up(bin, 1);   // (by all lanes: one that is switched off gives no value)
+    return (unsigned)__builtin_popcountll(wave_ballot(pair)) << 16 |
+           (unsigned)__builtin_popcountll(wave_ballot(pair && bin != before));
+}
+
 // The bins for this list: the box of the sampled points, the bins over it, left in memory for the
-// kernels that follow (one workgroup)
-template <typename T>
-__global__ __launch_bounds__(kScanBlock) void k_locality_bins(const T *__restrict__ positions, int N, int pd,
-                                                               LocalityScratch scratch) {
+// kernels that follow (one workgroup).  TELL: and how often the samples change their bin, for the
+// kernel that counts in histograms; everyone waits for the bins then, 1 us, which short lists and
+// lists expected in order (k_locality_count tells there) do not pay.
+template <typename T, bool TELL>
+__device__ __forceinline__ void locality_bins(const T *__restrict__ positions, int N, int pd,
+                                              const LocalityScratch &scratch, unsigned *order_tally) {
     __shared__ Box wave_part[kScanBlock / 64];
     // (all the loads first, none behind a branch: a sample past the end reads the last point)
     constexpr int kPerThread = kBoxSamples / kScanBlock;
@@ -202,40 +212,56 @@ __global__ __launch_bounds__(kScanBlock) void k_locality_bins(const T *__restric
         }
     }
     v = block_box(v, wave_part);
-    __shared__ LocalityBins shared_bins;
-    __shared__ int changes;
-    if (threadIdx.x == 0) {
-        shared_bins = bins_over(v, N, pd, scratch.max_bins);
-        changes = 0;
-    }
-    __syncthreads();
-    const LocalityBins bins = shared_bins;
-    if (scratch.table) {
-        // how often a sample's bin is not that of the point before it in its run (64 of the runs)
-        const int bin = (int)bin_of(bins, p[0]);
-        const int before = __shfl_up(bin, 1);   // (by all lanes: one that is switched off gives no value)
-        const int changed = __builtin_popcountll(wave_ballot(threadIdx.x % kSampleRun != 0 && bin != before));
-        if ((threadIdx.x & 63) == 0) atomicAdd(&changes, changed);
+    if constexpr (TELL) {
+        __shared__ LocalityBins shared_bins;
+        __shared__ unsigned tally;
+        if (threadIdx.x == 0) {
+            shared_bins = bins_over(v, N, pd, scratch.max_bins);
+            tally = 0;
+        }
         __syncthreads();
-    }
-    if (threadIdx.x == 0) {
+        const LocalityBins bins = shared_bins;
+        const unsigned changed = bin_changes((int)bin_of(bins, p[0]), threadIdx.x % kSampleRun != 0);
+        if ((threadIdx.x & 63) == 0) atomicAdd(&tally, changed);
+        __syncthreads();
+        if (threadIdx.x == 0) {
+            *bins_record(scratch) = bins;
+            *order_tally = tally;
+            scratch.range0[0] = bins.lo[0];
+            scratch.range0[1] = bins.hi0;
+        }
+    } else if (threadIdx.x == 0) {
+        const LocalityBins bins = bins_over(v, N, pd, scratch.max_bins);
         *bins_record(scratch) = bins;
-        constexpr int kPairs = kScanBlock - kScanBlock / (int)kSampleRun;   // (a run's first point has none before it)
-        *scratch.in_order = 4 * changes < kPairs ? 1u : 0u;
         scratch.range0[0] = bins.lo[0];
         scratch.range0[1] = bins.hi0;
     }
+}
+
+template <typename T>
+__global__ __launch_bounds__(kScanBlock) void k_locality_bins(const T *__restrict__ positions, int N, int pd,
+                                                               LocalityScratch scratch) {
+    locality_bins<T, false>(positions, N, pd, scratch, nullptr);
+}
+template <typename T>
+__global__ __launch_bounds__(kScanBlock) void k_locality_bins_told(const T *__restrict__ positions, int N, int pd,
+                                                                    LocalityScratch scratch, unsigned *order_tally) {
+    locality_bins<T, true>(positions, N, pd, scratch, order_tally);
 }
 
 // Every point draws its rank in its bin.  The lanes of a wavefront that share a bin (in a list
 // that has any order at all, most of them) draw their ranks with one atomic.  A thread takes
 // kCountPoints points, 256 apart, so that their loads and their atomics are in flight together.
 // (Also: every place of the order set to "no point".)
+// TELL (on a handle with a table): a wavefront each of up to kTallyWaves workgroups spread over the list also says how often its
+// points change their bin.
 constexpr int kCountPoints = 2;
-template <typename T>
-__global__ __launch_bounds__(kBlock) void k_locality_count(const T *__restrict__ positions, int N, int pd,
-                                                            LocalityScratch scratch, int *__restrict__ order,
-                                                            size_t order_entries) {
+constexpr unsigned kTallyWaves = 16;
+static_assert(kTallyWaves * 64 < 65536 && kScanBlock < 65536, "the tally's halves");
+template <typename T, bool TELL>
+__device__ __forceinline__ void locality_count(const T *__restrict__ positions, int N, int pd,
+                                               const LocalityScratch &scratch, int *__restrict__ order,
+                                               size_t order_entries, unsigned *order_tally) {
     const int lane = threadIdx.x & 63;
     // (the places of the order that the scatter will leave empty)
     for (size_t i = (size_t)blockIdx.x * kBlock + threadIdx.x; i < order_entries;
@@ -258,6 +284,10 @@ __global__ __launch_bounds__(kBlock) void k_locality_count(const T *__restrict__
 #pragma unroll
     for (int k = 0; k < kCountPoints; ++k) {
         bin[k] = valid[k] ? (int)bin_of(bins, p[k]) : 0;
+        if (TELL && k == 0 && threadIdx.x < 64 && blockIdx.x % (gridDim.x / kTallyWaves + 1u) == 0u) {
+            const unsigned changed = bin_changes(bin[k], valid[k] && lane != 0);
+            if (lane == 0) atomicAdd(order_tally, changed);
+        }
         // after 16 different bins the lanes that are left draw their ranks one by one
         uint64_t todo = wave_ballot(valid[k]);
         leader[k] = lane;
@@ -288,6 +318,19 @@ __global__ __launch_bounds__(kBlock) void k_locality_count(const T *__restrict__
     }
 }
 
+template <typename T>
+__global__ __launch_bounds__(kBlock) void k_locality_count(const T *__restrict__ positions, int N, int pd,
+                                                            LocalityScratch scratch, int *__restrict__ order,
+                                                            size_t order_entries) {
+    locality_count<T, false>(positions, N, pd, scratch, order, order_entries, nullptr);
+}
+template <typename T>
+__global__ __launch_bounds__(kBlock) void k_locality_count_told(const T *__restrict__ positions, int N, int pd,
+                                                                 LocalityScratch scratch, int *__restrict__ order,
+                                                                 size_t order_entries, unsigned *order_tally) {
+    locality_count<T, true>(positions, N, pd, scratch, order, order_entries, order_tally);
+}
+
 // The same for lists of many points, without an atomic on memory where the list has no order: a
 // workgroup of kScanBlock threads counts its points (kPerThread a thread) in a histogram of all bins in
 // LDS, two 16-bit counts to a word (the LDS atomic returns the point's rank among the workgroup's), and
@@ -304,16 +347,17 @@ __global__ __launch_bounds__(kBlock) void k_locality_count(const T *__restrict__
 // then have nothing to do, and fewer workgroups cost 3 to 7 us a call; telling costs 1 us.)
 template <typename T, int kPerThread>
 __global__ __launch_bounds__(kScanBlock) void k_locality_table(const T *__restrict__ positions, int N, int pd,
-                                                                LocalityScratch scratch, int *__restrict__ order,
-                                                                size_t order_entries) {
+                                                                LocalityScratch scratch, unsigned *__restrict__ histograms,
+                                                                const unsigned *order_tally, int *__restrict__ order) {
     __shared__ unsigned count[kLocalityTableBins / 2];
     static_assert(kScanBlock * kPerThread < 65536, "16-bit counts");
     const int lane = threadIdx.x & 63;
+    const size_t order_entries = (size_t)scratch.max_tiles * kBlock;
     for (size_t i = (size_t)blockIdx.x * kScanBlock + threadIdx.x; i < order_entries;
          i += (size_t)gridDim.x * kScanBlock)
         order[i] = -1;
     const LocalityBins bins = *bins_record(scratch);
-    const bool table = *scratch.in_order == 0u;
+    const bool table = !locality_in_order(*order_tally);
     const unsigned n_bins = bins.n_bins < scratch.max_bins ? bins.n_bins : scratch.max_bins;
     if (table)
         for (unsigned i = threadIdx.x; 2u * i < n_bins; i += kScanBlock) count[i] = 0u;
@@ -371,7 +415,7 @@ __global__ __launch_bounds__(kScanBlock) void k_locality_table(const T *__restri
     }
     if (!table) return;
     __syncthreads();
-    unsigned *__restrict__ row = scratch.table + (size_t)blockIdx.x * n_bins;
+    unsigned *__restrict__ row = histograms + (size_t)blockIdx.x * n_bins;
     for (unsigned i = threadIdx.x; i < n_bins; i += kScanBlock)
         row[i] = (count[i >> 1] >> ((i & 1u) * 16u)) & 0xffffu;
 }
@@ -379,11 +423,12 @@ __global__ __launch_bounds__(kScanBlock) void k_locality_table(const T *__restri
 // Sixty-four columns per workgroup, its sixteen wavefronts a sixteenth of the rows each.
 constexpr unsigned kTableGroups = kScanBlock / 64;
 constexpr unsigned kTableHeld = (kLocalityTableRows + kTableGroups - 1) / kTableGroups;
-__global__ __launch_bounds__(kScanBlock) void k_locality_table_columns(LocalityScratch scratch, unsigned rows) {
+__global__ __launch_bounds__(kScanBlock) void k_locality_table_columns(LocalityScratch scratch, unsigned *__restrict__ table,
+                                                                        const unsigned *order_tally, unsigned rows) {
     __shared__ unsigned group_sum[kTableGroups][64];
     unsigned n_bins = bins_record(scratch)->n_bins;
     if (n_bins > scratch.max_bins) n_bins = scratch.max_bins;
-    if (blockIdx.x * 64u >= n_bins || *scratch.in_order) return;     // (the whole workgroup)
+    if (blockIdx.x * 64u >= n_bins || locality_in_order(*order_tally)) return;     // (the whole workgroup)
     const unsigned lane = threadIdx.x & 63u, group = threadIdx.x >> 6;
     const unsigned bin = blockIdx.x * 64u + lane;
     const unsigned column = bin < n_bins ? bin : n_bins - 1u;
@@ -393,7 +438,7 @@ __global__ __launch_bounds__(kScanBlock) void k_locality_table_columns(LocalityS
 #pragma unroll
     for (unsigned k = 0; k < kTableHeld; ++k) {
         const unsigned r = begin + k;
-        held[k] = scratch.table[(size_t)(k < per && r < rows ? r : 0u) * n_bins + column];
+        held[k] = table[(size_t)(k < per && r < rows ? r : 0u) * n_bins + column];
     }
 #pragma unroll
     for (unsigned k = 0; k < kTableHeld; ++k) {
@@ -408,7 +453,7 @@ __global__ __launch_bounds__(kScanBlock) void k_locality_table_columns(LocalityS
 #pragma unroll
     for (unsigned k = 0; k < kTableHeld; ++k) {
         const unsigned r = begin + k;
-        if (k < per && r < rows) scratch.table[(size_t)r * n_bins + bin] = before;
+        if (k < per && r < rows) table[(size_t)r * n_bins + bin] = before;
         before += held[k];
     }
     if (group == kTableGroups - 1u) scratch.bin_count[bin] = before;
@@ -597,38 +642,59 @@ __global__ __launch_bounds__(kBlock) void k_locality_chunk_scan(LocalityScratch 
     }
 }
 
+__device__ __forceinline__ void put_in_order(const LocalityScratch &scratch, int *__restrict__ order, size_t n,
+                                             unsigned place) {
+    // (ranks come from atomics on counts that started at zero, so the place is the point's own)
+    if ((size_t)place < (size_t)scratch.max_tiles * kBlock) order[place] = (int)n;
+}
 __global__ __launch_bounds__(kBlock) void k_locality_scatter(LocalityScratch scratch, int N,
-                                                              unsigned points_per_row, int *__restrict__ order) {
+                                                              int *__restrict__ order) {
+    const size_t n = (size_t)blockIdx.x * kBlock + threadIdx.x;
+    if (n >= (size_t)N) return;
+    const uint2 br = scratch.bin_rank[n];
+    put_in_order(scratch, order, n, scratch.bin_first[br.x] + br.y);
+}
+// (a rank from the table of histograms is among the points of one row)
+__global__ __launch_bounds__(kBlock) void k_locality_scatter_rows(LocalityScratch scratch, int N,
+                                                                   int *__restrict__ order,
+                                                                   const unsigned *__restrict__ table,
+                                                                   const unsigned *order_tally,
+                                                                   unsigned points_per_row) {
     const size_t n = (size_t)blockIdx.x * kBlock + threadIdx.x;
     if (n >= (size_t)N) return;
     const uint2 br = scratch.bin_rank[n];
     unsigned place = scratch.bin_first[br.x] + br.y;
-    // (a rank from the table of histograms is among the points of one row)
-    if (points_per_row && !*scratch.in_order) {
+    if (!locality_in_order(*order_tally)) {
         const unsigned n_bins = bins_record(scratch)->n_bins;
-        place += scratch.table[n / points_per_row * (n_bins < scratch.max_bins ? n_bins : scratch.max_bins) + br.x];
+        place += table[n / points_per_row * (n_bins < scratch.max_bins ? n_bins : scratch.max_bins) + br.x];
     }
-    // (ranks come from atomics on counts that started at zero, so the place is the point's own)
-    if ((size_t)place < (size_t)scratch.max_tiles * kBlock) order[place] = (int)n;
+    put_in_order(scratch, order, n, place);
 }
 
 template <typename T>
-hipError_t order_points(const T *positions, int N, int pd, const LocalityScratch &scratch, int *order,
-                        hipStream_t s) {
+hipError_t order_points(const T *positions, int N, int pd, const LocalityScratch &scratch,
+                        const LocalityTable &counting, int *order, hipStream_t s) {
     const unsigned blocks = (unsigned)(((size_t)N + kBlock - 1) / kBlock);
-    hipLaunchKernelGGL((k_locality_bins<T>), dim3(1), dim3(kScanBlock), 0, s, positions, N, pd, scratch);
-    const unsigned table_rows = scratch.table && !scratch.expect_in_order ? locality_table_rows(N) : 0u;
+    const unsigned table_rows = counting.table && !counting.expect_in_order ? locality_table_rows(N) : 0u;
     const unsigned per_thread = locality_table_points(N) / kScanBlock;
     if (table_rows) {
+        hipLaunchKernelGGL((k_locality_bins_told<T>), dim3(1), dim3(kScanBlock), 0, s, positions, N, pd, scratch,
+                           counting.order_tally);
         const auto count = per_thread == 1 ? k_locality_table<T, 1> : per_thread == 2 ? k_locality_table<T, 2> : k_locality_table<T, 4>;
-        hipLaunchKernelGGL(count, dim3(table_rows), dim3(kScanBlock), 0, s, positions, N, pd, scratch, order,
-                           (size_t)scratch.max_tiles * kBlock);
+        hipLaunchKernelGGL(count, dim3(table_rows), dim3(kScanBlock), 0, s, positions, N, pd, scratch, counting.table,
+                           counting.order_tally, order);
         hipLaunchKernelGGL(k_locality_table_columns, dim3((scratch.max_bins + 63u) / 64u), dim3(kScanBlock), 0, s,
-                           scratch, table_rows);
+                           scratch, counting.table, counting.order_tally, table_rows);
     } else {
+        hipLaunchKernelGGL((k_locality_bins<T>), dim3(1), dim3(kScanBlock), 0, s, positions, N, pd, scratch);
         const unsigned count_blocks = (blocks + kCountPoints - 1) / kCountPoints;
-        hipLaunchKernelGGL((k_locality_count<T>), dim3(count_blocks), dim3(kBlock), 0, s, positions, N, pd, scratch,
-                           order, (size_t)scratch.max_tiles * kBlock);
+        const size_t order_entries = (size_t)scratch.max_tiles * kBlock;
+        if (counting.table)
+            hipLaunchKernelGGL((k_locality_count_told<T>), dim3(count_blocks), dim3(kBlock), 0, s, positions, N, pd, scratch,
+                               order, order_entries, counting.order_tally);
+        else
+            hipLaunchKernelGGL((k_locality_count<T>), dim3(count_blocks), dim3(kBlock), 0, s, positions, N, pd, scratch,
+                               order, order_entries);
     }
     if (scratch.max_bins <= kOneWorkgroupScans) {
         hipLaunchKernelGGL(k_locality_scan, dim3(1), dim3(kScanBlock), 0, s, scratch, N);
@@ -639,25 +705,29 @@ hipError_t order_points(const T *positions, int N, int pd, const LocalityScratch
         hipLaunchKernelGGL(k_locality_chunk_places, dim3(1), dim3(64), 0, s, scratch, N, n_chunks);
         hipLaunchKernelGGL(k_locality_chunk_scan, dim3(n_chunks), dim3(kBlock), 0, s, scratch, n_chunks);
     }
-    hipLaunchKernelGGL(k_locality_scatter, dim3(blocks), dim3(kBlock), 0, s, scratch, N,
-                       table_rows ? locality_table_points(N) : 0u, order);
+    if (table_rows)
+        hipLaunchKernelGGL(k_locality_scatter_rows, dim3(blocks), dim3(kBlock), 0, s, scratch, N, order, counting.table,
+                           counting.order_tally, locality_table_points(N));
+    else
+        hipLaunchKernelGGL(k_locality_scatter, dim3(blocks), dim3(kBlock), 0, s, scratch, N, order);
     return hipGetLastError();
 }
 
 }  // namespace
 
 hipError_t order_by_locality(const float *positions, const double *positions64, int N, int pd,
-                             const LocalityScratch &scratch, int *order, hipStream_t s) {
+                             const LocalityScratch &scratch, const LocalityTable &counting, int *order,
+                             hipStream_t s) {
     if (N <= 0) return hipSuccess;
     if (!scratch.bins || !scratch.range0 || !scratch.bin_count || !scratch.bin_first ||
-        !scratch.bin_rank || !order || !scratch.n_tiles || !scratch.in_order || !scratch.chunk_sums || !scratch.chunk_first ||
+        !scratch.bin_rank || !order || !scratch.n_tiles || !counting.order_tally || !scratch.chunk_sums || !scratch.chunk_first ||
         scratch.max_bins < 4u ||
         (size_t)scratch.max_tiles * kBlock < (size_t)N || scratch.max_bins % 4u != 0u ||
         (reinterpret_cast<uintptr_t>(scratch.bin_count) | reinterpret_cast<uintptr_t>(scratch.bin_first)) % 16u != 0u ||
-        pd < 1 || (scratch.table && locality_table_rows(N) && scratch.max_bins > kLocalityTableBins))
+        pd < 1 || (counting.table && locality_table_rows(N) && scratch.max_bins > kLocalityTableBins))
         return hipErrorInvalidValue;
-    if (positions64) return order_points<double>(positions64, N, pd, scratch, order, s);
-    if (positions) return order_points<float>(positions, N, pd, scratch, order, s);
+    if (positions64) return order_points<double>(positions64, N, pd, scratch, counting, order, s);
+    if (positions) return order_points<float>(positions, N, pd, scratch, counting, order, s);
     return hipErrorInvalidValue;
 }
 
