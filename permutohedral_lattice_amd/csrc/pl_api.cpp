@@ -185,7 +185,7 @@ struct pl_lattice {
     unsigned *locality_words = nullptr;    // the bins, range of feature 0, counts and firsts of the bins
     uint2 *bin_rank = nullptr;             // [N]
     unsigned *bin_table = nullptr;         // histograms of the bins (plk::locality_table_rows)
-    bool list_in_order = false;            // the last list that was ordered ran from a bin to the next
+    int expect_in_order_for = 0;           // lists to be counted as lists that run from a bin to the next
     int list_counted = -1;                 // PL_INFO_LIST_COUNTED (1 until the build reports: perhaps)
     int order_capacity = 0;
     hipEvent_t ev[EV_COUNT] = {};
@@ -479,7 +479,7 @@ int enqueue_build(pl_lattice *h, const plk::PointFeatures &features, const doubl
     h->counter_set = 1 - previous_set;
     h->list_counted = -1;
     if (h->map.mode == 1) {
-        const plk::LocalityTable counting{h->bin_table, &h->counters()->order_tally, h->list_in_order};
+        const plk::LocalityTable counting{h->bin_table, &h->counters()->order_tally, h->expect_in_order_for > 0};
         h->list_counted = counting.table && !counting.expect_in_order ? 1 : 0;
         PL_HIP(plk::order_by_locality(h->f64 ? nullptr : features.positions,
                                       h->f64 ? positions64 : nullptr, h->N, h->pd,
@@ -759,8 +759,14 @@ int verify_build(pl_lattice *h, uint32_t *retry_cells) {
     const int flags = status.flags;
     const int m = status.num_vertices;
     if (h->map.mode == 1) {
-        h->list_in_order = (flags & plk::kFlagListInOrder) != 0;
-        if (h->list_in_order) h->list_counted = 0;
+        // (two lists in no order before histograms are tried again: a program whose lists alternate
+        // would get every one of them counted the wrong way)
+        if (flags & plk::kFlagListInOrder) {
+            h->expect_in_order_for = 2;
+            h->list_counted = 0;
+        } else if (h->expect_in_order_for > 0) {
+            h->expect_in_order_for -= 1;
+        }
     }
     h->last_n_segments = status.n_segments;
     h->last_max_segment = status.max_segment;

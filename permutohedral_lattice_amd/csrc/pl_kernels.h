@@ -502,7 +502,7 @@ struct LocalityScratch {
 struct LocalityTable {
     unsigned *table;       // [locality_table_rows(N) * max_bins], none where that is 0
     unsigned *order_tally; // Counters::order_tally of the build, zero
-    bool expect_in_order;  // the handle's last list ran from a bin to the next
+    bool expect_in_order;  // one of the handle's last two lists ran from a bin to the next
 };
 // A list that runs from a bin to the next: fewer than a quarter of the points change it (k_locality_table)
 constexpr bool locality_in_order(unsigned order_tally) { return 4u * (order_tally & 0xffffu) < order_tally >> 16; }

@@ -343,8 +343,10 @@ __global__ __launch_bounds__(kBlock) void k_locality_count_told(const T *__restr
 // their bin at fewer than a quarter of their points, ranks are drawn from memory as above.  (A filter of
 // 65536 points that change it at 0.20 of them 47.9 us with atomics, 48.1 with the table, at 0.28 50.3 and
 // 48.9; a million at 0.28 95.0 and 103.6, at 0.36 112.1 and 100.7.)  (A handle
-// whose last list was in order takes the kernel above at once: the launches here and below, which
-// then have nothing to do, and fewer workgroups cost 3 to 7 us a call; telling costs 1 us.)
+// that had a list in order among its last two takes the kernel above at once: the launches here and below,
+// which then have nothing to do, and fewer workgroups cost a list in order 3 to 7 us.  Two, so that lists
+// that alternate are all counted above: 20000 points in order and 20000 in none, by turns, 90.9 us with
+// the last list deciding, 85.1 with the last two, 84.1 without the table at all.)
 template <typename T, int kPerThread>
 __global__ __launch_bounds__(kScanBlock) void k_locality_table(const T *__restrict__ positions, int N, int pd,
                                                                 LocalityScratch scratch, unsigned *__restrict__ histograms,
