@@ -200,7 +200,8 @@ typedef enum pl_info {
                                   estimate from every eighth workgroup); else -1 */
     PL_INFO_LIST_COUNTED = 5   /* when the last build put a plain list in an order (PL_OPT_ORDER_POINTS):
                                   1 if its points were counted in histograms, 0 if with atomics on memory
-                                  (short, very long and already ordered lists); else -1 */
+                                  (short, very long and already ordered lists, or no memory for the
+                                  histograms); else -1 */
 } pl_info;
 int pl_get_info(pl_handle h, int what, long *value);
 

@@ -36,7 +36,10 @@ inline int hip_failed(hipError_t e) {
 
 void *default_alloc(void *, size_t bytes) {
     void *p = nullptr;
-    if (hipMalloc(&p, bytes ? bytes : 1) != hipSuccess) return nullptr;
+    if (hipMalloc(&p, bytes ? bytes : 1) != hipSuccess) {
+        (void)hipGetLastError();   // (the caller says so, or does without: not the next launch's error)
+        return nullptr;
+    }
     return p;
 }
 void default_free(void *, void *p) {
@@ -389,9 +392,9 @@ int ensure_order(pl_lattice *h) {
     h->locality_words = (unsigned *)h->dmalloc(sizeof(unsigned) * words);
     h->bin_rank = (uint2 *)h->dmalloc(sizeof(uint2) * (size_t)h->N);
     const size_t table_words = (size_t)plk::locality_table_rows(h->N) * max_bins;
+    if (!h->point_order || !h->locality_words || !h->bin_rank) return PL_ENOMEM;
+    // (a list can be counted without it)
     if (table_words) h->bin_table = (unsigned *)h->dmalloc(sizeof(unsigned) * table_words);
-    if (!h->point_order || !h->locality_words || !h->bin_rank || (table_words && !h->bin_table))
-        return PL_ENOMEM;
     // (the pass leaves its counts zero for the next call)
     PL_HIP(plk::fill_zero(reinterpret_cast<float *>(h->locality_words), words, h->stream));
     h->order_capacity = h->N;
@@ -1442,7 +1445,7 @@ int pl_get_info(pl_handle h, int what, long *value) {
                      sizeof(uint2) * (size_t)h->order_capacity +
                      sizeof(unsigned) * (33 + 2 * (size_t)max_bins +
                                          3 * (size_t)plk::locality_scan_chunks(max_bins) +
-                                         (size_t)plk::locality_table_rows(h->order_capacity) * max_bins);
+                                         (h->bin_table ? (size_t)plk::locality_table_rows(h->order_capacity) * max_bins : 0));
             }
             *value = (long)b;
             return PL_OK;

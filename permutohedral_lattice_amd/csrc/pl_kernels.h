@@ -500,7 +500,7 @@ struct LocalityScratch {
 // instantiations without it: three more words in the arguments of each, and the tally taken and reported
 // where nobody asks for it, cost lists too short for a table 0.5 to 2 us of 46 to 49.)
 struct LocalityTable {
-    unsigned *table;       // [locality_table_rows(N) * max_bins], none where that is 0
+    unsigned *table;       // [locality_table_rows(N) * max_bins], none where that is 0 or there is no memory
     unsigned *order_tally; // Counters::order_tally of the build, zero
     bool expect_in_order;  // one of the handle's last two lists ran from a bin to the next
 };

@@ -27,15 +27,18 @@ class PlAlloc(C.Structure):
 class TorchScratch:
     """Allocator callbacks over torch tensors, with a budget after which alloc returns NULL."""
 
-    def __init__(self, fail_after=None):
+    def __init__(self, fail_after=None, refuse=None):
         self.live, self.n_alloc, self.n_free, self.bytes = {}, 0, 0, 0
-        self.fail_after = fail_after
+        self.fail_after, self.refuse, self.refused = fail_after, refuse, 0
         self._alloc = ALLOC_FN(self.alloc)
         self._free = FREE_FN(self.free)
         self.struct = PlAlloc(self._alloc, self._free, None)
 
     def alloc(self, _ctx, nbytes):
         if self.fail_after is not None and self.n_alloc >= self.fail_after:
+            return None
+        if nbytes == self.refuse:
+            self.refused += 1
             return None
         t = torch.empty(max(int(nbytes), 1), dtype=torch.uint8, device="cuda")
         self.live[t.data_ptr()] = t
@@ -107,6 +110,34 @@ def test_allocation_failure_is_reported_and_leaks_nothing(fail_after):
     else:
         assert rc == pla.PL_ENOMEM and not handle.value
     assert not scratch.live and scratch.n_free == scratch.n_alloc
+
+
+def test_a_list_does_without_the_histograms_there_is_no_memory_for():
+    """The table a long list is counted with is large (36 to 50 bytes a point) and can be done without."""
+    pd, vd, n = 2, 2, 1 << 18
+    gen = torch.Generator("cuda").manual_seed(1)
+    pos = torch.rand((n, pd), device="cuda", generator=gen) * 40.0
+    val = torch.rand((n, 1), device="cuda", generator=gen)
+    bins, rows = (n // 32 + 1024) & ~3, n // 1024
+    outs = []
+    for refuse in (None, 4 * bins * rows):
+        scratch = TorchScratch(refuse=refuse)
+        handle, counted = C.c_void_p(), C.c_long()
+        lib = pla._lib
+        assert lib.pl_create(pd, vd, n, None, C.byref(scratch.struct), C.byref(handle)) == pla.PL_OK
+        assert lib.pl_set_option(handle, pla.PL_OPT_GUESS_GRID, 0) == pla.PL_OK
+        out = torch.full((n, 1), float("nan"), device="cuda")
+        torch.cuda.synchronize()
+        for _ in range(2):
+            assert lib.pl_filter(handle, out.data_ptr(), val.data_ptr(), pos.data_ptr(), 0) == pla.PL_OK
+            assert lib.pl_get_info(handle, pla.PL_INFO_LIST_COUNTED, C.byref(counted)) == pla.PL_OK
+            assert counted.value == (1 if refuse is None else 0)
+        torch.cuda.synchronize()
+        assert scratch.refused == (0 if refuse is None else 1)     # (and is not asked for again)
+        outs.append(out)
+        assert lib.pl_destroy(handle) == pla.PL_OK
+        assert scratch.n_free == scratch.n_alloc and not scratch.live
+    assert float((outs[0] - outs[1]).abs().max()) <= 2e-5
 
 
 def test_op_with_caller_scratch_returns_everything_before_it_returns():
