@@ -107,9 +107,8 @@ class MeanField:
         """-> Q after ``iterations`` mean-field updates, shaped like ``logits``."""
         flat = logits.contiguous().view(self.batch, self.n, self.n_classes)
         q = torch.softmax(flat, dim=-1)
-        if type(self).messages is not MeanField.messages or not mean_field_update_supported(flat):
-            # (messages of a class derived from this one; logits that autograd follows into the last
-            # softmax, among others)
+        if not self._own_messages() or not mean_field_update_supported(flat):
+            # (logits that autograd follows into the last softmax, among others)
             for _ in range(iterations):
                 q = torch.softmax(flat + self.messages(q), dim=-1)
             return q.view(logits.shape)
@@ -123,7 +122,13 @@ class MeanField:
     def reverse(self, upstream):
         """The op's registered gradient of one message-passing step with respect to its input:
         both filters with ``reverse=True`` on ``upstream``, summed."""
-        return self.messages(upstream, reverse=True).view(upstream.shape)
+        total = self.messages(upstream, reverse=True).view(upstream.shape)
+        # (messages put in the place of this class's may give the same tensor again on the next call)
+        return total if self._own_messages() else total.clone()
+
+    def _own_messages(self):
+        """Whether ``messages`` is this class's, neither a derived class's nor put on the object."""
+        return getattr(self.messages, "__func__", None) is MeanField.messages
 
     def close(self):
         for lat in self.bilateral + self.spatial:

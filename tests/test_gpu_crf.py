@@ -107,3 +107,29 @@ def test_mean_field_update_leaves_other_calls_to_torch():
     with torch.no_grad():
         assert float((mf.infer(logits, iterations=2) - q).abs().max()) <= 1e-6
     mf.close()
+
+
+def test_messages_put_in_the_place_of_the_class_s():
+    """On the object or in a derived class: ``infer`` calls them, and what ``reverse`` gives does not
+    change with the next call where they return one tensor again and again."""
+    class Scaled(MeanField):
+        def messages(self, q, reverse=False):
+            self._msg_bi.copy_(super().messages(q, reverse) * 0.5)
+            return self._msg_bi
+
+    guide = torch.rand((1, 24, 32, 3), device="cuda") * 255.0
+    logits, upstream = (torch.randn((1, 24, 32, 4), device="cuda") for _ in range(2))
+    derived, plain = Scaled(guide, 4), MeanField(guide, 4)
+    step = torch.softmax(logits, dim=-1)
+    for _ in range(2):
+        step = torch.softmax(logits + 0.5 * plain.messages(step).view(logits.shape), dim=-1)
+    assert float((derived.infer(logits, 2) - step).abs().max()) <= 1e-6
+    first = derived.reverse(upstream)
+    kept = first.clone()
+    derived.reverse(3.0 * upstream)
+    assert torch.equal(first, kept)
+    own = plain.messages
+    plain.messages = lambda q, reverse=False: 0.5 * own(q, reverse)
+    assert float((plain.infer(logits, 2) - step).abs().max()) <= 1e-6
+    derived.close()
+    plain.close()
