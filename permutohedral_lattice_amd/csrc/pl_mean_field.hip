@@ -14,14 +14,12 @@ namespace {
 // A workgroup takes `kRows` points: their sums go to LDS as they lie in memory (16-byte loads of
 // consecutive lanes), every thread then has one point's row there to itself (rows an odd number of
 // words apart: no bank conflicts), and the results leave as the logits came.  What bounds it is the
-// four arrays' way through memory, each once: two sums and a softmax as separate passes moved
+// four arrays' way through memory, each once (q may be one of the others: no __restrict__, everything is
+// read before the first barrier and written behind the second): two sums and a softmax as separate passes moved
 // eight (2 x 512x512 points of 21 classes: 73.5 us, now 32.3, 5.4 TB/s).
 template <int kRows>
-__global__ __launch_bounds__(kRows) void k_mean_field_update(float *__restrict__ q,
-                                                              const float *__restrict__ logits,
-                                                              const float *__restrict__ message_a,
-                                                              const float *__restrict__ message_b,
-                                                              size_t n_points, int classes) {
+__global__ __launch_bounds__(kRows) void k_mean_field_update(float *q, const float *logits, const float *message_a,
+                                                              const float *message_b, size_t n_points, int classes) {
     extern __shared__ float rows[];   // [kRows][classes | 1]
     const int pitch = classes | 1;
     const size_t first = (size_t)blockIdx.x * kRows;

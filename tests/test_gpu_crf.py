@@ -71,8 +71,10 @@ def test_mean_field_update_is_the_softmax_of_the_sums(classes, n):
     want = torch.softmax((logits + (a + b)).double(), dim=-1)
     # e^x and the quotient to an ulp or two each, a sum of `classes` terms
     assert float((q.double() - want).abs().max()) <= (classes + 8) * 6e-8
-    pla.mean_field_update(logits, logits, a, b)     # in place
-    assert torch.equal(logits, q)
+    for which in range(3):                          # in place of each array
+        arrays = [t.clone() for t in (logits, a, b)]
+        pla.mean_field_update(arrays[which], *arrays)
+        assert torch.equal(arrays[which], q)
 
 
 @pytest.mark.parametrize("classes", [2, 5, 21, 40, 41, 64, 128])
