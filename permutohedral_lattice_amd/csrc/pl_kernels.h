@@ -300,8 +300,8 @@ hipError_t splat(int pd, int vd, const PointMap &map, const float *input, int in
                  ReplayEntry *replay, const int *cell_vertex, float *values,
                  int xcd_aware, hipStream_t s);
 
-// The same for rows of 5 to 32 channels when the workgroups' points share their vertices, as after a
-// merging build (any points are splatted correctly): pairs sorted by vertex in LDS, see pl_splat_tile.hip.
+// The same for rows of 5 to 32 channels after a merging build, whose workgroups' points have at most
+// kTileSlots vertices: pairs sorted by vertex in LDS, see pl_splat_tile.hip.
 // (up to 32 channels and nine corners the pairs and the points' rows fit 64 KB of LDS)
 inline bool splat_tile_takes(int vd) { return vd >= 5 && vd <= 32; }
 hipError_t splat_tile(int pd, int vd, const PointMap &map, const float *input, int in_channels, ReplayEntry *replay,

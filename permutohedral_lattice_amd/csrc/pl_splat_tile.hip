@@ -24,8 +24,8 @@ using namespace device;
 // 130 rows a workgroup.  k_splat_channels, which takes a wavefront's pairs vertex by vertex, loads the
 // rows once per two corners and sends a row per wavefront and vertex (about 165): 2 x 321x481 points, pd = 5,
 // vd = 22: 37.0 us a launch, this 26.5.
-// A vertex that finds no slot (more than kTileSlots of them in one workgroup, which a merging build
-// does not leave behind) has its rows added one by one.
+// After a merging build only: it leaves a workgroup at most kTileSlots vertices (a build with more is
+// repeated without merging), so that every vertex finds a slot.
 // Two threads to a point, which share its corners (one thread to a point, 16 groups of lanes: 27.6 us;
 // every lane looking for its slot instead of the first of a run: 27.1).
 constexpr unsigned kSides = 2, kThreads = kSides * kBlock;
@@ -163,20 +163,11 @@ __global__ __launch_bounds__(kThreads) void k_splat_tile(int d1, int vd, PointMa
 
 #pragma unroll
     for (int r = 0; r < (int)kMaxCorners; ++r) {
-        if (index[r] < 0) continue;
-        int v;
-        if (place[r] != kNoPlace) {
-            const unsigned slot = place[r] & 0xffffu;
-            sorted[slot_count[slot] + (place[r] >> 16)] =
-                make_uint2(__float_as_uint(weight[r]), (unsigned)point | slot << 8);
-            v = slot_index[slot];
-        } else {
-            v = cell_vertex ? cell_vertex[index[r]] : index[r];
-            for (int c = 0; c < vd; ++c)
-                atomicAdd(values + ((unsigned)v * (unsigned)vd + (unsigned)c),
-                          weight[r] * (c < in_channels ? rows[point * in_channels + c] : 1.0f));
-        }
-        if (cell_vertex) replay[(size_t)((int)kSides * r + side) * T + t].index = v;
+        if (place[r] == kNoPlace) continue;
+        const unsigned slot = place[r] & 0xffffu;
+        sorted[slot_count[slot] + (place[r] >> 16)] =
+            make_uint2(__float_as_uint(weight[r]), (unsigned)point | slot << 8);
+        if (cell_vertex) replay[(size_t)((int)kSides * r + side) * T + t].index = slot_index[slot];
     }
     __syncthreads();   // the pairs are in the order of their slots
 
