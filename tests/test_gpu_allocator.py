@@ -113,7 +113,7 @@ def test_allocation_failure_is_reported_and_leaks_nothing(fail_after):
 
 
 def test_a_list_does_without_the_histograms_there_is_no_memory_for():
-    """The table a long list is counted with is large (36 to 50 bytes a point) and can be done without."""
+    """The table a long list is counted with is large (here 36 bytes a point) and can be done without."""
     pd, vd, n = 2, 2, 1 << 18
     gen = torch.Generator("cuda").manual_seed(1)
     pos = torch.rand((n, pd), device="cuda", generator=gen) * 40.0

@@ -69,8 +69,9 @@ def test_mean_field_update_is_the_softmax_of_the_sums(classes, n):
     assert pla.mean_field_update_supported(logits)
     q = pla.mean_field_update(torch.full_like(logits, float("nan")), logits, a, b)
     want = torch.softmax((logits + (a + b)).double(), dim=-1)
-    # e^x and the quotient to an ulp or two each, a sum of `classes` terms
-    assert float((q.double() - want).abs().max()) <= (classes + 8) * 6e-8
+    # in halves of an ulp of 1, 6e-8: the argument's rounding at most 0.37 (d e^-d), e^x 2, the quotient 1,
+    # and the sum, of doubles, the terms' own 2.4 and 1 for its rounding: less than 8 for any number of classes
+    assert float((q.double() - want).abs().max()) <= 8 * 6e-8
     for which in range(3):                          # in place of each array
         arrays = [t.clone() for t in (logits, a, b)]
         pla.mean_field_update(arrays[which], *arrays)
