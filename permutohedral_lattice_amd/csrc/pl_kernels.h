@@ -302,7 +302,10 @@ hipError_t splat(int pd, int vd, const PointMap &map, const float *input, int in
 
 // The same for rows of 5 to 32 channels after a merging build, whose workgroups' points have at most
 // kTileSlots vertices: pairs sorted by vertex in LDS, see pl_splat_tile.hip.
-// (up to 32 channels and nine corners the pairs and the points' rows fit 64 KB of LDS)
+// (Up to 32 channels and nine corners the pairs and the points' rows fit 64 KB of LDS.  Filters of
+// 64x64 to 800x1000 points, splat by wavefronts and this, us: 64x64 pd 2 vd 5 32.4 and 29.7, pd 5 vd 32
+// 56.9 and 53.0; 120x160 pd 3 vd 17 41.0 and 37.5; 321x481 pd 2 vd 22 54.9 and 53.5, pd 5 vd 5 84.8 and 65.1;
+// 800x1000 pd 2 vd 32 150 and 131, pd 3 vd 8 133 and 97, pd 5 vd 16 278 and 194; in none of 60 shapes slower.)
 inline bool splat_tile_takes(int vd) { return vd >= 5 && vd <= 32; }
 hipError_t splat_tile(int pd, int vd, const PointMap &map, const float *input, int in_channels, ReplayEntry *replay,
                       const int *cell_vertex, float *values, int xcd_aware, hipStream_t s);
@@ -479,7 +482,8 @@ hipError_t guess_grid(const float *positions, int N, int pd, GridGuess *guess, h
 // max_tiles workgroups (a quarter more than the points fill).  Otherwise the bins follow each
 // other without gaps and a wavefront takes parts of two.  Four launches: the bins (from the
 // bounding box of a sample of the points), count (every point draws its rank in its bin), scan of
-// the counts, scatter.
+// the counts, scatter; five where the points are counted in histograms (LocalityTable), whose columns
+// are added up by a launch of their own.
 // The order inside a bin is whatever the atomics gave; it only orders the work.
 // bin_count must be zero before the first call; every call leaves it so.
 constexpr size_t kLocalityBinsBytes = 64;
@@ -511,9 +515,12 @@ inline unsigned locality_bins_for(int N) { return ((unsigned)N / 32u + 1024u) & 
 // The table of histograms a list of N points is counted with (k_locality_table): a row per
 // locality_table_points(N) points (one, two or four per thread of a workgroup, so that there are
 // enough workgroups and few rows), locality_table_rows(N) of them; 0: no table, ranks are drawn with
-// atomics on memory.  At most as many points as have their bins in one workgroup's LDS, and no
-// fewer than kLocalityTableFrom (a filter of a cloud
-// of 16384 points 54.3 us with atomics, 49.7 with the table; 131072: 86.3 and 60.6; a million: 237 and 173)
+// atomics on memory.  At most as many points as have their bins in 80 KB of LDS, which leaves a CU room
+// for two workgroups (1 278 079 points, 313 rows: within the 320 whose counts k_locality_table_columns holds
+// in registers), and no fewer than kLocalityTableFrom (a filter of a cloud
+// of 16384 points 54.3 us with atomics, 49.7 with the table; 131072: 86.3 and 60.6; a million: 237 and 173).
+// A word a count: 0.1 to 51 MB a handle (16 of the 105 that a handle of 500 009 points holds); the
+// first filter of a new handle, bound by its allocations, takes as long as without (1.44 and 1.43 ms).
 constexpr unsigned kLocalityTableBins = 40960, kLocalityTableRows = 320;
 constexpr int kLocalityTableFrom = 16384;
 inline unsigned locality_table_points(int N) { return N <= (1 << 18) ? 1024u : N <= (1 << 19) ? 2048u : 4096u; }
