@@ -479,10 +479,10 @@ int enqueue_build(pl_lattice *h, const plk::PointFeatures &features, const doubl
     h->stage_ran[3] = true;
     // the previous vertex-numbering kernel (or pl_create) left the other counter set zeroed
     const int previous_set = h->counter_set;
-    h->counter_set = 1 - previous_set;
     h->list_counted = -1;
     if (h->map.mode == 1) {
-        const plk::LocalityTable counting{h->bin_table, &h->counters()->order_tally, h->expect_in_order_for > 0};
+        const plk::LocalityTable counting{h->bin_table, &h->d_counters[1 - previous_set].order_tally,
+                                          h->expect_in_order_for > 0};
         h->list_counted = counting.table && !counting.expect_in_order ? 1 : 0;
         PL_HIP(plk::order_by_locality(h->f64 ? nullptr : features.positions,
                                       h->f64 ? positions64 : nullptr, h->N, h->pd,
@@ -494,6 +494,7 @@ int enqueue_build(pl_lattice *h, const plk::PointFeatures &features, const doubl
     h->table_clean = false;
     h->n_cells = cells;
     h->mark(EV_CLEAR);
+    h->counter_set = 1 - previous_set;
     const plk::VertexTables vertices{h->cell_vertex, h->vertex_keys, h->vertex_cell, h->neighbours,
                                      h->max_vertices()};
     const plk::CreatedLists lists = h->lists(h->counter_set);
