@@ -548,21 +548,117 @@ __device__ __forceinline__ int wave_leader_of_equal(T x, bool active, int lane) 
     }
     return leader;
 }
-// The same, and the mask of the lanes whose group has at most small_size members.
+// The groups of lanes that hold the same value of `x`, as an order of the lanes in which every group's
+// are next to each other.  Per lane: its place in that order (bits 0..7), the place of its group's
+// first lane (8..15), and that lane, the lowest of the group (16..23).  The lanes outside `among` come
+// last, each a group of its own.  All 64 lanes must call it.
 template <typename T>
-__device__ __forceinline__ int wave_leader_of_equal(T x, bool active, int lane, int small_size, uint64_t &small) {
-    int leader = lane;
-    small = 0;
-    const uint64_t among = wave_ballot(active);
+__device__ __forceinline__ unsigned wave_groups_in_order(T x, uint64_t among) {
+    unsigned own = 0, filled = 0;   // filled: how many lanes are placed, in both of the low bytes
     uint64_t remaining = among;
     while (remaining) {
         const int first = __builtin_ctzll(remaining);
-        const uint64_t same = lanes_equal(x, lane_value(x, first)) & among;
-        set_in_lanes(leader, same, first);
+        const uint64_t same = lanes_equal(x, lane_value(x, first)) & remaining;
+        const unsigned rank = __builtin_amdgcn_mbcnt_hi((uint32_t)(same >> 32),
+                                                        __builtin_amdgcn_mbcnt_lo((uint32_t)same, 0u));
+        // (one addition under a narrowed exec mask, as in set_in_lanes)
+        asm volatile(
+            "s_mov_b64 exec, %2\n\t"
+            "v_add_u32_e32 %0, %3, %1\n\t"
+            "s_mov_b64 exec, -1"
+            : "+v"(own)
+            : "v"(rank), "s"(same), "s"(filled + ((unsigned)first << 16)));
+        filled += (unsigned)lanes_in(same) * 0x101u;
         remaining &= ~same;
-        if (lanes_in(same) <= small_size) small |= same;
     }
-    return leader;
+    if (among != ~0ull) {
+        const uint64_t rest = ~among;
+        const unsigned rank = __builtin_amdgcn_mbcnt_hi((uint32_t)(rest >> 32),
+                                                        __builtin_amdgcn_mbcnt_lo((uint32_t)rest, 0u));
+        if (lane_in(rest)) own = filled + rank * 0x101u;
+    }
+    return own;
+}
+__device__ __forceinline__ int place_of(unsigned group) { return (int)(group & 0xffu); }
+__device__ __forceinline__ int first_place_of(unsigned group) { return (int)((group >> 8) & 0xffu); }
+__device__ __forceinline__ int leader_of(unsigned group) { return (int)(group >> 16); }
+
+// x of the lane that has place `lane` in the order (each lane gives its own place)
+__device__ __forceinline__ int to_place(int place, int x) {
+    return __builtin_amdgcn_ds_permute(place << 2, x);
+}
+__device__ __forceinline__ float to_place(int place, float x) {
+    return __int_as_float(to_place(place, __float_as_int(x)));
+}
+__device__ __forceinline__ double to_place(int place, double x) {
+    return __hiloint2double(to_place(place, __double2hiint(x)), to_place(place, __double2loint(x)));
+}
+
+// The lanes being in the order above, and first_place the place of a lane's group's first: x := the
+// sum of x over the lanes of the group up to this one, so that the last lane of every group holds the
+// group's sum.  Six steps for all groups of the wavefront together: the lane 1, 2, 4, 8 below in the
+// row of 16, the last lane of the row below, the last lane of the lower half, each added where it is
+// of the same group.  The terms must be finite and far from overflowing (what does not count is
+// multiplied by 0, so that a step is one instruction per channel).  All 64 lanes must call it.
+struct StepsCount {
+    float step[6];   // 1 where the lane a step looks at is of this lane's group, else 0
+};
+__device__ __forceinline__ StepsCount steps_that_count(int lane, int first_place) {
+    float before = (float)(lane - first_place);   // lanes of the group before this one
+    asm("" : "+v"(before));                       // (a float from here on: one instruction a step)
+    auto zero_to_one = [](float x) { return __builtin_amdgcn_fmed3f(x, 0.0f, 1.0f); };
+    return StepsCount{{zero_to_one(before), zero_to_one(before - 1.0f), zero_to_one(before - 3.0f),
+                       zero_to_one(before - 7.0f), zero_to_one(before - (float)(lane & 15)),
+                       zero_to_one(before - (float)(lane & 31))}};
+}
+// (A DPP operand written by one of the last two instructions is not seen: between a step's
+// instruction and the next step's on the same register there are two others.)
+template <int C>
+__device__ __forceinline__ void sum_groups_in_order(float (&x)[C], const StepsCount &counts) {
+    static_assert(C >= 2 && C <= 4, "the register splats");
+#define PLK_ADD_LANE(R, STEP, CONTROL) "v_fmac_f32_dpp " R ", " R ", " STEP " " CONTROL " bank_mask:0xf\n\t"
+#define PLK_SUM_STEPS(ADD)                                                                       \
+    "s_nop 1\n\t"                                                                              \
+    ADD("%[s0]", "row_shr:1 row_mask:0xf") ADD("%[s1]", "row_shr:2 row_mask:0xf")                  \
+    ADD("%[s2]", "row_shr:4 row_mask:0xf") ADD("%[s3]", "row_shr:8 row_mask:0xf")                  \
+    ADD("%[s4]", "row_bcast:15 row_mask:0xa") ADD("%[s5]", "row_bcast:31 row_mask:0xc")
+#define PLK_ADD2(S, C) PLK_ADD_LANE("%0", S, C) PLK_ADD_LANE("%1", S, C) "s_nop 0\n\t"
+#define PLK_ADD3(S, C) PLK_ADD_LANE("%0", S, C) PLK_ADD_LANE("%1", S, C) PLK_ADD_LANE("%2", S, C)
+#define PLK_ADD4(S, C) PLK_ADD3(S, C) PLK_ADD_LANE("%3", S, C)
+#define PLK_STEPS                                                                                \
+    [s0] "v"(counts.step[0]), [s1] "v"(counts.step[1]), [s2] "v"(counts.step[2]),                \
+        [s3] "v"(counts.step[3]), [s4] "v"(counts.step[4]), [s5] "v"(counts.step[5])
+    if constexpr (C == 2)
+        asm volatile(PLK_SUM_STEPS(PLK_ADD2) : "+v"(x[0]), "+v"(x[1]) : PLK_STEPS);
+    else if constexpr (C == 3)
+        asm volatile(PLK_SUM_STEPS(PLK_ADD3) : "+v"(x[0]), "+v"(x[1]), "+v"(x[2]) : PLK_STEPS);
+    else
+        asm volatile(PLK_SUM_STEPS(PLK_ADD4) : "+v"(x[0]), "+v"(x[1]), "+v"(x[2]), "+v"(x[3]) : PLK_STEPS);
+#undef PLK_ADD_LANE
+#undef PLK_SUM_STEPS
+#undef PLK_ADD2
+#undef PLK_ADD3
+#undef PLK_ADD4
+#undef PLK_STEPS
+}
+// (doubles: the other lane's in two moves)
+template <int CTRL, int ROW_MASK, int C>
+__device__ __forceinline__ void add_lane_f64(double (&x)[C], float counts) {
+#pragma unroll
+    for (int j = 0; j < C; ++j) {
+        const int lo = __builtin_amdgcn_update_dpp(0, __double2loint(x[j]), CTRL, ROW_MASK, 0xf, true);
+        const int hi = __builtin_amdgcn_update_dpp(0, __double2hiint(x[j]), CTRL, ROW_MASK, 0xf, true);
+        x[j] = __builtin_fma(__hiloint2double(hi, lo), (double)counts, x[j]);
+    }
+}
+template <int C>
+__device__ __forceinline__ void sum_groups_in_order(double (&x)[C], const StepsCount &counts) {
+    add_lane_f64<0x111, 0xf>(x, counts.step[0]);   // row_shr:1, 2, 4, 8
+    add_lane_f64<0x112, 0xf>(x, counts.step[1]);
+    add_lane_f64<0x114, 0xf>(x, counts.step[2]);
+    add_lane_f64<0x118, 0xf>(x, counts.step[3]);
+    add_lane_f64<0x142, 0xa>(x, counts.step[4]);   // row_bcast:15 (rows 1 and 3), row_bcast:31 (rows 2 and 3)
+    add_lane_f64<0x143, 0xc>(x, counts.step[5]);
 }
 
 // What a build counts in, as the build after next must find it

@@ -508,13 +508,9 @@ __global__ __launch_bounds__(kBlock) void k_build_tile(PointFeatures features, P
     if (valid && !in_range) atomicOr(&counters->flags, kFlagKeyRange);
     const bool active = valid && in_range;
 
-    unsigned leaders[(D1 + 4) / 5] = {};
-    auto leader_of = [&](int r) { return (int)((leaders[r / 5] >> (6 * (r % 5))) & 63u); };
+    unsigned group[D1];     // the lanes that hold the same key r, put in order (SPLAT_VD), and their leader
     int slot[D1];           // the LDS slot of key r, at first in the lanes of the leaders only
-    // Groups of a few lanes add their terms to the slot's row one by one; the tree that sums a
-    // group costs the same for two lanes as for sixty-four, and half the groups have four or fewer.
-    constexpr int kSmallGroup = SPLAT_VD ? 4 : 0;
-    uint64_t small[D1];
+    const uint64_t among = wave_ballot(active);
     __syncthreads();        // the LDS table is empty
     {
         uint64_t key[D1];
@@ -522,9 +518,11 @@ __global__ __launch_bounds__(kBlock) void k_build_tile(PointFeatures features, P
         vertex_keys_of<PD>(s, key);
 #pragma unroll
         for (int r = 0; r < D1; ++r) {
-            const int leader = wave_leader_of_equal(key[r], active, lane, kSmallGroup, small[r]);
-            leaders[r / 5] |= (unsigned)leader << (6 * (r % 5));
-            if (active && leader == lane) open |= 1u << r;
+            if constexpr (SPLAT_VD != 0)
+                group[r] = wave_groups_in_order(key[r], among);
+            else
+                group[r] = (unsigned)wave_leader_of_equal(key[r], active, lane) << 16;
+            if (active && leader_of(group[r]) == lane) open |= 1u << r;
             static_assert(kTileSlots == 1 << (32 - kTileSlotShift), "the slot is the hash's high bits");
             slot[r] = (int)(hash_key(key[r]) >> kTileSlotShift);
         }
@@ -564,44 +562,53 @@ __global__ __launch_bounds__(kBlock) void k_build_tile(PointFeatures features, P
                 if (j < in_channels) val[j] = input[(size_t)n * in_channels + j];
         }
     }
+    // (what sum_groups_in_order asks of its terms: the wavefront's values and weights finite and, as
+    // the weights are at most one, their sums far from overflowing; a NaN fails the comparison)
+    bool tame = true;
+    if (SPLAT_VD) {
+        T all = (T)0;
+#pragma unroll
+        for (int r = 0; r < D1; ++r) all += s.weight[r];
+#pragma unroll
+        for (int j = 0; j < VD; ++j) all += val[j] < (T)0 ? -val[j] : val[j];
+        tame = wave_ballot(!(all < (kDouble ? (T)1e290 : (T)1e30))) == 0;
+    }
 #pragma unroll
     for (int r = 0; r < D1; ++r) {
-        const int leader = leader_of(r);
-        const int own = slot[r];
-        slot[r] = active ? __shfl(own, leader) : -1;
-        if (SPLAT_VD) {
-            const T w = s.weight[r];
-            const T term[4] = {w * val[0], w * val[1], w * val[2], w * val[3]};
-            const uint64_t among = wave_ballot(active) & ~small[r];
-            uint64_t remaining = among;
-            if constexpr (kDouble) {
-                while (remaining) {
-                    const int first = __builtin_ctzll(remaining);
-                    const uint64_t group = lanes_equal(leader, first) & among;
-                    remaining &= ~group;
-                    const int group_slot = lane_value(own, first);
-                    const double sum = wave_sums_to_quads_f64(lane_in(group), term, lane);
-                    if (group_slot >= 0 && lane < 4 && channel_of_quad_lane(lane) < VD)
-                        atomicAdd(&slot_sum[group_slot * P + channel_of_quad_lane(lane)], sum);
-                }
-            } else {
-                const QuadTerms quad = quad_terms<VD>(term, lane);
-                // (one group per turn: two side by side, to overlap their chains of cross-lane
-                // additions, cost more for the odd group out than they gain)
-                while (remaining) {
-                    const int first = __builtin_ctzll(remaining);
-                    const uint64_t group = lanes_equal(leader, first) & among;
-                    remaining &= ~group;
-                    const bool same = lane_in(group);
-                    const int group_slot = lane_value(own, first);
-                    const float sum = wave_sum_to_last_lanes<VD>(same, quad, lane);
-                    if (group_slot >= 0 && lane >= 64 - P && channel_of_lane<VD>(lane) < VD)
-                        atomicAdd(&slot_sum[group_slot * P + channel_of_lane<VD>(lane)], sum);
-                }
-            }
-            if (lane_in(small[r]) && slot[r] >= 0) {
+        const int of_group = __shfl(slot[r], leader_of(group[r]));
+        slot[r] = active ? of_group : -1;
+    }
+    if (SPLAT_VD && tame) {
+        // The lanes in the order of their groups, the groups summed side by side; the last lane of
+        // each adds the sums to the slot's row.  About 45 vector instructions a corner, however many
+        // groups it has, where a tree of 26 for each group above four lanes and LDS additions lane by
+        // lane for the rest were about 95 (the kernel is bound by its vector and scalar instructions:
+        // a filter of 1024x1024 points, pd 5, vd 4, 123 and 115 us; 128x256x256 voxels, pd 4, vd 2, 506
+        // and 482; 601x803 points in doubles 102 and 97).
+        unsigned where[D1];   // of the lane at a place: the slot and the first place of its group
 #pragma unroll
-                for (int j = 0; j < VD; ++j) atomicAdd(&slot_sum[slot[r] * P + j], term[j]);
+        for (int r = 0; r < D1; ++r)
+            where[r] = (unsigned)to_place(place_of(group[r]),
+                                          (int)((unsigned)slot[r] << 20 | (unsigned)first_place_of(group[r])));
+#pragma unroll
+        for (int r = 0; r < D1; ++r) {
+            T term[VD];
+#pragma unroll
+            for (int j = 0; j < VD; ++j) term[j] = to_place(place_of(group[r]), s.weight[r] * val[j]);
+            sum_groups_in_order(term, steps_that_count(lane, (int)(where[r] & 0xffu)));
+            // (wave_shl:1, nothing above lane 63)
+            const unsigned above = (unsigned)__builtin_amdgcn_update_dpp(-1, (int)where[r], 0x130, 0xf, 0xf, false);
+            if (above != where[r] && where[r] < 0xfff00000u) {
+#pragma unroll
+                for (int j = 0; j < VD; ++j) atomicAdd(&slot_sum[(where[r] >> 20) * P + j], term[j]);
+            }
+        }
+    } else if (SPLAT_VD) {
+#pragma unroll
+        for (int r = 0; r < D1; ++r) {
+            if (slot[r] >= 0) {
+#pragma unroll
+                for (int j = 0; j < VD; ++j) atomicAdd(&slot_sum[slot[r] * P + j], s.weight[r] * val[j]);
             }
         }
     }
