@@ -1125,6 +1125,7 @@ int features_from_image(pl_lattice *h, const float *reference, int n_reference_c
     f.feature_std = feature_std;
     for (int i = 0; i < plk::kMaxSpatialDims; ++i) f.dims.v[i] = 1;
     for (int i = 0; i < n_spatial_dims; ++i) f.dims.v[i] = spatial_dims[i];
+    plk::set_inverse_widths(f);
     if (n_spatial_dims > 0) {
         // also checks that the extents are positive and that their product is N
         const int rc = pl_set_point_grid(h, n_spatial_dims, spatial_dims);

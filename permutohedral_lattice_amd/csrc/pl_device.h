@@ -214,11 +214,29 @@ struct Simplex {
     T weight[PD + 1];
 };
 
+// (float)((double)x * (1.0 / D1)), the reference's expression, in two single-precision operations: the
+// product with 1/D1 as the float below it and the rest, rounded once.  The error before that rounding
+// is some 2^-48 of the result, and no quotient by D1's odd factor comes closer than 1/18 ulp to the middle
+// between two floats (compared for all 2^23 mantissas and D1 = 2..9; |x| at least 2^-90 or 0).
+template <int D1>
+__device__ __forceinline__ float scaled_down(float x) {
+    constexpr double inverse = 1.0 / (double)D1;
+    if constexpr ((D1 & (D1 - 1)) == 0) {
+        return x * (float)inverse;
+    } else {
+        // (the rest is positive: an infinite x stays infinite)
+        constexpr float nearest = (float)inverse;
+        constexpr float below = (double)nearest > inverse
+                                    ? __builtin_bit_cast(float, __builtin_bit_cast(uint32_t, nearest) - 1u) : nearest;
+        constexpr float rest = (float)(inverse - (double)below);
+        return __builtin_fmaf(x, below, x * rest);
+    }
+}
+
 template <int PD>
 __device__ __forceinline__ void enclosing_simplex(const float (&pos)[PD], const ScaleFactor &scale,
                                                   Simplex<PD> &s) {
     constexpr int D1 = PD + 1;
-    const double inv_d1 = 1.0 / (double)D1;
 
     // elevate onto the hyperplane sum(x) = 0 (float, unfused)
     float el[D1];
@@ -240,7 +258,7 @@ __device__ __forceinline__ void enclosing_simplex(const float (&pos)[PD], const 
         // (The reference rounds between ceil(v) and floor(v) times pd+1.  The ceiling is the
         // floor plus one unless v is whole, and then both of its candidates are the same point:
         // one step above the floor's multiple decides the same, without a second rounding.)
-        const float v = (float)((double)el[i] * inv_d1);
+        const float v = scaled_down<D1>(el[i]);
         const float fl = floorf(v);
         const float below = fl * (float)D1, above = below + (float)D1;
         const bool up = (above - el[i]) < (el[i] - below);
@@ -269,13 +287,15 @@ __device__ __forceinline__ void enclosing_simplex(const float (&pos)[PD], const 
             rk[j] -= lt;
         }
     }
-    // ranks that left 0..pd wrap round, and their coordinate moves one step
+    // ranks that left 0..pd wrap round, and their coordinate moves one step (all the same way)
+    const int step = qsum < 0 ? 1 : -1;
+    const float step_rem = qsum < 0 ? (float)D1 : -(float)D1;
 #pragma unroll
     for (int i = 0; i < D1; ++i) {
-        const int step = rk[i] < 0 ? 1 : (rk[i] > PD ? -1 : 0);
-        s.rank[i] = rk[i] + step * D1;
-        s.q[i] += step;
-        rem[i] += (float)(step * D1);
+        const bool wraps = (unsigned)rk[i] > (unsigned)PD;
+        s.rank[i] = rk[i] + (wraps ? step * D1 : 0);
+        s.q[i] += wraps ? step : 0;
+        rem[i] += wraps ? step_rem : 0.0f;
     }
 
     // barycentric weights.  by_rank[k] is the scaled residual of the coordinate of rank k; the
@@ -286,7 +306,7 @@ __device__ __forceinline__ void enclosing_simplex(const float (&pos)[PD], const 
     // residuals are equal in either place.  Sorted by a network of compare-and-swaps.
     float by_rank[D1];
 #pragma unroll
-    for (int i = 0; i < D1; ++i) by_rank[i] = (float)((double)(el[i] - rem[i]) * inv_d1);
+    for (int i = 0; i < D1; ++i) by_rank[i] = scaled_down<D1>(el[i] - rem[i]);
     sort_descending<D1>(by_rank);
 #pragma unroll
     for (int k = 1; k < D1; ++k) s.weight[k] = by_rank[PD - k] - by_rank[PD - k + 1];
@@ -431,7 +451,9 @@ __device__ __forceinline__ void wide_keys_of(const Simplex<PD, T> &s, Key128 (&k
 // consecutive points.  The mapping only changes the order of work, never a result.
 // Per-point scratch (the replay arrays) is stored in thread order, so it stays coalesced.
 // ------------------------------------------------------------------------------------------------
-__device__ __forceinline__ int point_of_thread(const PointMap &m, unsigned vblock, unsigned tid) {
+// at: the point's grid coordinates as the map has them, slowest first (modes 2 and 3; else zeros).
+__device__ __forceinline__ int point_of_thread(const PointMap &m, unsigned vblock, unsigned tid, int (&at)[3]) {
+    at[0] = at[1] = at[2] = 0;
     if (m.mode == 0) {
         const size_t n = (size_t)vblock * kBlock + tid;
         return n < (size_t)m.N ? (int)n : -1;
@@ -443,9 +465,9 @@ __device__ __forceinline__ int point_of_thread(const PointMap &m, unsigned vbloc
     }
     const unsigned wave = tid >> 6, lane = tid & 63;
     const unsigned tiles_yx = (unsigned)m.tiles[1] * (unsigned)m.tiles[2];
-    const unsigned tz = vblock / tiles_yx;
+    const unsigned tz = m.mode == 2 ? 0u : m.by_tiles_yx(vblock);
     const unsigned rest = vblock - tz * tiles_yx;
-    const unsigned ty = rest / (unsigned)m.tiles[2];
+    const unsigned ty = m.by_tiles_x(rest);
     const unsigned tx = rest - ty * (unsigned)m.tiles[2];
     unsigned z, y, x;
     if (m.mode == 2) {
@@ -458,7 +480,14 @@ __device__ __forceinline__ int point_of_thread(const PointMap &m, unsigned vbloc
         x = tx * 8 + (wave & 1) * 4 + (lane & 3);
     }
     if (z >= (unsigned)m.dims[0] || y >= (unsigned)m.dims[1] || x >= (unsigned)m.dims[2]) return -1;
+    at[0] = (int)z;
+    at[1] = (int)y;
+    at[2] = (int)x;
     return (int)(((size_t)z * m.dims[1] + y) * m.dims[2] + x);
+}
+__device__ __forceinline__ int point_of_thread(const PointMap &m, unsigned vblock, unsigned tid) {
+    int at[3];
+    return point_of_thread(m, vblock, tid, at);
 }
 
 // The share of the points this workgroup takes (vblock; each XCD a contiguous range of shares when
@@ -477,6 +506,16 @@ __device__ __forceinline__ bool block_of_points(const PointMap &m, int xcd_aware
     }
     vblock = xcd_contiguous_block(blockIdx.x, nb, xcd_aware);
     return true;
+}
+
+// a / b, correctly rounded as the division is, from inverse = 1 / b, itself correctly rounded: two steps
+// of Markstein's correction (P. Markstein, IBM J. Res. Dev. 34 (1990): the first leaves the quotient within
+// an ulp, the second rounds it right).  For a of a size whose remainder does not leave the number range,
+// b as FeatureWidths allows it.
+__device__ __forceinline__ float divided(float a, float b, float inverse) {
+    float q = a * inverse;
+    q = __builtin_fmaf(__builtin_fmaf(-q, b, a), inverse, q);
+    return __builtin_fmaf(__builtin_fmaf(-q, b, a), inverse, q);
 }
 
 // Mask of the lanes whose predicate holds (the compare result itself, no detour through 0/1)
@@ -548,64 +587,85 @@ __device__ __forceinline__ int wave_leader_of_equal(T x, bool active, int lane) 
     }
     return leader;
 }
-// The groups of lanes that hold the same value of `x`, as an order of the lanes in which every group's
-// are next to each other.  Per lane: its place in that order (bits 0..7), the place of its group's
-// first lane (8..15), and that lane, the lowest of the group (16..23).  The lanes outside `among` come
-// last, each a group of its own.  All 64 lanes must call it.
-template <typename T>
-__device__ __forceinline__ unsigned wave_groups_in_order(T x, uint64_t among) {
-    unsigned own = 0, filled = 0;   // filled: how many lanes are placed, in both of the low bytes
-    uint64_t remaining = among;
-    while (remaining) {
-        const int first = __builtin_ctzll(remaining);
-        const uint64_t same = lanes_equal(x, lane_value(x, first)) & remaining;
-        const unsigned rank = __builtin_amdgcn_mbcnt_hi((uint32_t)(same >> 32),
-                                                        __builtin_amdgcn_mbcnt_lo((uint32_t)same, 0u));
-        // (one addition under a narrowed exec mask, as in set_in_lanes)
+// The groups of lanes that hold the same value of `x`, numbered from *n_groups on, which counts them, and
+// an order of the lanes in which every group's are next to each other.  Per lane: the number of its group
+// (bits 0..9), its rank in it (10..16; the lowest lane 0) and its place in the order (17..23).  The lanes
+// outside `among` come last, each with rank 0.  All 64 lanes must call it.
+// Written out: a wavefront's forty turns are a chain of scalar and vector instructions that wait for each
+// other, the longest stretch of the build.  exec holds the lanes still to be found, so that
+// v_readfirstlane gives the next group's value (its two words are used two instructions later, as
+// registers written by a vector instruction must be); s_lshl_b32 leaves in scc whether there was a group
+// to count.  A turn without a lane left changes nothing, so turns go in pairs.  Cycles a turn, alone on
+// the SIMD or with seven other wavefronts: the compiler's loop 178, this 93 (one turn at a time 111, with
+// s_ff1_i32_b64 and v_readlane 130; two lists side by side 93 a turn: it is the number of instructions).
+__device__ __forceinline__ unsigned wave_groups_in_order(uint64_t x, uint64_t among, unsigned *n_groups) {
+    unsigned own = 0;
+    unsigned filled = *n_groups;   // the number of the next group, and (from bit 17) how many lanes are placed
+    if (among != 0) {
+        uint64_t left, same;
+        unsigned count, rank;
+#define PLK_FIND_GROUP                                         \
+    "v_readfirstlane_b32 vcc_lo, %[lo]\n\t"                    \
+    "v_readfirstlane_b32 vcc_hi, %[hi]\n\t"                    \
+    "s_nop 1\n\t"                                              \
+    "v_cmp_eq_u64_e64 %[same], vcc, %[x]\n\t"                  \
+    "s_and_saveexec_b64 %[left], %[same]\n\t"                  \
+    "v_mbcnt_lo_u32_b32 %[rank], exec_lo, 0\n\t"               \
+    "v_mbcnt_hi_u32_b32 %[rank], exec_hi, %[rank]\n\t"         \
+    "v_mad_u32_u24 %[own], %[rank], %[both], %[filled]\n\t"    \
+    "s_bcnt1_i32_b64 %[count], %[same]\n\t"                    \
+    "s_lshl_b32 %[count], %[count], 17\n\t"                    \
+    "s_addc_u32 %[filled], %[filled], %[count]\n\t"            \
+    "s_andn2_b64 exec, %[left], %[same]\n\t"
         asm volatile(
-            "s_mov_b64 exec, %2\n\t"
-            "v_add_u32_e32 %0, %3, %1\n\t"
+            "s_mov_b64 exec, %[among]\n"
+            "1:\n\t"
+            PLK_FIND_GROUP
+            PLK_FIND_GROUP
+            "s_cbranch_execnz 1b\n\t"
             "s_mov_b64 exec, -1"
-            : "+v"(own)
-            : "v"(rank), "s"(same), "s"(filled + ((unsigned)first << 16)));
-        filled += (unsigned)lanes_in(same) * 0x101u;
-        remaining &= ~same;
+            : [own] "+v"(own), [filled] "+s"(filled), [left] "=&s"(left), [same] "=&s"(same),
+              [count] "=&s"(count), [rank] "=&v"(rank)
+            : [x] "v"(x), [lo] "v"((uint32_t)x), [hi] "v"((uint32_t)(x >> 32)), [among] "s"(among),
+              [both] "v"((1u << 10) + (1u << 17))
+            : "vcc", "scc");
+#undef PLK_FIND_GROUP
     }
+    *n_groups = filled & 0x3ffu;
     if (among != ~0ull) {
         const uint64_t rest = ~among;
         const unsigned rank = __builtin_amdgcn_mbcnt_hi((uint32_t)(rest >> 32),
                                                         __builtin_amdgcn_mbcnt_lo((uint32_t)rest, 0u));
-        if (lane_in(rest)) own = filled + rank * 0x101u;
+        if (lane_in(rest)) own = (filled & ~0x1ffffu) + (rank << 17);
     }
     return own;
 }
-__device__ __forceinline__ int place_of(unsigned group) { return (int)(group & 0xffu); }
-__device__ __forceinline__ int first_place_of(unsigned group) { return (int)((group >> 8) & 0xffu); }
-__device__ __forceinline__ int leader_of(unsigned group) { return (int)(group >> 16); }
+__device__ __forceinline__ unsigned number_of(unsigned group) { return group & 0x3ffu; }
+__device__ __forceinline__ unsigned rank_of(unsigned group) { return (group >> 10) & 0x7fu; }
 
-// x of the lane that has place `lane` in the order (each lane gives its own place)
-__device__ __forceinline__ int to_place(int place, int x) {
-    return __builtin_amdgcn_ds_permute(place << 2, x);
+// x of the lane whose place in the order (of its own `group`) is this lane.  (The address of ds_permute
+// is the lane times four; the bits below are not looked at, and those above are zero.)
+__device__ __forceinline__ int to_place(unsigned group, int x) {
+    return __builtin_amdgcn_ds_permute((int)(group >> 15), x);
 }
-__device__ __forceinline__ float to_place(int place, float x) {
-    return __int_as_float(to_place(place, __float_as_int(x)));
+__device__ __forceinline__ float to_place(unsigned group, float x) {
+    return __int_as_float(to_place(group, __float_as_int(x)));
 }
-__device__ __forceinline__ double to_place(int place, double x) {
-    return __hiloint2double(to_place(place, __double2hiint(x)), to_place(place, __double2loint(x)));
+__device__ __forceinline__ double to_place(unsigned group, double x) {
+    return __hiloint2double(to_place(group, __double2hiint(x)), to_place(group, __double2loint(x)));
 }
 
-// The lanes being in the order above, and first_place the place of a lane's group's first: x := the
-// sum of x over the lanes of the group up to this one, so that the last lane of every group holds the
-// group's sum.  Six steps for all groups of the wavefront together: the lane 1, 2, 4, 8 below in the
+// The lanes being in the order above, and rank a lane's rank in its group: x := the sum of x over the
+// lanes of the group up to this one, so that the last lane of every group holds the group's sum.  Six steps for all groups of the wavefront together: the lane 1, 2, 4, 8 below in the
 // row of 16, the last lane of the row below, the last lane of the lower half, each added where it is
 // of the same group.  The terms must be finite and far from overflowing (what does not count is
 // multiplied by 0, so that a step is one instruction per channel).  All 64 lanes must call it.
 struct StepsCount {
     float step[6];   // 1 where the lane a step looks at is of this lane's group, else 0
 };
-__device__ __forceinline__ StepsCount steps_that_count(int lane, int first_place) {
-    float before = (float)(lane - first_place);   // lanes of the group before this one
-    asm("" : "+v"(before));                       // (a float from here on: one instruction a step)
+__device__ __forceinline__ StepsCount steps_that_count(int lane, unsigned rank) {
+    float before = (float)rank;   // lanes of the group before this one
+    asm("" : "+v"(before));       // (a float from here on: one instruction a step)
     auto zero_to_one = [](float x) { return __builtin_amdgcn_fmed3f(x, 0.0f, 1.0f); };
     return StepsCount{{zero_to_one(before), zero_to_one(before - 1.0f), zero_to_one(before - 3.0f),
                        zero_to_one(before - 7.0f), zero_to_one(before - (float)(lane & 15)),

@@ -177,7 +177,18 @@ struct PointFeatures {
     int n_spatial_dims, n_reference_channels;
     SpatialDims dims;         // slowest first, the last runs fastest
     float spatial_std, feature_std;
+    // their reciprocals, and whether the kernels may divide by multiplying with them (set_inverse_widths)
+    float inverse_spatial_std, inverse_feature_std;
+    int multiply;
 };
+// Widths of 2^-40 .. 2^40: quotients and remainders of coordinates, and of channels below 2^80, are then
+// ordinary numbers.  (A channel below 2^-100 may be an ulp off.)
+inline void set_inverse_widths(PointFeatures &f) {
+    auto ordinary = [](float x) { return (x < 0.0f ? -x : x) >= 0x1p-40f && (x < 0.0f ? -x : x) <= 0x1p40f; };
+    f.multiply = (f.n_spatial_dims == 0 || ordinary(f.spatial_std)) && (f.n_reference_channels == 0 || ordinary(f.feature_std));
+    f.inverse_spatial_std = f.multiply && f.n_spatial_dims ? 1.0f / f.spatial_std : 0.0f;
+    f.inverse_feature_std = f.multiply && f.n_reference_channels ? 1.0f / f.feature_std : 0.0f;
+}
 
 // How threads are laid over the points (see point_of_thread in pl_kernels.hip).
 struct PointMap {
@@ -192,6 +203,12 @@ struct PointMap {
     // (in device memory: the launch is enqueued before the order is known)
     const int *order;
     const unsigned *n_tiles;
+    // x / tiles[2] and x / (tiles[1] * tiles[2]) as a product and a shift (make_point_map)
+    struct Divisor {
+        uint64_t factor;
+        unsigned shift;
+        __host__ __device__ unsigned operator()(unsigned x) const { return (unsigned)((x * factor) >> shift); }
+    } by_tiles_x, by_tiles_yx;
 };
 
 // Where feature 0 of the first and of the last point can be read (one of the two pointers, or

@@ -43,34 +43,62 @@ __device__ __forceinline__ void load_position(const float *positions, int n, flo
 // The feature vector from a positions array, or built on the fly exactly as k_positions builds it
 // (reference: src/PermutohedralLatticeCPU.h:464-473): IEEE float division of the grid coordinate
 // and of the reference channels.
+// On a grid of up to three extents the coordinates are the point map's, and the divisions are
+// multiplications that round the same (divided): with the coordinates taken out of the point's number by
+// integer divisions and the features divided the build of 128x256x256 voxels executed 1101 vector
+// instructions per wavefront, with this 1014 (489 and 484 us a filter).
 template <int PD>
-__device__ __forceinline__ void load_features(const PointFeatures &f, int n, float (&pos)[PD]) {
+__device__ __forceinline__ void load_features(const PointFeatures &f, const PointMap &map, int n,
+                                              const int (&at)[3], float (&pos)[PD]) {
     if (f.positions) {
         load_position<PD>(f.positions, n, pos);
         return;
     }
-    int rest = n;
-#pragma unroll
-    for (int i = PD - 1; i >= 0; --i) {
-        if (i < f.n_spatial_dims) {
-            const int next = rest / f.dims.v[i];
-            pos[i] = (float)(rest - next * f.dims.v[i]) / f.spatial_std;
-            rest = next;
-        }
-    }
+    float channel[PD];
     if (f.n_reference_channels > 0) {
         // (every channel is asked for at once, from an element that exists, and taken or not
         // afterwards: loads behind the condition would wait for one another)
         const float *row = f.reference + (size_t)n * f.n_reference_channels;
-        float channel[PD];
 #pragma unroll
         for (int i = 0; i < PD; ++i) {
             const int j = i - f.n_spatial_dims;
             channel[i] = row[j >= 0 && j < f.n_reference_channels ? j : 0];
         }
+    }
+    const bool quick = f.multiply && map.mode >= 2 && f.n_spatial_dims <= 3;
+    if (quick) {
+        // (a grid has at least two extents)
+        const float z = divided((float)at[0], f.spatial_std, f.inverse_spatial_std);
+        const float y = divided((float)at[1], f.spatial_std, f.inverse_spatial_std);
+        const float x = divided((float)at[2], f.spatial_std, f.inverse_spatial_std);
+        pos[0] = f.n_spatial_dims == 3 ? z : y;
+        if constexpr (PD >= 2) pos[1] = f.n_spatial_dims == 3 ? y : x;
+        if constexpr (PD >= 3) pos[2] = x;
+    } else {
+        int rest = n;
 #pragma unroll
-        for (int i = 0; i < PD; ++i)
-            if (i >= f.n_spatial_dims) pos[i] = channel[i] / f.feature_std;
+        for (int i = PD - 1; i >= 0; --i) {
+            if (i < f.n_spatial_dims) {
+                const int next = rest / f.dims.v[i];
+                pos[i] = (float)(rest - next * f.dims.v[i]) / f.spatial_std;
+                rest = next;
+            }
+        }
+    }
+    if (f.n_reference_channels > 0) {
+#pragma unroll
+        for (int i = 0; i < PD; ++i) {
+            if (i >= f.n_spatial_dims) {
+                if (quick) {
+                    // (a quotient that is none, infinite or far beyond any lattice stays what it is)
+                    const float q = channel[i] * f.inverse_feature_std;
+                    pos[i] = __builtin_fabsf(q) < 0x1p80f
+                                 ? divided(channel[i], f.feature_std, f.inverse_feature_std) : q;
+                } else {
+                    pos[i] = channel[i] / f.feature_std;
+                }
+            }
+        }
     }
 }
 
@@ -207,7 +235,8 @@ __global__ __launch_bounds__(kBlock) void k_build(PointFeatures features, PointM
     const unsigned vblock = xcd_contiguous_block(blockIdx.x, gridDim.x, xcd_aware);
     const size_t t = (size_t)vblock * kBlock * D1 + threadIdx.x;   // slot in the replay arrays
     constexpr size_t n_slots = kBlock;
-    const int n = point_of_thread(map, vblock, threadIdx.x);
+    int at[3];
+    const int n = point_of_thread(map, vblock, threadIdx.x, at);
     const int lane = threadIdx.x & 63;
     const bool valid = n >= 0;
 
@@ -221,7 +250,7 @@ __global__ __launch_bounds__(kBlock) void k_build(PointFeatures features, PointM
         float pos[PD];
 #pragma unroll
         for (int i = 0; i < PD; ++i) pos[i] = 0.0f;
-        if (valid) load_features<PD>(features, n, pos);
+        if (valid) load_features<PD>(features, map, n, at, pos);
         enclosing_simplex<PD>(pos, scale, s);
     }
 
@@ -443,8 +472,9 @@ __global__ __launch_bounds__(kBlock) void k_build(PointFeatures features, PointM
 static_assert(kTileSlots == 2 * kBlock, "a thread places at most two slots in the table");
 constexpr int kTileProbeLimit = 48;
 
+// (at most 102 scalar registers: with more a SIMD holds seven wavefronts, not eight)
 template <int PD, int SPLAT_VD, typename T = float>
-__global__ __launch_bounds__(kBlock) void k_build_tile(PointFeatures features, PointMap map,
+__global__ __launch_bounds__(kBlock) __attribute__((amdgpu_num_sgpr(102))) void k_build_tile(PointFeatures features, PointMap map,
                                                         ScaleFactor scale, uint64_t *cell_keys,
                                                         uint32_t mask, Counters *counters,
                                                         ReplayEntry *__restrict__ replay,
@@ -474,6 +504,7 @@ __global__ __launch_bounds__(kBlock) void k_build_tile(PointFeatures features, P
     __shared__ unsigned short slot_rank[kTileSlots];
     constexpr unsigned short kNotCreated = 0xffffu;
     __shared__ int group_created;
+    __shared__ uint64_t group_keys[kBlock / 64][64];
     const int tid = threadIdx.x;
     for (int i = tid; i < kTileSlots; i += kBlock) slot_key[i] = kEmptyCell;
     if (SPLAT_VD)
@@ -485,7 +516,8 @@ __global__ __launch_bounds__(kBlock) void k_build_tile(PointFeatures features, P
 
     const size_t t = (size_t)vblock * kBlock * D1 + tid;   // slot in the replay arrays
     constexpr size_t n_slots = kBlock;
-    const int n = point_of_thread(map, vblock, tid);
+    int at[3];
+    const int n = point_of_thread(map, vblock, tid, at);
     const int lane = tid & 63;
     const bool valid = n >= 0;
 
@@ -499,7 +531,7 @@ __global__ __launch_bounds__(kBlock) void k_build_tile(PointFeatures features, P
         float pos[PD];
 #pragma unroll
         for (int i = 0; i < PD; ++i) pos[i] = 0.0f;
-        if (valid) load_features<PD>(features, n, pos);
+        if (valid) load_features<PD>(features, map, n, at, pos);
         enclosing_simplex<PD>(pos, scale, s);
     }
 #pragma unroll
@@ -508,48 +540,62 @@ __global__ __launch_bounds__(kBlock) void k_build_tile(PointFeatures features, P
     if (valid && !in_range) atomicOr(&counters->flags, kFlagKeyRange);
     const bool active = valid && in_range;
 
-    unsigned group[D1];     // the lanes that hold the same key r, put in order (SPLAT_VD), and their leader
-    int slot[D1];           // the LDS slot of key r, at first in the lanes of the leaders only
+    unsigned group[D1];     // the lanes that hold the same key r, numbered and put in order
+    int slot[D1];           // the LDS slot of key r
     const uint64_t among = wave_ballot(active);
     __syncthreads();        // the LDS table is empty
     {
         uint64_t key[D1];
-        unsigned open = 0;
+        unsigned n_groups = 0;      // of the wavefront, all corners counted through
         vertex_keys_of<PD>(s, key);
 #pragma unroll
-        for (int r = 0; r < D1; ++r) {
-            if constexpr (SPLAT_VD != 0)
-                group[r] = wave_groups_in_order(key[r], among);
-            else
-                group[r] = (unsigned)wave_leader_of_equal(key[r], active, lane) << 16;
-            if (active && leader_of(group[r]) == lane) open |= 1u << r;
-            static_assert(kTileSlots == 1 << (32 - kTileSlotShift), "the slot is the hash's high bits");
-            slot[r] = (int)(hash_key(key[r]) >> kTileSlotShift);
-        }
-        bool any_open = open != 0;
-        for (int probe = 0; any_open && probe < kTileProbeLimit; ++probe) {
+        for (int r = 0; r < D1; ++r) group[r] = wave_groups_in_order(key[r], among, &n_groups);
+        // The leaders' keys go to lane after lane of the wavefront, whatever corner they are of (an
+        // image's 8x8 pixels have about forty), and every lane places one in the table, where a lane
+        // with a leader for each of its corners would place up to pd+1, one behind the other; the
+        // slots come back the same way.  (More than 64 groups: 64 at a time.)
+        uint64_t *wave_keys = group_keys[tid >> 6];
+        int *wave_slots = reinterpret_cast<int *>(wave_keys);
+#pragma unroll
+        for (int r = 0; r < D1; ++r) slot[r] = -1;
+        for (unsigned from = 0; from < n_groups; from += 64) {
 #pragma unroll
             for (int r = 0; r < D1; ++r) {
-                if ((open >> r) & 1u) {
-                    const uint64_t seen =
-                        atomicCAS((unsigned long long *)&slot_key[slot[r]],
-                                  (unsigned long long)kEmptyCell, (unsigned long long)key[r]);
-                    if (seen == kEmptyCell || seen == key[r]) {
-                        open &= ~(1u << r);
-                        // the slot was empty: it joins the list of slots in use
-                        if (seen == kEmptyCell)
-                            occupied[atomicAdd(&n_occupied, 1)] = (unsigned short)slot[r];
-                    } else {
-                        slot[r] = (slot[r] + 1) & (kTileSlots - 1);
-                    }
+                const unsigned to = number_of(group[r]) - from;
+                if (active && rank_of(group[r]) == 0 && to < 64u) wave_keys[to] = key[r];
+            }
+            __builtin_amdgcn_wave_barrier();
+            const uint64_t mine = wave_keys[lane];
+            static_assert(kTileSlots == 1 << (32 - kTileSlotShift), "the slot is the hash's high bits");
+            int at_slot = (int)(hash_key(mine) >> kTileSlotShift);
+            bool open = from + (unsigned)lane < n_groups, was_empty = false;
+            if (!open) at_slot = -1;
+            for (int probe = 0; open && probe < kTileProbeLimit; ++probe) {
+                const uint64_t seen = atomicCAS((unsigned long long *)&slot_key[at_slot],
+                                                (unsigned long long)kEmptyCell, (unsigned long long)mine);
+                if (seen == kEmptyCell || seen == mine) {
+                    open = false;
+                    was_empty = seen == kEmptyCell;
+                } else {
+                    at_slot = (at_slot + 1) & (kTileSlots - 1);
                 }
             }
-            any_open = open != 0;
-        }
-        if (any_open) atomicOr(&counters->flags, kFlagTileFull);
+            if (open) {
+                atomicOr(&counters->flags, kFlagTileFull);
+                at_slot = -1;
+            }
+            __builtin_amdgcn_wave_barrier();
+            wave_slots[2 * lane] = at_slot;
+            __builtin_amdgcn_wave_barrier();
 #pragma unroll
-        for (int r = 0; r < D1; ++r)
-            if ((open >> r) & 1u) slot[r] = -1;
+            for (int r = 0; r < D1; ++r) {
+                const unsigned to = number_of(group[r]) - from;
+                if (active && to < 64u) slot[r] = wave_slots[2 * to];
+            }
+            // the slots that were empty join the list of slots in use
+            if (was_empty) occupied[atomicAdd(&n_occupied, 1)] = (unsigned short)at_slot;
+            __builtin_amdgcn_wave_barrier();
+        }
     }
 
     T val[4] = {(T)0, (T)0, (T)0, (T)0};
@@ -573,32 +619,25 @@ __global__ __launch_bounds__(kBlock) void k_build_tile(PointFeatures features, P
         for (int j = 0; j < VD; ++j) all += val[j] < (T)0 ? -val[j] : val[j];
         tame = wave_ballot(!(all < (kDouble ? (T)1e290 : (T)1e30))) == 0;
     }
-#pragma unroll
-    for (int r = 0; r < D1; ++r) {
-        const int of_group = __shfl(slot[r], leader_of(group[r]));
-        slot[r] = active ? of_group : -1;
-    }
     if (SPLAT_VD && tame) {
         // The lanes in the order of their groups, the groups summed side by side; the last lane of
         // each adds the sums to the slot's row.  About 45 vector instructions a corner, however many
         // groups it has, where a tree of 26 for each group above four lanes and LDS additions lane by
-        // lane for the rest were about 95 (the kernel is bound by its vector and scalar instructions:
-        // a filter of 1024x1024 points, pd 5, vd 4, 123 and 115 us; 128x256x256 voxels, pd 4, vd 2, 506
-        // and 482; 601x803 points in doubles 102 and 97).
-        unsigned where[D1];   // of the lane at a place: the slot and the first place of its group
+        // lane for the rest were about 95 (a filter of 1024x1024 points, pd 5, vd 4, 123 and 115 us;
+        // 128x256x256 voxels, pd 4, vd 2, 506 and 482; 601x803 points in doubles 102 and 97).
+        unsigned where[D1];   // of the lane at a place: its slot and its rank
 #pragma unroll
         for (int r = 0; r < D1; ++r)
-            where[r] = (unsigned)to_place(place_of(group[r]),
-                                          (int)((unsigned)slot[r] << 20 | (unsigned)first_place_of(group[r])));
+            where[r] = (unsigned)to_place(group[r], (int)((unsigned)slot[r] << 20 | rank_of(group[r])));
 #pragma unroll
         for (int r = 0; r < D1; ++r) {
             T term[VD];
 #pragma unroll
-            for (int j = 0; j < VD; ++j) term[j] = to_place(place_of(group[r]), s.weight[r] * val[j]);
-            sum_groups_in_order(term, steps_that_count(lane, (int)(where[r] & 0xffu)));
-            // (wave_shl:1, nothing above lane 63)
-            const unsigned above = (unsigned)__builtin_amdgcn_update_dpp(-1, (int)where[r], 0x130, 0xf, 0xf, false);
-            if (above != where[r] && where[r] < 0xfff00000u) {
+            for (int j = 0; j < VD; ++j) term[j] = to_place(group[r], s.weight[r] * val[j]);
+            sum_groups_in_order(term, steps_that_count(lane, where[r] & 0xffu));
+            // (wave_shl:1, a zero above lane 63)
+            const unsigned above = (unsigned)__builtin_amdgcn_update_dpp(0, (int)where[r], 0x130, 0xf, 0xf, true);
+            if ((above & 0xffu) == 0 && where[r] < 0xfff00000u) {
 #pragma unroll
                 for (int j = 0; j < VD; ++j) atomicAdd(&slot_sum[(where[r] >> 20) * P + j], term[j]);
             }
@@ -2083,6 +2122,15 @@ int key_field_bits(int pd) {
     return b > 16 ? 16 : b;
 }
 
+// x / d == (x * factor) >> shift for every x below 2^31: factor = ceil(2^shift / d) with 2^shift at least
+// 2^32 d, so x * factor exceeds x * 2^shift / d by less than 2^shift / d, and stays below 2^64.
+static PointMap::Divisor divisor(unsigned d) {
+    unsigned bits = 0;
+    while ((1ull << bits) < d) ++bits;
+    const unsigned shift = 31u + bits;
+    return PointMap::Divisor{((1ull << shift) + d - 1u) / d, shift};
+}
+
 PointMap make_point_map(int N, int n_dims, const int *dims) {
     PointMap m{};
     m.N = N;
@@ -2119,6 +2167,8 @@ PointMap make_point_map(int N, int n_dims, const int *dims) {
         }
     }
     if (N == 0) m.n_blocks = 0;
+    m.by_tiles_x = divisor((unsigned)m.tiles[2]);
+    m.by_tiles_yx = divisor((unsigned)m.tiles[1] * (unsigned)m.tiles[2]);
     return m;
 }
 

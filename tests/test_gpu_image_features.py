@@ -1,0 +1,35 @@
+"""Features made from the grid in the build against the same features as a positions array: keys and
+barycentric weights of every point, bit for bit, over widths that divide by a multiplication and widths
+that do not, and grids of every number of extents."""
+import numpy as np
+import pytest
+import torch
+
+import permutohedral_lattice_amd as pla
+
+pytestmark = pytest.mark.gpu
+
+
+def rows(lat, build):
+    build()
+    vertex, weight = (x.cpu().numpy() for x in lat.debug_replay())
+    keys = lat.debug_keys().cpu().numpy()
+    return keys[vertex], weight
+
+
+@pytest.mark.parametrize("dims", [(5,), (17, 23), (1, 40), (64, 1, 48), (3, 9, 21), (1, 30, 33), (2, 3, 9, 17), (33, 70)])
+@pytest.mark.parametrize("channels", [0, 1, 3])
+@pytest.mark.parametrize("widths", [(8.0, 0.125), (3.3, 0.07), (0.37, 13.0), (2.0 ** 41, 2.0 ** -41), (1e30, -1.7)])
+def test_features_of_the_grid(dims, channels, widths):
+    n, pd = int(np.prod(dims)), len(dims) + channels
+    rng = np.random.default_rng(n + channels)
+    image = rng.uniform(0, 1, (n, channels)).astype(np.float32) if channels else None
+    if channels and widths[1] < 1e-6:
+        image *= np.float32(widths[1])
+    image = torch.from_numpy(image).cuda() if channels else None
+    lat = pla.PermutohedralLattice(pd, 2, n)
+    got = rows(lat, lambda: lat.build_image(image, dims, *widths))
+    positions = pla.compute_positions(image, dims, *widths)
+    want = rows(lat, lambda: lat.build(positions))
+    assert (got[0] == want[0]).all() and (got[1] == want[1]).all()
+    lat.close()
