@@ -367,6 +367,25 @@ int pl_mean_field_update(float *q, const float *logits, const float *message_a,
                          const float *message_b, long long n_points, int n_classes,
                          pl_stream stream);
 
+/* ----------------------------------------------------------------------------------------
+ * Message passing of a dense CRF over n images, each with a lattice of its coordinates and colours
+ * (bilateral) and one of its coordinates (spatial), built by pl_build / pl_build_image over the same N
+ * points, with as many value channels as there are classes and one.  Arrays are [n][N][n_classes].
+ *   pl_mean_field_messages: output = bilateral(input) + spatial(input), blurred in reverse order if asked.
+ *   pl_mean_field_infer: q = softmax(logits), then `iterations` times
+ *                        q = softmax(logits + bilateral(q) + spatial(q)); q and logits 16-byte aligned.
+ * The same as pl_apply on every lattice and pl_mean_field_update, with each pass of all lattices in one launch
+ * on `stream`: enqueued behind what the lattices' own streams hold, and what these are given next comes
+ * behind it.  output and q are arrays of their own.  PL_EUNSUPPORTED (nothing is enqueued) where the
+ * lattices must be applied one by one: no vertex lists, options that change an apply, 4 classes to 31 only,
+ * two or three spatial dimensions with a guide of one or three channels, a stream that is being captured.
+ * ---------------------------------------------------------------------------------------- */
+int pl_mean_field_messages(int n, const pl_handle *bilateral, const pl_handle *spatial, float *output,
+                           const float *input, int reverse, pl_stream stream);
+int pl_mean_field_infer(int n, const pl_handle *bilateral, const pl_handle *spatial, float *q,
+                        const float *logits, int iterations, pl_stream stream);
+
+
 #ifdef __cplusplus
 }
 #endif

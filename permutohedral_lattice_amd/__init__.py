@@ -45,7 +45,7 @@ EXPORTS = (
     "pl_debug_keys", "pl_debug_values", "pl_debug_replay", "pl_compute_positions", "pl_filter_image", "pl_build_image",
     "pl_filter_begin", "pl_filter_image_begin", "pl_filter_end",
     "pl_build_begin", "pl_build_image_begin", "pl_build_end", "pl_lattice_filter_op",
-    "pl_set_op_concurrency", "pl_mean_field_update",
+    "pl_set_op_concurrency", "pl_mean_field_update", "pl_mean_field_messages", "pl_mean_field_infer",
     "pl_create_f64", "pl_filter_f64", "pl_build_f64", "pl_apply_f64", "pl_debug_simplex_f64",
     "pl_compute_positions_f64", "pl_lattice_filter_op_f64",
 )
@@ -116,6 +116,8 @@ def _load(path=LIB_PATH):
     lib.pl_build_end.argtypes = [vp]
     lib.pl_set_op_concurrency.argtypes = [ci]
     lib.pl_mean_field_update.argtypes = [vp, vp, vp, vp, C.c_longlong, ci, vp]
+    lib.pl_mean_field_messages.argtypes = [ci, C.POINTER(vp), C.POINTER(vp), vp, vp, ci, vp]
+    lib.pl_mean_field_infer.argtypes = [ci, C.POINTER(vp), C.POINTER(vp), vp, vp, ci, vp]
     lib.pl_lattice_filter_op.argtypes = [vp, vp, vp, ci, ci, C.POINTER(ci), ci, ci, ci, cf, cf, cf,
                                          ci, vp, vp]
     # T = double
@@ -424,6 +426,35 @@ def mean_field_update(q, logits, message_a, message_b):
                                      n // int(logits.shape[-1]), int(logits.shape[-1]), _stream_ptr()),
            "pl_mean_field_update")
     return q
+
+
+def _handles(lattices):
+    return (C.c_void_p * len(lattices))(*(lat._h for lat in lattices))
+
+
+def mean_field_messages(bilateral, spatial, output, input, reverse=False):
+    """``output = bilateral(input) + spatial(input)`` for ``[n, N, classes]`` arrays and n lattices each,
+    on the current stream.  False: these lattices must be applied one by one."""
+    n = len(bilateral) * bilateral[0].N * (bilateral[0].vd - 1)
+    status = _lib.pl_mean_field_messages(len(bilateral), _handles(bilateral), _handles(spatial),
+                                         _dev_f32(output, "output", n), _dev_f32(input, "input", n),
+                                         int(bool(reverse)), _stream_ptr())
+    if status == PL_EUNSUPPORTED:
+        return False
+    _check(status, "pl_mean_field_messages")
+    return True
+
+
+def mean_field_infer(bilateral, spatial, q, logits, iterations):
+    """Mean-field updates of ``q`` from ``softmax(logits)`` on, likewise."""
+    n = len(bilateral) * bilateral[0].N * (bilateral[0].vd - 1)
+    status = _lib.pl_mean_field_infer(len(bilateral), _handles(bilateral), _handles(spatial),
+                                      _dev_f32(q, "q", n), _dev_f32(logits, "logits", n), int(iterations),
+                                      _stream_ptr())
+    if status == PL_EUNSUPPORTED:
+        return False
+    _check(status, "pl_mean_field_infer")
+    return True
 
 
 def _lattice_filter_raw(input_image, reference_image, bilateral, theta_alpha, theta_beta,

@@ -12,17 +12,19 @@ each batch item builds its two lattices once (``pl_build_image``) and every mess
 gradient.
 
 The 2 x batch lattices of a step are independent of each other, and at image sizes like 512 x 512
-one apply is a chain of short kernels that leaves most of the GPU idle, so every lattice works on a
-HIP stream of its own (default priority): a message-passing step waits for its input on the
-caller's stream, runs the applies of all lattices side by side, and the caller's stream waits for
-all of them before it adds the messages up.
+one apply is a chain of short kernels that leaves most of the GPU idle.  They are applied together, every
+pass of all of them in one launch on the caller's stream; where that cannot be (see
+``pl_mean_field_messages``) every lattice works on a HIP stream of its own (default priority), as the builds
+do: a message-passing step waits for its input on the caller's stream, runs the applies of all lattices side
+by side, and the caller's stream waits for all of them before it adds the messages up.
 
 torch carries the tensors; the filters, and the softmax over the logits and both messages, are the
 HIP library's.
 """
 import torch
 
-from . import PermutohedralLattice, mean_field_update, mean_field_update_supported
+from . import (PermutohedralLattice, mean_field_infer, mean_field_messages, mean_field_update,
+               mean_field_update_supported)
 
 
 class MeanField:
@@ -100,14 +102,24 @@ class MeanField:
 
     def messages(self, q, reverse=False):
         """bilateral(q) + spatial(q) for ``q [B, ..., n_classes]`` (any spatial shape of N points)."""
+        if self.batch and q.is_cuda and q.device == self._msg_bi.device:
+            flat = q.contiguous().view(self.batch, self.n, self.n_classes)
+            total = torch.empty_like(self._msg_bi)
+            if mean_field_messages(self.bilateral, self.spatial, total, flat.detach(), reverse):
+                return total
         self._apply_all(q, reverse)
         return self._msg_bi + self._msg_sp
 
     def infer(self, logits, iterations=5):
         """-> Q after ``iterations`` mean-field updates, shaped like ``logits``."""
         flat = logits.contiguous().view(self.batch, self.n, self.n_classes)
+        own = self._own_messages() and mean_field_update_supported(flat)
+        if own and self.batch:
+            q = torch.empty_like(flat)
+            if mean_field_infer(self.bilateral, self.spatial, q, flat, iterations):
+                return q.view(logits.shape)
         q = torch.softmax(flat, dim=-1)
-        if not self._own_messages() or not mean_field_update_supported(flat):
+        if not own:
             # (logits that autograd follows into the last softmax, among others)
             for _ in range(iterations):
                 q = torch.softmax(flat + self.messages(q), dim=-1)

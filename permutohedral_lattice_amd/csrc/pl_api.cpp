@@ -193,6 +193,11 @@ struct pl_lattice {
     int order_capacity = 0;
     hipEvent_t ev[EV_COUNT] = {};
     bool ev_recorded[EV_COUNT] = {};
+    // pl_mean_field_*, which work on another stream than this lattice's: the event that orders the two, the
+    // stream they worked on last, and whether this lattice's own has been given work since
+    hipEvent_t handover = nullptr;
+    hipStream_t worked_on = nullptr;
+    bool own_stream_used = true;
     // which of the eight stages pl_stage_ms reports launched a kernel in the last build / apply
     // (an interval between two events with nothing in between still reads a few microseconds)
     bool stage_ran[8] = {};
@@ -428,6 +433,7 @@ int enqueue_build(pl_lattice *h, const plk::PointFeatures &features, const doubl
                   uint32_t cells, const void *splat_input) {
     // keys of two words while a build that needed them is recent (the plain build only)
     const bool wide = h->wide_for > 0;
+    h->own_stream_used = true;
     if (h->wide_for > 0) h->wide_for -= 1;
     if (wide != h->wide_keys) h->table_clean = false;   // (cells of another width)
     h->wide_keys = wide;
@@ -646,6 +652,7 @@ int enqueue_apply_f64(pl_lattice *h, double *output, const double *input, int re
 
 // output and input are arrays of the lattice's value type
 int enqueue_apply(pl_lattice *h, void *output_any, const void *input_any, int reverse) {
+    h->own_stream_used = true;
     if (h->f64)
         return enqueue_apply_f64(h, static_cast<double *>(output_any),
                                  static_cast<const double *>(input_any), reverse);
@@ -973,6 +980,7 @@ int pl_destroy(pl_handle h) {
     if (h->h_status) (void)hipHostFree(h->h_status);
     for (int i = 0; i < EV_COUNT; ++i)
         if (h->ev[i]) (void)hipEventDestroy(h->ev[i]);
+    if (h->handover) (void)hipEventDestroy(h->handover);
     delete h;
     return PL_OK;
 }
@@ -1590,6 +1598,162 @@ extern "C" int pl_mean_field_update(float *q, const float *logits, const float *
     PL_HIP(plk::mean_field_update(q, logits, message_a, message_b, (size_t)n_points, n_classes,
                                   (hipStream_t)stream));
     return PL_OK;
+}
+
+// ------------------------------------------------------------------------------------------------
+// Message passing of a dense CRF: the applies of all its lattices, pass by pass in one launch each
+// (pl_many.hip), on the caller's stream.
+// ------------------------------------------------------------------------------------------------
+namespace {
+
+constexpr int kPairsPerLaunch = plk::kManyItems / 2;
+
+bool same_points(const plk::PointMap &a, const plk::PointMap &b) {
+    return a.mode == b.mode && a.mode != 1 && a.N == b.N && a.n_blocks == b.n_blocks && a.dims[0] == b.dims[0] &&
+           a.dims[1] == b.dims[1] && a.dims[2] == b.dims[2];
+}
+
+// Whether these lattices' applies can be enqueued together; PL_EUNSUPPORTED: one by one (pl_apply).
+int pairs_status(int n, const pl_handle *bilateral, const pl_handle *spatial, hipStream_t stream) {
+    if (n < 1 || !bilateral || !spatial) return PL_EINVAL;
+    for (int i = 0; i < n; ++i) {
+        const pl_lattice *const pair[2] = {bilateral[i], spatial[i]};
+        for (const pl_lattice *h : pair) {
+            if (!h || h->f64) return PL_EINVAL;
+            if (!h->built || !h->verified || h->pending.active) return PL_ESTATE;
+            if (h->vd != bilateral[0]->vd || h->N != bilateral[0]->N) return PL_EINVAL;
+            if (h->N == 0 || !h->lists_valid || h->values_splatted || h->replay_holds_cells || !h->normalize ||
+                h->stop_after != 0 || h->profile || !h->pair_blur || h->device != bilateral[0]->device)
+                return PL_EUNSUPPORTED;
+        }
+        if (pair[0]->pd != bilateral[0]->pd || pair[1]->pd != spatial[0]->pd ||
+            !same_points(pair[0]->map, pair[1]->map) || !plk::slice_pairs_take(pair[0]->pd, pair[1]->pd, pair[0]->vd))
+            return PL_EUNSUPPORTED;
+        for (int j = 0; j < i; ++j)
+            if (bilateral[j] == bilateral[i] || spatial[j] == spatial[i]) return PL_EUNSUPPORTED;
+    }
+    int device = -1;
+    PL_HIP(hipGetDevice(&device));
+    if (device != bilateral[0]->device) return PL_EUNSUPPORTED;
+    // (a stream that is being captured cannot wait for the lattices' streams, which are not)
+    hipStreamCaptureStatus capturing = hipStreamCaptureStatusNone;
+    PL_HIP(hipStreamIsCapturing(stream, &capturing));
+    return capturing == hipStreamCaptureStatusNone ? PL_OK : PL_EUNSUPPORTED;
+}
+
+// The lattices' streams and `stream`: what is enqueued on `stream` comes after what theirs hold (enter),
+// and what they are given next after what `stream` then holds (leave).
+int enter_stream(int n, const pl_handle *lattices, hipStream_t stream) {
+    for (int i = 0; i < n; ++i) {
+        pl_lattice *h = lattices[i];
+        if (h->stream == stream || (!h->own_stream_used && h->worked_on == stream)) continue;
+        if (!h->handover) PL_HIP(hipEventCreateWithFlags(&h->handover, hipEventDisableTiming));
+        PL_HIP(hipEventRecord(h->handover, h->stream));
+        PL_HIP(hipStreamWaitEvent(stream, h->handover, 0));
+    }
+    return PL_OK;
+}
+int leave_stream(int n, const pl_handle *lattices, hipStream_t stream) {
+    hipEvent_t done = nullptr;
+    for (int i = 0; i < n; ++i) {
+        pl_lattice *h = lattices[i];
+        if (h->stream == stream) continue;
+        if (!done) {
+            done = h->handover;
+            PL_HIP(hipEventRecord(done, stream));
+        }
+        PL_HIP(hipStreamWaitEvent(h->stream, done, 0));
+        h->worked_on = stream;
+        h->own_stream_used = false;
+    }
+    return PL_OK;
+}
+
+// output := softmax(logits + bilateral(input) + spatial(input)) per item, or without logits the sum of the
+// two; all are [n][N][vd-1].
+int enqueue_pairs(int n, const pl_handle *bilateral, const pl_handle *spatial, float *output, const float *input,
+                  const float *logits, int reverse, hipStream_t stream) {
+    const int vd = bilateral[0]->vd;
+    const size_t item = (size_t)bilateral[0]->N * (size_t)(vd - 1);
+    for (int first = 0; first < n; first += kPairsPerLaunch) {
+        const int pairs = n - first < kPairsPerLaunch ? n - first : kPairsPerLaunch;
+        pl_lattice *lattice[plk::kManyItems];
+        plk::GatherWork gather[plk::kManyItems];
+        for (int i = 0; i < 2 * pairs; ++i) {
+            pl_lattice *h = lattice[i] = i < pairs ? bilateral[first + i] : spatial[first + i - pairs];
+            const plk::VertexLists &l = h->lists_of_vertices;
+            gather[i] = plk::GatherWork{l.chunks, l.entries, input + (size_t)(first + i % pairs) * item, h->values[0],
+                                        h->list_chunks, h->long_lists};
+            h->values_zeroed = false;
+            h->current_values = 0;
+        }
+        PL_HIP(plk::splat_gather_many(vd, vd - 1, 2 * pairs, gather, stream));
+        for (int step = 0;; step += 2) {
+            plk::BlurWork blur[plk::kManyItems];
+            int left = 0;
+            for (int i = 0; i < 2 * pairs; ++i) {
+                pl_lattice *h = lattice[i];
+                if (step > h->pd) continue;
+                const int mv = h->max_vertices(), cur = h->current_values;
+                const int axis = reverse ? h->pd - step : step, second = reverse ? axis - 1 : axis + 1;
+                const bool reset = !h->table_clean && step == 0 && !h->wide_keys;
+                blur[left++] = plk::BlurWork{h->counters(), h->values[cur], h->values[1 - cur],
+                                             h->neighbours + (size_t)axis * mv,
+                                             step + 1 <= h->pd ? h->neighbours + (size_t)second * mv : nullptr,
+                                             reset ? h->cell_keys : nullptr, h->vertex_cell, mv, h->launch_vertices()};
+                if (reset) h->table_clean = true;
+                h->current_values = 1 - cur;
+            }
+            if (!left) break;
+            PL_HIP(plk::blur_many(vd, left, blur, stream));
+        }
+        plk::SlicePair slice[kPairsPerLaunch];
+        for (int i = 0; i < pairs; ++i) {
+            const pl_lattice *a = lattice[i], *b = lattice[pairs + i];
+            slice[i] = plk::SlicePair{a->map, a->replay, b->replay, a->values[a->current_values],
+                                      b->values[b->current_values],
+                                      logits ? logits + (size_t)(first + i) * item : nullptr,
+                                      output + (size_t)(first + i) * item};
+        }
+        PL_HIP(plk::slice_pairs(lattice[0]->pd, lattice[pairs]->pd, vd, pairs, slice, stream));
+    }
+    return PL_OK;
+}
+
+}  // namespace
+
+extern "C" int pl_mean_field_messages(int n, const pl_handle *bilateral, const pl_handle *spatial, float *output,
+                                      const float *input, int reverse, pl_stream stream) {
+    int rc = pairs_status(n, bilateral, spatial, (hipStream_t)stream);
+    if (rc != PL_OK) return rc;
+    if (!output || !input || output == input) return PL_EINVAL;
+    rc = enter_stream(n, bilateral, (hipStream_t)stream);
+    if (rc == PL_OK) rc = enter_stream(n, spatial, (hipStream_t)stream);
+    if (rc == PL_OK)
+        rc = enqueue_pairs(n, bilateral, spatial, output, input, nullptr, reverse, (hipStream_t)stream);
+    const int left = leave_stream(n, bilateral, (hipStream_t)stream);
+    const int left_too = leave_stream(n, spatial, (hipStream_t)stream);
+    return rc != PL_OK ? rc : left != PL_OK ? left : left_too;
+}
+
+extern "C" int pl_mean_field_infer(int n, const pl_handle *bilateral, const pl_handle *spatial, float *q,
+                                   const float *logits, int iterations, pl_stream stream) {
+    int rc = pairs_status(n, bilateral, spatial, (hipStream_t)stream);
+    if (rc != PL_OK) return rc;
+    if (!q || !logits || q == logits || iterations < 0) return PL_EINVAL;
+    if ((reinterpret_cast<uintptr_t>(q) | reinterpret_cast<uintptr_t>(logits)) % 16u != 0u) return PL_EINVAL;
+    const int classes = bilateral[0]->vd - 1;
+    rc = enter_stream(n, bilateral, (hipStream_t)stream);
+    if (rc == PL_OK) rc = enter_stream(n, spatial, (hipStream_t)stream);
+    if (rc == PL_OK && hip_failed(plk::mean_field_update(q, logits, nullptr, nullptr,
+                                                         (size_t)n * (size_t)bilateral[0]->N, classes,
+                                                         (hipStream_t)stream)))
+        rc = PL_EHIP;
+    for (int i = 0; i < iterations && rc == PL_OK; ++i)
+        rc = enqueue_pairs(n, bilateral, spatial, q, q, logits, 0, (hipStream_t)stream);
+    const int left = leave_stream(n, bilateral, (hipStream_t)stream);
+    const int left_too = leave_stream(n, spatial, (hipStream_t)stream);
+    return rc != PL_OK ? rc : left != PL_OK ? left : left_too;
 }
 
 // ------------------------------------------------------------------------------------------------

@@ -812,6 +812,40 @@ inline unsigned vertex_blocks(size_t n_items) {
 }
 
 // ------------------------------------------------------------------------------------------------
+// Blur
+// ------------------------------------------------------------------------------------------------
+// One tap (reference: src/PermutohedralLatticeCPU.h:403-405, evaluated in double and rounded once)
+__device__ __forceinline__ float blur_tap(float a, float self, float b) {
+    return (float)(0.25 * (double)a + 0.5 * (double)self + 0.25 * (double)b);
+}
+
+// (S = double: the values of a lattice of doubles)
+__device__ __forceinline__ double blur_tap(double a, double self, double b) {
+    return 0.25 * a + 0.5 * self + 0.25 * b;
+}
+
+// The vertices whose values the taps along axis a, then axis b at vertex v combine (nine; -1
+// where there is none: an absent b-neighbour stands for three zeros, whose tap is zero).
+__device__ __forceinline__ void two_axis_sources(const int2 *__restrict__ nbr_a,
+                                                 const int2 *__restrict__ nbr_b, int v,
+                                                 int (&u)[9]) {
+    const int2 nb = nbr_b[v];
+    const int2 na_self = nbr_a[v];
+    int2 na_x = nbr_a[nb.x >= 0 ? nb.x : 0];
+    int2 na_y = nbr_a[nb.y >= 0 ? nb.y : 0];
+    asm volatile("" : "+v"(na_x.x), "+v"(na_x.y), "+v"(na_y.x), "+v"(na_y.y));
+    u[0] = nb.x >= 0 ? na_x.x : -1;
+    u[1] = nb.x;
+    u[2] = nb.x >= 0 ? na_x.y : -1;
+    u[3] = na_self.x;
+    u[4] = v;
+    u[5] = na_self.y;
+    u[6] = nb.y >= 0 ? na_y.x : -1;
+    u[7] = nb.y;
+    u[8] = nb.y >= 0 ? na_y.y : -1;
+}
+
+// ------------------------------------------------------------------------------------------------
 // Wavefront sums of doubles (the splat of a lattice of doubles)
 // ------------------------------------------------------------------------------------------------
 // The double of another lane (by DPP control; both words moved alike)
@@ -856,6 +890,31 @@ __device__ __forceinline__ double wave_sums_to_quads_f64(bool member, const doub
     }
     return x;
 }
+
+// Which item of a launch a workgroup works for: the items' workgroups follow each other, every item's a
+// multiple of eight, so that workgroup b of an item runs on XCD b % 8 as in a launch of its own.
+template <typename Item, int N = kManyItems>
+struct Items {
+    Item item[N];
+    unsigned blocks[N];   // workgroups of the items
+    int n;
+};
+template <typename Item, int N>
+__device__ __forceinline__ const Item &item_of(const Items<Item, N> &items, unsigned &block, unsigned &blocks) {
+    int i = 0;
+    block = blockIdx.x;
+    if (N > 1)
+        while (i + 1 < items.n && block >= items.blocks[i]) block -= items.blocks[i++];
+    blocks = items.blocks[i];
+    return items.item[i];
+}
+template <typename Item, int N>
+unsigned all_blocks(const Items<Item, N> &items) {
+    unsigned b = 0;
+    for (int i = 0; i < items.n; ++i) b += items.blocks[i];
+    return b;
+}
+inline unsigned multiple_of_xcds(unsigned b) { return (b + kXcds - 1u) / kXcds * kXcds; }
 
 // (keys of two words exist for the dimensions whose packed key has fields of less than 16 bits)
 #define PLK_DISPATCH_WIDE_PD(pd, CALL)            \

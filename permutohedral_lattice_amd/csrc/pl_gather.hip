@@ -408,18 +408,23 @@ __device__ __forceinline__ float pick(const float (&x)[4], int i) {
     return i == 0 ? x[0] : i == 1 ? x[1] : i == 2 ? x[2] : x[3];
 }
 
-template <int L>
-__global__ __launch_bounds__(kBlock) void k_splat_gather_channels(ListChunks chunks, unsigned n_chunks,
-                                                                   int vd,
-                                                                   const ListEntry *__restrict__ entries,
-                                                                   const float *__restrict__ input,
-                                                                   int in_channels, float *values) {
+// N: lattices a launch may be given
+template <int L, int N>
+__global__ __launch_bounds__(kBlock) void k_splat_gather_channels(Items<GatherWork, N> items, int vd,
+                                                                   int in_channels) {
+    unsigned block, blocks;
+    const GatherWork &lattice = item_of(items, block, blocks);
+    const ListChunks &chunks = lattice.chunks;
+    const unsigned n_chunks = lattice.n_chunks;
+    const ListEntry *__restrict__ entries = lattice.entries;
+    const float *__restrict__ input = lattice.input;
+    float *values = lattice.values;
     constexpr unsigned per_block = kBlock / L;
     constexpr int E = kChannelChunk / L;          // entries per lane
     constexpr int kBatch = 16;                    // rows in flight (8: 6 % slower, 32: 2 %)
     const int sub = threadIdx.x % L;
-    const unsigned first_block = xcd_contiguous_block(blockIdx.x, gridDim.x, 1);
-    for (unsigned c0 = first_block * per_block; c0 < n_chunks; c0 += gridDim.x * per_block) {
+    const unsigned first_block = xcd_contiguous_block(block, blocks, 1);
+    for (unsigned c0 = first_block * per_block; c0 < n_chunks; c0 += blocks * per_block) {
         const ChunkWork work = chunk_work(c0 + threadIdx.x / L, n_chunks, chunks, vd, values);
         const unsigned rows = work.to - work.from;
         // (entries past the end of the chunk: its first row, weight zero)
@@ -472,11 +477,16 @@ __global__ __launch_bounds__(kBlock) void k_splat_gather_channels(ListChunks chu
 // alone: the same order on every call.
 constexpr int kSumInFlight = 16;
 
-__global__ __launch_bounds__(kBlock) void k_sum_partial_rows(ListChunks chunks, unsigned n_long, int vd,
-                                                              float *values) {
+template <int N>
+__global__ __launch_bounds__(kBlock) void k_sum_partial_rows(Items<GatherWork, N> items, int vd) {
+    unsigned block, blocks;
+    const GatherWork &lattice = item_of(items, block, blocks);
+    const ListChunks &chunks = lattice.chunks;
+    const unsigned n_long = lattice.n_long;
+    float *values = lattice.values;
     const int lane = threadIdx.x & 63, half = lane >> 5, sub = lane & 31;
-    const unsigned waves = gridDim.x * (kBlock / 64);
-    for (unsigned i = blockIdx.x * (kBlock / 64) + (threadIdx.x >> 6); i < n_long; i += waves) {
+    const unsigned waves = blocks * (kBlock / 64);
+    for (unsigned i = block * (kBlock / 64) + (threadIdx.x >> 6); i < n_long; i += waves) {
         const LongList list = chunks.long_lists[i];
         const unsigned from = list.chunk_from;
         unsigned to = from + chunks_of(list.to - list.from, chunks.rows);
@@ -541,9 +551,46 @@ hipError_t build_vertex_lists(int pd, const PointMap &map, ReplayEntry *replay, 
     return hipGetLastError();
 }
 
+template <int N>
+static hipError_t sum_partial_rows(int vd, int n, const GatherWork *work, hipStream_t s) {
+    Items<GatherWork, N> items{};
+    for (int i = 0; i < n; ++i) {
+        if (!work[i].n_long) continue;
+        items.item[items.n] = work[i];
+        items.blocks[items.n++] = multiple_of_xcds(blocks_for(work[i].n_long, kBlock / 64));
+    }
+    if (items.n) hipLaunchKernelGGL((k_sum_partial_rows<N>), dim3(all_blocks(items)), dim3(kBlock), 0, s, items, vd);
+    return hipGetLastError();
+}
+
+// (rows of more than four channels)
+template <int N>
+static hipError_t splat_gather_channels(int vd, int in_channels, int n, const GatherWork *work, hipStream_t s) {
+    if (in_channels < 4) return hipErrorInvalidValue;
+    const int lanes = vd <= 16 ? 4 : vd <= 32 ? 8 : 16;
+    Items<GatherWork, N> items{};
+    for (int i = 0; i < n; ++i) {
+        if (work[i].chunks.rows > (unsigned)kChannelChunk) return hipErrorInvalidValue;
+        if (!work[i].n_chunks) continue;
+        items.item[items.n] = work[i];
+        items.blocks[items.n++] = multiple_of_xcds(blocks_for(work[i].n_chunks, kBlock / lanes));
+    }
+    if (!items.n) return hipSuccess;
+    const auto kernel = lanes == 4 ? k_splat_gather_channels<4, N>
+                                   : lanes == 8 ? k_splat_gather_channels<8, N> : k_splat_gather_channels<16, N>;
+    hipLaunchKernelGGL(kernel, dim3(all_blocks(items)), dim3(kBlock), 0, s, items, vd, in_channels);
+    return sum_partial_rows<N>(vd, n, work, s);
+}
+
+hipError_t splat_gather_many(int vd, int in_channels, int n, const GatherWork *work, hipStream_t s) {
+    if (n < 1 || n > kManyItems || vd < 5) return hipErrorInvalidValue;
+    return splat_gather_channels<kManyItems>(vd, in_channels, n, work, s);
+}
+
 hipError_t splat_gather(int vd, const VertexLists &lists, unsigned n_chunks, unsigned n_long,
                         const float *input, int in_channels, float *values, hipStream_t s) {
     if (n_chunks == 0) return hipSuccess;
+    const GatherWork work{lists.chunks, lists.entries, input, values, n_chunks, n_long};
     const dim3 block(kBlock);
 #define PLK_GATHER(VD)                                                                               \
     case VD:                                                                                        \
@@ -559,28 +606,10 @@ hipError_t splat_gather(int vd, const VertexLists &lists, unsigned n_chunks, uns
         break;
     switch (vd) {
         PLK_GATHER(2) PLK_GATHER(3) PLK_GATHER(4)
-        default:
-            if (lists.chunks.rows > (unsigned)kChannelChunk) return hipErrorInvalidValue;
-            if (in_channels < 4) return hipErrorInvalidValue;
-            if (vd <= 16)
-                hipLaunchKernelGGL(k_splat_gather_channels<4>, dim3(blocks_for(n_chunks, kBlock / 4)),
-                                   block, 0, s, lists.chunks, n_chunks, vd, lists.entries, input,
-                                   in_channels, values);
-            else if (vd <= 32)
-                hipLaunchKernelGGL(k_splat_gather_channels<8>, dim3(blocks_for(n_chunks, kBlock / 8)),
-                                   block, 0, s, lists.chunks, n_chunks, vd, lists.entries, input,
-                                   in_channels, values);
-            else
-                hipLaunchKernelGGL(k_splat_gather_channels<16>, dim3(blocks_for(n_chunks, kBlock / 16)),
-                                   block, 0, s, lists.chunks, n_chunks, vd, lists.entries, input,
-                                   in_channels, values);
-            break;
+        default: return splat_gather_channels<1>(vd, in_channels, 1, &work, s);
     }
 #undef PLK_GATHER
-    if (n_long)
-        hipLaunchKernelGGL(k_sum_partial_rows, dim3(blocks_for(n_long, kBlock / 64)), block, 0, s,
-                           lists.chunks, n_long, vd, values);
-    return hipGetLastError();
+    return sum_partial_rows<1>(vd, 1, &work, s);
 }
 
 }  // namespace plk

@@ -386,6 +386,39 @@ hipError_t build_vertex_lists(int pd, const PointMap &map, ReplayEntry *replay, 
 hipError_t splat_gather(int vd, const VertexLists &lists, unsigned n_chunks, unsigned n_long,
                         const float *input, int in_channels, float *values, hipStream_t s);
 
+// The same for several lattices of rows of five channels and more in one launch each (pl_many.hip).
+constexpr int kManyItems = 8;
+struct GatherWork {
+    ListChunks chunks;
+    const ListEntry *entries;
+    const float *input;
+    float *values;
+    unsigned n_chunks, n_long;
+};
+hipError_t splat_gather_many(int vd, int in_channels, int n, const GatherWork *work, hipStream_t s);
+// Stage 4 of several lattices: one axis each, or two (nbr_second), in one launch.
+struct BlurWork {
+    const Counters *counters;
+    const float *src;
+    float *dst;
+    const int2 *nbr_first, *nbr_second;
+    uint64_t *reset_cell_keys;
+    const int *vertex_cell;
+    int max_vertices, launch_vertices;
+};
+hipError_t blur_many(int vd, int n, const BlurWork *work, hipStream_t s);
+// Stage 5 of pairs of lattices over the same points (same point map, normalising): output := the sum of
+// both slices, or, with logits, softmax(logits + sum) over the vd-1 channels.
+struct SlicePair {
+    PointMap map;
+    const ReplayEntry *replay_a, *replay_b;
+    const float *values_a, *values_b;
+    const float *logits;
+    float *output;
+};
+bool slice_pairs_take(int pd_a, int pd_b, int vd);
+hipError_t slice_pairs(int pd_a, int pd_b, int vd, int n, const SlicePair *work, hipStream_t s);
+
 // Stage 4, one axis: dst[v] = 1/4 src[n1] + 1/2 src[v] + 1/4 src[n2] for v < counters->num_vertices.
 // reset_cell_keys != nullptr: also empty the hash cell of every vertex (vertex_cell[v]).
 hipError_t blur_axis(int vd, const Counters *counters, int max_vertices, const float *src, float *dst,
@@ -558,8 +591,8 @@ hipError_t compute_positions(const float *reference, float *positions, int N, in
                              int n_spatial_dims, const SpatialDims &dims, float spatial_std,
                              float feature_std, hipStream_t s);
 
-// q = softmax(logits + (message_a + message_b)) over the classes of every point: the mean field's step.
-// All four are [n_points][classes], 16-byte aligned; q may be one of the others.
+// q = softmax(logits + (message_a + message_b)) over the classes of every point: the mean field's step;
+// without messages (both null) softmax(logits).  All four are [n_points][classes], 16-byte aligned; q may be one of the others.
 constexpr int kMeanFieldMaxClasses = 128;
 hipError_t mean_field_update(float *q, const float *logits, const float *message_a, const float *message_b,
                              size_t n_points, int classes, hipStream_t s);

@@ -1468,15 +1468,6 @@ __global__ __launch_bounds__(kBlock) void k_splat_channels(int d1, int vd, Point
 // after a build also empties the hash cells of its vertices (reset_cell_keys != nullptr), which
 // leaves the table clean for the next build without a pass over all cells.
 // ------------------------------------------------------------------------------------------------
-__device__ __forceinline__ float blur_tap(float a, float self, float b) {
-    return (float)(0.25 * (double)a + 0.5 * (double)self + 0.25 * (double)b);
-}
-
-// (S = double: the values of a lattice of doubles)
-__device__ __forceinline__ double blur_tap(double a, double self, double b) {
-    return 0.25 * a + 0.5 * self + 0.25 * b;
-}
-
 // Loads never depend on a branch: an absent neighbour (-1) reads vertex 0 and the value is then
 // replaced by zero, so that all the loads of one level of the gather are in flight together
 // (with a branch per neighbour each load is waited for before the next is asked for: thirteen
@@ -1491,27 +1482,6 @@ __device__ __forceinline__ void gather_elements(const S *__restrict__ src, int v
     for (int k = 0; k < N; ++k) asm volatile("" : "+v"(x[k]));
 #pragma unroll
     for (int k = 0; k < N; ++k) x[k] = u[k] >= 0 ? x[k] : (S)0;
-}
-
-// The vertices whose values the taps along axis a, then axis b at vertex v combine (nine; -1
-// where there is none: an absent b-neighbour stands for three zeros, whose tap is zero).
-__device__ __forceinline__ void two_axis_sources(const int2 *__restrict__ nbr_a,
-                                                 const int2 *__restrict__ nbr_b, int v,
-                                                 int (&u)[9]) {
-    const int2 nb = nbr_b[v];
-    const int2 na_self = nbr_a[v];
-    int2 na_x = nbr_a[nb.x >= 0 ? nb.x : 0];
-    int2 na_y = nbr_a[nb.y >= 0 ? nb.y : 0];
-    asm volatile("" : "+v"(na_x.x), "+v"(na_x.y), "+v"(na_y.x), "+v"(na_y.y));
-    u[0] = nb.x >= 0 ? na_x.x : -1;
-    u[1] = nb.x;
-    u[2] = nb.x >= 0 ? na_x.y : -1;
-    u[3] = na_self.x;
-    u[4] = v;
-    u[5] = na_self.y;
-    u[6] = nb.y >= 0 ? na_y.x : -1;
-    u[7] = nb.y;
-    u[8] = nb.y >= 0 ? na_y.y : -1;
 }
 
 // one thread per (vertex, channel), any vd

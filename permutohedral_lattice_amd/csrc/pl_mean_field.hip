@@ -39,7 +39,9 @@ __global__ __launch_bounds__(kRows) void k_mean_field_update(float *q, const flo
     int row = 4 * (int)threadIdx.x / classes, cls = 4 * (int)threadIdx.x - row * classes;
     const int row0 = row, cls0 = cls;
     for (int i = threadIdx.x; i < n4; i += kRows) {
-        const float4 l = l4[i], a = a4[i], b = b4[i];
+        const float4 l = l4[i];
+        const float4 a = message_a ? a4[i] : make_float4(0.0f, 0.0f, 0.0f, 0.0f);
+        const float4 b = message_a ? b4[i] : make_float4(0.0f, 0.0f, 0.0f, 0.0f);
         const float x[4] = {l.x + (a.x + b.x), l.y + (a.y + b.y), l.z + (a.z + b.z), l.w + (a.w + b.w)};
         int r = row, c = cls;
 #pragma unroll
@@ -58,7 +60,8 @@ __global__ __launch_bounds__(kRows) void k_mean_field_update(float *q, const flo
         }
     }
     for (int e = 4 * n4 + (int)threadIdx.x; e < n; e += kRows)
-        rows[(e / classes) * pitch + e % classes] = logits[base + e] + (message_a[base + e] + message_b[base + e]);
+        rows[(e / classes) * pitch + e % classes] =
+            logits[base + e] + (message_a ? message_a[base + e] + message_b[base + e] : 0.0f);
     __syncthreads();
     if ((int)threadIdx.x < n_rows) {
         float *own = rows + (int)threadIdx.x * pitch;
@@ -108,7 +111,7 @@ hipError_t mean_field_update(float *q, const float *logits, const float *message
     if (n_points == 0) return hipSuccess;
     const uintptr_t all = reinterpret_cast<uintptr_t>(q) | reinterpret_cast<uintptr_t>(logits) |
                           reinterpret_cast<uintptr_t>(message_a) | reinterpret_cast<uintptr_t>(message_b);
-    if (!q || !logits || !message_a || !message_b || all % 16u != 0u || classes < 1 ||
+    if (!q || !logits || !message_a != !message_b || all % 16u != 0u || classes < 1 ||
         classes > kMeanFieldMaxClasses)
         return hipErrorInvalidValue;
     // (256 rows of up to 40 classes are 42 KB of LDS, three workgroups a CU; 64 rows of up to 128, 33 KB)

@@ -136,3 +136,80 @@ def test_messages_put_in_the_place_of_the_class_s():
     assert float((plain.infer(logits, 2) - step).abs().max()) <= 1e-6
     derived.close()
     plain.close()
+
+
+@pytest.mark.parametrize("shape,guide_channels,classes,batch", [
+    ((33, 47), 3, 4, 1), ((64, 80), 1, 5, 3), ((40, 24), 3, 15, 2), ((40, 24), 3, 16, 5), ((24, 33), 3, 31, 1),
+    ((9, 17, 20), 1, 21, 2), ((8, 12, 16), 3, 7, 2), ((72, 100), 3, 21, 6),
+    ((30, 2), 3, 21, 2)])                       # (a grid too thin for tiles)
+def test_lattices_applied_together_equal_them_one_by_one(shape, guide_channels, classes, batch):
+    """Every pass of all lattices in one launch, both messages sliced at once: the same sums in the same
+    order as an apply each, so equal to an ulp or two of the weighted means."""
+    import permutohedral_lattice_amd as pla
+    gen = torch.Generator("cuda").manual_seed(batch * 100 + classes)
+    guide = torch.rand((batch,) + shape + (guide_channels,), device="cuda", generator=gen) * 255.0
+    x = torch.randn((batch,) + shape + (classes,), device="cuda", generator=gen)
+    mf = MeanField(guide, classes, 10.0, 60.0, 3.0)
+    n = mf.n
+    flat = x.view(batch, n, classes)
+    for reverse in (False, True):
+        together = torch.full_like(flat, float("nan"))
+        assert pla.mean_field_messages(mf.bilateral, mf.spatial, together, flat, reverse)
+        mf._apply_all(flat, reverse)
+        one_by_one = mf._msg_bi + mf._msg_sp
+        scale = float(one_by_one.abs().max())
+        assert float((together - one_by_one).abs().max()) <= 4 * 1.2e-7 * scale
+    q = torch.full_like(flat, float("nan"))
+    assert pla.mean_field_infer(mf.bilateral, mf.spatial, q, flat, 3)
+    want = torch.softmax(flat, dim=-1)
+    for _ in range(3):
+        mf._apply_all(want, False)
+        want = torch.softmax(flat + (mf._msg_bi + mf._msg_sp), dim=-1)
+    # (an error of a few ulps of a logit of size s moves its probability by that many times s ulps)
+    assert float((q - want).abs().max()) <= 3 * 8 * 1.2e-7 * float(flat.abs().max() + 2)
+    mf.close()
+
+
+def test_what_cannot_be_applied_together_is_applied_one_by_one():
+    import permutohedral_lattice_amd as pla
+    gen = torch.Generator("cuda").manual_seed(3)
+    guide = torch.rand((2, 40, 56, 3), device="cuda", generator=gen) * 255.0
+    for classes, option, together in ((33, None, False), (3, None, False), (21, (pla.PL_OPT_VERTEX_LISTS, 0), False),
+                                      (21, (pla.PL_OPT_PAIR_BLUR, 0), False), (21, None, True)):
+        x = torch.randn((2, 40, 56, classes), device="cuda", generator=gen)
+        mf = MeanField(guide, classes)
+        if option:
+            mf.spatial[1].set_option(*option)
+        out = torch.empty((2, 40 * 56, classes), device="cuda")
+        assert pla.mean_field_messages(mf.bilateral, mf.spatial, out, x.view(out.shape)) == together
+        got = mf.messages(x).view(x.shape)
+        want = pla.lattice_filter(x, guide, True, 80.0, 13.0, 3.0) + pla.lattice_filter(x, guide, False, 80.0, 13.0, 3.0)
+        assert float((got - want).abs().max()) <= 1e-4
+        mf.close()
+
+
+def test_lattices_applied_together_from_two_streams():
+    """The lattices' own streams, and applies of single lattices on them, stay in order with it."""
+    gen = torch.Generator("cuda").manual_seed(5)
+    guides = [torch.rand((2, 96, 120, 3), device="cuda", generator=gen) * 255.0 for _ in range(2)]
+    x = torch.randn((2, 96, 120, 21), device="cuda", generator=gen)
+    mf, want = None, []
+    for guide in guides:
+        fresh = MeanField(guide, 21)
+        want.append((fresh.infer(x, 3), fresh.messages(x, True)))
+        torch.cuda.synchronize()
+        fresh.close()
+    mf = MeanField(guides[0], 21)
+    streams = [torch.cuda.Stream(), torch.cuda.Stream()]
+    torch.cuda.synchronize()
+    for turn in range(6):
+        with torch.cuda.stream(streams[turn % 2]):
+            streams[turn % 2].wait_stream(streams[1 - turn % 2])
+            mf.rebuild(guides[turn % 2])
+            q = mf.infer(x, 3)
+            mf.bilateral[1].apply(mf._msg_bi[1], x[1].reshape(-1, 21))
+            back = mf.messages(x, True).view(x.shape)
+        streams[turn % 2].synchronize()
+        assert float((q - want[turn % 2][0]).abs().max()) <= 1e-6
+        assert float((back - want[turn % 2][1].view(x.shape)).abs().max()) <= 1e-5
+    mf.close()
