@@ -677,7 +677,9 @@ int enqueue_apply(pl_lattice *h, void *output_any, const void *input_any, int re
         const size_t filled = h->verified && h->n_segments == 0 ? (size_t)h->M : (size_t)mv;
         if (!h->values_zeroed) PL_HIP(plk::fill_zero(h->values[0], filled * vd, h->stream));
         h->mark(EV_FILL);
-        const auto splat = h->last_build_merged && plk::splat_tile_takes(vd) ? plk::splat_tile : plk::splat;
+        const auto splat = !h->last_build_merged ? plk::splat
+                           : vd <= 4             ? plk::splat_merge
+                           : plk::splat_tile_takes(vd) ? plk::splat_tile : plk::splat;
         PL_HIP(splat(pd, vd, h->map, input, in_channels, h->replay,
                      h->replay_holds_cells ? h->cell_vertex : nullptr, h->values[0],
                      h->xcd_aware ? 1 : 0, h->stream));

@@ -317,6 +317,10 @@ hipError_t splat(int pd, int vd, const PointMap &map, const float *input, int in
                  ReplayEntry *replay, const int *cell_vertex, float *values,
                  int xcd_aware, hipStream_t s);
 
+// The same for rows of 2 to 4 channels after a merging build: sums merged per workgroup in LDS.
+hipError_t splat_merge(int pd, int vd, const PointMap &map, const float *input, int in_channels,
+                       ReplayEntry *replay, const int *cell_vertex, float *values, int xcd_aware, hipStream_t s);
+
 // The same for rows of 5 to 32 channels after a merging build, whose workgroups' points have at most
 // kTileSlots vertices: pairs sorted by vertex in LDS, see pl_splat_tile.hip.
 // (Up to 32 channels and nine corners the pairs and the points' rows fit 64 KB of LDS.  Filters of

@@ -460,6 +460,112 @@ __global__ __launch_bounds__(kBlock) void k_build(PointFeatures features, PointM
     }
 }
 
+// What the kernels that merge a workgroup's rows in LDS share.
+static_assert(kTileSlots == 1 << (32 - kTileSlotShift), "the slot is the hash's high bits");
+
+// A slot of the workgroup's table for every group of the wavefront (wave_groups_in_order of each corner,
+// numbered through): slot[r] := that of the lane's group of corner r, -1 where it has none (bit r of
+// `present` clear) or no slot was found; new slots join the list `occupied`.  True: every key of this lane's
+// has its slot.
+// The leaders' keys go to lane after lane of the wavefront, whatever corner they are of (an image's 8x8
+// pixels have about forty), and every lane places one, where a lane with a leader for each of its
+// corners would place up to D1, one behind the other; the slots come back the same way.  (More than 64
+// groups: 64 at a time.)  wave_keys: 64 keys of the wavefront's own, in LDS.
+template <int PROBES, int D1, typename Key, typename Hash>
+__device__ __forceinline__ bool place_groups(const Key (&key)[D1], const unsigned (&group)[D1], unsigned present,
+                                             unsigned n_groups, int lane, Key *wave_keys, Key *table, Key empty,
+                                             Hash hash, unsigned short *occupied, int *n_occupied,
+                                             int (&slot)[D1]) {
+    using Word = std::conditional_t<sizeof(Key) == 8, unsigned long long, int>;
+    constexpr int kStride = sizeof(Key) / sizeof(int);
+    int *wave_slots = reinterpret_cast<int *>(wave_keys);
+    bool placed = true;
+#pragma unroll
+    for (int r = 0; r < D1; ++r) slot[r] = -1;
+    for (unsigned from = 0; from < n_groups; from += 64) {
+#pragma unroll
+        for (int r = 0; r < D1; ++r) {
+            const unsigned to = number_of(group[r]) - from;
+            if (((present >> r) & 1u) && rank_of(group[r]) == 0 && to < 64u) wave_keys[to] = key[r];
+        }
+        __builtin_amdgcn_wave_barrier();
+        const Key mine = wave_keys[lane];
+        int at_slot = (int)(hash(mine) >> kTileSlotShift);
+        bool open = from + (unsigned)lane < n_groups, was_empty = false;
+        if (!open) at_slot = -1;
+        for (int probe = 0; open && probe < PROBES; ++probe) {
+            const Key seen = (Key)atomicCAS((Word *)&table[at_slot], (Word)empty, (Word)mine);
+            if (seen == empty || seen == mine) {
+                open = false;
+                was_empty = seen == empty;
+            } else {
+                at_slot = (at_slot + 1) & (kTileSlots - 1);
+            }
+        }
+        if (open) {
+            placed = false;
+            at_slot = -1;
+        }
+        __builtin_amdgcn_wave_barrier();
+        wave_slots[kStride * lane] = at_slot;
+        __builtin_amdgcn_wave_barrier();
+#pragma unroll
+        for (int r = 0; r < D1; ++r) {
+            const unsigned to = number_of(group[r]) - from;
+            if (((present >> r) & 1u) && to < 64u) slot[r] = wave_slots[kStride * to];
+        }
+        // the slots that were empty join the list of slots in use
+        if (was_empty) occupied[atomicAdd(n_occupied, 1)] = (unsigned short)at_slot;
+        __builtin_amdgcn_wave_barrier();
+    }
+    return placed;
+}
+
+// Weight times value of every corner of the wavefront's points, added to the rows (of P values) of their
+// slots in LDS.  The lanes in the order of their groups, the groups summed side by side; the last lane of
+// each adds the sums to the slot's row.  About 45 vector instructions a corner, however many groups it
+// has, where a tree of 26 for each group above four lanes and LDS additions lane by lane for the rest
+// were about 95 (a filter of 1024x1024 points, pd 5, vd 4, 123 and 115 us; 128x256x256 voxels, pd 4, vd 2,
+// 506 and 482; 601x803 points in doubles 102 and 97).
+template <int VD, int P, int D1, typename T>
+__device__ __forceinline__ void add_to_slots(T *slot_sum, const unsigned (&group)[D1], const int (&slot)[D1],
+                                             const T (&weight)[D1], const T (&val)[4], int lane) {
+    // (what sum_groups_in_order asks of its terms: the wavefront's values and weights finite and, as
+    // the weights are at most one, their sums far from overflowing; a NaN fails the comparison)
+    T all = (T)0;
+#pragma unroll
+    for (int r = 0; r < D1; ++r) all += weight[r];
+#pragma unroll
+    for (int j = 0; j < VD; ++j) all += val[j] < (T)0 ? -val[j] : val[j];
+    if (wave_ballot(!(all < (sizeof(T) == sizeof(double) ? (T)1e290 : (T)1e30))) == 0) {
+        unsigned where[D1];   // of the lane at a place: its slot and its rank
+#pragma unroll
+        for (int r = 0; r < D1; ++r)
+            where[r] = (unsigned)to_place(group[r], (int)((unsigned)slot[r] << 20 | rank_of(group[r])));
+#pragma unroll
+        for (int r = 0; r < D1; ++r) {
+            T term[VD];
+#pragma unroll
+            for (int j = 0; j < VD; ++j) term[j] = to_place(group[r], weight[r] * val[j]);
+            sum_groups_in_order(term, steps_that_count(lane, where[r] & 0xffu));
+            // (wave_shl:1, a zero above lane 63)
+            const unsigned above = (unsigned)__builtin_amdgcn_update_dpp(0, (int)where[r], 0x130, 0xf, 0xf, true);
+            if ((above & 0xffu) == 0 && where[r] < 0xfff00000u) {
+#pragma unroll
+                for (int j = 0; j < VD; ++j) atomicAdd(&slot_sum[(where[r] >> 20) * P + j], term[j]);
+            }
+        }
+    } else {
+#pragma unroll
+        for (int r = 0; r < D1; ++r) {
+            if (slot[r] >= 0) {
+#pragma unroll
+                for (int j = 0; j < VD; ++j) atomicAdd(&slot_sum[slot[r] * P + j], weight[r] * val[j]);
+            }
+        }
+    }
+}
+
 // The same stage with the keys and sums of a whole workgroup merged in LDS before they go to the
 // table: for an image tile of 16x16 pixels the four wavefronts hold about 165 (wavefront, vertex)
 // pairs but only about 100 distinct vertices, and what limits the build is the number of requests
@@ -550,52 +656,10 @@ __global__ __launch_bounds__(kBlock) __attribute__((amdgpu_num_sgpr(102))) void 
         vertex_keys_of<PD>(s, key);
 #pragma unroll
         for (int r = 0; r < D1; ++r) group[r] = wave_groups_in_order(key[r], among, &n_groups);
-        // The leaders' keys go to lane after lane of the wavefront, whatever corner they are of (an
-        // image's 8x8 pixels have about forty), and every lane places one in the table, where a lane
-        // with a leader for each of its corners would place up to pd+1, one behind the other; the
-        // slots come back the same way.  (More than 64 groups: 64 at a time.)
-        uint64_t *wave_keys = group_keys[tid >> 6];
-        int *wave_slots = reinterpret_cast<int *>(wave_keys);
-#pragma unroll
-        for (int r = 0; r < D1; ++r) slot[r] = -1;
-        for (unsigned from = 0; from < n_groups; from += 64) {
-#pragma unroll
-            for (int r = 0; r < D1; ++r) {
-                const unsigned to = number_of(group[r]) - from;
-                if (active && rank_of(group[r]) == 0 && to < 64u) wave_keys[to] = key[r];
-            }
-            __builtin_amdgcn_wave_barrier();
-            const uint64_t mine = wave_keys[lane];
-            static_assert(kTileSlots == 1 << (32 - kTileSlotShift), "the slot is the hash's high bits");
-            int at_slot = (int)(hash_key(mine) >> kTileSlotShift);
-            bool open = from + (unsigned)lane < n_groups, was_empty = false;
-            if (!open) at_slot = -1;
-            for (int probe = 0; open && probe < kTileProbeLimit; ++probe) {
-                const uint64_t seen = atomicCAS((unsigned long long *)&slot_key[at_slot],
-                                                (unsigned long long)kEmptyCell, (unsigned long long)mine);
-                if (seen == kEmptyCell || seen == mine) {
-                    open = false;
-                    was_empty = seen == kEmptyCell;
-                } else {
-                    at_slot = (at_slot + 1) & (kTileSlots - 1);
-                }
-            }
-            if (open) {
-                atomicOr(&counters->flags, kFlagTileFull);
-                at_slot = -1;
-            }
-            __builtin_amdgcn_wave_barrier();
-            wave_slots[2 * lane] = at_slot;
-            __builtin_amdgcn_wave_barrier();
-#pragma unroll
-            for (int r = 0; r < D1; ++r) {
-                const unsigned to = number_of(group[r]) - from;
-                if (active && to < 64u) slot[r] = wave_slots[2 * to];
-            }
-            // the slots that were empty join the list of slots in use
-            if (was_empty) occupied[atomicAdd(&n_occupied, 1)] = (unsigned short)at_slot;
-            __builtin_amdgcn_wave_barrier();
-        }
+        const bool all_placed = place_groups<kTileProbeLimit>(
+            key, group, active ? (1u << D1) - 1u : 0u, n_groups, lane, group_keys[tid >> 6], slot_key, kEmptyCell,
+            [](uint64_t k) { return hash_key(k); }, occupied, &n_occupied, slot);
+        if (!all_placed) atomicOr(&counters->flags, kFlagTileFull);
     }
 
     T val[4] = {(T)0, (T)0, (T)0, (T)0};
@@ -608,49 +672,7 @@ __global__ __launch_bounds__(kBlock) __attribute__((amdgpu_num_sgpr(102))) void 
                 if (j < in_channels) val[j] = input[(size_t)n * in_channels + j];
         }
     }
-    // (what sum_groups_in_order asks of its terms: the wavefront's values and weights finite and, as
-    // the weights are at most one, their sums far from overflowing; a NaN fails the comparison)
-    bool tame = true;
-    if (SPLAT_VD) {
-        T all = (T)0;
-#pragma unroll
-        for (int r = 0; r < D1; ++r) all += s.weight[r];
-#pragma unroll
-        for (int j = 0; j < VD; ++j) all += val[j] < (T)0 ? -val[j] : val[j];
-        tame = wave_ballot(!(all < (kDouble ? (T)1e290 : (T)1e30))) == 0;
-    }
-    if (SPLAT_VD && tame) {
-        // The lanes in the order of their groups, the groups summed side by side; the last lane of
-        // each adds the sums to the slot's row.  About 45 vector instructions a corner, however many
-        // groups it has, where a tree of 26 for each group above four lanes and LDS additions lane by
-        // lane for the rest were about 95 (a filter of 1024x1024 points, pd 5, vd 4, 123 and 115 us;
-        // 128x256x256 voxels, pd 4, vd 2, 506 and 482; 601x803 points in doubles 102 and 97).
-        unsigned where[D1];   // of the lane at a place: its slot and its rank
-#pragma unroll
-        for (int r = 0; r < D1; ++r)
-            where[r] = (unsigned)to_place(group[r], (int)((unsigned)slot[r] << 20 | rank_of(group[r])));
-#pragma unroll
-        for (int r = 0; r < D1; ++r) {
-            T term[VD];
-#pragma unroll
-            for (int j = 0; j < VD; ++j) term[j] = to_place(group[r], s.weight[r] * val[j]);
-            sum_groups_in_order(term, steps_that_count(lane, where[r] & 0xffu));
-            // (wave_shl:1, a zero above lane 63)
-            const unsigned above = (unsigned)__builtin_amdgcn_update_dpp(0, (int)where[r], 0x130, 0xf, 0xf, true);
-            if ((above & 0xffu) == 0 && where[r] < 0xfff00000u) {
-#pragma unroll
-                for (int j = 0; j < VD; ++j) atomicAdd(&slot_sum[(where[r] >> 20) * P + j], term[j]);
-            }
-        }
-    } else if (SPLAT_VD) {
-#pragma unroll
-        for (int r = 0; r < D1; ++r) {
-            if (slot[r] >= 0) {
-#pragma unroll
-                for (int j = 0; j < VD; ++j) atomicAdd(&slot_sum[slot[r] * P + j], s.weight[r] * val[j]);
-            }
-        }
-    }
+    if constexpr (SPLAT_VD != 0) add_to_slots<VD, P>(slot_sum, group, slot, s.weight, val, lane);
     __syncthreads();        // the keys and sums of all four wavefronts are in the LDS table
 
     // Every slot in use goes to the table in HBM: thread i takes the i-th of them (and the
@@ -1275,6 +1297,78 @@ __global__ __launch_bounds__(kBlock) void k_splat_dpp(PointMap map,
                 atomicAdd(values + (size_t)k * VD + my_channel, sum);
         }
     }
+}
+
+// The same after a merging build, which leaves a workgroup's points at most kTileSlots vertices: the rows
+// of sums of its four wavefronts meet in LDS first, as in the build, and go out with one request each
+// (1024x1024 points, pd 5: 99 rows a workgroup instead of 165), and the vertices are told from the hash
+// cells once a slot instead of once a row.  What bounds it is the chain of its instructions; 1024x1024
+// points, pd 5, vd 2: 30.7 us a launch, k_splat_dpp 50.2.
+template <int VD, int D1>
+__global__ __launch_bounds__(kBlock) void k_splat_merge(PointMap map, const float *__restrict__ input,
+                                                         int in_channels, ReplayEntry *replay,
+                                                         const int *__restrict__ cell_vertex, float *values,
+                                                         int xcd_aware) {
+    static_assert(VD >= 2 && VD <= 4, "register splat handles 2..4 channels");
+    constexpr int P = VD == 2 ? 2 : 4;   // values per LDS row of sums
+    unsigned vblock;
+    if (!block_of_points(map, xcd_aware, vblock)) return;
+    __shared__ int slot_index[kTileSlots];
+    __shared__ float slot_sum[kTileSlots * P];
+    __shared__ unsigned short occupied[kTileSlots];
+    __shared__ int n_occupied;
+    __shared__ int group_index[kBlock / 64][64];
+    const int tid = threadIdx.x, lane = tid & 63;
+    for (int i = tid; i < kTileSlots; i += kBlock) slot_index[i] = -1;
+    for (int i = tid; i < kTileSlots * P; i += kBlock) slot_sum[i] = 0.0f;
+    if (tid == 0) n_occupied = 0;
+    const size_t t = (size_t)vblock * kBlock * D1 + tid;
+    constexpr size_t T = kBlock;
+    const int n = point_of_thread(map, vblock, tid);
+    // (a lane without a point reads point 0 and takes no part)
+    float val[4] = {0.0f, 0.0f, 0.0f, 0.0f};
+#pragma unroll
+    for (int j = 0; j < VD; ++j) {
+        const float x = input[(size_t)(n >= 0 ? n : 0) * in_channels + (j < in_channels ? j : 0)];
+        val[j] = j < in_channels ? (n >= 0 ? x : 0.0f) : 1.0f;   // the homogeneous channel when vd-1 are given
+    }
+    int index[D1];
+    float weight[D1];
+#pragma unroll
+    for (int r = 0; r < D1; ++r) {
+        const ReplayEntry e = replay[(size_t)r * T + t];
+        index[r] = n >= 0 ? e.index : -1;
+        weight[r] = n >= 0 ? e.weight : 0.0f;
+    }
+    __syncthreads();        // the slots are empty
+    unsigned group[D1], n_groups = 0, present = 0;
+    int slot[D1];
+#pragma unroll
+    for (int r = 0; r < D1; ++r) {
+        if (index[r] >= 0) present |= 1u << r;
+        group[r] = wave_groups_in_order((uint64_t)(uint32_t)index[r], wave_ballot(index[r] >= 0), &n_groups);
+    }
+    place_groups<kTileSlots>(index, group, present, n_groups, lane, group_index[tid >> 6], slot_index, -1,
+                             [](int i) { return (uint32_t)i * 0x9E3779B1u; }, occupied, &n_occupied, slot);
+    add_to_slots<VD, P>(slot_sum, group, slot, weight, val, lane);
+    __syncthreads();        // the sums of all four wavefronts are in the rows
+    const int n_in_use = n_occupied, channel = tid % P;
+    for (int i = tid / P; i < n_in_use; i += kBlock / P) {
+        const int sl = (int)occupied[i];
+        int v = slot_index[sl];
+        if (cell_vertex) v = cell_vertex[v];
+        if (channel < VD) atomicAdd(values + (size_t)v * VD + channel, slot_sum[sl * P + channel]);
+        // (read by this lane's row alone until the barrier below)
+        if (cell_vertex) {
+            __builtin_amdgcn_wave_barrier();
+            if (channel == 0) slot_index[sl] = v;
+        }
+    }
+    if (!cell_vertex) return;
+    __syncthreads();
+#pragma unroll
+    for (int r = 0; r < D1; ++r)
+        if (slot[r] >= 0) replay[(size_t)r * T + t].index = slot_index[slot[r]];
 }
 
 // Any vd: the same, four channels at a time.  The deduplication loop runs once per block of four
@@ -2283,6 +2377,24 @@ hipError_t fill_ranges(FillRanges ranges, hipStream_t s) {
 hipError_t fill_zero(float *p, size_t n, hipStream_t s) {
     if (n == 0) return hipSuccess;
     hipLaunchKernelGGL(k_fill_zero, dim3(blocks_for(n)), dim3(kBlock), 0, s, p, n);
+    return hipGetLastError();
+}
+
+hipError_t splat_merge(int pd, int vd, const PointMap &map, const float *input, int in_channels,
+                       ReplayEntry *replay, const int *cell_vertex, float *values, int xcd_aware, hipStream_t s) {
+    if (map.n_blocks == 0) return hipSuccess;
+    const dim3 grid(map.n_blocks), block(kBlock);
+#define PLK_SPLAT_MERGE(VD)                                                                             \
+    case VD:                                                                                            \
+        PLK_DISPATCH_PD(pd, hipLaunchKernelGGL((k_splat_merge<VD, PD + 1>), grid, block, 0, s, map,     \
+                                               input, in_channels, replay, cell_vertex, values,         \
+                                               xcd_aware));                                             \
+        break;
+    switch (vd) {
+        PLK_SPLAT_MERGE(2) PLK_SPLAT_MERGE(3) PLK_SPLAT_MERGE(4)
+        default: return hipErrorInvalidValue;
+    }
+#undef PLK_SPLAT_MERGE
     return hipGetLastError();
 }
 
