@@ -154,7 +154,9 @@ struct pl_lattice {
     // has many thousands of workgroups (they draw their numbers one after the other), or when
     // the last such build of these points held so many rows of sums for vertices of other
     // workgroups that adding them afterwards, an atomic each, outweighs the numbering pass.
-    bool numbering_pass_pays = false;
+    // (The pass then serves the next numbering_pass_backoff builds, doubled every time it is found to pay
+    // again, up to 1024, before a build counts such rows anew: inputs change.)
+    int numbering_pass_for = 0, numbering_pass_backoff = 32;
     long foreign_rows = -1;            // of the last build (an estimate from a sample); -1: it listed none
     bool built = false;                // a build has been enqueued and, if verified, fitted
     bool verified = false;             // its status has been read on the host
@@ -468,7 +470,8 @@ int enqueue_build(pl_lattice *h, const plk::PointFeatures &features, const doubl
     // (a build for one filter: a lattice built to be applied many times is numbered by the
     // numbering pass, in the order of the image tiles, which the passes over the vertices walk
     // a few per cent faster than the order in which the workgroups happened to finish)
-    const bool numbers_in_build = merge && fused && !h->numbering_pass_pays && h->forced_segments >= 0;
+    const bool numbers_in_build = merge && fused && h->numbering_pass_for == 0 && h->forced_segments >= 0;
+    if (merge && fused && h->numbering_pass_for > 0) h->numbering_pass_for -= 1;
     const size_t floats_per_value = h->f64 ? 2 : 1;
     if (fused && !numbers_in_build && !h->cell_values_clean) {
         PL_HIP(plk::fill_zero(h->cell_values, (size_t)h->n_cells_alloc * h->vd * floats_per_value,
@@ -837,8 +840,12 @@ int verify_build(pl_lattice *h, uint32_t *retry_cells) {
     // workgroups: 41 us), and the build 1500 longer with all its rows going out as atomics)
     h->foreign_rows = status.n_segments != 0 ? (long)status.foreign_rows : -1;
     if (status.n_segments != 0 &&
-        0.037 * status.foreign_rows > 1.25 * h->working_blocks() + 0.02 * m + 1500.0)
-        h->numbering_pass_pays = true;
+        0.037 * status.foreign_rows > 1.25 * h->working_blocks() + 0.02 * m + 1500.0) {
+        h->numbering_pass_for = h->numbering_pass_backoff;
+        h->numbering_pass_backoff = h->numbering_pass_backoff >= 512 ? 1024 : h->numbering_pass_backoff * 2;
+    } else if (status.n_segments != 0) {
+        h->numbering_pass_backoff = 32;
+    }
     h->verified = true;
     if (h->last_build_merged) h->tiles_backoff = 32;
     return PL_OK;
@@ -1050,10 +1057,20 @@ int pl_set_point_grid(pl_handle h, int n_dims, const int *dims) {
     }
     h->built = false;
     h->grid_given = n_dims > 0;
+    const plk::PointMap before = h->map;
     h->map = plk::make_point_map(h->N, n_dims, dims);
-    h->numbering_pass_pays = false;
-    h->one_segment_for = 0;
-    h->one_segment_backoff = 32;
+    // (the *_image entry points set the grid on every call: what the last builds of these points have
+    // shown about the way to number their vertices holds for as long as the grid is the same.  128x256x256
+    // voxels under their intensities: forgetting it, the build numbered its vertices every time and 1.3
+    // million rows of sums for other workgroups' vertices followed it as atomics, 473 us; 430 with the
+    // numbering pass from the second call on.)
+    if (h->map.mode < 2 || h->map.mode != before.mode || h->map.dims[0] != before.dims[0] ||
+        h->map.dims[1] != before.dims[1] || h->map.dims[2] != before.dims[2]) {
+        h->numbering_pass_for = 0;
+        h->numbering_pass_backoff = 32;
+        h->one_segment_for = 0;
+        h->one_segment_backoff = 32;
+    }
     return ensure_replay(h, false);
 }
 
@@ -1112,7 +1129,8 @@ int guess_point_grid(pl_lattice *h, const float *positions) {
     }
     if (dims[0] < 2) return PL_OK;
     h->map = plk::make_point_map(h->N, n_dims, dims);
-    h->numbering_pass_pays = false;
+    h->numbering_pass_for = 0;
+    h->numbering_pass_backoff = 32;
     h->one_segment_for = 0;
     h->one_segment_backoff = 32;
     return ensure_replay(h, false);

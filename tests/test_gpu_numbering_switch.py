@@ -59,3 +59,28 @@ def test_a_handle_that_returns_to_merging_again_and_again():
         assert lat.info(pla.PL_INFO_BUILD_MERGED) == 0, call
         assert lat.num_vertices == cpu.num_vertices
         assert float(np.abs(out.cpu().numpy() - want).max()) <= 1e-5
+
+
+def test_the_way_to_number_is_kept_while_the_grid_is_the_same():
+    """``filter_image`` sets the grid on every call.  A volume whose tiles share most of their vertices: the
+    pass numbers them from the second call on, until another grid (or, after 32 builds, another count)."""
+    import torch
+    import permutohedral_lattice_amd as pla
+    dims = (48, 96, 96)
+    n = dims[0] * dims[1] * dims[2]
+    gen = torch.Generator("cuda").manual_seed(11)
+    guide = torch.rand((n, 1), device="cuda", generator=gen)
+    val = torch.rand((n, 1), device="cuda", generator=gen)
+    lat = pla.PermutohedralLattice(4, 2, n)
+    outs, rows = [], []
+    for call in range(36):
+        out = torch.empty_like(val)
+        lat.filter_image(out, val, guide, dims if call < 35 else (96, 48, 96), 6.0, 0.2)
+        rows.append(lat.info(pla.PL_INFO_FOREIGN_ROWS))
+        if call < 35:
+            outs.append(out)
+    assert rows[0] > 0 and rows[1] == -1 and rows[32] == -1     # (-1: numbered by the pass)
+    assert rows[33] > 0 and rows[34] == -1 and rows[35] != -1
+    for out in outs[1:]:
+        assert float((out - outs[0]).abs().max()) <= 2e-6
+    lat.close()
