@@ -83,6 +83,7 @@ struct pl_lattice {
     bool f64 = false;
     plk::ScaleFactor64 scale64{};
     double *weights64 = nullptr;       // barycentric weights, layout of the replay rows
+    plk::Points64 image64{};           // the features of a call that gives no positions array (the op's)
 
     // hash table and the per-vertex arrays; a table of n_cells holds at most 3/4 n_cells vertices
     uint64_t *cell_keys = nullptr;     // [n_cells_alloc]
@@ -541,8 +542,16 @@ int enqueue_build(pl_lattice *h, const plk::PointFeatures &features, const doubl
             regions.enabled = 0;
         }
     }
+    if (h->f64 && !positions64) {
+        regions.first = 0.0f;
+        regions.last = (float)((double)((h->map.mode == 3 ? h->map.dims[0] : h->image64.n_spatial_dims == 3 ? 1 : h->map.dims[1]) - 1) /
+                               h->image64.spatial_std);
+    }
     if (h->f64) {
-        const plk::Points64 points{positions64, h->weights64, h->scale64};
+        plk::Points64 points = h->image64;
+        points.positions = positions64;
+        points.weights = h->weights64;
+        points.scale = h->scale64;
         PL_HIP(plk::build_f64(h->pd, points, h->map, h->cell_keys, cells, h->counters(), h->replay,
                               h->xcd_aware ? 1 : 0, lists, regions, merge ? &numbering : nullptr,
                               fused ? h->vd : 0,
@@ -1991,17 +2000,30 @@ extern "C" int pl_lattice_filter_op_f64(const double *input, const double *refer
     if (batch == 0) return PL_OK;
     if (!input || !output) return PL_EINVAL;
 
-    // pl_filter_f64 returns after the build has been waited for, and the build's kernel is the
-    // only reader of the positions, so the next item may overwrite them
+    // The features are made in the build where they can be (features64_from_grid), else as an
+    // array per item, as the reference does: pl_filter_f64 returns after the build has been waited for,
+    // and the build's kernel is the only reader of the positions, so the next item may overwrite them.
+    plk::Points64 image{};
+    image.n_spatial_dims = n_spatial_dims;
+    image.n_reference_channels = ref_ch;
+    image.spatial_std = spatial_std;
+    image.feature_std = feature_std;
+    const bool on_grid = plk::features64_from_grid(image, plk::make_point_map(N, n_spatial_dims, spatial_dims).mode);
     auto filter_items = [&](pl_handle lattice, double *positions) {
         int rc = pl_set_point_grid(lattice, n_spatial_dims, spatial_dims);
         for (int b = 0; b < batch && rc == PL_OK; ++b) {
             const double *ref_b = ref_ch ? reference + (size_t)b * N * ref_ch : nullptr;
+            double *out_b = output + (size_t)b * N * n_input_channels;
+            const double *in_b = input + (size_t)b * N * n_input_channels;
+            if (on_grid) {
+                lattice->image64 = image;
+                lattice->image64.reference = ref_b;
+                rc = filter_lattice(lattice, out_b, in_b, plk::PointFeatures{}, reverse);
+                continue;
+            }
             rc = pl_compute_positions_f64(ref_b, positions, N, ref_ch, n_spatial_dims,
                                           spatial_dims, spatial_std, feature_std, stream);
-            if (rc == PL_OK)
-                rc = pl_filter_f64(lattice, output + (size_t)b * N * n_input_channels,
-                                   input + (size_t)b * N * n_input_channels, positions, reverse);
+            if (rc == PL_OK) rc = pl_filter_f64(lattice, out_b, in_b, positions, reverse);
         }
         return rc;
     };
@@ -2011,7 +2033,7 @@ extern "C" int pl_lattice_filter_op_f64(const double *input, const double *refer
         pl_handle lattice = nullptr;
         int rc = pl_create_f64(pd, vd, N, stream, alloc, &lattice);
         double *positions = nullptr;
-        if (rc == PL_OK) {
+        if (rc == PL_OK && !on_grid) {
             positions = (double *)alloc->alloc(alloc->ctx, position_bytes);
             if (!positions) rc = PL_ENOMEM;
         }
@@ -2027,7 +2049,7 @@ extern "C" int pl_lattice_filter_op_f64(const double *input, const double *refer
     OpCacheEntry *entry = op_cache_entry(device, pd, vd, N, (hipStream_t)stream, true);
     int rc = ensure_lanes(*entry, 1);
     if (rc != PL_OK) return rc;
-    if (!entry->positions64 &&
+    if (!on_grid && !entry->positions64 &&
         hip_failed(hipMalloc((void **)&entry->positions64, position_bytes))) {
         entry->positions64 = nullptr;
         return PL_ENOMEM;

@@ -518,6 +518,12 @@ __device__ __forceinline__ float divided(float a, float b, float inverse) {
     return __builtin_fmaf(__builtin_fmaf(-q, b, a), inverse, q);
 }
 
+__device__ __forceinline__ double divided(double a, double b, double inverse) {
+    double q = a * inverse;
+    q = __builtin_fma(__builtin_fma(-q, b, a), inverse, q);
+    return __builtin_fma(__builtin_fma(-q, b, a), inverse, q);
+}
+
 // Mask of the lanes whose predicate holds (the compare result itself, no detour through 0/1)
 __device__ __forceinline__ uint64_t wave_ballot(bool predicate) {
     return __builtin_amdgcn_ballot_w64(predicate);

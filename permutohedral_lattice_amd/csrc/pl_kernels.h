@@ -122,6 +122,11 @@ struct Points64 {
     const double *positions;
     double *weights;
     ScaleFactor64 scale;
+    // positions == nullptr: the point's grid coordinates (a map of mode 2 or 3, two or three extents)
+    // divided by spatial_std, then its reference channels divided by feature_std (features64_from_grid)
+    const double *reference;
+    int n_spatial_dims, n_reference_channels;
+    double spatial_std, feature_std, inverse_spatial_std, inverse_feature_std;
 };
 
 struct SpatialDims {
@@ -188,6 +193,18 @@ inline void set_inverse_widths(PointFeatures &f) {
     f.multiply = (f.n_spatial_dims == 0 || ordinary(f.spatial_std)) && (f.n_reference_channels == 0 || ordinary(f.feature_std));
     f.inverse_spatial_std = f.multiply && f.n_spatial_dims ? 1.0f / f.spatial_std : 0.0f;
     f.inverse_feature_std = f.multiply && f.n_reference_channels ? 1.0f / f.feature_std : 0.0f;
+}
+
+// The same for doubles; false: these features are made as an array (compute_positions_f64).
+inline bool features64_from_grid(Points64 &p, int map_mode) {
+    auto ordinary = [](double x) { return (x < 0.0 ? -x : x) >= 0x1p-40 && (x < 0.0 ? -x : x) <= 0x1p40; };
+    if (map_mode < 2 || p.n_spatial_dims < 2 || p.n_spatial_dims > 3 || !ordinary(p.spatial_std) ||
+        (p.n_reference_channels > 0 && !ordinary(p.feature_std)))
+        return false;
+    p.positions = nullptr;
+    p.inverse_spatial_std = 1.0 / p.spatial_std;
+    p.inverse_feature_std = p.n_reference_channels > 0 ? 1.0 / p.feature_std : 0.0;
+    return true;
 }
 
 // How threads are laid over the points (see point_of_thread in pl_kernels.hip).

@@ -102,6 +102,43 @@ __device__ __forceinline__ void load_features(const PointFeatures &f, const Poin
     }
 }
 
+// Features of doubles: the positions array's row, or made from the grid as k_positions_f64 makes them (its
+// divisions rounded the same; the array's way through memory and its launch were 13 of 93 us of a call on
+// 601x803 points, pd 5).
+template <int PD>
+__device__ __forceinline__ void load_features64(const Points64 &p, int n, const int (&at)[3], double (&pos)[PD]) {
+    if (p.positions) {
+#pragma unroll
+        for (int i = 0; i < PD; ++i) pos[i] = p.positions[(size_t)n * PD + i];
+        return;
+    }
+    double channel[PD];
+    if (p.n_reference_channels > 0) {
+        const double *row = p.reference + (size_t)n * p.n_reference_channels;
+#pragma unroll
+        for (int i = 0; i < PD; ++i) {
+            const int j = i - p.n_spatial_dims;
+            channel[i] = row[j >= 0 && j < p.n_reference_channels ? j : 0];
+        }
+    }
+    const double z = divided((double)at[0], p.spatial_std, p.inverse_spatial_std);
+    const double y = divided((double)at[1], p.spatial_std, p.inverse_spatial_std);
+    const double x = divided((double)at[2], p.spatial_std, p.inverse_spatial_std);
+    pos[0] = p.n_spatial_dims == 3 ? z : y;
+    if constexpr (PD >= 2) pos[1] = p.n_spatial_dims == 3 ? y : x;
+    if constexpr (PD >= 3) pos[2] = x;
+    if (p.n_reference_channels > 0) {
+#pragma unroll
+        for (int i = 0; i < PD; ++i) {
+            if (i >= p.n_spatial_dims) {
+                // (a quotient that is none, infinite or far beyond any lattice stays what it is)
+                const double q = channel[i] * p.inverse_feature_std;
+                pos[i] = __builtin_fabs(q) < 0x1p80 ? divided(channel[i], p.feature_std, p.inverse_feature_std) : q;
+            }
+        }
+    }
+}
+
 // ------------------------------------------------------------------------------------------------
 // Hash table
 // ------------------------------------------------------------------------------------------------
@@ -244,7 +281,8 @@ __global__ __launch_bounds__(kBlock) void k_build(PointFeatures features, PointM
     if constexpr (kDouble) {
         double pos[PD];
 #pragma unroll
-        for (int i = 0; i < PD; ++i) pos[i] = valid ? points64.positions[(size_t)n * PD + i] : 0.0;
+        for (int i = 0; i < PD; ++i) pos[i] = 0.0;
+        if (valid) load_features64<PD>(points64, n, at, pos);
         enclosing_simplex<PD>(pos, points64.scale, s);
     } else {
         float pos[PD];
@@ -631,7 +669,8 @@ __global__ __launch_bounds__(kBlock) __attribute__((amdgpu_num_sgpr(102))) void 
     if constexpr (kDouble) {
         double pos[PD];
 #pragma unroll
-        for (int i = 0; i < PD; ++i) pos[i] = valid ? points64.positions[(size_t)n * PD + i] : 0.0;
+        for (int i = 0; i < PD; ++i) pos[i] = 0.0;
+        if (valid) load_features64<PD>(points64, n, at, pos);
         enclosing_simplex<PD>(pos, points64.scale, s);
     } else {
         float pos[PD];

@@ -33,3 +33,28 @@ def test_features_of_the_grid(dims, channels, widths):
     want = rows(lat, lambda: lat.build(positions))
     assert (got[0] == want[0]).all() and (got[1] == want[1]).all()
     lat.close()
+
+
+@pytest.mark.parametrize("dims", [(5,), (17, 23), (1, 40), (64, 1, 48), (3, 9, 21), (1, 30, 33), (2, 3, 9, 17), (33, 70), (40, 2)])
+@pytest.mark.parametrize("channels", [0, 1, 3])
+@pytest.mark.parametrize("widths", [(8.0, 0.125), (3.3, 0.07), (0.37, 13.0), (2.0 ** 41, 0.2)])
+def test_features_of_doubles_from_the_grid(dims, channels, widths):
+    """The op makes them in the build where the points are a grid of two or three extents: the same filter as
+    under the positions array, up to the order of additions (the sums of a vertex are at most some
+    hundred terms: 1e-13 of values in [0, 1])."""
+    n, pd = int(np.prod(dims)), len(dims) + channels
+    rng = np.random.default_rng(n + channels)
+    value = torch.from_numpy(rng.uniform(0, 1, (2, n, 2))).cuda()
+    image = torch.from_numpy(rng.uniform(0, 1, (2, n, channels))).cuda() if channels else None
+    got = pla.lattice_filter(value.view((2,) + dims + (2,)), image.view((2,) + dims + (channels,)) if channels else None,
+                             bilateral=channels > 0, theta_alpha=widths[0], theta_beta=widths[1], theta_gamma=widths[0])
+    want = torch.empty_like(value)
+    for b in range(2):
+        # (the op's attributes are floats for every value type)
+        positions = pla.compute_positions(image[b] if channels else None, dims, float(np.float32(widths[0])),
+                                          float(np.float32(widths[1])), dtype=torch.float64)
+        lat = pla.PermutohedralLattice(pd, 3, n, dtype=torch.float64)
+        lat.set_point_grid(dims)
+        lat.filter(want[b], value[b], positions)
+        lat.close()
+    assert float((got.view(want.shape) - want).abs().max()) <= 1e-13
