@@ -1617,7 +1617,7 @@ __device__ __forceinline__ void gather_elements(const S *__restrict__ src, int v
     for (int k = 0; k < N; ++k) x[k] = u[k] >= 0 ? x[k] : (S)0;
 }
 
-// one thread per (vertex, channel), any vd
+// one thread per (vertex, channel): doubles of more than four channels (floats: k_blur_runs, pl_many.hip)
 template <typename S>
 __global__ __launch_bounds__(kBlock) void k_blur_element(const Counters *counters, int max_vertices,
                                                           int vd, const S *__restrict__ src,
@@ -2491,9 +2491,8 @@ hipError_t blur_axis(int vd, const Counters *counters, int max_vertices, const f
         default: break;
     }
 #undef PLK_BLUR_ROW
-    hipLaunchKernelGGL(k_blur_element<float>, dim3(vertex_blocks((size_t)launch_vertices * vd)), dim3(kBlock), 0, s,
-                       counters, max_vertices, vd, src, dst, nbr, reset_cell_keys, vertex_cell);
-    return hipGetLastError();
+    const BlurWork work{counters, src, dst, nbr, nullptr, reset_cell_keys, vertex_cell, max_vertices, launch_vertices};
+    return blur_many(vd, 1, &work, s);
 }
 
 hipError_t blur_two_axes(int vd, const Counters *counters, int max_vertices, const float *src,
@@ -2514,10 +2513,9 @@ hipError_t blur_two_axes(int vd, const Counters *counters, int max_vertices, con
         default: break;
     }
 #undef PLK_BLUR2_ROW
-    hipLaunchKernelGGL(k_blur2_element<float>, dim3(vertex_blocks((size_t)launch_vertices * vd)), dim3(kBlock), 0, s,
-                       counters, max_vertices, vd, src, dst, nbr_first, nbr_second, reset_cell_keys,
-                       vertex_cell);
-    return hipGetLastError();
+    const BlurWork work{counters, src, dst, nbr_first, nbr_second, reset_cell_keys, vertex_cell, max_vertices,
+                        launch_vertices};
+    return blur_many(vd, 1, &work, s);
 }
 
 // The blur of a lattice of doubles: the same kernels over the value type.

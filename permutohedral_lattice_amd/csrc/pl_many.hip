@@ -26,7 +26,8 @@ struct alignas(4) FourFloats {
 // twice, the same), one axis or two as k_blur_element and k_blur2_element of pl_kernels.hip apply them: same
 // arithmetic, same results, a quarter of the load instructions.  Bound by three round trips to memory, in
 // one launch for all lattices (two images, 97 000 vertices of 22 channels: 8.8 us a pass of two axes; a
-// launch a lattice 5.4 us each).
+// launch a lattice, a thread per channel, 5.4 us each).  A lattice alone takes it too (an op and its
+// gradient on 2 x 321x481 points of 21 channels, twelve passes of two axes: 306.7 and 292.8 us).
 // ------------------------------------------------------------------------------------------------
 __device__ __forceinline__ FourFloats blur_taps(const FourFloats &a, const FourFloats &self, const FourFloats &b) {
     FourFloats out;
@@ -52,7 +53,8 @@ __device__ __forceinline__ void gather_runs(const float *__restrict__ src, int v
         for (int j = 0; j < 4; ++j) x[k].c[j] = u[k] >= 0 ? x[k].c[j] : 0.0f;
     }
 }
-__global__ __launch_bounds__(kBlock) void k_blur_runs(Items<BlurWork> items, int vd) {
+template <int N>   // lattices a launch may be given
+__global__ __launch_bounds__(kBlock) void k_blur_runs(Items<BlurWork, N> items, int vd) {
     unsigned block, blocks;
     const BlurWork &work = item_of(items, block, blocks);
     const unsigned runs = (unsigned)(vd + 3) / 4u;
@@ -212,17 +214,21 @@ __global__ __launch_bounds__(kBlock) void k_slice_pairs(Items<SlicePair> items, 
 
 }  // namespace
 
-hipError_t blur_many(int vd, int n, const BlurWork *work, hipStream_t s) {
-    if (n < 1 || n > kManyItems || vd < 4) return hipErrorInvalidValue;
-    Items<BlurWork> items{};
+template <int N>
+static hipError_t blur_runs(int vd, int n, const BlurWork *work, hipStream_t s) {
+    Items<BlurWork, N> items{};
     items.n = n;
     const unsigned runs = (unsigned)(vd + 3) / 4u;
     for (int i = 0; i < n; ++i) {
         items.item[i] = work[i];
         items.blocks[i] = vertex_blocks((size_t)work[i].launch_vertices * runs);
     }
-    hipLaunchKernelGGL(k_blur_runs, dim3(all_blocks(items)), dim3(kBlock), 0, s, items, vd);
+    hipLaunchKernelGGL((k_blur_runs<N>), dim3(all_blocks(items)), dim3(kBlock), 0, s, items, vd);
     return hipGetLastError();
+}
+hipError_t blur_many(int vd, int n, const BlurWork *work, hipStream_t s) {
+    if (n < 1 || n > kManyItems || vd < 5) return hipErrorInvalidValue;
+    return n == 1 ? blur_runs<1>(vd, n, work, s) : blur_runs<kManyItems>(vd, n, work, s);
 }
 
 bool slice_pairs_take(int pd_a, int pd_b, int vd) {
