@@ -305,17 +305,20 @@ __global__ __launch_bounds__(kBlock) void k_build(PointFeatures features, PointM
     // table.
     using Key = std::conditional_t<WIDE, Key128, uint64_t>;
     Key key[D1];
-    // (leader lanes are kept five to a register, six bits each: registers decide how many
-    // wavefronts a CU holds)
-    unsigned leaders[(D1 + 4) / 5] = {};
-    auto leader_of = [&](int r) { return (int)((leaders[r / 5] >> (6 * (r % 5))) & 63u); };
-    if constexpr (WIDE)
+    // (keys of one word: the groups also in order, for the sums; of two words: the leaders' lanes)
+    unsigned group[D1];
+    if constexpr (WIDE) {
         wide_keys_of<PD>(s, key);
-    else
-        vertex_keys_of<PD>(s, key);
 #pragma unroll
-    for (int r = 0; r < D1; ++r)
-        leaders[r / 5] |= (unsigned)wave_leader_of_equal(key[r], active, lane) << (6 * (r % 5));
+        for (int r = 0; r < D1; ++r) group[r] = (unsigned)wave_leader_of_equal(key[r], active, lane);
+    } else {
+        vertex_keys_of<PD>(s, key);
+        const uint64_t among = wave_ballot(active);
+        unsigned n_groups = 0;
+#pragma unroll
+        for (int r = 0; r < D1; ++r) group[r] = wave_groups_in_order(key[r], among, &n_groups);
+    }
+    auto leads = [&](int r) { return active && (WIDE ? (int)group[r] == lane : rank_of(group[r]) == 0); };
 
     // Insertion of a lane's pd+1 keys proceeds in rounds over all of them at once, so that the
     // loads and compare-and-swaps of one round are in flight together: a round loads the current
@@ -332,7 +335,7 @@ __global__ __launch_bounds__(kBlock) void k_build(PointFeatures features, PointM
     unsigned created = 0;   // bit r: this lane's swap made the vertex of rank r
 #pragma unroll
     for (int r = 0; r < D1; ++r)
-        if (active && leader_of(r) == lane) open |= 1u << r;
+        if (leads(r)) open |= 1u << r;
     bool any_open = open != 0;
     if constexpr (WIDE) {
         // Rounds as below.  Words are read past the first-level cache: a second word may arrive
@@ -469,16 +472,33 @@ __global__ __launch_bounds__(kBlock) void k_build(PointFeatures features, PointM
         }
     }
 
+    // the sums of a wavefront's groups, one corner at a time: rows of P values, and their cells
+    constexpr int VD = SPLAT_VD ? SPLAT_VD : 2, P = VD == 2 ? 2 : 4;
+    __shared__ float group_row[SPLAT_VD && !WIDE ? kBlock / 64 : 1][64 * P];
+    __shared__ int group_cell[SPLAT_VD && !WIDE ? kBlock / 64 : 1][64];
+    bool tame = false;   // (what sum_groups_in_order asks of its terms, as in add_to_slots)
+    if constexpr (SPLAT_VD != 0 && !WIDE) {
+        float all = 0.0f;
+#pragma unroll
+        for (int r = 0; r < D1; ++r) all += (float)s.weight[r];
+#pragma unroll
+        for (int j = 0; j < VD; ++j) all += __builtin_fabsf(val[j]);
+        tame = wave_ballot(!(all < 1e30f)) == 0;
+    }
 #pragma unroll
     for (int r = 0; r < D1; ++r) {
         const int own = (open >> r) & 1u ? -1 : (int)cell[r];
-        const int leader = leader_of(r);
-        const int c = __shfl(own, leader);
+        int c;
+        if constexpr (WIDE) {
+            c = __shfl(own, (int)group[r]);
+        } else {
+            // (the lowest lane of a group is the first of it in the order)
+            const int in_order = to_place(group[r], own);
+            c = __shfl(in_order, (int)(group[r] >> 17) - (int)rank_of(group[r]));
+        }
         replay[(size_t)r * n_slots + t] = ReplayEntry{active ? c : -1, valid ? (float)s.weight[r] : 0.0f};
         if constexpr (kDouble) points64.weights[(size_t)r * n_slots + t] = valid ? s.weight[r] : 0.0;
-        if (SPLAT_VD) {
-            constexpr int VD = SPLAT_VD ? SPLAT_VD : 2;
-            constexpr int P = VD == 2 ? 2 : 4;
+        if constexpr (SPLAT_VD != 0 && WIDE) {
             const float w = (float)s.weight[r];
             const float term[4] = {w * val[0], w * val[1], w * val[2], w * val[3]};
             const QuadTerms quad = quad_terms<VD>(term, lane);
@@ -486,13 +506,49 @@ __global__ __launch_bounds__(kBlock) void k_build(PointFeatures features, PointM
             uint64_t remaining = among;
             while (remaining) {
                 const int first = __builtin_ctzll(remaining);
-                const uint64_t group = lanes_equal(leader, first) & among;
-                remaining &= ~group;
-                const bool same = lane_in(group);
-                const int group_cell = lane_value(own, first);
+                const uint64_t of_group = lanes_equal((int)group[r], first) & among;
+                remaining &= ~of_group;
+                const bool same = lane_in(of_group);
+                const int cell_of_group = lane_value(own, first);
                 const float sum = wave_sum_to_last_lanes<VD>(same, quad, lane);
-                if (group_cell >= 0 && lane >= 64 - P && channel_of_lane<VD>(lane) < VD)
-                    atomicAdd(cell_values + (size_t)group_cell * VD + channel_of_lane<VD>(lane), sum);
+                if (cell_of_group >= 0 && lane >= 64 - P && channel_of_lane<VD>(lane) < VD)
+                    atomicAdd(cell_values + (size_t)cell_of_group * VD + channel_of_lane<VD>(lane), sum);
+            }
+        } else if constexpr (SPLAT_VD != 0) {
+            // All groups of the corner side by side (sum_groups_in_order); their rows meet in LDS, so
+            // that P consecutive lanes send a row as one request.  What bounds the kernel is a
+            // wavefront's instructions in their turn: 120x160 points, pd 5, vd 4, about a hundred groups a
+            // wavefront, 32.4 us with a tree and a request for every group in turn and the grouping
+            // compiled from a loop, this 18.4.
+            if (tame) {
+                const int at = to_place(group[r], active ? c : -1);
+                const unsigned rank = (unsigned)to_place(group[r], (int)rank_of(group[r]));
+                float term[VD];
+#pragma unroll
+                for (int j = 0; j < VD; ++j) term[j] = to_place(group[r], (float)s.weight[r] * val[j]);
+                sum_groups_in_order(term, steps_that_count(lane, rank));
+                // (wave_shl:1, a zero above lane 63)
+                const unsigned above = (unsigned)__builtin_amdgcn_update_dpp(0, (int)rank, 0x130, 0xf, 0xf, true);
+                const bool ends = above == 0 && at >= 0;
+                const uint64_t ending = wave_ballot(ends);
+                const int n_rows = lanes_in(ending), wave = threadIdx.x >> 6;
+                if (ends) {
+                    const int i = (int)__builtin_amdgcn_mbcnt_hi((uint32_t)(ending >> 32),
+                                                                 __builtin_amdgcn_mbcnt_lo((uint32_t)ending, 0u));
+                    group_cell[wave][i] = at;
+#pragma unroll
+                    for (int j = 0; j < VD; ++j) group_row[wave][i * P + j] = term[j];
+                }
+                __builtin_amdgcn_wave_barrier();
+                const int channel = lane % P;
+                for (int i = lane / P; i < n_rows; i += 64 / P)
+                    if (channel < VD)
+                        atomicAdd(cell_values + (size_t)group_cell[wave][i] * VD + channel, group_row[wave][i * P + channel]);
+                __builtin_amdgcn_wave_barrier();
+            } else if (active && c >= 0) {
+#pragma unroll
+                for (int j = 0; j < VD; ++j)
+                    atomicAdd(cell_values + (size_t)c * VD + j, (float)s.weight[r] * val[j]);
             }
         }
     }

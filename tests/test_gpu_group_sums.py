@@ -1,4 +1,4 @@
-"""The sums of the merging build: groups of one lane, of a whole wavefront and of lanes that are not next
+"""The sums of the builds, with tiles merged and without: groups of one lane, of a whole wavefront and of lanes that are not next
 to each other, tiles that are not full, and values that are not finite or near the largest, which take
 the sums lane by lane; filter against the oracle."""
 import numpy as np
@@ -54,3 +54,29 @@ def test_sums_of_groups(kind, h, w, vd, dtype):
             if fine.any():
                 assert np.abs(got - want).max() <= MAX_ABS_TOL and rel_l2(got, want) <= REL_L2_TOL
     lat.close()
+
+
+@pytest.mark.parametrize("vd", [2, 3, 4])
+@pytest.mark.parametrize("kind,h,w", [("one", 16, 16), ("own", 16, 16), ("mixed", 17, 23), ("noise", 40, 33),
+                                      ("own", 1, 1), ("noise", 9, 7)])
+def test_sums_of_groups_without_merging(kind, h, w, vd):
+    rng = np.random.default_rng(100 * vd + h * w)
+    pos = np.ascontiguousarray(positions(kind, h, w, rng), dtype=np.float32)
+    n, pd = pos.shape
+    out = torch.empty((n, vd - 1), dtype=torch.float32, device="cuda")
+    large = float(np.finfo(np.float32).max) / 4
+    for extreme in (None, large, np.inf, np.nan):
+        val = rng.uniform(0.1, 1, (n, vd - 1)).astype(np.float32)
+        if extreme is not None:
+            val[n // 2, -1] = extreme
+        pla.filter_static(out, torch.from_numpy(val).cuda(), torch.from_numpy(pos).cuda(), pd, vd)
+        with np.errstate(all="ignore"):
+            want = oracle.Lattice(pd, vd, n, dtype=np.float32).filter(val, pos, False)
+        got = out.cpu().numpy()
+        fine = np.isfinite(want)
+        assert (np.isfinite(got) == fine).all()
+        assert (np.isnan(got) == np.isnan(want)).all()
+        scale = large if extreme == large else 1.0
+        got, want = got[fine] / scale, want[fine] / scale
+        if fine.any():
+            assert np.abs(got - want).max() <= MAX_ABS_TOL and rel_l2(got, want) <= REL_L2_TOL
