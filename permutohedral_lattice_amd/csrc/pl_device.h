@@ -649,6 +649,15 @@ __device__ __forceinline__ unsigned wave_groups_in_order(uint64_t x, uint64_t am
 __device__ __forceinline__ unsigned number_of(unsigned group) { return group & 0x3ffu; }
 __device__ __forceinline__ unsigned rank_of(unsigned group) { return (group >> 10) & 0x7fu; }
 
+// What the lanes of the wavefront have written to LDS is there for its others, and what they have read is
+// read, before anything behind: an order for the compiler (also between accesses of different types); the
+// LDS takes a wavefront's instructions in their turn by itself, so this is no instruction.
+__device__ __forceinline__ void wave_exchange_in_lds() {
+    __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
+    __builtin_amdgcn_wave_barrier();
+    __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
+}
+
 // x of the lane whose place in the order (of its own `group`) is this lane.  (The address of ds_permute
 // is the lane times four; the bits below are not looked at, and those above are zero.)
 __device__ __forceinline__ int to_place(unsigned group, int x) {

@@ -539,12 +539,12 @@ __global__ __launch_bounds__(kBlock) void k_build(PointFeatures features, PointM
 #pragma unroll
                     for (int j = 0; j < VD; ++j) group_row[wave][i * P + j] = term[j];
                 }
-                __builtin_amdgcn_wave_barrier();
+                wave_exchange_in_lds();
                 const int channel = lane % P;
                 for (int i = lane / P; i < n_rows; i += 64 / P)
                     if (channel < VD)
                         atomicAdd(cell_values + (size_t)group_cell[wave][i] * VD + channel, group_row[wave][i * P + channel]);
-                __builtin_amdgcn_wave_barrier();
+                wave_exchange_in_lds();
             } else if (active && c >= 0) {
 #pragma unroll
                 for (int j = 0; j < VD; ++j)
@@ -582,7 +582,7 @@ __device__ __forceinline__ bool place_groups(const Key (&key)[D1], const unsigne
             const unsigned to = number_of(group[r]) - from;
             if (((present >> r) & 1u) && rank_of(group[r]) == 0 && to < 64u) wave_keys[to] = key[r];
         }
-        __builtin_amdgcn_wave_barrier();
+        wave_exchange_in_lds();
         const Key mine = wave_keys[lane];
         int at_slot = (int)(hash(mine) >> kTileSlotShift);
         bool open = from + (unsigned)lane < n_groups, was_empty = false;
@@ -600,9 +600,9 @@ __device__ __forceinline__ bool place_groups(const Key (&key)[D1], const unsigne
             placed = false;
             at_slot = -1;
         }
-        __builtin_amdgcn_wave_barrier();
+        wave_exchange_in_lds();
         wave_slots[kStride * lane] = at_slot;
-        __builtin_amdgcn_wave_barrier();
+        wave_exchange_in_lds();
 #pragma unroll
         for (int r = 0; r < D1; ++r) {
             const unsigned to = number_of(group[r]) - from;
@@ -610,7 +610,7 @@ __device__ __forceinline__ bool place_groups(const Key (&key)[D1], const unsigne
         }
         // the slots that were empty join the list of slots in use
         if (was_empty) occupied[atomicAdd(n_occupied, 1)] = (unsigned short)at_slot;
-        __builtin_amdgcn_wave_barrier();
+        wave_exchange_in_lds();
     }
     return placed;
 }
@@ -1457,7 +1457,7 @@ __global__ __launch_bounds__(kBlock) void k_splat_merge(PointMap map, const floa
         if (channel < VD) atomicAdd(values + (size_t)v * VD + channel, slot_sum[sl * P + channel]);
         // (read by this lane's row alone until the barrier below)
         if (cell_vertex) {
-            __builtin_amdgcn_wave_barrier();
+            wave_exchange_in_lds();
             if (channel == 0) slot_index[sl] = v;
         }
     }
