@@ -375,10 +375,12 @@ int pl_mean_field_update(float *q, const float *logits, const float *message_a,
  *   pl_mean_field_infer: q = softmax(logits), then `iterations` times
  *                        q = softmax(logits + bilateral(q) + spatial(q)); q and logits 16-byte aligned.
  * The same as pl_apply on every lattice and pl_mean_field_update, with each pass of all lattices in one launch
- * on `stream`: enqueued behind what the lattices' own streams hold, and what these are given next comes
- * behind it.  output and q are arrays of their own.  PL_EUNSUPPORTED (nothing is enqueued) where the
+ * on `stream`: enqueued behind all that has been enqueued on the lattices (by other calls, or as the replay of
+ * a captured pl_apply on a lattice's own stream), and what their own streams are given next comes behind it;
+ * the arrays are read and written in the order of `stream`.  output and q are arrays of their own.  PL_EUNSUPPORTED (nothing is enqueued) where the
  * lattices must be applied one by one: no vertex lists, options that change an apply, 4 classes to 31 only,
- * two or three spatial dimensions with a guide of one or three channels, a stream that is being captured.
+ * two or three spatial dimensions with a guide of one or three channels, `stream` or a lattice's own being
+ * captured.
  * ---------------------------------------------------------------------------------------- */
 int pl_mean_field_messages(int n, const pl_handle *bilateral, const pl_handle *spatial, float *output,
                            const float *input, int reverse, pl_stream stream);

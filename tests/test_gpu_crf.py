@@ -213,3 +213,81 @@ def test_lattices_applied_together_from_two_streams():
         assert float((q - want[turn % 2][0]).abs().max()) <= 1e-6
         assert float((back - want[turn % 2][1].view(x.shape)).abs().max()) <= 1e-5
     mf.close()
+
+
+def _one_by_one(mf, x):
+    mf._apply_all(x, False)
+    out = mf._msg_bi + mf._msg_sp
+    torch.cuda.synchronize()
+    return out
+
+
+def test_lattices_on_one_stream_applied_together_from_it_and_another():
+    """Calls on another stream, the lattices' own and the other again, nothing built or applied in between
+    and no wait by the caller: they share the lattices' value tables alone."""
+    gen = torch.Generator("cuda").manual_seed(6)
+    guide = torch.rand((2, 96, 120, 3), device="cuda", generator=gen) * 255.0
+    own, other = torch.cuda.Stream(), torch.cuda.Stream()
+    torch.cuda.synchronize()
+    with torch.cuda.stream(own):
+        mf = MeanField(guide, 21, concurrent=False)
+    xs = [torch.randn((2, 96, 120, 21), device="cuda", generator=gen) for _ in range(6)]
+    torch.cuda.synchronize()
+    with torch.cuda.stream(own):
+        want = [_one_by_one(mf, x) for x in xs]
+    got = []
+    for i, x in enumerate(xs):
+        with torch.cuda.stream(own if i in (1, 3, 4) else other):
+            got.append(mf.messages(x))
+    torch.cuda.synchronize()
+    for g, w in zip(got, want):
+        assert float((g - w).abs().max()) <= 1e-5
+    mf.close()
+
+
+def test_work_on_a_lattice_s_own_stream_between_calls_that_apply_them_together():
+    """An export of the vertex values, and the replay of a captured apply: both only on the lattice's own
+    stream, the calls before and behind on the same other one."""
+    gen = torch.Generator("cuda").manual_seed(7)
+    guide = torch.rand((2, 96, 120, 3), device="cuda", generator=gen) * 255.0
+    xs = [torch.randn((2, 96, 120, 21), device="cuda", generator=gen) for _ in range(2)]
+    mf = MeanField(guide, 21)
+    own, other = mf._streams[2], torch.cuda.Stream()   # (own: of the second image's bilateral lattice)
+    lat = mf.bilateral[1]
+    want = [_one_by_one(mf, x) for x in xs]
+    q = [mf.infer(x, 2) for x in xs]
+    torch.cuda.synchronize()
+    values = lat.debug_values()
+    torch.cuda.synchronize()
+    with torch.cuda.stream(other):
+        again = mf.infer(xs[1], 2)
+        exported = lat.debug_values()
+        behind = mf.infer(xs[0], 2)
+    torch.cuda.synchronize()
+    assert torch.equal(exported, values)
+    assert float((again - q[1]).abs().max()) <= 1e-6 and float((behind - q[0]).abs().max()) <= 1e-6
+    static_in = xs[0][1].reshape(-1, 21).contiguous()
+    static_out, alone = torch.empty_like(static_in), torch.empty_like(static_in)
+    torch.cuda.synchronize()
+    with torch.cuda.stream(own):
+        lat.apply(alone, static_in)
+    torch.cuda.synchronize()
+    graph = torch.cuda.CUDAGraph()
+    with torch.cuda.graph(graph, stream=own):
+        lat.apply(static_out, static_in)
+    for _ in range(3):
+        with torch.cuda.stream(own):
+            static_out.zero_()
+        got = []
+        for i in (1, 0):
+            with torch.cuda.stream(other):
+                got.append(mf.messages(xs[i]))
+            with torch.cuda.stream(own):
+                graph.replay()
+        with torch.cuda.stream(other):
+            got.append(mf.messages(xs[1]))
+        torch.cuda.synchronize()
+        assert float((static_out - alone).abs().max()) <= 1e-5
+        for g, i in zip(got, (1, 0, 1)):
+            assert float((g - want[i]).abs().max()) <= 1e-5
+    mf.close()
