@@ -1743,6 +1743,7 @@ int enqueue_pairs(int n, const pl_handle *bilateral, const pl_handle *spatial, f
         PL_HIP(plk::splat_gather_many(vd, vd - 1, 2 * pairs, gather, stream));
         for (int step = 0;; step += 2) {
             plk::BlurWork blur[plk::kManyItems];
+            pl_lattice *blurred[plk::kManyItems];
             int left = 0;
             for (int i = 0; i < 2 * pairs; ++i) {
                 pl_lattice *h = lattice[i];
@@ -1750,15 +1751,18 @@ int enqueue_pairs(int n, const pl_handle *bilateral, const pl_handle *spatial, f
                 const int mv = h->max_vertices(), cur = h->current_values;
                 const int axis = reverse ? h->pd - step : step, second = reverse ? axis - 1 : axis + 1;
                 const bool reset = !h->table_clean && step == 0 && !h->wide_keys;
+                blurred[left] = h;
                 blur[left++] = plk::BlurWork{h->counters(), h->values[cur], h->values[1 - cur],
                                              h->neighbours + (size_t)axis * mv,
                                              step + 1 <= h->pd ? h->neighbours + (size_t)second * mv : nullptr,
                                              reset ? h->cell_keys : nullptr, h->vertex_cell, mv, h->launch_vertices()};
-                if (reset) h->table_clean = true;
-                h->current_values = 1 - cur;
             }
             if (!left) break;
             PL_HIP(plk::blur_many(vd, left, blur, stream));
+            for (int i = 0; i < left; ++i) {
+                if (blur[i].reset_cell_keys) blurred[i]->table_clean = true;
+                blurred[i]->current_values = 1 - blurred[i]->current_values;
+            }
         }
         plk::SlicePair slice[kPairsPerLaunch];
         for (int i = 0; i < pairs; ++i) {

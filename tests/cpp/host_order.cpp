@@ -64,9 +64,14 @@ struct Array {
 };
 std::map<const void *, Array> g_arrays;
 std::vector<std::string> g_launches;
+std::string g_fail_next;   // the launch of this name fails, once
 
 hipError_t launch(const char *name, hipStream_t s, const std::vector<const void *> &reads,
                   const std::vector<const void *> &writes) {
+    if (g_fail_next == name) {
+        g_fail_next.clear();
+        return hipErrorInvalidValue;
+    }
     g_launches.push_back(name);
     Stream &stream = stream_of(s);
     if (stream.capturing) return hipSuccess;
@@ -81,6 +86,11 @@ hipError_t launch(const char *name, hipStream_t s, const std::vector<const void 
     for (const void *p : writes)
         if (p) behind(g_arrays[p].writes), behind(g_arrays[p].reads), g_arrays[p].writes.push_back(now);
     return hipSuccess;
+}
+bool launched(const char *name) {
+    for (const auto &l : g_launches)
+        if (l == name) return true;
+    return false;
 }
 
 const float *g_values[2];             // value tables of the lattice blurred last in a joint pass
@@ -349,6 +359,16 @@ void own_stream_captured() {
     expect(g_launches.size() == before, "something was enqueued");
 }
 
+// the launch that would have emptied the hash cells fails: the next build empties the table
+void failed_blur() {
+    Pairs p(four_streams());
+    g_fail_next = "blur_many";
+    expect(p.send(named_stream(9)) == PL_EHIP, "a launch failed");
+    g_launches.clear();
+    p.build();
+    expect(launched("clear_table"), "the table is taken to be empty");
+}
+
 }  // namespace
 
 int main(int argc, char **argv) {
@@ -359,6 +379,7 @@ int main(int argc, char **argv) {
         {"handle_given_out_again", handle_given_out_again},
         {"two_callers_and_builds", two_callers_and_builds},
         {"own_stream_captured", own_stream_captured},
+        {"failed_blur", failed_blur},
     };
     const auto found = scenarios.find(argc > 1 ? argv[1] : "");
     if (found == scenarios.end()) {
