@@ -111,7 +111,8 @@ class MeanField:
         return self._msg_bi + self._msg_sp
 
     def infer(self, logits, iterations=5):
-        """-> Q after ``iterations`` mean-field updates, shaped like ``logits``."""
+        """-> Q after ``iterations`` mean-field updates, shaped like ``logits`` (none for a negative count)."""
+        iterations = len(range(iterations))
         flat = logits.contiguous().view(self.batch, self.n, self.n_classes)
         own = self._own_messages() and mean_field_update_supported(flat)
         if own and self.batch:

@@ -291,3 +291,18 @@ def test_work_on_a_lattice_s_own_stream_between_calls_that_apply_them_together()
         for g, i in zip(got, (1, 0, 1)):
             assert float((g - want[i]).abs().max()) <= 1e-5
     mf.close()
+
+
+def test_the_number_of_iterations_is_what_range_makes_of_it():
+    """A negative count is none, a whole number of any type counts, and a fraction is refused, whether the
+    lattices are applied together or one by one."""
+    guide = torch.rand((1, 24, 32, 3), device="cuda") * 255.0
+    for classes in (5, 3):
+        logits = torch.randn((1, 24, 32, classes), device="cuda")
+        mf = MeanField(guide, classes)
+        for none in (0, -1, np.int64(-3)):
+            assert float((mf.infer(logits, none) - torch.softmax(logits, dim=-1)).abs().max()) <= 1e-6
+        assert float((mf.infer(logits, np.int32(2)) - mf.infer(logits, 2)).abs().max()) <= 1e-6
+        with pytest.raises(TypeError):
+            mf.infer(logits, 2.0)
+        mf.close()
