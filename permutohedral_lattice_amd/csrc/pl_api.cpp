@@ -83,7 +83,7 @@ struct pl_lattice {
     bool f64 = false;
     plk::ScaleFactor64 scale64{};
     double *weights64 = nullptr;       // barycentric weights, layout of the replay rows
-    plk::Points64 image64{};           // the features of a call that gives no positions array (the op's)
+    plk::Points64 image64{};           // the features while a call runs that gives no positions array (the op's)
 
     // hash table and the per-vertex arrays; a table of n_cells holds at most 3/4 n_cells vertices
     uint64_t *cell_keys = nullptr;     // [n_cells_alloc]
@@ -2044,6 +2044,7 @@ extern "C" int pl_lattice_filter_op_f64(const double *input, const double *refer
                 lattice->image64 = image;
                 lattice->image64.reference = ref_b;
                 rc = filter_lattice(lattice, out_b, in_b, plk::PointFeatures{}, reverse);
+                lattice->image64 = plk::Points64{};   // (the reference image is the caller's)
                 continue;
             }
             rc = pl_compute_positions_f64(ref_b, positions, N, ref_ch, n_spatial_dims,

@@ -93,6 +93,7 @@ bool launched(const char *name) {
     return false;
 }
 
+plk::Points64 g_points64;             // of the last build of doubles
 const float *g_values[2];             // value tables of the lattice blurred last in a joint pass
 
 void report(plk::HostReport to) {
@@ -180,6 +181,12 @@ hipError_t build(int, const PointFeatures &, const PointMap &, const ScaleFactor
                  const RegionSource &, const InBuildNumbering *, bool, hipStream_t s) {
     return launch("build", s, {}, {keys, replay});
 }
+hipError_t build_f64(int, const Points64 &points, const PointMap &, uint64_t *keys, uint32_t, Counters *,
+                     ReplayEntry *replay, int, const CreatedLists &, const RegionSource &, const InBuildNumbering *,
+                     int, const double *, int, double *, bool, hipStream_t s) {
+    g_points64 = points;
+    return launch("build_f64", s, {}, {keys, replay});
+}
 hipError_t number_vertices(int, const PointMap &, const CreatedLists &, int *, unsigned, const VertexTables &,
                            float *values, int, float *, Counters *, Counters *, HostReport to, bool, hipStream_t s) {
     report(to);
@@ -208,6 +215,10 @@ hipError_t splat_gather_many(int, int, int n, const GatherWork *work, hipStream_
         e = launch("splat_gather_many", s, {work[i].entries, work[i].input}, {work[i].values});
     return e;
 }
+hipError_t splat_f64(int, int, const PointMap &, const double *input, int, ReplayEntry *replay, const double *,
+                     const int *, double *values, int, hipStream_t s) {
+    return launch("splat_f64", s, {input, replay}, {values});
+}
 hipError_t blur_many(int, int n, const BlurWork *work, hipStream_t s) {
     hipError_t e = hipSuccess;
     for (int i = 0; i < n && e == hipSuccess; ++i) {
@@ -225,9 +236,21 @@ hipError_t blur_axis(int, const Counters *, int, const float *src, float *dst, c
                      const int *, int, hipStream_t s) {
     return launch("blur_axis", s, {src}, {dst, reset});
 }
+hipError_t blur_two_axes_f64(int, const Counters *, int, const double *src, double *dst, const int2 *, const int2 *,
+                             uint64_t *reset, const int *, int, hipStream_t s) {
+    return launch("blur_two_axes_f64", s, {src}, {dst, reset});
+}
+hipError_t blur_axis_f64(int, const Counters *, int, const double *src, double *dst, const int2 *, uint64_t *reset,
+                         const int *, int, hipStream_t s) {
+    return launch("blur_axis_f64", s, {src}, {dst, reset});
+}
 hipError_t slice(int, int, const PointMap &, const ReplayEntry *replay, const int *, const float *values,
                  float *output, int, hipStream_t s) {
     return launch("slice", s, {replay, values}, {output});
+}
+hipError_t slice_f64(int, int, const PointMap &, const ReplayEntry *replay, const double *, const int *,
+                     const double *values, double *output, int, hipStream_t s) {
+    return launch("slice_f64", s, {replay, values}, {output});
 }
 hipError_t slice_pairs(int, int, int, int n, const SlicePair *work, hipStream_t s) {
     hipError_t e = hipSuccess;
@@ -238,6 +261,10 @@ hipError_t slice_pairs(int, int, int, int n, const SlicePair *work, hipStream_t 
 }
 hipError_t mean_field_update(float *q, const float *logits, const float *, const float *, size_t, int, hipStream_t s) {
     return launch("mean_field_update", s, {logits}, {q});
+}
+hipError_t compute_positions_f64(const double *reference, double *positions, int, int, int, const SpatialDims &, double,
+                                 double, hipStream_t s) {
+    return launch("compute_positions_f64", s, {reference}, {positions});
 }
 hipError_t export_values(const float *values, int, const VertexNumbers &, float *out, hipStream_t s) {
     return launch("export_values", s, {values}, {out});
@@ -369,6 +396,21 @@ void failed_blur() {
     expect(launched("clear_table"), "the table is taken to be empty");
 }
 
+// the op of doubles leaves no pointer to its reference image in its lattice
+void no_pointer_kept() {
+    const int dims[2] = {kH, kW};
+    double *in = nullptr, *out = nullptr, *reference = nullptr, *positions = nullptr;
+    for (double **p : {&in, &out, &reference, &positions}) (void)hipMalloc((void **)p, sizeof(double) * kH * kW * 5);
+    expect(pl_lattice_filter_op_f64(in, reference, out, 1, 2, dims, 2, 3, 1, 8.0f, 0.1f, 1.0f, 0, nullptr, nullptr) ==
+               PL_OK, "the op");
+    expect(g_points64.reference == reference, "the features come from the reference image");
+    // (the pooled lattice is filtered from a positions array by an op whose points are no grid of tiles)
+    const int flat[1] = {kH * kW};
+    expect(pl_lattice_filter_op_f64(in, reference, out, 1, 1, flat, 2, 4, 1, 8.0f, 0.1f, 1.0f, 0, nullptr, nullptr) ==
+               PL_OK, "the op on a list");
+    expect(g_points64.positions && !g_points64.reference, "the reference image of a call that has returned");
+}
+
 }  // namespace
 
 int main(int argc, char **argv) {
@@ -380,6 +422,7 @@ int main(int argc, char **argv) {
         {"two_callers_and_builds", two_callers_and_builds},
         {"own_stream_captured", own_stream_captured},
         {"failed_blur", failed_blur},
+        {"no_pointer_kept", no_pointer_kept},
     };
     const auto found = scenarios.find(argc > 1 ? argv[1] : "");
     if (found == scenarios.end()) {
