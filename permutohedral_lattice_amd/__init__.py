@@ -428,17 +428,19 @@ def mean_field_update(q, logits, message_a, message_b):
     return q
 
 
-def _handles(lattices):
-    return (C.c_void_p * len(lattices))(*(lat._h for lat in lattices))
+def _handles_of_pairs(bilateral, spatial):
+    if len(bilateral) != len(spatial):
+        raise ValueError("%d bilateral and %d spatial lattices" % (len(bilateral), len(spatial)))
+    return [(C.c_void_p * len(lattices))(*(lat._h for lat in lattices)) for lattices in (bilateral, spatial)]
 
 
 def mean_field_messages(bilateral, spatial, output, input, reverse=False):
     """``output = bilateral(input) + spatial(input)`` for ``[n, N, classes]`` arrays and n lattices each,
     on the current stream.  False: these lattices must be applied one by one."""
+    handles = _handles_of_pairs(bilateral, spatial)
     n = len(bilateral) * bilateral[0].N * (bilateral[0].vd - 1)
-    status = _lib.pl_mean_field_messages(len(bilateral), _handles(bilateral), _handles(spatial),
-                                         _dev_f32(output, "output", n), _dev_f32(input, "input", n),
-                                         int(bool(reverse)), _stream_ptr())
+    status = _lib.pl_mean_field_messages(len(bilateral), *handles, _dev_f32(output, "output", n),
+                                         _dev_f32(input, "input", n), int(bool(reverse)), _stream_ptr())
     if status == PL_EUNSUPPORTED:
         return False
     _check(status, "pl_mean_field_messages")
@@ -447,10 +449,10 @@ def mean_field_messages(bilateral, spatial, output, input, reverse=False):
 
 def mean_field_infer(bilateral, spatial, q, logits, iterations):
     """Mean-field updates of ``q`` from ``softmax(logits)`` on, likewise."""
+    handles = _handles_of_pairs(bilateral, spatial)
     n = len(bilateral) * bilateral[0].N * (bilateral[0].vd - 1)
-    status = _lib.pl_mean_field_infer(len(bilateral), _handles(bilateral), _handles(spatial),
-                                      _dev_f32(q, "q", n), _dev_f32(logits, "logits", n), int(iterations),
-                                      _stream_ptr())
+    status = _lib.pl_mean_field_infer(len(bilateral), *handles, _dev_f32(q, "q", n),
+                                      _dev_f32(logits, "logits", n), int(iterations), _stream_ptr())
     if status == PL_EUNSUPPORTED:
         return False
     _check(status, "pl_mean_field_infer")

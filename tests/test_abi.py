@@ -152,6 +152,18 @@ def test_a_library_with_another_array_layout_is_refused(tmp_path):
         pla._load(_stub_library(tmp_path, pla.LAYOUT_VERSION + 1, pla.REPLAY_ROW_BYTES))
 
 
+def test_pairs_of_lattices_are_counted_before_they_are_handed_on():
+    """(The library reads as many handles of either kind as there are bilateral ones.)"""
+    class Lattice:
+        N, vd, _h = 4, 3, None
+
+    for call in (lambda a, b: pla.mean_field_messages(a, b, None, None),
+                 lambda a, b: pla.mean_field_infer(a, b, None, None, 1)):
+        for a, b in ((2, 1), (1, 2), (1, 0)):
+            with pytest.raises(ValueError, match="lattices"):
+                call([Lattice()] * a, [Lattice()] * b)
+
+
 def test_documented_build_command_lists_every_source():
     from permutohedral_lattice_amd import build
     text = open(os.path.join(ROOT, "INTEGRATION.md")).read()
