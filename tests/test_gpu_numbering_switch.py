@@ -84,3 +84,33 @@ def test_the_way_to_number_is_kept_while_the_grid_is_the_same():
     for out in outs[1:]:
         assert float((out - outs[0]).abs().max()) <= 2e-6
     lat.close()
+
+
+def test_the_way_to_number_follows_a_handle_s_inputs():
+    """Volumes of one grid by turns, with vertices enough for the numbering pass and with few: a build goes by
+    the vertices of the one before it, and the rows are counted anew after 32 builds however often."""
+    import torch
+    import permutohedral_lattice_amd as pla
+    dims = (48, 96, 96)
+    n = dims[0] * dims[1] * dims[2]
+    gen = torch.Generator("cuda").manual_seed(12)
+    noisy = torch.rand((n, 1), device="cuda", generator=gen)
+    smooth = torch.linspace(0.0, 1.0, n, device="cuda").view(n, 1)
+    val = torch.rand((n, 1), device="cuda", generator=gen)
+    lat = pla.PermutohedralLattice(4, 2, n)
+    want = {}
+    for _ in range(3):
+        for guide in (noisy, smooth):
+            for call in range(3):
+                out = torch.empty_like(val)
+                lat.filter_image(out, val, guide, dims, 6.0, 0.2)
+                passed = lat.info(pla.PL_INFO_FOREIGN_ROWS) == -1
+                # (the first of the same kind is numbered as the one before it asked for)
+                assert passed == ((call > 0) == (guide is noisy))
+                assert float((out - want.setdefault(id(guide), out)).abs().max()) <= 2e-6
+    rows = []
+    for call in range(101):
+        lat.filter_image(out, val, noisy, dims, 6.0, 0.2)
+        rows.append(lat.info(pla.PL_INFO_FOREIGN_ROWS))
+    assert [call for call, r in enumerate(rows) if r != -1] == [0, 33, 66, 99]
+    lat.close()
