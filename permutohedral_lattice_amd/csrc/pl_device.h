@@ -219,7 +219,7 @@ struct Simplex {
 // is some 2^-48 of the result, and no quotient by D1's odd factor comes closer than 1/18 ulp to the middle
 // between two floats (compared for all 2^23 mantissas and D1 = 2..9; |x| at least 2^-90 or 0).
 template <int D1>
-__device__ __forceinline__ float scaled_down(float x) {
+__host__ __device__ __forceinline__ float scaled_down(float x) {
     constexpr double inverse = 1.0 / (double)D1;
     if constexpr ((D1 & (D1 - 1)) == 0) {
         return x * (float)inverse;
@@ -510,15 +510,16 @@ __device__ __forceinline__ bool block_of_points(const PointMap &m, int xcd_aware
 
 // a / b, correctly rounded as the division is, from inverse = 1 / b, itself correctly rounded: two steps
 // of Markstein's correction (P. Markstein, IBM J. Res. Dev. 34 (1990): the first leaves the quotient within
-// an ulp, the second rounds it right).  For a of a size whose remainder does not leave the number range,
-// b as FeatureWidths allows it.
-__device__ __forceinline__ float divided(float a, float b, float inverse) {
+// an ulp, the second rounds it right).  For a of a size whose remainder does not leave the number range
+// (2^-100 and up, or 0; below that it may be an ulp off,
+// which reaches no key), b as set_inverse_widths allows it.  The sign of a zero is not kept.
+__host__ __device__ __forceinline__ float divided(float a, float b, float inverse) {
     float q = a * inverse;
     q = __builtin_fmaf(__builtin_fmaf(-q, b, a), inverse, q);
     return __builtin_fmaf(__builtin_fmaf(-q, b, a), inverse, q);
 }
 
-__device__ __forceinline__ double divided(double a, double b, double inverse) {
+__host__ __device__ __forceinline__ double divided(double a, double b, double inverse) {
     double q = a * inverse;
     q = __builtin_fma(__builtin_fma(-q, b, a), inverse, q);
     return __builtin_fma(__builtin_fma(-q, b, a), inverse, q);
