@@ -198,7 +198,7 @@ struct pl_lattice {
     hipEvent_t ev[EV_COUNT] = {};
     bool ev_recorded[EV_COUNT] = {};
     // pl_mean_field_* work on another stream than this lattice's.  handover: where they last ended; whether
-    // this lattice's own stream has been given work on its arrays since; and whether such work was ever
+    // this lattice's own stream has been given work on its arrays since; and whether an apply was ever
     // captured there, to be replayed when this library does not see it
     hipEvent_t handover = nullptr;
     bool own_stream_used = true, captured = false;
@@ -437,12 +437,6 @@ bool is_captured(hipStream_t stream) {
     return true;
 }
 
-// The lattice's own stream is about to be given work on its arrays.
-void own_stream_takes_over(pl_lattice *h) {
-    h->own_stream_used = true;
-    if (!h->captured) h->captured = is_captured(h->stream);
-}
-
 // Enqueue one build with a table of `cells` cells.  Nothing here waits for the device.
 // splat_input != nullptr: the build kernel also splats these values (when it can for this vd),
 // and the value table holds them when the build is done.
@@ -451,7 +445,7 @@ int enqueue_build(pl_lattice *h, const plk::PointFeatures &features, const doubl
                   uint32_t cells, const void *splat_input) {
     // keys of two words while a build that needed them is recent (the plain build only)
     const bool wide = h->wide_for > 0;
-    own_stream_takes_over(h);
+    h->own_stream_used = true;
     if (h->wide_for > 0) h->wide_for -= 1;
     if (wide != h->wide_keys) h->table_clean = false;   // (cells of another width)
     h->wide_keys = wide;
@@ -679,7 +673,10 @@ int enqueue_apply_f64(pl_lattice *h, double *output, const double *input, int re
 
 // output and input are arrays of the lattice's value type
 int enqueue_apply(pl_lattice *h, void *output_any, const void *input_any, int reverse) {
-    own_stream_takes_over(h);
+    h->own_stream_used = true;
+    // (only lattices that pl_mean_field_* may take need to know: the question costs the host 0.3 us, of
+    // passes of 28 to 44 us on small images)
+    if (h->vd >= plk::kManyChannels && !h->f64 && !h->captured) h->captured = is_captured(h->stream);
     if (h->f64)
         return enqueue_apply_f64(h, static_cast<double *>(output_any),
                                  static_cast<const double *>(input_any), reverse);
@@ -1535,7 +1532,7 @@ int pl_debug_simplex(pl_handle h, const float *positions, short *rem0, short *ra
 // The debug exports count the vertices densely, whatever numbers the build gave them: read how
 // many each segment holds (these calls are for tests; they wait for the stream).
 static int vertex_numbers(pl_lattice *h, plk::VertexNumbers *numbers) {
-    own_stream_takes_over(h);
+    h->own_stream_used = true;
     plk::Counters counters;
     PL_HIP(hipMemcpyAsync(&counters, h->counters(), sizeof(counters), hipMemcpyDeviceToHost,
                           h->stream));

@@ -583,7 +583,7 @@ static hipError_t splat_gather_channels(int vd, int in_channels, int n, const Ga
 }
 
 hipError_t splat_gather_many(int vd, int in_channels, int n, const GatherWork *work, hipStream_t s) {
-    if (n < 1 || n > kManyItems || vd < 5) return hipErrorInvalidValue;
+    if (n < 1 || n > kManyItems || vd < kManyChannels) return hipErrorInvalidValue;
     return splat_gather_channels<kManyItems>(vd, in_channels, n, work, s);
 }
 

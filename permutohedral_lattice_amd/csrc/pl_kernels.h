@@ -408,7 +408,7 @@ hipError_t splat_gather(int vd, const VertexLists &lists, unsigned n_chunks, uns
                         const float *input, int in_channels, float *values, hipStream_t s);
 
 // The same for several lattices of rows of five channels and more in one launch each (pl_many.hip).
-constexpr int kManyItems = 8;
+constexpr int kManyItems = 8, kManyChannels = 5;
 struct GatherWork {
     ListChunks chunks;
     const ListEntry *entries;
