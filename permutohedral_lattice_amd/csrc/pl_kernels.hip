@@ -2283,8 +2283,10 @@ int key_field_bits(int pd) {
     return b > 16 ? 16 : b;
 }
 
-// x / d == (x * factor) >> shift for every x below 2^31: factor = ceil(2^shift / d) with 2^shift at least
-// 2^32 d, so x * factor exceeds x * 2^shift / d by less than 2^shift / d, and stays below 2^64.
+// x / d == (x * factor) >> shift for every x below 2^31: factor = ceil(2^shift / d), so factor * d exceeds
+// 2^shift by less than d, and x * factor / 2^shift exceeds x / d by less than x / 2^shift.  With 2^shift at
+// least 2^31 d that is less than 1 / d, too little to reach the next whole number; and x * factor, at most
+// 2^31 (2^32 + 1), stays below 2^64.
 static PointMap::Divisor divisor(unsigned d) {
     unsigned bits = 0;
     while ((1ull << bits) < d) ++bits;
