@@ -155,9 +155,10 @@ struct pl_lattice {
     // has many thousands of workgroups (they draw their numbers one after the other), or when
     // the last such build of these points held so many rows of sums for vertices of other
     // workgroups that adding them afterwards, an atomic each, outweighs the numbering pass.
-    // (The pass then serves the next builds for as long as rows in proportion to their vertices would
-    // outweigh it as well, and at most 32 before a build counts such rows anew: inputs change.)
-    int numbering_pass_for = 0;
+    // (The pass then serves the next builds for as long as rows in proportion to their vertices would cost
+    // three quarters of it as well, and at most numbering_pass_backoff, doubled every time it is found to
+    // pay again, up to 128, before a build counts such rows anew: inputs change.)
+    int numbering_pass_for = 0, numbering_pass_backoff = 32;
     double foreign_rows_per_vertex = 0.0;   // of the last build that counted them
     long foreign_rows = -1;            // of the last build (an estimate from a sample); -1: it listed none
     bool built = false;                // a build has been enqueued and, if verified, fitted
@@ -860,14 +861,22 @@ int verify_build(pl_lattice *h, uint32_t *retry_cells) {
     // numbering pass 1.25 per workgroup of the build and 0.02 per vertex (the volume's 32 768
     // workgroups: 41 us), and the build 1500 longer with all its rows going out as atomics)
     // A build that the pass numbered counts no rows; those of the same grid go with its vertices (4.5 to 5.7
-    // a vertex on volumes, smooth or noisy).  Without a look at the vertices smooth volumes of 48x96x96
-    // points kept the pass that a noisy one had asked for: 64.3 us a filter instead of 58.5.
+    // a vertex on volumes, smooth or noisy, under the same widths).  Without a look at the vertices smooth
+    // volumes of 48x96x96 points kept the pass that a noisy one had asked for: 64.3 us a filter instead of
+    // 58.5.  (Three quarters: inputs about the line would go back and forth; 128x256x256 voxels, 1.04 M rows
+    // where the line is 1.25 M, 414 us with the pass and 451 without.)
     h->foreign_rows = status.n_segments != 0 ? (long)status.foreign_rows : -1;
-    if (status.n_segments != 0 && m > 0) h->foreign_rows_per_vertex = (double)status.foreign_rows / m;
-    if (status.n_segments != 0 || h->numbering_pass_for > 0) {
-        const bool pays = 0.037 * h->foreign_rows_per_vertex * m > 1.25 * h->working_blocks() + 0.02 * m + 1500.0;
-        if (!pays) h->numbering_pass_for = 0;
-        else if (status.n_segments != 0) h->numbering_pass_for = 32;
+    const double pass_ns = 1.25 * h->working_blocks() + 0.02 * m + 1500.0;
+    if (status.n_segments != 0) {
+        if (m > 0) h->foreign_rows_per_vertex = (double)status.foreign_rows / m;
+        if (0.037 * status.foreign_rows > pass_ns) {
+            h->numbering_pass_for = h->numbering_pass_backoff;
+            h->numbering_pass_backoff = h->numbering_pass_backoff >= 64 ? 128 : h->numbering_pass_backoff * 2;
+        } else {
+            h->numbering_pass_backoff = 32;
+        }
+    } else if (0.037 * h->foreign_rows_per_vertex * m < 0.75 * pass_ns) {
+        h->numbering_pass_for = 0;
     }
     h->verified = true;
     if (h->last_build_merged) h->tiles_backoff = 32;
@@ -1090,6 +1099,7 @@ int pl_set_point_grid(pl_handle h, int n_dims, const int *dims) {
     if (h->map.mode < 2 || h->map.mode != before.mode || h->map.dims[0] != before.dims[0] ||
         h->map.dims[1] != before.dims[1] || h->map.dims[2] != before.dims[2]) {
         h->numbering_pass_for = 0;
+        h->numbering_pass_backoff = 32;
         h->one_segment_for = 0;
         h->one_segment_backoff = 32;
     }
@@ -1152,6 +1162,7 @@ int guess_point_grid(pl_lattice *h, const float *positions) {
     if (dims[0] < 2) return PL_OK;
     h->map = plk::make_point_map(h->N, n_dims, dims);
     h->numbering_pass_for = 0;
+    h->numbering_pass_backoff = 32;
     h->one_segment_for = 0;
     h->one_segment_backoff = 32;
     return ensure_replay(h, false);

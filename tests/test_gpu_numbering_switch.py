@@ -88,7 +88,7 @@ def test_the_way_to_number_is_kept_while_the_grid_is_the_same():
 
 def test_the_way_to_number_follows_a_handle_s_inputs():
     """Volumes of one grid by turns, with vertices enough for the numbering pass and with few: a build goes by
-    the vertices of the one before it, and the rows are counted anew after 32 builds however often."""
+    the vertices of the one before it, and the rows are counted anew after 32, 64 and then every 128 builds."""
     import torch
     import permutohedral_lattice_amd as pla
     dims = (48, 96, 96)
@@ -109,8 +109,8 @@ def test_the_way_to_number_follows_a_handle_s_inputs():
                 assert passed == ((call > 0) == (guide is noisy))
                 assert float((out - want.setdefault(id(guide), out)).abs().max()) <= 2e-6
     rows = []
-    for call in range(101):
+    for call in range(360):
         lat.filter_image(out, val, noisy, dims, 6.0, 0.2)
         rows.append(lat.info(pla.PL_INFO_FOREIGN_ROWS))
-    assert [call for call, r in enumerate(rows) if r != -1] == [0, 33, 66, 99]
+    assert [call for call, r in enumerate(rows) if r != -1] == [0, 33, 98, 227, 356]
     lat.close()
