@@ -132,17 +132,20 @@ hipError_t hipStreamIsCapturing(hipStream_t s, hipStreamCaptureStatus *status) {
 }
 hipError_t hipStreamGetDevice(hipStream_t, hipDevice_t *d) { return *d = 0, hipSuccess; }
 hipError_t hipStreamWaitEvent(hipStream_t s, hipEvent_t e, unsigned) {
-    if (!e) return hipErrorInvalidHandle;
+    if (!g_events.count((void *)e)) return hipErrorInvalidHandle;
     return join(stream_of(s).clock, g_events[(void *)e]), hipSuccess;
 }
 hipError_t hipEventCreate(hipEvent_t *e) {
     static long made = 0;
-    return *e = (hipEvent_t)(++made * 64), hipSuccess;
+    *e = (hipEvent_t)(++made * 64);
+    return g_events[(void *)*e] = {}, hipSuccess;
 }
 hipError_t hipEventCreateWithFlags(hipEvent_t *e, unsigned) { return hipEventCreate(e); }
-hipError_t hipEventDestroy(hipEvent_t) { return hipSuccess; }
+hipError_t hipEventDestroy(hipEvent_t e) {
+    return g_events.erase((void *)e) ? hipSuccess : hipErrorInvalidHandle;
+}
 hipError_t hipEventRecord(hipEvent_t e, hipStream_t s) {
-    if (!e) return hipErrorInvalidHandle;
+    if (!g_events.count((void *)e)) return hipErrorInvalidHandle;
     expect(!stream_of(s).capturing, "an event is recorded on a stream that is being captured");
     join(stream_of(s).clock, g_host);
     return g_events[(void *)e] = stream_of(s).clock, hipSuccess;
@@ -373,6 +376,41 @@ void two_callers_and_builds() {
     }
 }
 
+// calls with some of the lattices, in changing order and company, some destroyed in between: the events that
+// they refer to are one another's
+void changing_company() {
+    for (int destroyed = 0; destroyed <= 4; ++destroyed) {
+        Pairs p(four_streams()), other({named_stream(5), named_stream(5), named_stream(1), named_stream(6)});
+        auto call = [&](const std::vector<pl_handle> &bilateral, const std::vector<pl_handle> &spatial, long stream) {
+            float *out = nullptr;
+            (void)hipMalloc((void **)&out, 4);
+            expect(pl_mean_field_messages((int)bilateral.size(), bilateral.data(), spatial.data(), out, p.logits, 0,
+                                          named_stream(stream)) == PL_OK, "messages");
+        };
+        const pl_handle *a = p.bilateral, *b = p.spatial, *c = other.bilateral, *d = other.spatial;
+        call({a[0], a[1]}, {b[0], b[1]}, 9);
+        call({c[0], a[1]}, {b[1], d[1]}, 8);
+        call({a[0]}, {b[0]}, 2);
+        call({a[1], a[0], c[1]}, {d[0], b[0], b[1]}, 9);
+        call({c[0], c[1]}, {d[1], d[0]}, 7);
+        float *out = nullptr;
+        (void)hipMalloc((void **)&out, 4);
+        expect(pl_apply(a[1], out, p.logits, 0) == PL_OK, "pl_apply");
+        call({a[1]}, {d[1]}, 3);
+        const pl_handle all[] = {a[0], a[1], b[0], c[0]};
+        for (int i = 0; i < destroyed; ++i) expect(pl_destroy(all[i]) == PL_OK, "pl_destroy");
+        if (destroyed < 1) call({a[0], c[0]}, {b[1], d[0]}, 8);
+        if (destroyed < 2) call({a[1]}, {b[0]}, 9);
+        if (destroyed < 4) call({c[0]}, {d[1]}, 8);
+        call({c[1]}, {b[1]}, 7);
+        call({c[1]}, {d[0]}, 9);
+        for (int i = destroyed; i < 4; ++i) (void)pl_destroy(all[i]);
+        for (const pl_handle h : {b[1], c[1], d[0], d[1]}) (void)pl_destroy(h);
+        expect(g_events.empty(), "events are left");
+        g_arrays.clear();   // (freed memory comes back as other arrays)
+    }
+}
+
 // a lattice's own stream is being captured: nothing may be recorded there, nothing is enqueued
 void own_stream_captured() {
     Pairs p(four_streams());
@@ -420,6 +458,7 @@ int main(int argc, char **argv) {
         {"one_stream_for_all", one_stream_for_all},
         {"handle_given_out_again", handle_given_out_again},
         {"two_callers_and_builds", two_callers_and_builds},
+        {"changing_company", changing_company},
         {"own_stream_captured", own_stream_captured},
         {"failed_blur", failed_blur},
         {"no_pointer_kept", no_pointer_kept},
