@@ -112,7 +112,7 @@ typedef enum pl_library_property {
     PL_LIB_SOURCE_HASH = 3       /* first 48 bits of the SHA-256 over the library's source files as its
                                     build script hashed them (0 when built without the script) */
 } pl_library_property;
-#define PL_LAYOUT_VERSION 4
+#define PL_LAYOUT_VERSION 5
 int pl_library_info(int what, long long *value);
 
 /*

@@ -35,7 +35,7 @@ PL_LIB_LAYOUT_VERSION, PL_LIB_REPLAY_ROW_BYTES, PL_LIB_SOURCE_HASH = 1, 2, 3
 # written for: PL_LAYOUT_VERSION of include/permutohedral_lattice.h and the size of a replay row.
 # A library that reports other values is not driven at all: its kernels would read each other's
 # arrays in a layout this side knows nothing of.
-LAYOUT_VERSION = 4
+LAYOUT_VERSION = 5
 REPLAY_ROW_BYTES = 8
 
 # every symbol include/permutohedral_lattice.h declares

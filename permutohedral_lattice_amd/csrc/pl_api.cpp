@@ -114,7 +114,8 @@ struct pl_lattice {
     // what each workgroup of the build created (see plk::CreatedLists); the chunk counts exist
     // twice and alternate between builds like the counters
     uint4 *created_entries = nullptr;      // [n_blocks * list_stride()]
-    int *block_count = nullptr;            // [n_blocks]
+    int *block_count = nullptr;            // [n_blocks], and behind them tiles.used
+    plk::TileVertices tiles{};             // in created_entries and block_count
     int *chunk_count = nullptr;            // [2][n_chunks]
     // which of the two sets is zero: the numbering pass of a build zeroes the other set, but a
     // build that numbers its vertices itself leaves both as they are
@@ -256,7 +257,7 @@ struct pl_lattice {
     int list_stride() const { return plk::created_list_stride(pd, f64) * (lists_wide ? 2 : 1); }
     plk::CreatedLists lists(int set) const {
         return plk::CreatedLists{created_entries, block_count, chunk_count + (size_t)set * n_chunks,
-                                 list_stride()};
+                                 list_stride(), map.tile_vertices, false};
     }
 };
 
@@ -313,12 +314,14 @@ int ensure_replay(pl_lattice *h, bool wide) {
     h->replay = (plk::ReplayEntry *)h->dmalloc(sizeof(plk::ReplayEntry) * (want ? want : 1));
     const size_t entries = (size_t)h->map.n_blocks * (size_t)h->list_stride();
     h->created_entries = (uint4 *)h->dmalloc(sizeof(uint4) * (entries ? entries : 1));
-    h->block_count = (int *)h->dmalloc(sizeof(int) * (h->map.n_blocks ? h->map.n_blocks : 1));
+    h->block_count = (int *)h->dmalloc(sizeof(int) * (h->map.n_blocks ? h->map.n_blocks : 1) * 2);
     h->chunk_count = (int *)h->dmalloc(sizeof(int) * 2 * h->n_chunks);
     if (h->f64) h->weights64 = (double *)h->dmalloc(sizeof(double) * (want ? want : 1));
     if (!h->replay || !h->created_entries || !h->block_count || !h->chunk_count ||
         (h->f64 && !h->weights64))
         return PL_ENOMEM;
+    h->tiles = plk::TileVertices{reinterpret_cast<int *>(h->created_entries + plk::tile_table_from(h->f64)),
+                                 h->block_count + h->map.n_blocks, 4u * (unsigned)h->list_stride()};
     if (!h->cleared_by_caller)
         PL_HIP(plk::fill_zero(reinterpret_cast<float *>(h->chunk_count), 2 * h->n_chunks, h->stream));
     h->chunk_count_clean[0] = h->chunk_count_clean[1] = true;
@@ -477,6 +480,7 @@ int enqueue_build(pl_lattice *h, const plk::PointFeatures &features, const doubl
     rc = ensure_replay(h, wide);
     if (rc != PL_OK) return rc;
     // (a lattice of doubles splats in its build only in the merging kernel)
+    h->map.tile_vertices = merge ? h->tiles : plk::TileVertices{};
     const bool fused = splat_input && plk::build_can_splat(h->vd) && (!h->f64 || merge);
     // (a build for one filter: a lattice built to be applied many times is numbered by the
     // numbering pass, in the order of the image tiles, which the passes over the vertices walk
@@ -517,7 +521,8 @@ int enqueue_build(pl_lattice *h, const plk::PointFeatures &features, const doubl
     h->counter_set = 1 - previous_set;
     const plk::VertexTables vertices{h->cell_vertex, h->vertex_keys, h->vertex_cell, h->neighbours,
                                      h->max_vertices()};
-    const plk::CreatedLists lists = h->lists(h->counter_set);
+    plk::CreatedLists lists = h->lists(h->counter_set);
+    lists.foreign_rows = numbers_in_build;
     if (!numbers_in_build) {
         // (sums of an earlier build would shift the numbers of this one's vertices past the
         // tables' filled rows)
@@ -586,15 +591,16 @@ int enqueue_build(pl_lattice *h, const plk::PointFeatures &features, const doubl
                                     h->d_counters + previous_set, report_to, wide, h->stream));
     }
     h->mark(EV_IDS);
-    // (the rows a build that numbered its vertices listed for vertices of other workgroups join
-    // the value table here, and its counts reach the host from here)
+    // (the vertices that a merging build's workgroups did not number get their numbers in the workgroups'
+    // tables here; the rows a build that numbered its vertices listed for them join the value
+    // table, and its counts reach the host from here)
     PL_HIP(plk::neighbours(h->pd, vertices, h->counters(), h->cell_keys, cells,
-                           h->launch_vertices(), numbers_in_build && fused ? &lists : nullptr,
+                           h->launch_vertices(), merge ? &lists : nullptr,
                            h->map.n_blocks, h->values[0], h->vd, h->f64,
                            numbers_in_build ? h->counters() : nullptr,
                            h->d_counters + previous_set, report_to, wide, h->stream));
     h->mark(EV_NBR);
-    h->replay_holds_cells = true;
+    h->replay_holds_cells = !merge;
     h->values_zeroed = !fused;
     h->values_splatted = fused;
     h->built = true;
@@ -1776,7 +1782,7 @@ int enqueue_pairs(int n, const pl_handle *bilateral, const pl_handle *spatial, f
         plk::SlicePair slice[kPairsPerLaunch];
         for (int i = 0; i < pairs; ++i) {
             const pl_lattice *a = lattice[i], *b = lattice[pairs + i];
-            slice[i] = plk::SlicePair{a->map, a->replay, b->replay, a->values[a->current_values],
+            slice[i] = plk::SlicePair{a->map, b->map.tile_vertices, a->replay, b->replay, a->values[a->current_values],
                                       b->values[b->current_values],
                                       logits ? logits + (size_t)(first + i) * item : nullptr,
                                       output + (size_t)(first + i) * item};

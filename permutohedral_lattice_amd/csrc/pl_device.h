@@ -508,6 +508,57 @@ __device__ __forceinline__ bool block_of_points(const PointMap &m, int xcd_aware
     return true;
 }
 
+// The words and the weights of a workgroup's points in the replay of a merging build (TileVertices).
+template <bool DOUBLES = false>
+__device__ __forceinline__ uint32_t *words_of_tile(ReplayEntry *replay, unsigned vblock, int d1) {
+    return reinterpret_cast<uint32_t *>(replay) + (size_t)vblock * kBlock * (replay_words(d1) + (DOUBLES ? 0 : d1));
+}
+template <bool DOUBLES = false>
+__device__ __forceinline__ const uint32_t *words_of_tile(const ReplayEntry *replay, unsigned vblock, int d1) {
+    return words_of_tile<DOUBLES>(const_cast<ReplayEntry *>(replay), vblock, d1);
+}
+__device__ __forceinline__ const float *weights_behind(const uint32_t *words, int d1) {
+    return reinterpret_cast<const float *>(words + kBlock * replay_words(d1));
+}
+__device__ __forceinline__ uint32_t place_of_corner(uint32_t word, int r) {
+    return (word >> (kPlaceBits * (r % kPlacesPerWord))) & kNoPlace;
+}
+// Corner r of the point of thread tid, from the replay of any build: its vertex (hash cell where rows still
+// hold them), -1: none, and its weight (lattices of floats).
+template <bool DOUBLES = false>
+__device__ __forceinline__ ReplayEntry replay_corner(const ReplayEntry *replay, const TileVertices &tiles,
+                                                     unsigned vblock, int d1, int r, unsigned tid) {
+    if (!tiles.table) return replay[((size_t)vblock * d1 + r) * kBlock + tid];
+    const uint32_t *words = words_of_tile<DOUBLES>(replay, vblock, d1);
+    const uint32_t place = place_of_corner(words[(r / kPlacesPerWord) * kBlock + tid], r);
+    ReplayEntry e{place < kTileSlots ? tiles.of(vblock)[place] : -1, 0.0f};
+    if (!DOUBLES) e.weight = weights_behind(words, d1)[r * kBlock + tid];
+    return e;
+}
+// All corners at once, their loads in flight together
+template <int D1, bool DOUBLES = false>
+__device__ __forceinline__ void replay_corners(const ReplayEntry *replay, const TileVertices &tiles, unsigned vblock,
+                                               unsigned tid, ReplayEntry (&e)[D1]) {
+    if (!tiles.table) {
+#pragma unroll
+        for (int r = 0; r < D1; ++r) e[r] = replay[((size_t)vblock * D1 + r) * kBlock + tid];
+        return;
+    }
+    const uint32_t *words = words_of_tile<DOUBLES>(replay, vblock, D1);
+    uint32_t word[replay_words(D1)];
+#pragma unroll
+    for (int w = 0; w < replay_words(D1); ++w) word[w] = words[w * kBlock + tid];
+#pragma unroll
+    for (int r = 0; r < D1; ++r) e[r].weight = DOUBLES ? 0.0f : weights_behind(words, D1)[r * kBlock + tid];
+    int vertex[D1];
+#pragma unroll
+    for (int r = 0; r < D1; ++r)
+        vertex[r] = tiles.of(vblock)[place_of_corner(word[r / kPlacesPerWord], r) & (kTileSlots - 1u)];
+#pragma unroll
+    for (int r = 0; r < D1; ++r)
+        e[r].index = place_of_corner(word[r / kPlacesPerWord], r) != kNoPlace ? vertex[r] : -1;
+}
+
 // a / b, correctly rounded as the division is, from inverse = 1 / b, itself correctly rounded: two steps
 // of Markstein's correction (P. Markstein, IBM J. Res. Dev. 34 (1990): the first leaves the quotient within
 // an ulp, the second rounds it right).  For a of a size whose remainder does not leave the number range

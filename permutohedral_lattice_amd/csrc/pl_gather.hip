@@ -48,8 +48,10 @@ __global__ __launch_bounds__(kBlock) void k_list_places(PointMap map, ReplayEntr
     const int lane = threadIdx.x & 63;
 
     int vertex[D1];
+    ReplayEntry corner[D1];
+    replay_corners<D1>(replay, map.tile_vertices, vblock, threadIdx.x, corner);
 #pragma unroll
-    for (int r = 0; r < D1; ++r) vertex[r] = n >= 0 ? replay[(size_t)r * T + t].index : -1;
+    for (int r = 0; r < D1; ++r) vertex[r] = n >= 0 ? corner[r].index : -1;
     if (cell_vertex) {
 #pragma unroll
         for (int r = 0; r < D1; ++r)
@@ -274,11 +276,9 @@ __global__ __launch_bounds__(kBlock) void k_list_fill(PointMap map,
     if (n < 0) return;
     ReplayEntry e[D1];
     unsigned place[D1], first[D1];
+    replay_corners<D1>(replay, map.tile_vertices, vblock, threadIdx.x, e);
 #pragma unroll
-    for (int r = 0; r < D1; ++r) {
-        e[r] = replay[(size_t)r * T + t];
-        place[r] = places[(size_t)r * T + t];
-    }
+    for (int r = 0; r < D1; ++r) place[r] = places[(size_t)r * T + t];
 #pragma unroll
     for (int r = 0; r < D1; ++r)
         first[r] = start[(unsigned)e[r].index < (unsigned)max_vertices ? e[r].index : 0];

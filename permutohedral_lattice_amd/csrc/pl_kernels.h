@@ -104,7 +104,8 @@ struct VertexTables {
 __host__ __device__ inline uint32_t max_vertices_for(uint32_t n_cells) { return n_cells / 4u * 3u; }
 
 // One row of the replay matrix (reference: MatrixEntry, src/PermutohedralLatticeCPU.h:187-190):
-// which vertex a point's simplex corner is (hash cell until the first splat) and its weight.
+// which vertex a point's simplex corner is (hash cell until the first splat) and its weight.  (After a
+// merging build: TileVertices.)
 struct ReplayEntry {
     int index;
     float weight;
@@ -133,6 +134,26 @@ struct SpatialDims {
     int v[kMaxSpatialDims];
 };
 
+// The replay of a merging build.  The 256 points of one of its workgroups touch at most kTileSlots vertices
+// between them (about a hundred on an image), so their corners name the vertex by its place in the
+// workgroup's own table, and a pass over the points reads every vertex once a workgroup instead of once
+// a corner.  In the memory of the replay rows, per workgroup and in thread order, replay_words(pd + 1)
+// words a point, three corners' places in each (corner r in bits 10 (r % 3) .. of word r / 3; kNoPlace: no
+// point), [word][thread], and behind them, in a lattice of floats, the barycentric weights [r][thread]:
+// 8 + 24 bytes a point for pd = 5 where rows are 48.
+constexpr int kTileSlots = 512;    // vertices of a workgroup of the merging build
+constexpr int kPlaceBits = 10, kPlacesPerWord = 3;
+constexpr uint32_t kNoPlace = (1u << kPlaceBits) - 1u;
+__host__ __device__ constexpr int replay_words(int d1) { return (d1 + kPlacesPerWord - 1) / kPlacesPerWord; }
+// (table == nullptr: a build that did not merge, which leaves rows)
+struct TileVertices {
+    int *table;         // per workgroup, `stride` apart, kTileSlots places: the vertices (behind neighbours(); a
+                        // build leaves the hash cells of those it has not numbered), -1: none
+    int *used;          // [workgroups] how many of a workgroup's
+    unsigned stride;
+    __host__ __device__ int *of(unsigned workgroup) const { return table + (size_t)workgroup * stride; }
+};
+
 // Per-workgroup lists, `stride` uint4 per workgroup of the build (in the build's virtual order).
 // A build that leaves the numbering to number_vertices lists what it created: workgroup b has
 // block_count[b] new vertices, one uint4 each: (key low word, key high word, hash cell, 0);
@@ -140,22 +161,25 @@ struct SpatialDims {
 // before the build.
 // A merging build that numbers its vertices itself lists, when it splats, the rows of sums it
 // holds for vertices that another workgroup created (their numbers are not known yet):
-// block_count[b] of them, the rows (four values each) from the start of the workgroup's part and
-// their hash cells, as ints, behind kTileSlots rows.  neighbours() adds them to the value table.
+// block_count[b] of them, the rows (four values each) from the start of the workgroup's part and, behind
+// kTileSlots rows, their hash cells and places in the workgroup's table, as pairs of ints.  neighbours() adds
+// them to the value table.
 constexpr int kBlocksPerChunk = 64;
-constexpr int kTileSlots = 512;    // LDS slots of a workgroup of the merging build
 struct CreatedLists {
     uint4 *entries;
     int *block_count;
     int *chunk_count;
     int stride;
+    TileVertices tiles;   // of a merging build
+    bool foreign_rows;    // it numbered its vertices and lists such rows
 };
 // uint4 a workgroup's part must hold: its 256 * (pd+1) possible vertices, or kTileSlots rows of
-// four values and as many cells
+// four values, as many pairs of a cell and a place, and, at tile_table_from, the workgroup's table (which is
+// kept with the replay: no other allocation of megabytes for a new handle)
+inline int tile_table_from(bool f64) { return kTileSlots * (f64 ? 2 : 1) + kTileSlots / 2; }
 inline int created_list_stride(int pd, bool f64) {
-    const int vertices = 256 * (pd + 1);
-    const int rows = kTileSlots * (f64 ? 2 : 1) + kTileSlots / 4;
-    return vertices > rows ? vertices : rows;
+    const int vertices = 256 * (pd + 1), tile = tile_table_from(f64) + kTileSlots / 4;
+    return vertices > tile ? vertices : tile;
 }
 
 // What the merging build needs to number its vertices: the per-vertex tables and the value table
@@ -220,6 +244,8 @@ struct PointMap {
     // (in device memory: the launch is enqueued before the order is known)
     const int *order;
     const unsigned *n_tiles;
+    // the replay that the last build left on this map
+    TileVertices tile_vertices;
     // x / tiles[2] and x / (tiles[1] * tiles[2]) as a product and a shift (make_point_map)
     struct Divisor {
         uint64_t factor;
@@ -301,15 +327,15 @@ hipError_t number_vertices(int pd, const PointMap &map, const CreatedLists &list
 // launch_vertices (here and below): the vertex count the grid is sized for; any count is
 // covered, a wrong estimate only costs time.
 // Keys are looked for where the build put them: counters->region_* as the build left them.
-// foreign_rows != nullptr (after a merging build that numbered its vertices and splatted): the
-// launch also adds the rows the build's n_lists workgroups listed to `values` (rows of vd floats
-// or doubles).
+// tiles != nullptr (after a merging build of n_lists workgroups): the launch also puts vertices in the place of
+// the hash cells in their tables and, with tiles->foreign_rows, adds the rows they listed to `values` (rows
+// of vd floats or doubles).
 // report != nullptr (after a merging build that numbered its vertices): the launch also sums the
 // segments' counts in *report (the build's counters, == counters), copies them and the flags to
 // *host_status and zeroes *next_counters, as number_vertices does otherwise.
 hipError_t neighbours(int pd, const VertexTables &vertices, const Counters *counters,
                       const uint64_t *cell_keys, uint32_t n_cells, int launch_vertices,
-                      const CreatedLists *foreign_rows, unsigned n_lists, void *values, int vd,
+                      const CreatedLists *tiles, unsigned n_lists, void *values, int vd,
                       bool values_are_double, Counters *report, Counters *next_counters,
                       HostReport host_report, bool wide_keys, hipStream_t s);
 
@@ -431,7 +457,8 @@ hipError_t blur_many(int vd, int n, const BlurWork *work, hipStream_t s);
 // Stage 5 of pairs of lattices over the same points (same point map, normalising): output := the sum of
 // both slices, or, with logits, softmax(logits + sum) over the vd-1 channels.
 struct SlicePair {
-    PointMap map;
+    PointMap map;              // (its tile_vertices: a's)
+    TileVertices tiles_b;
     const ReplayEntry *replay_a, *replay_b;
     const float *values_a, *values_b;
     const float *logits;
@@ -469,6 +496,10 @@ hipError_t blur_three_axes_f64(int vd, const Counters *counters, int max_vertice
 hipError_t slice(int pd, int vd, const PointMap &map, const ReplayEntry *replay,
                  const int *cell_vertex, const float *values,
                  float *output, int normalize, hipStream_t s);
+
+// Five to sixty-four channels of a lattice whose build merged (pl_many.hip).
+hipError_t slice_tile_channels(int pd, int vd, const PointMap &map, const ReplayEntry *replay, const float *values,
+                            float *output, int normalize, hipStream_t s);
 
 hipError_t debug_simplex(int pd, const float *positions, int N, const ScaleFactor &scale,
                          short *rem0, short *rank, short *keys, float *barycentric, hipStream_t s);

@@ -12,7 +12,8 @@
 //   neighbours[(pd+1)*M]   int2 per blur axis a and vertex v: indices of v's two neighbours or -1
 //   values[M*vd]           f32  vertex values, two buffers (ping-pong across blur axes)
 //   replay[(pd+1)*T] {i32, f32} [workgroup][r][thread]: vertex r of the thread's point (hash cell until the
-//                                first splat) and its barycentric weight
+//                                first splat) and its barycentric weight; after a merging build in
+//                                another form (TileVertices in pl_kernels.h)
 //
 // Packed key.  Every coordinate of lattice vertex with remainder r is (pd+1)*q_i + r, so a key is
 // (r, q_0..q_{pd-1}): r in bits 60..63, q_i biased into a field of B = min(16, 60/pd) bits.
@@ -559,8 +560,8 @@ static_assert(kTileSlots == 1 << (32 - kTileSlotShift), "the slot is the hash's 
 
 // A slot of the workgroup's table for every group of the wavefront (wave_groups_in_order of each corner,
 // numbered through): slot[r] := that of the lane's group of corner r, -1 where it has none (bit r of
-// `present` clear) or no slot was found; new slots join the list `occupied`.  True: every key of this lane's
-// has its slot.
+// `present` clear) or no slot was found; new slots join the list `occupied`, at place_of_slot.  True: every key
+// of this lane's has its slot.
 // The leaders' keys go to lane after lane of the wavefront, whatever corner they are of (an image's 8x8
 // pixels have about forty), and every lane places one, where a lane with a leader for each of its
 // corners would place up to D1, one behind the other; the slots come back the same way.  (More than 64
@@ -568,8 +569,8 @@ static_assert(kTileSlots == 1 << (32 - kTileSlotShift), "the slot is the hash's 
 template <int PROBES, int D1, typename Key, typename Hash>
 __device__ __forceinline__ bool place_groups(const Key (&key)[D1], const unsigned (&group)[D1], unsigned present,
                                              unsigned n_groups, int lane, Key *wave_keys, Key *table, Key empty,
-                                             Hash hash, unsigned short *occupied, int *n_occupied,
-                                             int (&slot)[D1]) {
+                                             Hash hash, unsigned short *occupied, unsigned short *place_of_slot,
+                                             int *n_occupied, int (&slot)[D1]) {
     using Word = std::conditional_t<sizeof(Key) == 8, unsigned long long, int>;
     constexpr int kStride = sizeof(Key) / sizeof(int);
     int *wave_slots = reinterpret_cast<int *>(wave_keys);
@@ -609,7 +610,11 @@ __device__ __forceinline__ bool place_groups(const Key (&key)[D1], const unsigne
             if (((present >> r) & 1u) && to < 64u) slot[r] = wave_slots[kStride * to];
         }
         // the slots that were empty join the list of slots in use
-        if (was_empty) occupied[atomicAdd(n_occupied, 1)] = (unsigned short)at_slot;
+        if (was_empty) {
+            const int i = atomicAdd(n_occupied, 1);
+            occupied[i] = (unsigned short)at_slot;
+            place_of_slot[at_slot] = (unsigned short)i;
+        }
         wave_exchange_in_lds();
     }
     return placed;
@@ -693,20 +698,23 @@ __global__ __launch_bounds__(kBlock) __attribute__((amdgpu_num_sgpr(102))) void 
     unsigned vblock;
     if (!block_of_points(map, xcd_aware, vblock)) {
         // (no points: nothing created, no rows of sums for the passes that walk the lists)
-        if (threadIdx.x == 0) created_lists.block_count[vblock] = 0;
+        if (threadIdx.x == 0) created_lists.block_count[vblock] = created_lists.tiles.used[vblock] = 0;
         return;
     }
     __shared__ uint64_t slot_key[kTileSlots];
-    __shared__ int slot_cell[kTileSlots];
     __shared__ T slot_sum[SPLAT_VD ? kTileSlots * P : 1];
-    // the slots in use, in the order their keys arrived: the last phases walk these, not all slots
-    __shared__ unsigned short occupied[kTileSlots];
+    // the slots in use, in the order their keys arrived: the last phases walk these, not all slots, and
+    // the place in this order is what the points' corners name the vertex by
+    __shared__ unsigned short occupied[kTileSlots], place_of_slot[kTileSlots];
     __shared__ int n_occupied;
-    // which of the vertices this workgroup created a slot's key is (kNotCreated: none of them)
-    __shared__ unsigned short slot_rank[kTileSlots];
+    // per place: which of the vertices this workgroup created it is (kNotCreated: none of them), and the
+    // cell; the cells come where the wavefronts' keys have been, which are done with by then
+    __shared__ unsigned short created_rank[kTileSlots];
     constexpr unsigned short kNotCreated = 0xffffu;
     __shared__ int group_created;
     __shared__ uint64_t group_keys[kBlock / 64][64];
+    static_assert(sizeof(group_keys) == kTileSlots * sizeof(int), "a cell per place");
+    int *const place_cell = reinterpret_cast<int *>(group_keys);
     const int tid = threadIdx.x;
     for (int i = tid; i < kTileSlots; i += kBlock) slot_key[i] = kEmptyCell;
     if (SPLAT_VD)
@@ -716,8 +724,6 @@ __global__ __launch_bounds__(kBlock) __attribute__((amdgpu_num_sgpr(102))) void 
         group_created = 0;
     }
 
-    const size_t t = (size_t)vblock * kBlock * D1 + tid;   // slot in the replay arrays
-    constexpr size_t n_slots = kBlock;
     int at[3];
     const int n = point_of_thread(map, vblock, tid, at);
     const int lane = tid & 63;
@@ -755,7 +761,7 @@ __global__ __launch_bounds__(kBlock) __attribute__((amdgpu_num_sgpr(102))) void 
         for (int r = 0; r < D1; ++r) group[r] = wave_groups_in_order(key[r], among, &n_groups);
         const bool all_placed = place_groups<kTileProbeLimit>(
             key, group, active ? (1u << D1) - 1u : 0u, n_groups, lane, group_keys[tid >> 6], slot_key, kEmptyCell,
-            [](uint64_t k) { return hash_key(k); }, occupied, &n_occupied, slot);
+            [](uint64_t k) { return hash_key(k); }, occupied, place_of_slot, &n_occupied, slot);
         if (!all_placed) atomicOr(&counters->flags, kFlagTileFull);
     }
 
@@ -794,12 +800,10 @@ __global__ __launch_bounds__(kBlock) __attribute__((amdgpu_num_sgpr(102))) void 
         uint32_t cell[H], pair_index[H];
         ulonglong2 seen[H];
         unsigned open = 0, created = 0;
-        int in_slot[H];
 #pragma unroll
         for (int h = 0; h < H; ++h) {
             const bool has = tid + h * kBlock < n_in_use;
-            in_slot[h] = has ? (int)occupied[tid + h * kBlock] : 0;
-            key[h] = has ? slot_key[in_slot[h]] : kEmptyCell;
+            key[h] = has ? slot_key[occupied[tid + h * kBlock]] : kEmptyCell;
             if (has) open |= 1u << h;
             cell[h] = cell_of_key<PD>(key[h], mask, regions);
             pair_index[h] = 0;
@@ -851,7 +855,7 @@ __global__ __launch_bounds__(kBlock) __attribute__((amdgpu_num_sgpr(102))) void 
 #pragma unroll
         for (int h = 0; h < H; ++h)
             if (tid + h * kBlock < n_in_use)
-                slot_cell[in_slot[h]] = (open >> h) & 1u ? -1 : (int)cell[h];
+                place_cell[tid + h * kBlock] = (open >> h) & 1u ? -1 : (int)cell[h];
 
         // the vertices this workgroup created, as in k_build
         int offset[H];
@@ -869,7 +873,7 @@ __global__ __launch_bounds__(kBlock) __attribute__((amdgpu_num_sgpr(102))) void 
 #pragma unroll
         for (int h = 0; h < H; ++h)
             if (tid + h * kBlock < n_in_use)
-                slot_rank[in_slot[h]] =
+                created_rank[tid + h * kBlock] =
                     (created >> h) & 1u ? (unsigned short)(base + offset[h]) : kNotCreated;
         if (!numbers_here) {
             // (for the numbering pass: what this workgroup created, as in k_build)
@@ -891,11 +895,38 @@ __global__ __launch_bounds__(kBlock) __attribute__((amdgpu_num_sgpr(102))) void 
     }
     __syncthreads();        // every slot's cell is known
 
+    // What the points are in the workgroup's own table.  (Behind the keys' way to the table in HBM: a
+    // wavefront's loads wait for its stores before them; thumbnail of 64x64 points 1 us longer, 1024x1024
+    // points pd 2 vd 2 2 us, with the stores first.)
+    auto write_replay = [&]() {
+        uint32_t *words = words_of_tile<kDouble>(replay, vblock, D1);
+#pragma unroll
+        for (int w = 0; w < replay_words(D1); ++w) {
+            uint32_t word = 0;
+#pragma unroll
+            for (int i = 0; i < kPlacesPerWord && kPlacesPerWord * w + i < D1; ++i) {
+                const int in = slot[kPlacesPerWord * w + i];
+                word |= (in >= 0 ? (uint32_t)place_of_slot[in] : kNoPlace) << (kPlaceBits * i);
+            }
+            words[w * kBlock + tid] = word;
+        }
+#pragma unroll
+        for (int r = 0; r < D1; ++r) {
+            if constexpr (kDouble)
+                points64.weights[((size_t)vblock * D1 + r) * kBlock + tid] = valid ? s.weight[r] : 0.0;
+            else
+                reinterpret_cast<float *>(words)[(replay_words(D1) + r) * kBlock + tid] = valid ? s.weight[r] : 0.0f;
+        }
+    };
+
+    int *const table = created_lists.tiles.of(vblock);
     if (!numbers_here) {
         // The numbering pass follows: it needs the length of the workgroup's list, and moves the
         // rows of sums from the hash cells to the vertices.
+        for (int i = tid; i < n_in_use; i += kBlock) table[i] = place_cell[i];
         if (tid == 0) {
             const int sum = group_created;
+            created_lists.tiles.used[vblock] = n_in_use;
             created_lists.block_count[vblock] = sum;
             if (sum) atomicAdd(&created_lists.chunk_count[vblock / kBlocksPerChunk], sum);
         }
@@ -905,17 +936,12 @@ __global__ __launch_bounds__(kBlock) __attribute__((amdgpu_num_sgpr(102))) void 
             const int channel = tid % P;
             for (int i = tid / P; i < n_in_use; i += kBlock / P) {
                 const int sl = (int)occupied[i];
-                const int cell = slot_cell[sl];
+                const int cell = place_cell[i];
                 if (cell >= 0 && channel < VD)
                     atomicAdd(cell_values + (size_t)cell * VD + channel, slot_sum[sl * P + channel]);
             }
         }
-#pragma unroll
-        for (int r = 0; r < D1; ++r) {
-            const int c = slot[r] >= 0 ? slot_cell[slot[r]] : -1;
-            replay[(size_t)r * n_slots + t] = ReplayEntry{c, valid ? (float)s.weight[r] : 0.0f};
-            if constexpr (kDouble) points64.weights[(size_t)r * n_slots + t] = valid ? s.weight[r] : 0.0;
-        }
+        write_replay();
         return;
     }
 
@@ -923,7 +949,7 @@ __global__ __launch_bounds__(kBlock) __attribute__((amdgpu_num_sgpr(102))) void 
     // atomic (the segment is the eighth of the image the workgroup lies in, which is the XCD it
     // runs on when the workgroups are dealt out that way; a small table has one segment).  The
     // atomic takes a microsecond or more to come back -- a segment's workgroups all add to one
-    // address -- so only the first wavefront waits for it: the others end behind their replay rows
+    // address -- so only the first wavefront waits for it: the others end behind their stores
     // and leave their places to the wavefronts of the next workgroup.
     const unsigned stride = segment_stride((uint32_t)numbering.max_vertices, numbering.n_segments);
     unsigned segment = 0;
@@ -944,12 +970,7 @@ __global__ __launch_bounds__(kBlock) __attribute__((amdgpu_num_sgpr(102))) void 
     const unsigned count = (unsigned)group_created;
     unsigned first = 0;
     if (tid == 0 && count) first = atomicAdd(&counters->segment_count[segment].n, count);
-#pragma unroll
-    for (int r = 0; r < D1; ++r) {
-        const int c = slot[r] >= 0 ? slot_cell[slot[r]] : -1;
-        replay[(size_t)r * n_slots + t] = ReplayEntry{c, valid ? (float)s.weight[r] : 0.0f};
-        if constexpr (kDouble) points64.weights[(size_t)r * n_slots + t] = valid ? s.weight[r] : 0.0;
-    }
+    write_replay();
     if (blockIdx.x == 0 && tid < kMaxSegments) {
         counters->n_segments = numbering.n_segments;
         counters->segment_count[tid].n_segments = numbering.n_segments;
@@ -968,14 +989,14 @@ __global__ __launch_bounds__(kBlock) __attribute__((amdgpu_num_sgpr(102))) void 
     const int numbers_from = (int)(segment * stride);
     uint4 *part = created_lists.entries + (size_t)vblock * (size_t)created_lists.stride;
     T *foreign_rows = reinterpret_cast<T *>(part);
-    int *foreign_cells = reinterpret_cast<int *>(part + kTileSlots * (kDouble ? 2 : 1));
+    int2 *foreign_cells = reinterpret_cast<int2 *>(part + kTileSlots * (kDouble ? 2 : 1));
     int n_foreign = 0;
     for (int i0 = 0; i0 < n_in_use; i0 += 64) {
         const int i = i0 + lane;
         const bool has = i < n_in_use;
         const int sl = has ? (int)occupied[i] : 0;
-        const int cell = has ? slot_cell[sl] : -1;
-        const unsigned short rank = slot_rank[sl];
+        const int cell = has ? place_cell[i] : -1;
+        const unsigned short rank = created_rank[has ? i : 0];
         const bool mine = cell >= 0 && rank != kNotCreated;
         const bool foreign = SPLAT_VD != 0 && cell >= 0 && rank == kNotCreated;
         T row[4] = {(T)0, (T)0, (T)0, (T)0};
@@ -983,12 +1004,13 @@ __global__ __launch_bounds__(kBlock) __attribute__((amdgpu_num_sgpr(102))) void 
 #pragma unroll
             for (int j = 0; j < P; ++j) row[j] = slot_sum[sl * P + j];
         }
+        int own = cell < 0 ? -1 : 0;   // (another workgroup's: neighbours())
         if (mine) {
             // (a number beyond the segment is not given out: what runs until the host repeats
             // the build must find a valid one)
             const bool fits = first + rank < stride;
             const int v = fits ? numbers_from + (int)(first + rank) : 0;
-            numbering.cell_vertex[cell] = v;
+            numbering.cell_vertex[cell] = own = v;
             if (fits) {
                 numbering.vertex_keys[v] = slot_key[sl];
                 numbering.vertex_cell[v] = cell;
@@ -1010,13 +1032,14 @@ __global__ __launch_bounds__(kBlock) __attribute__((amdgpu_num_sgpr(102))) void 
                 }
             }
         }
+        if (has) table[i] = own;
         if (SPLAT_VD) {
             const uint64_t b = wave_ballot(foreign);
             const int offset = n_foreign + (int)__builtin_amdgcn_mbcnt_hi(
                                                (uint32_t)(b >> 32), __builtin_amdgcn_mbcnt_lo((uint32_t)b, 0u));
             n_foreign += (int)__builtin_popcountll(b);
             if (foreign) {
-                foreign_cells[offset] = cell;
+                foreign_cells[offset] = make_int2(cell, i);
 #pragma unroll
                 for (int j = 0; j < 4; ++j) foreign_rows[(size_t)offset * 4 + j] = row[j];
             }
@@ -1024,6 +1047,7 @@ __global__ __launch_bounds__(kBlock) __attribute__((amdgpu_num_sgpr(102))) void 
     }
     if (lane == 0) {
         created_lists.block_count[vblock] = n_foreign;
+        created_lists.tiles.used[vblock] = n_in_use;
         // (how many such rows there are in all tells the host whether numbering here pays)
         if ((blockIdx.x / kXcds) % kForeignSampling == 0 && n_foreign)
             atomicAdd(&counters->foreign_rows_sampled.n, (unsigned)n_foreign);
@@ -1168,27 +1192,27 @@ __global__ __launch_bounds__(64) void k_number_vertices(CreatedLists lists, int 
 // vertices follow each other.  u is the + neighbour of v exactly when v is the - neighbour of u:
 // one lookup fills out[a][v].x and out[a][u].y (all entries start as -1).
 // ------------------------------------------------------------------------------------------------
-// After a merging build that numbered its vertices and splatted, the launch also adds the rows of
-// sums that the build's workgroups hold for vertices other workgroups created (ForeignRows) to the
-// value table, now that every vertex has its number: its first foreign_blocks workgroups (a
-// multiple of 8, or 0) take four workgroups' lists each, one per wavefront, a row per group of
-// four lanes.  S: the value type.
+// After a merging build the launch also completes what the build's workgroups left of vertices they did not
+// number themselves, now that every vertex has its number: its first tile_blocks workgroups (a multiple of
+// 8, or 0) take four workgroups' tables each, one per wavefront, and put vertices in the place of hash
+// cells; where the build numbered its vertices and splatted, they add the rows of sums that it holds for
+// vertices of other workgroups to the value table, a row per group of four lanes.  S: the value type.
 template <typename S>
-__device__ __forceinline__ void add_foreign_rows(const CreatedLists &lists, unsigned n_lists,
-                                                 unsigned group, int vd,
+__device__ __forceinline__ void add_foreign_rows(const CreatedLists &lists, unsigned list, int vd,
                                                  const int *__restrict__ cell_vertex, S *values) {
-    const unsigned list = group * (kBlock / 64) + (threadIdx.x >> 6);
-    if (list >= n_lists) return;
     const int lane = threadIdx.x & 63;
     const int n = lists.block_count[list];
     const uint4 *part = lists.entries + (size_t)list * (size_t)lists.stride;
     const S *rows = reinterpret_cast<const S *>(part);
-    const int *cells = reinterpret_cast<const int *>(part + kTileSlots * (sizeof(S) / sizeof(float)));
+    const int2 *cells = reinterpret_cast<const int2 *>(part + kTileSlots * (sizeof(S) / sizeof(float)));
+    int *const table = lists.tiles.of(list);
     const int channel = lane & 3;
     // (what bounds this is the atomic unit, a request per row: asking for all rows of the four
     // lists at once instead of sixteen rows at a time per list made it slower)
     for (int e = lane >> 2; e < n; e += 16) {
-        const int v = cell_vertex[cells[e]];
+        const int2 cell = cells[e];   // (and its place in the workgroup's table)
+        const int v = cell_vertex[cell.x];
+        if (channel == 0) table[cell.y] = v;
         if (channel < vd) atomicAdd(values + (size_t)v * vd + channel, rows[(size_t)e * 4 + channel]);
     }
 }
@@ -1198,7 +1222,7 @@ template <int PD, bool WIDE = false>
 __global__ __launch_bounds__(kBlock) void k_neighbours(VertexTables vertices,
                                                         const Counters *counters,
                                                         const uint64_t *__restrict__ cell_keys,
-                                                        uint32_t mask, unsigned foreign_blocks,
+                                                        uint32_t mask, unsigned tile_blocks,
                                                         CreatedLists lists, unsigned n_lists,
                                                         void *values, int vd, int values_are_double,
                                                         Counters *report, Counters *next_counters,
@@ -1209,7 +1233,7 @@ __global__ __launch_bounds__(kBlock) void k_neighbours(VertexTables vertices,
     // are summed here, and what the next build will count in is cleared.
     // (by the first wavefront of the first workgroup that looks up neighbours, which starts with
     // the launch: a lane per segment)
-    if (report && blockIdx.x == foreign_blocks && threadIdx.x < 64) {
+    if (report && blockIdx.x == tile_blocks && threadIdx.x < 64) {
         static_assert(kMaxSegments <= 64, "a lane per segment");
         const int n_segments = report->n_segments;
         const unsigned c = (int)threadIdx.x < n_segments ? report->segment_count[threadIdx.x].n : 0u;
@@ -1236,17 +1260,26 @@ __global__ __launch_bounds__(kBlock) void k_neighbours(VertexTables vertices,
             reset_counters(next_counters);
         }
     }
-    if (blockIdx.x < foreign_blocks) {
-        const unsigned group = xcd_contiguous_block(blockIdx.x, foreign_blocks, 1);
-        if (values_are_double)
-            add_foreign_rows(lists, n_lists, group, vd, vertices.cell_vertex, static_cast<double *>(values));
-        else
-            add_foreign_rows(lists, n_lists, group, vd, vertices.cell_vertex, static_cast<float *>(values));
+    if (blockIdx.x < tile_blocks) {
+        const unsigned list = xcd_contiguous_block(blockIdx.x, tile_blocks, 1) * (kBlock / 64) + (threadIdx.x >> 6);
+        if (list >= n_lists) return;
+        if (!lists.foreign_rows) {
+            int *const table = lists.tiles.of(list);
+            const int used = lists.tiles.used[list];
+            for (int i = threadIdx.x & 63; i < used; i += 64) {
+                const int cell = table[i];
+                if (cell >= 0) table[i] = vertices.cell_vertex[cell];
+            }
+        } else if (values_are_double) {
+            add_foreign_rows(lists, list, vd, vertices.cell_vertex, static_cast<double *>(values));
+        } else {
+            add_foreign_rows(lists, list, vd, vertices.cell_vertex, static_cast<float *>(values));
+        }
         return;
     }
     const KeyRegions regions{counters->region_lo, counters->region_per_unit};
     const int max_vertices = vertices.max_vertices;
-    SegmentWalk walk(counters, max_vertices, blockIdx.x - foreign_blocks, gridDim.x - foreign_blocks);
+    SegmentWalk walk(counters, max_vertices, blockIdx.x - tile_blocks, gridDim.x - tile_blocks);
     unsigned ib;
     while (walk.next(1u, D1, ib)) {
     const int a = (int)(ib % D1);
@@ -1396,32 +1429,30 @@ __global__ __launch_bounds__(kBlock) void k_splat_dpp(PointMap map,
     }
 }
 
-// The same after a merging build, which leaves a workgroup's points at most kTileSlots vertices: the rows
-// of sums of its four wavefronts meet in LDS first, as in the build, and go out with one request each
-// (1024x1024 points, pd 5: 99 rows a workgroup instead of 165), and the vertices are told from the hash
-// cells once a slot instead of once a row.  What bounds it is the chain of its instructions; 1024x1024
-// points, pd 5, vd 2: 30.7 us a launch, k_splat_dpp 50.2.
+// The same after a merging build, whose workgroups' corners name their vertex by its place in the workgroup's
+// table: the rows of sums of the four wavefronts meet in LDS first, as in the build, and go out with one
+// request each (1024x1024 points, pd 5: 99 rows a workgroup instead of 165).  What bounds it is the chain of
+// its instructions and the requests to the L2 atomic unit; 1024x1024 points, pd 5, vd 2: 21.5 us a launch, 30.8
+// when it looked its vertices up in a table of hashes first.
 template <int VD, int D1>
 __global__ __launch_bounds__(kBlock) void k_splat_merge(PointMap map, const float *__restrict__ input,
-                                                         int in_channels, ReplayEntry *replay,
-                                                         const int *__restrict__ cell_vertex, float *values,
-                                                         int xcd_aware) {
+                                                         int in_channels, const ReplayEntry *__restrict__ replay,
+                                                         float *values, int xcd_aware) {
     static_assert(VD >= 2 && VD <= 4, "register splat handles 2..4 channels");
     constexpr int P = VD == 2 ? 2 : 4;   // values per LDS row of sums
     unsigned vblock;
     if (!block_of_points(map, xcd_aware, vblock)) return;
-    __shared__ int slot_index[kTileSlots];
-    __shared__ float slot_sum[kTileSlots * P];
-    __shared__ unsigned short occupied[kTileSlots];
-    __shared__ int n_occupied;
-    __shared__ int group_index[kBlock / 64][64];
+    __shared__ float place_sum[kTileSlots * P];
     const int tid = threadIdx.x, lane = tid & 63;
-    for (int i = tid; i < kTileSlots; i += kBlock) slot_index[i] = -1;
-    for (int i = tid; i < kTileSlots * P; i += kBlock) slot_sum[i] = 0.0f;
-    if (tid == 0) n_occupied = 0;
-    const size_t t = (size_t)vblock * kBlock * D1 + tid;
-    constexpr size_t T = kBlock;
+    for (int i = tid; i < kTileSlots * P; i += kBlock) place_sum[i] = 0.0f;
     const int n = point_of_thread(map, vblock, tid);
+    const uint32_t *words = words_of_tile(replay, vblock, D1);
+    uint32_t word[replay_words(D1)];
+    float weight[D1];
+#pragma unroll
+    for (int w = 0; w < replay_words(D1); ++w) word[w] = words[w * kBlock + tid];
+#pragma unroll
+    for (int r = 0; r < D1; ++r) weight[r] = weights_behind(words, D1)[r * kBlock + tid];
     // (a lane without a point reads point 0 and takes no part)
     float val[4] = {0.0f, 0.0f, 0.0f, 0.0f};
 #pragma unroll
@@ -1429,43 +1460,24 @@ __global__ __launch_bounds__(kBlock) void k_splat_merge(PointMap map, const floa
         const float x = input[(size_t)(n >= 0 ? n : 0) * in_channels + (j < in_channels ? j : 0)];
         val[j] = j < in_channels ? (n >= 0 ? x : 0.0f) : 1.0f;   // the homogeneous channel when vd-1 are given
     }
-    int index[D1];
-    float weight[D1];
+    unsigned group[D1], n_groups = 0;
+    int place[D1];
 #pragma unroll
     for (int r = 0; r < D1; ++r) {
-        const ReplayEntry e = replay[(size_t)r * T + t];
-        index[r] = n >= 0 ? e.index : -1;
-        weight[r] = n >= 0 ? e.weight : 0.0f;
+        const uint32_t p = place_of_corner(word[r / kPlacesPerWord], r);
+        place[r] = n >= 0 && p < (uint32_t)kTileSlots ? (int)p : -1;
+        if (n < 0) weight[r] = 0.0f;
+        group[r] = wave_groups_in_order((uint64_t)(uint32_t)place[r], wave_ballot(place[r] >= 0), &n_groups);
     }
-    __syncthreads();        // the slots are empty
-    unsigned group[D1], n_groups = 0, present = 0;
-    int slot[D1];
-#pragma unroll
-    for (int r = 0; r < D1; ++r) {
-        if (index[r] >= 0) present |= 1u << r;
-        group[r] = wave_groups_in_order((uint64_t)(uint32_t)index[r], wave_ballot(index[r] >= 0), &n_groups);
-    }
-    place_groups<kTileSlots>(index, group, present, n_groups, lane, group_index[tid >> 6], slot_index, -1,
-                             [](int i) { return (uint32_t)i * 0x9E3779B1u; }, occupied, &n_occupied, slot);
-    add_to_slots<VD, P>(slot_sum, group, slot, weight, val, lane);
+    __syncthreads();        // the rows of sums are zero
+    add_to_slots<VD, P>(place_sum, group, place, weight, val, lane);
     __syncthreads();        // the sums of all four wavefronts are in the rows
-    const int n_in_use = n_occupied, channel = tid % P;
-    for (int i = tid / P; i < n_in_use; i += kBlock / P) {
-        const int sl = (int)occupied[i];
-        int v = slot_index[sl];
-        if (cell_vertex) v = cell_vertex[v];
-        if (channel < VD) atomicAdd(values + (size_t)v * VD + channel, slot_sum[sl * P + channel]);
-        // (read by this lane's row alone until the barrier below)
-        if (cell_vertex) {
-            wave_exchange_in_lds();
-            if (channel == 0) slot_index[sl] = v;
-        }
+    const int used = map.tile_vertices.used[vblock], channel = tid % P;
+    const int *table = map.tile_vertices.of(vblock);
+    for (int i = tid / P; i < used; i += kBlock / P) {
+        const int v = table[i];
+        if (v >= 0 && channel < VD) atomicAdd(values + (size_t)v * VD + channel, place_sum[i * P + channel]);
     }
-    if (!cell_vertex) return;
-    __syncthreads();
-#pragma unroll
-    for (int r = 0; r < D1; ++r)
-        if (slot[r] >= 0) replay[(size_t)r * T + t].index = slot_index[slot[r]];
 }
 
 // Any vd: the same, four channels at a time.  The deduplication loop runs once per block of four
@@ -1486,11 +1498,12 @@ __global__ __launch_bounds__(kBlock) void k_splat_dpp_blocks(int vd, PointMap ma
 
     int vertex[D1];
     float weight[D1];
+    ReplayEntry e[D1];
+    replay_corners<D1>(replay, map.tile_vertices, vblock, threadIdx.x, e);
 #pragma unroll
     for (int r = 0; r < D1; ++r) {
-        const ReplayEntry e = replay[(size_t)r * T + t];
-        vertex[r] = n >= 0 ? e.index : -1;
-        weight[r] = e.weight;
+        vertex[r] = n >= 0 ? e[r].index : -1;
+        weight[r] = e[r].weight;
     }
     if (cell_vertex) {
 #pragma unroll
@@ -1567,7 +1580,7 @@ __global__ __launch_bounds__(kBlock) void k_splat_channels(int d1, int vd, Point
         vertex[i] = -1;
         weight[i] = 0.0f;
         if (r < d1) {
-            const ReplayEntry e = replay[(size_t)r * T + t];
+            const ReplayEntry e = replay_corner(replay, map.tile_vertices, vblock, d1, r, threadIdx.x);
             vertex[i] = n >= 0 ? e.index : -1;
             weight[i] = e.weight;
             if (cell_vertex) {
@@ -1996,6 +2009,76 @@ __global__ __launch_bounds__(kBlock) void k_slice_rows_f64(PointMap map,
     }
 }
 
+// The same after a merging build: the workgroup's vertices' rows go to LDS, each read once, and the points'
+// corners find them there by their places in its table.  Rows of floats and of doubles (the weights of
+// those in weights64); arithmetic as in k_slice_point and k_slice_point_f64.
+// Bound by the stream of weights and places (32 bytes a point for pd = 5) and its chain of three round trips
+// (table, rows, LDS).  From replay rows of 48 bytes a point, every corner gathering its vertex and row, and
+// this, us: 1024x1024 points pd 5 vd 4 15.1 and 10.1, vd 2 12.2 and 8.5; 128x256x256 voxels pd 4 vd 2 103.8
+// and 57.3; 601x803 points in doubles 14.3 and 8.8.
+template <int VD, int D1, typename S>
+__global__ __launch_bounds__(kBlock) void k_slice_tile(PointMap map, const ReplayEntry *__restrict__ replay,
+                                                        const double *__restrict__ weights64,
+                                                        const S *__restrict__ values, S *__restrict__ output,
+                                                        int normalize) {
+    constexpr bool kDouble = sizeof(S) == sizeof(double);
+    constexpr int P = VD == 2 ? 2 : 4;   // values per row in LDS
+    struct alignas(16) Row {
+        S c[P];
+    };
+    using Packed = std::conditional_t<P == 2 && !kDouble, float2, Row>;
+    static_assert(sizeof(Packed) == P * sizeof(S), "rows without gaps");
+    __shared__ Packed rows[kTileSlots];
+    unsigned vblock;
+    if (!block_of_points(map, 1, vblock)) return;
+    const int tid = threadIdx.x;
+    const uint32_t *words = words_of_tile<kDouble>(replay, vblock, D1);
+    const int *table = map.tile_vertices.of(vblock);
+    // (what does not depend on anything read is asked for at once; a table has room for kTileSlots)
+    uint32_t word[replay_words(D1)];
+    S weight[D1];
+#pragma unroll
+    for (int w = 0; w < replay_words(D1); ++w) word[w] = words[w * kBlock + tid];
+#pragma unroll
+    for (int r = 0; r < D1; ++r) {
+        if constexpr (kDouble)
+            weight[r] = weights64[((size_t)vblock * D1 + r) * kBlock + tid];
+        else
+            weight[r] = weights_behind(words, D1)[r * kBlock + tid];
+    }
+    const int used = map.tile_vertices.used[vblock];
+    for (int i = tid; i < used; i += kBlock) {
+        const int v = table[i];
+        const ValueRow<VD, S> row = reinterpret_cast<const ValueRow<VD, S> *>(values)[v >= 0 ? v : 0];
+        Packed packed;
+        S *c = reinterpret_cast<S *>(&packed);
+#pragma unroll
+        for (int j = 0; j < P; ++j) c[j] = j < VD ? row.c[j < VD ? j : 0] : (S)0;
+        rows[i] = packed;
+    }
+    const int n = point_of_thread(map, vblock, tid);
+    __syncthreads();
+    if (n < 0) return;
+    S acc[VD];
+#pragma unroll
+    for (int j = 0; j < VD; ++j) acc[j] = (S)0;
+#pragma unroll
+    for (int r = 0; r < D1; ++r) {
+        const Packed packed = rows[place_of_corner(word[r / kPlacesPerWord], r) & (kTileSlots - 1u)];
+        const S *c = reinterpret_cast<const S *>(&packed);
+#pragma unroll
+        for (int j = 0; j < VD; ++j) acc[j] += weight[r] * c[j];
+    }
+    if (normalize) {
+        const S scale = (S)(1.0 / (double)acc[VD - 1]);
+#pragma unroll
+        for (int j = 0; j < VD - 1; ++j) output[(size_t)n * (VD - 1) + j] = acc[j] * scale;
+    } else {
+#pragma unroll
+        for (int j = 0; j < VD; ++j) output[(size_t)n * VD + j] = acc[j];
+    }
+}
+
 // Any vd: one thread per point and run of four channels.  The pd+1 replay rows, then the value
 // rows, are all requested before the first is used (with a run-time loop the passes waited for
 // two memory round trips per vertex, one after the other); the channels of a run share the index
@@ -2016,13 +2099,10 @@ __global__ __launch_bounds__(kBlock) void k_slice_channels(int vd, PointMap map,
     const int j0 = kSliceRun * (int)(item - slot * runs);
     unsigned vblock;   // as in k_slice_point
     if (!block_of_points(map, 1, vblock)) return;
-    constexpr size_t T = kBlock;
-    const size_t t = (size_t)vblock * kBlock * D1 + slot;
     const int n = point_of_thread(map, vblock, slot);
     if (n < 0) return;
     ReplayEntry e[D1];
-#pragma unroll
-    for (int r = 0; r < D1; ++r) e[r] = replay[(size_t)r * T + t];
+    replay_corners<D1>(replay, map.tile_vertices, vblock, slot, e);
     float own[D1][kSliceRun], last[D1];
 #pragma unroll
     for (int r = 0; r < D1; ++r) {
@@ -2216,12 +2296,10 @@ __global__ __launch_bounds__(kBlock) void k_export_replay(int d1, PointMap map,
                                                            const int *__restrict__ cell_vertex,
                                                            VertexNumbers numbers,
                                                            int *vertex, float *weight) {
-    const size_t t = (size_t)blockIdx.x * kBlock * d1 + threadIdx.x;
-    constexpr size_t T = kBlock;
     const int n = point_of_thread(map, blockIdx.x, threadIdx.x);
     if (n < 0) return;
     for (int r = 0; r < d1; ++r) {
-        const ReplayEntry e = replay[(size_t)r * T + t];
+        const ReplayEntry e = replay_corner(replay, map.tile_vertices, blockIdx.x, d1, r, threadIdx.x);
         if (vertex) {
             int v = e.index;
             if (cell_vertex && v >= 0) v = cell_vertex[v];
@@ -2437,19 +2515,18 @@ hipError_t number_vertices(int pd, const PointMap &map, const CreatedLists &list
 
 hipError_t neighbours(int pd, const VertexTables &vertices, const Counters *counters,
                       const uint64_t *cell_keys, uint32_t n_cells, int launch_vertices,
-                      const CreatedLists *foreign_rows, unsigned n_lists, void *values, int vd,
+                      const CreatedLists *tiles, unsigned n_lists, void *values, int vd,
                       bool values_are_double, Counters *report, Counters *next_counters,
                       HostReport host_report, bool wide_keys, hipStream_t s) {
     if (vertices.max_vertices <= 0) return hipErrorInvalidValue;
     const size_t items = (size_t)(pd + 1) * (size_t)launch_vertices;
-    const unsigned foreign_blocks =
-        foreign_rows ? (blocks_for(n_lists, kBlock / 64) + kXcds - 1u) / kXcds * kXcds : 0u;
+    const unsigned tile_blocks = tiles ? (blocks_for(n_lists, kBlock / 64) + kXcds - 1u) / kXcds * kXcds : 0u;
 #define PLK_NEIGHBOURS(WIDE, DISPATCH)                                                             \
     DISPATCH(pd, hipLaunchKernelGGL((k_neighbours<PD, WIDE>),                                      \
-                                           dim3(foreign_blocks + vertex_blocks(items)),            \
+                                           dim3(tile_blocks + vertex_blocks(items)),            \
                                            dim3(kBlock), 0, s, vertices, counters, cell_keys,      \
-                                           n_cells - 1u, foreign_blocks,                           \
-                                           foreign_rows ? *foreign_rows : CreatedLists{}, n_lists, \
+                                           n_cells - 1u, tile_blocks,                           \
+                                           tiles ? *tiles : CreatedLists{}, n_lists,               \
                                            values, vd, values_are_double ? 1 : 0, report,          \
                                            next_counters, host_report))
     if (wide_keys) {
@@ -2480,14 +2557,14 @@ hipError_t fill_zero(float *p, size_t n, hipStream_t s) {
 }
 
 hipError_t splat_merge(int pd, int vd, const PointMap &map, const float *input, int in_channels,
-                       ReplayEntry *replay, const int *cell_vertex, float *values, int xcd_aware, hipStream_t s) {
+                       ReplayEntry *replay, const int *, float *values, int xcd_aware, hipStream_t s) {
     if (map.n_blocks == 0) return hipSuccess;
+    if (!map.tile_vertices.table) return hipErrorInvalidValue;
     const dim3 grid(map.n_blocks), block(kBlock);
 #define PLK_SPLAT_MERGE(VD)                                                                             \
     case VD:                                                                                            \
         PLK_DISPATCH_PD(pd, hipLaunchKernelGGL((k_splat_merge<VD, PD + 1>), grid, block, 0, s, map,     \
-                                               input, in_channels, replay, cell_vertex, values,         \
-                                               xcd_aware));                                             \
+                                               input, in_channels, replay, values, xcd_aware));         \
         break;
     switch (vd) {
         PLK_SPLAT_MERGE(2) PLK_SPLAT_MERGE(3) PLK_SPLAT_MERGE(4)
@@ -2669,6 +2746,20 @@ hipError_t slice(int pd, int vd, const PointMap &map, const ReplayEntry *replay,
     if (map.n_blocks == 0) return hipSuccess;
     const int d1 = pd + 1;
     const dim3 grid(map.n_blocks), block(kBlock);
+    if (map.tile_vertices.table && vd <= 4) {
+#define PLK_SLICE_TILE(VD)                                                                             \
+    case VD:                                                                                           \
+        PLK_DISPATCH_PD(pd, hipLaunchKernelGGL((k_slice_tile<VD, PD + 1, float>), grid, block, 0, s, map, \
+                                               replay, (const double *)nullptr, values, output, normalize)); \
+        break;
+        switch (vd) {
+            PLK_SLICE_TILE(2) PLK_SLICE_TILE(3) PLK_SLICE_TILE(4)
+            default: return hipErrorInvalidValue;
+        }
+#undef PLK_SLICE_TILE
+        return hipGetLastError();
+    }
+    if (map.tile_vertices.table && vd <= 64) return slice_tile_channels(pd, vd, map, replay, values, output, normalize, s);
 #define PLK_SLICE(VD)                                                                          \
     case VD:                                                                                   \
         hipLaunchKernelGGL(k_slice_point<VD>, grid, block, 0, s, d1, map, replay,              \
@@ -2718,9 +2809,13 @@ hipError_t slice_rows_f64(int pd, int vd, const PointMap &map, const ReplayEntry
     const dim3 grid(map.n_blocks), block(kBlock);
 #define PLK_SLICE_ROWS(VD)                                                                     \
     case VD:                                                                                   \
-        PLK_DISPATCH_PD(pd, hipLaunchKernelGGL((k_slice_rows_f64<VD, PD + 1>), grid, block, 0, \
-                                               s, map, replay, weights, cell_vertex, values,   \
-                                               output, normalize));                            \
+        if (map.tile_vertices.table)                                                                   \
+            PLK_DISPATCH_PD(pd, hipLaunchKernelGGL((k_slice_tile<VD, PD + 1, double>), grid, block, 0, s, map, \
+                                                   replay, weights, values, output, normalize)) \
+        else                                                                                   \
+            PLK_DISPATCH_PD(pd, hipLaunchKernelGGL((k_slice_rows_f64<VD, PD + 1>), grid, block, 0, \
+                                                   s, map, replay, weights, cell_vertex, values, \
+                                                   output, normalize))                         \
         break;
     switch (vd) {
         PLK_SLICE_ROWS(2) PLK_SLICE_ROWS(3) PLK_SLICE_ROWS(4)

@@ -45,9 +45,11 @@ __global__ __launch_bounds__(kBlock) void k_splat_f64(int vd, PointMap map,
     // place (it has said so), carry vertex -1 and belong to no group
     int vertex[D1];
     double weight[D1];
+    ReplayEntry corner[D1];
+    replay_corners<D1, true>(replay, map.tile_vertices, vblock, threadIdx.x, corner);
 #pragma unroll
     for (int r = 0; r < D1; ++r) {
-        vertex[r] = n >= 0 ? replay[(size_t)r * n_slots + t].index : -1;
+        vertex[r] = n >= 0 ? corner[r].index : -1;
         weight[r] = weights[(size_t)r * n_slots + t];
     }
     if (cell_vertex) {
@@ -110,9 +112,11 @@ __global__ __launch_bounds__(kBlock) void k_slice_point_f64(int vd, PointMap map
     if (n < 0) return;
     int vertex[D1];
     double weight[D1];
+    ReplayEntry corner[D1];
+    replay_corners<D1, true>(replay, map.tile_vertices, vblock, threadIdx.x, corner);
 #pragma unroll
     for (int r = 0; r < D1; ++r) {
-        vertex[r] = replay[(size_t)r * n_slots + t].index;
+        vertex[r] = corner[r].index;
         weight[r] = weights[(size_t)r * n_slots + t];
     }
     if (cell_vertex) {
@@ -166,9 +170,11 @@ __global__ __launch_bounds__(kBlock) void k_slice_f64(int vd, PointMap map,
     if (n < 0) return;
     const int j = blockIdx.y;
     double sum = 0.0, homogeneous = 0.0;
+    ReplayEntry corner[D1];
+    replay_corners<D1, true>(replay, map.tile_vertices, vblock, threadIdx.x, corner);
 #pragma unroll
     for (int r = 0; r < D1; ++r) {
-        int v = replay[(size_t)r * n_slots + t].index;
+        int v = corner[r].index;
         if (v < 0) continue;
         if (cell_vertex) v = cell_vertex[v];
         const double w = weights[(size_t)r * n_slots + t];

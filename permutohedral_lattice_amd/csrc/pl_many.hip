@@ -7,6 +7,8 @@
 // of the GPU, and an iteration on two images and their four lattices was 22 launches on four streams (and 13
 // events): the host needed as long for them as the GPU.  Here it is six or seven launches on one stream.
 // Two images, five iterations: 1154 us as launches of their own, 720 this way.
+#include <type_traits>
+
 #include "pl_device.h"
 #include "pl_kernels.h"
 
@@ -98,6 +100,7 @@ constexpr int kPairPoints = 2;
 
 template <int D1, int L>
 __device__ __forceinline__ void sliced_channels(int vd, const ReplayEntry *__restrict__ replay,
+                                                const TileVertices &tiles,
                                                 const float *__restrict__ values, unsigned vblock,
                                                 const unsigned (&slot)[kPairPoints], const int (&n)[kPairPoints],
                                                 int sub, float (&message)[kPairPoints][4]) {
@@ -105,11 +108,10 @@ __device__ __forceinline__ void sliced_channels(int vd, const ReplayEntry *__res
     ReplayEntry mine[kPairPoints][E];
 #pragma unroll
     for (int q = 0; q < kPairPoints; ++q) {
-        const size_t t = (size_t)vblock * kBlock * D1 + slot[q];
 #pragma unroll
         for (int u = 0; u < E; ++u) {
             const int r = u * L + sub;
-            mine[q][u] = replay[(size_t)(r < D1 ? r : 0) * kBlock + t];
+            mine[q][u] = replay_corner(replay, tiles, vblock, D1, r < D1 ? r : 0, slot[q]);
         }
     }
     const int c = 4 * sub;
@@ -166,8 +168,8 @@ __global__ __launch_bounds__(kBlock) void k_slice_pairs(Items<SlicePair> items, 
         n[q] = point_of_thread(work.map, vblock, slot[q]);   // (the same for all L lanes)
     }
     float a[kPairPoints][4], b[kPairPoints][4];
-    sliced_channels<D1A, L>(vd, work.replay_a, work.values_a, vblock, slot, n, sub, a);
-    sliced_channels<D1B, L>(vd, work.replay_b, work.values_b, vblock, slot, n, sub, b);
+    sliced_channels<D1A, L>(vd, work.replay_a, work.map.tile_vertices, work.values_a, vblock, slot, n, sub, a);
+    sliced_channels<D1B, L>(vd, work.replay_b, work.tiles_b, work.values_b, vblock, slot, n, sub, b);
     const int classes = vd - 1, c = 4 * sub;
 #pragma unroll
     for (int q = 0; q < kPairPoints; ++q) {
@@ -212,7 +214,407 @@ __global__ __launch_bounds__(kBlock) void k_slice_pairs(Items<SlicePair> items, 
     }
 }
 
+// ------------------------------------------------------------------------------------------------
+// The slices of many channels after a merging build.  A workgroup's points touch a hundred or two of
+// vertices between them, where its corners are 256 * D1: the vertices' rows go to LDS, each read once, and
+// two lanes a point sum the rows from there, every other piece of four channels each.  What they make of a
+// point goes out by way of LDS as well, so that a wavefront's stores are runs of memory.  Workgroups of more
+// vertices than there are rows in LDS gather from memory, corner by corner.  Sums in the order of k_slice_quads
+// and sliced_channels, each product and sum rounded once instead of twice.
+// Bound by what a workgroup waits for (table, rows, LDS, its stores), 32 wavefronts a CU for a lattice alone, 24
+// for two; vector instructions half of the time.  321x481 points, pd 5, vd 22: 9.2 us a launch (k_slice_quads on
+// replay rows 12.6, on places 14.0; a lane a point with its stores 84 bytes apart 14.8; eight lanes a point
+// 13.2).  Pairs of 2 x 512x512 points with the softmax, 21 classes: 43.7 us (k_slice_pairs on rows 56.5; a lane
+// a point 55.1; eight lanes 62.0; with five wavefronts a SIMD, not six, 49.3).
+// (A row in LDS is an odd number of 16-byte pieces: the same piece of sixteen rows lies in different banks.)
+// ------------------------------------------------------------------------------------------------
+constexpr int kTileLanes = 2, kTileThreads = kTileLanes * kBlock;
+constexpr int kTileChannels = 32;   // channels a workgroup takes at most
+// Channels from `from` on of the rows of one lattice of a workgroup's points
+struct Tile {
+    const int *table;
+    const float *values;
+    int used, vd, from;
+    float *rows, *last;   // in LDS: Q pieces of four channels, row_stride(Q) floats apart; the homogeneous channels
+};
+__host__ __device__ constexpr int row_stride(int Q) { return 4 * (Q | 1); }
+// Rows in LDS: with 28 KB a CU holds four workgroups, 32 wavefronts, and of 21 channels a workgroup 247 rows
+inline unsigned tile_rows(int Q) {
+    const unsigned rows = (28u << 10) / (sizeof(float) * (unsigned)(row_stride(Q) + 1));
+    return rows < (unsigned)kTileSlots ? rows : (unsigned)kTileSlots;
+}
+// (what the rows leave takes the 256 points' channels later)
+inline size_t tile_lds(int Q, unsigned rows) {
+    const size_t in = (size_t)rows * (row_stride(Q) + 1), out = (size_t)kBlock * 4 * Q;
+    return sizeof(float) * (in > out ? in : out);
+}
+__device__ __forceinline__ float one_of(int i, float a, float b, float c, float d) {
+    return i == 0 ? a : i == 1 ? b : i == 2 ? c : d;
+}
+// The four channels from c on of a row in memory (what is past vd: anything)
+__device__ __forceinline__ FourFloats piece_of_row(const float *row, int vd, int c) {
+    const int start = c < vd - 4 ? c : vd - 4, shift = c - start;
+    const FourFloats x = *reinterpret_cast<const FourFloats *>(row + start);
+    if (shift == 0) return x;
+    return FourFloats{{one_of(shift, x.c[0], x.c[1], x.c[2], x.c[3]), one_of(shift + 1, x.c[0], x.c[1], x.c[2], x.c[3]),
+                       x.c[3], x.c[3]}};
+}
+// (as many lanes a row as it has pieces, or some more; two rows a group of lanes in flight)
+template <int Q>
+__device__ __forceinline__ void rows_to_lds(const Tile &tile) {
+    constexpr int L = Q <= 2 ? 2 : Q <= 4 ? 4 : 8, kGroups = kTileThreads / L, kAhead = 2;
+    const int sub = threadIdx.x % L;
+    for (int i0 = threadIdx.x / L; i0 < tile.used; i0 += kAhead * kGroups) {
+        int v[kAhead];
+        FourFloats x[kAhead];
+        float last[kAhead];
+#pragma unroll
+        for (int u = 0; u < kAhead; ++u) v[u] = tile.table[i0 + u * kGroups < tile.used ? i0 + u * kGroups : i0];
+#pragma unroll
+        for (int u = 0; u < kAhead; ++u) {
+            const float *row = tile.values + (size_t)(v[u] >= 0 ? v[u] : 0) * tile.vd;
+            x[u] = piece_of_row(row, tile.vd, tile.from + 4 * sub);
+            last[u] = row[tile.vd - 1];
+        }
+#pragma unroll
+        for (int u = 0; u < kAhead; ++u) {
+            const int i = i0 + u * kGroups;
+            if (i >= tile.used) continue;
+            if (sub < Q)
+                *reinterpret_cast<float4 *>(tile.rows + i * row_stride(Q) + 4 * sub) =
+                    make_float4(x[u].c[0], x[u].c[1], x[u].c[2], x[u].c[3]);
+            if (sub == 0) tile.last[i] = last[u];
+        }
+    }
+}
+// A point's corners: places (of points that are none, or that the build could not place: 0) and weights
+template <int D1>
+struct Corners {
+    int place[D1];
+    float weight[D1];
+};
+template <int D1>
+__device__ __forceinline__ Corners<D1> corners_of(const ReplayEntry *__restrict__ replay, unsigned vblock, int point,
+                                                  int used) {
+    const uint32_t *words = words_of_tile(replay, vblock, D1);
+    uint32_t word[replay_words(D1)];
+#pragma unroll
+    for (int w = 0; w < replay_words(D1); ++w) word[w] = words[w * kBlock + point];
+    Corners<D1> corners;
+#pragma unroll
+    for (int r = 0; r < D1; ++r) {
+        corners.weight[r] = weights_behind(words, D1)[r * kBlock + point];
+        const int place = (int)place_of_corner(word[r / kPlacesPerWord], r);
+        corners.place[r] = place < used ? place : 0;
+    }
+    return corners;
+}
+// (a piece of all corners in flight, not all pieces: the next one's addresses come after this one's sums)
+template <int D1>
+__device__ __forceinline__ void next_piece(Corners<D1> &corners, float (&sums)[4]) {
+#pragma unroll
+    for (int j = 0; j < 4; ++j) asm volatile("" : "+v"(sums[j]));
+#pragma unroll
+    for (int r = 0; r < D1; ++r) asm volatile("" : "+v"(corners.place[r]), "+v"(sums[0]));
+}
+// acc := piece q of the point's channels
+template <int D1, int Q, bool IN_LDS>
+__device__ __forceinline__ void sum_corners(const Tile &tile, int q, const Corners<D1> &corners, float (&acc)[4]) {
+#pragma unroll
+    for (int j = 0; j < 4; ++j) acc[j] = 0.0f;
+#pragma unroll
+    for (int r = 0; r < D1; ++r) {
+        FourFloats y;
+        if constexpr (IN_LDS) {
+            const float4 x = *reinterpret_cast<const float4 *>(tile.rows + corners.place[r] * row_stride(Q) + 4 * q);
+            y = FourFloats{{x.x, x.y, x.z, x.w}};
+        } else {
+            const int v = tile.table[corners.place[r]];
+            y = piece_of_row(tile.values + (size_t)(v >= 0 ? v : 0) * tile.vd, tile.vd, tile.from + 4 * q);
+        }
+#pragma unroll
+        for (int j = 0; j < 4; ++j) acc[j] = __builtin_fmaf(corners.weight[r], y.c[j], acc[j]);
+    }
+}
+// The sum of the homogeneous channel
+template <int D1, bool IN_LDS>
+__device__ __forceinline__ float sum_of_last(const Tile &tile, const Corners<D1> &corners) {
+    float sum = 0.0f;
+#pragma unroll
+    for (int r = 0; r < D1; ++r) {
+        if constexpr (IN_LDS) {
+            sum = __builtin_fmaf(corners.weight[r], tile.last[corners.place[r]], sum);
+        } else {
+            const int v = tile.table[corners.place[r]];
+            sum = __builtin_fmaf(corners.weight[r], tile.values[(size_t)(v >= 0 ? v : 0) * tile.vd + tile.vd - 1], sum);
+        }
+    }
+    return sum;
+}
+
+// x of lane I of this lane's two (quad_perm [0,0,2,2] or [1,1,3,3])
+template <int I>
+__device__ __forceinline__ float lane_of_two(float x) {
+    return __int_as_float(__builtin_amdgcn_mov_dpp(__float_as_int(x), I == 0 ? 0xA0 : 0xF5, 0xf, 0xf, true));
+}
+
+// The workgroup's 256 points' rows of `channels` channels (at least four) in memory, `stride` floats apart and
+// offset by `from`, piece by piece: floats 4 i .. 4 i + 3 of the rows one behind the other, which lie one
+// behind the other in memory as well where neighbours in the workgroup are neighbours there.  per_channel:
+// 2^20 / channels, rounded up (i / channels for i < 2^14 as a product, channels < 64).
+struct PointRows {
+    int channels, stride, from;
+    unsigned per_channel;
+};
+struct Piece {
+    int p, c;      // its first float: point and channel
+    bool whole;    // four floats of memory
+};
+__device__ __forceinline__ Piece piece_at(int i, const PointRows &rows, const int *n_of) {
+    Piece piece;
+    piece.p = (int)(((unsigned)(4 * i) * rows.per_channel) >> 20);
+    piece.c = 4 * i - piece.p * rows.channels;
+    const int left = rows.channels - piece.c;   // of this point's
+    piece.whole = n_of[piece.p] >= 0 &&
+                  (left >= 4 || (rows.channels == rows.stride && n_of[piece.p + 1] == n_of[piece.p] + 1));
+    return piece;
+}
+__device__ __forceinline__ void store_points(const float *from_lds, float *output, const PointRows &rows, const int *n_of) {
+    for (int i = threadIdx.x; i < kBlock / 4 * rows.channels; i += kTileThreads) {
+        const Piece piece = piece_at(i, rows, n_of);
+        const float4 x = reinterpret_cast<const float4 *>(from_lds)[i];
+        const float y[4] = {x.x, x.y, x.z, x.w};
+        if (piece.whole) {
+            *reinterpret_cast<FourFloats *>(output + (size_t)n_of[piece.p] * rows.stride + rows.from + piece.c) =
+                FourFloats{{y[0], y[1], y[2], y[3]}};
+        } else {
+            int p = piece.p, c = piece.c;
+#pragma unroll
+            for (int j = 0; j < 4; ++j) {
+                const int n = n_of[p];
+                if (n >= 0) output[(size_t)n * rows.stride + rows.from + c] = y[j];
+                if (++c == rows.channels) c = 0, ++p;
+            }
+        }
+    }
+}
+// (the pieces this thread brings to LDS: read before the LDS is free for them, left there afterwards)
+template <int Q>
+__device__ __forceinline__ void load_points(const float *input, const PointRows &rows, const int *n_of,
+                                            FourFloats (&x)[(4 * Q * kBlock / 4 + kTileThreads - 1) / kTileThreads]) {
+#pragma unroll
+    for (int k = 0; k < (4 * Q * kBlock / 4 + kTileThreads - 1) / kTileThreads; ++k) {
+        const int i = (int)threadIdx.x + k * kTileThreads;
+        if (i >= kBlock / 4 * rows.channels) continue;
+        const Piece piece = piece_at(i, rows, n_of);
+        if (piece.whole) {
+            x[k] = *reinterpret_cast<const FourFloats *>(input + (size_t)n_of[piece.p] * rows.stride + rows.from + piece.c);
+        } else {
+            int p = piece.p, c = piece.c;
+#pragma unroll
+            for (int j = 0; j < 4; ++j) {
+                const int n = n_of[p];
+                x[k].c[j] = n >= 0 ? input[(size_t)n * rows.stride + rows.from + c] : 0.0f;
+                if (++c == rows.channels) c = 0, ++p;
+            }
+        }
+    }
+}
+template <int Q>
+__device__ __forceinline__ void points_to_lds(float *lds, const PointRows &rows,
+                                              const FourFloats (&x)[(4 * Q * kBlock / 4 + kTileThreads - 1) / kTileThreads]) {
+#pragma unroll
+    for (int k = 0; k < (4 * Q * kBlock / 4 + kTileThreads - 1) / kTileThreads; ++k) {
+        const int i = (int)threadIdx.x + k * kTileThreads;
+        if (i < kBlock / 4 * rows.channels)
+            reinterpret_cast<float4 *>(lds)[i] = make_float4(x[k].c[0], x[k].c[1], x[k].c[2], x[k].c[3]);
+    }
+}
+
+// workgroup (x, y): channels 32 y .. of the points of block x.  Q: pieces of four channels of a workgroup's.
+template <int D1, int Q>
+__global__ __launch_bounds__(kTileThreads) void k_slice_tile_channels(int vd, PointMap map,
+                                                                      const ReplayEntry *__restrict__ replay,
+                                                                      const float *__restrict__ values,
+                                                                      float *__restrict__ output, int normalize,
+                                                                      int n_rows, PointRows rows) {
+    extern __shared__ float4 lds4[];
+    __shared__ int n_of[kBlock + 1];
+    float *lds = reinterpret_cast<float *>(lds4);
+    unsigned vblock;
+    if (!block_of_points(map, 1, vblock)) return;
+    const int tid = threadIdx.x, sub = tid % kTileLanes, point = tid / kTileLanes;
+    rows.from = kTileChannels * (int)blockIdx.y;
+    if (rows.stride - rows.from < rows.channels) {   // (the last of several workgroups of a tile)
+        rows.channels = rows.stride - rows.from;
+        rows.per_channel = ((1u << 20) + (unsigned)rows.channels - 1u) / (unsigned)rows.channels;
+    }
+    const Tile tile{map.tile_vertices.of(vblock), values, map.tile_vertices.used[vblock],
+                    vd, rows.from, lds, lds + n_rows * row_stride(Q)};
+    Corners<D1> corners = corners_of<D1>(replay, vblock, point, tile.used);
+    const bool in_lds = tile.used <= n_rows;
+    if (in_lds) rows_to_lds<Q>(tile);
+    if (tid <= kBlock) n_of[tid] = tid < kBlock ? point_of_thread(map, vblock, tid) : -1;
+    __syncthreads();
+    constexpr int kOwn = (Q + kTileLanes - 1) / kTileLanes;   // pieces of a lane
+    float y[kOwn][4];
+    auto slice_point = [&](auto rows_in_lds) {
+        constexpr bool kInLds = decltype(rows_in_lds)::value;
+        const float scale = normalize ? (float)(1.0 / (double)sum_of_last<D1, kInLds>(tile, corners)) : 1.0f;
+#pragma unroll
+        for (int k = 0; k < kOwn; ++k) {
+            const int q = kTileLanes * k + sub;
+            sum_corners<D1, Q, kInLds>(tile, q < Q ? q : 0, corners, y[k]);
+#pragma unroll
+            for (int j = 0; j < 4; ++j) y[k][j] = normalize ? y[k][j] * scale : y[k][j];
+            next_piece(corners, y[k]);
+        }
+    };
+    if (in_lds)
+        slice_point(std::true_type{});
+    else
+        slice_point(std::false_type{});
+    __syncthreads();        // the rows are done with
+#pragma unroll
+    for (int k = 0; k < kOwn; ++k) {
+        const int c = 4 * (kTileLanes * k + sub);
+#pragma unroll
+        for (int j = 0; j < 4; ++j)
+            if (c + j < rows.channels) lds[point * rows.channels + c + j] = y[k][j];
+    }
+    __syncthreads();
+    store_points(lds, output, rows, n_of);
+}
+
+// Q: pieces of four classes
+template <int D1A, int D1B, int Q>
+__global__ __launch_bounds__(kTileThreads, D1A <= 6 ? 6 : 4) void k_slice_tile_pairs(Items<SlicePair> items, int vd, int n_rows,
+                                                                   PointRows rows) {
+    extern __shared__ float4 lds4[];
+    __shared__ int n_of[kBlock + 1];
+    float *lds = reinterpret_cast<float *>(lds4);
+    unsigned block, blocks;
+    const SlicePair &work = item_of(items, block, blocks);
+    if (block >= work.map.n_blocks) return;
+    const unsigned vblock = xcd_contiguous_block(block, work.map.n_blocks, 1);
+    const int tid = threadIdx.x, sub = tid % kTileLanes, point = tid / kTileLanes;
+    if (tid <= kBlock) n_of[tid] = tid < kBlock ? point_of_thread(work.map, vblock, tid) : -1;
+    const int used_a = work.map.tile_vertices.used[vblock], used_b = work.tiles_b.used[vblock];
+    const Tile a{work.map.tile_vertices.of(vblock), work.values_a, used_a, vd, 0, lds,
+                 lds + n_rows * row_stride(Q)};
+    const Tile b{work.tiles_b.of(vblock), work.values_b, used_b, vd, 0,
+                 a.rows + used_a * row_stride(Q), a.last + used_a};
+    Corners<D1A> corners_a = corners_of<D1A>(work.replay_a, vblock, point, used_a);
+    Corners<D1B> corners_b = corners_of<D1B>(work.replay_b, vblock, point, used_b);
+    const bool in_lds = used_a + used_b <= n_rows;
+    if (in_lds) {
+        rows_to_lds<Q>(a);
+        rows_to_lds<Q>(b);
+    }
+    __syncthreads();
+    FourFloats logits[(4 * Q * kBlock / 4 + kTileThreads - 1) / kTileThreads];
+    if (work.logits) load_points<Q>(work.logits, rows, n_of, logits);
+    constexpr int kOwn = (Q + kTileLanes - 1) / kTileLanes;   // pieces of a lane
+    float y[kOwn][4];
+    auto slice_point = [&](auto rows_in_lds) {
+        constexpr bool kInLds = decltype(rows_in_lds)::value;
+        // (a division a lane, one lattice's each)
+        const float last_a = sum_of_last<D1A, kInLds>(a, corners_a), last_b = sum_of_last<D1B, kInLds>(b, corners_b);
+        const float one_over = (float)(1.0 / (double)(sub == 0 ? last_a : last_b));
+        const float scale_a = lane_of_two<0>(one_over), scale_b = lane_of_two<1>(one_over);
+#pragma unroll
+        for (int k = 0; k < kOwn; ++k) {
+            const int q = kTileLanes * k + sub < Q ? kTileLanes * k + sub : 0;
+            float z[4];
+            sum_corners<D1A, Q, kInLds>(a, q, corners_a, y[k]);
+            sum_corners<D1B, Q, kInLds>(b, q, corners_b, z);
+#pragma unroll
+            for (int j = 0; j < 4; ++j) y[k][j] = y[k][j] * scale_a + z[j] * scale_b;
+            next_piece(corners_a, y[k]);
+            next_piece(corners_b, y[k]);
+        }
+    };
+    if (in_lds)
+        slice_point(std::true_type{});
+    else
+        slice_point(std::false_type{});
+    __syncthreads();        // the rows are done with
+    float *const own = lds + point * rows.channels;
+    if (work.logits) {
+        points_to_lds<Q>(lds, rows, logits);
+        __syncthreads();
+        float highest = -INFINITY;
+#pragma unroll
+        for (int k = 0; k < kOwn; ++k) {
+            const int c = 4 * (kTileLanes * k + sub);
+#pragma unroll
+            for (int j = 0; j < 4; ++j) {
+                if (c + j < rows.channels) {
+                    y[k][j] = own[c + j] + y[k][j];
+                    highest = fmaxf(highest, y[k][j]);
+                }
+            }
+        }
+        highest = fmaxf(lane_of_two<0>(highest), lane_of_two<1>(highest));
+        double wide_sum = 0.0;
+#pragma unroll
+        for (int k = 0; k < kOwn; ++k) {
+            const int c = 4 * (kTileLanes * k + sub);
+#pragma unroll
+            for (int j = 0; j < 4; ++j) {
+                y[k][j] = expf(y[k][j] - highest);
+                if (c + j < rows.channels) wide_sum += (double)y[k][j];
+            }
+        }
+        wide_sum += __shfl_xor(wide_sum, 1);
+        // (a product of doubles rounded once: within 2^-29 of an ulp of the quotient's rounding)
+        const double one_over = 1.0 / (double)(float)wide_sum;
+#pragma unroll
+        for (int k = 0; k < kOwn; ++k) {
+#pragma unroll
+            for (int j = 0; j < 4; ++j) y[k][j] = (float)((double)y[k][j] * one_over);
+        }
+    }
+    // (a point's channels are its own two lanes' in LDS)
+#pragma unroll
+    for (int k = 0; k < kOwn; ++k) {
+        const int c = 4 * (kTileLanes * k + sub);
+#pragma unroll
+        for (int j = 0; j < 4; ++j)
+            if (c + j < rows.channels) own[c + j] = y[k][j];
+    }
+    __syncthreads();
+    store_points(lds, work.output, rows, n_of);
+}
+
 }  // namespace
+
+static PointRows point_rows(int channels, int stride) {
+    return PointRows{channels, stride, 0, ((1u << 20) + (unsigned)channels - 1u) / (unsigned)channels};
+}
+
+hipError_t slice_tile_channels(int pd, int vd, const PointMap &map, const ReplayEntry *replay, const float *values,
+                               float *output, int normalize, hipStream_t s) {
+    if (map.n_blocks == 0) return hipSuccess;
+    if (!map.tile_vertices.table || vd < kManyChannels) return hipErrorInvalidValue;
+    const int out_ch = normalize ? vd - 1 : vd, channels = out_ch < kTileChannels ? out_ch : kTileChannels;
+    const int Q = (channels + 3) / 4;
+    const unsigned n_rows = tile_rows(Q);
+    const dim3 grid(map.n_blocks, (unsigned)((out_ch + kTileChannels - 1) / kTileChannels)), block(kTileThreads);
+#define PLK_SLICE_TILE(Q)                                                                                     \
+    case Q:                                                                                                   \
+        PLK_DISPATCH_PD(pd, hipLaunchKernelGGL((k_slice_tile_channels<PD + 1, Q>), grid, block,               \
+                                               tile_lds(Q, n_rows), s, vd, map, replay, values, output,       \
+                                               normalize, (int)n_rows, point_rows(channels, out_ch)));        \
+        break;
+    switch (Q) {
+        PLK_SLICE_TILE(1) PLK_SLICE_TILE(2) PLK_SLICE_TILE(3) PLK_SLICE_TILE(4) PLK_SLICE_TILE(5)
+        PLK_SLICE_TILE(6) PLK_SLICE_TILE(7) PLK_SLICE_TILE(8)
+        default: return hipErrorInvalidValue;
+    }
+#undef PLK_SLICE_TILE
+    return hipGetLastError();
+}
 
 template <int N>
 static hipError_t blur_runs(int vd, int n, const BlurWork *work, hipStream_t s) {
@@ -253,16 +655,32 @@ hipError_t slice_pairs(int pd_a, int pd_b, int vd, int n, const SlicePair *work,
     const unsigned blocks = all_blocks(items);
     if (!blocks) return hipSuccess;
     const int lanes = vd <= 16 ? 4 : 8;
-    const dim3 grid(blocks, (unsigned)(lanes / kPairPoints)), block(kBlock);
+    bool tiles = true;
+    for (int i = 0; i < n; ++i) tiles = tiles && work[i].map.tile_vertices.table && work[i].tiles_b.table;
+    const int Q = (vd - 1 + 3) / 4;
+    const unsigned n_rows = tile_rows(Q);
+    const dim3 grid(blocks, tiles ? 1u : (unsigned)(lanes / kPairPoints)), block(tiles ? kTileThreads : kBlock);
+#define PLK_PAIR_TILES(A, B, Q)                                                                            \
+    case Q:                                                                                                \
+        hipLaunchKernelGGL((k_slice_tile_pairs<A + 1, B + 1, Q>), grid, block, tile_lds(Q, n_rows), s, items, \
+                           vd, (int)n_rows, point_rows(vd - 1, vd - 1));                                   \
+        break;
 #define PLK_PAIR(A, B)                                                                                     \
     if (pd_a == A && pd_b == B) {                                                                          \
-        if (lanes == 4)                                                                                    \
+        if (tiles)                                                                                         \
+            switch (Q) {                                                                                   \
+                PLK_PAIR_TILES(A, B, 1) PLK_PAIR_TILES(A, B, 2) PLK_PAIR_TILES(A, B, 3) PLK_PAIR_TILES(A, B, 4)                    \
+                PLK_PAIR_TILES(A, B, 5) PLK_PAIR_TILES(A, B, 6) PLK_PAIR_TILES(A, B, 7)                    \
+                PLK_PAIR_TILES(A, B, 8)                                                                    \
+            }                                                                                              \
+        else if (lanes == 4)                                                                               \
             hipLaunchKernelGGL((k_slice_pairs<A + 1, B + 1, 4>), grid, block, 0, s, items, vd);            \
         else                                                                                               \
             hipLaunchKernelGGL((k_slice_pairs<A + 1, B + 1, 8>), grid, block, 0, s, items, vd);            \
     }
     PLK_PAIR(3, 2) PLK_PAIR(5, 2) PLK_PAIR(4, 3) PLK_PAIR(6, 3)
 #undef PLK_PAIR
+#undef PLK_PAIR_TILES
     return hipGetLastError();
 }
 

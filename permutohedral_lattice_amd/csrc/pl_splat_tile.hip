@@ -15,54 +15,47 @@ namespace {
 using namespace device;
 
 // A workgroup's 256 points have 256 * d1 (corner, vertex) pairs but only about a hundred distinct
-// vertices.  The pairs are sorted by vertex with a counting sort in LDS -- a small hash table gives
-// every vertex a slot and counts its pairs, each pair's rank in its slot comes back from the count --
-// and 32 groups of sixteen lanes, a lane on channels c, c + 16, ..., then run over their share of
+// vertices, which they name by a place in the workgroup's table.  The pairs are sorted by place with a
+// counting sort in LDS -- each pair's rank comes back from the count of its place -- and 32 groups of sixteen lanes, a lane on channels c, c + 16, ..., then run over their share of
 // the sorted pairs each: weight times the point's row (in LDS, loaded once) into registers until the
 // vertex changes, and one request per line of the vertex's row then.
 // What bounds it is the instructions of that last loop and the requests to the L2 atomic unit, about
 // 130 rows a workgroup.  k_splat_channels, which takes a wavefront's pairs vertex by vertex, loads the
 // rows once per two corners and sends a row per wavefront and vertex (about 165): 2 x 321x481 points, pd = 5,
-// vd = 22: 37.0 us a launch, this 26.5.
-// After a merging build only: it leaves a workgroup at most kTileSlots vertices (a build with more is
-// repeated without merging), so that every vertex finds a slot.
-// Two threads to a point, which share its corners (one thread to a point, 16 groups of lanes: 27.6 us;
-// every lane looking for its slot instead of the first of a run: 27.1).
+// vd = 22: 37.0 us a launch, this 25.5 (26.5 when it looked its vertices up in a table of hashes first).
+// After a merging build only (TileVertices).
+// Two threads to a point, which share its corners (one thread to a point, 16 groups of lanes: 27.6 us).
 constexpr unsigned kSides = 2, kThreads = kSides * kBlock;
 constexpr unsigned kMaxCorners = (kMaxPd + 1 + kSides - 1) / kSides;   // of a thread
 
 template <int K>
 __global__ __launch_bounds__(kThreads) void k_splat_tile(int d1, int vd, PointMap map, const float *__restrict__ input,
-                                                        int in_channels, ReplayEntry *replay,
-                                                        const int *__restrict__ cell_vertex, float *values,
-                                                        int xcd_aware) {
+                                                        int in_channels, const ReplayEntry *__restrict__ replay,
+                                                        float *values, int xcd_aware) {
     extern __shared__ uint2 sorted[];   // [kBlock * d1]: weight, point | slot << 8; then the points' rows
     __shared__ int slot_index[kTileSlots];
     __shared__ unsigned slot_count[kTileSlots];
-    __shared__ unsigned short occupied[kTileSlots];
-    __shared__ unsigned n_occupied;
     __shared__ unsigned wave_pairs[kThreads / 64];
     unsigned vblock;
     if (!block_of_points(map, xcd_aware, vblock)) return;
     float *rows = reinterpret_cast<float *>(sorted + (size_t)kBlock * d1);   // [kBlock][in_channels]
     const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
     const int point = tid % kBlock, side = tid / kBlock;   // (its corners: side, side + 2, ...)
-    const size_t t = (size_t)vblock * kBlock * d1 + point;
-    constexpr size_t T = kBlock;
     const int n = point_of_thread(map, vblock, point);
     static_assert(kTileSlots == kThreads, "a slot per thread");
-    slot_index[tid] = -1;
+    const uint32_t *words = words_of_tile(replay, vblock, d1);
+    const int used = map.tile_vertices.used[vblock];
+    const int own_vertex = map.tile_vertices.of(vblock)[tid];
     slot_count[tid] = 0u;
-    if (tid == 0) n_occupied = 0u;
 
     int index[kMaxCorners];
     float weight[kMaxCorners];
 #pragma unroll
     for (int i = 0; i < (int)kMaxCorners; ++i) {
         const int r = (int)kSides * i + side;
-        const ReplayEntry e = replay[(size_t)(r < d1 ? r : 0) * T + t];
-        index[i] = r < d1 && n >= 0 ? e.index : -1;
-        weight[i] = e.weight;
+        const uint32_t place = place_of_corner(words[(r < d1 ? r / kPlacesPerWord : 0) * kBlock + point], r);
+        index[i] = r < d1 && n >= 0 && place < (uint32_t)kTileSlots ? (int)place : -1;
+        weight[i] = weights_behind(words, d1)[(r < d1 ? r : 0) * kBlock + point];
     }
     // element i of the wavefront's 64 rows belongs to point i / in_channels, channel i % in_channels
     // (eight loads asked for before the first is stored; a point without data reads point 0; the two
@@ -98,8 +91,8 @@ __global__ __launch_bounds__(kThreads) void k_splat_tile(int d1, int vd, PointMa
     }
     __syncthreads();   // the slots are empty (and the rows there)
 
-    // place[r]: the slot of corner r's vertex and, above it, the pair's rank among the slot's.  The
-    // first lane of a run of lanes with one vertex looks for the slot and counts for the run (8x8
+    // place[r]: the slot of corner r's vertex (its place in the table) and, above it, the pair's rank among
+    // the slot's.  The first lane of a run of lanes with one vertex counts for the run (8x8
     // pixels: 29 runs; LDS atomics on one address take turns).
     unsigned place[kMaxCorners];
     constexpr unsigned kNoPlace = 0xffffffffu;
@@ -111,36 +104,15 @@ __global__ __launch_bounds__(kThreads) void k_splat_tile(int d1, int vd, PointMa
         const uint64_t behind = lane == 63 ? 0ull : opening >> (lane + 1);
         const unsigned length = behind ? (unsigned)__builtin_ctzll(behind) + 1u : 64u - (unsigned)lane;
         unsigned found = kNoPlace;
-        if (opens && index[r] >= 0) {
-            unsigned slot = ((unsigned)index[r] * 0x9E3779B1u) >> kTileSlotShift;
-            for (int probe = 0; probe < kTileSlots; ++probe) {
-                int seen = *(volatile int *)&slot_index[slot];
-                if (seen < 0) {
-                    seen = atomicCAS(&slot_index[slot], -1, index[r]);
-                    if (seen < 0) {
-                        occupied[atomicAdd(&n_occupied, 1u)] = (unsigned short)slot;
-                        seen = index[r];
-                    }
-                }
-                if (seen == index[r]) {
-                    found = slot | atomicAdd(&slot_count[slot], length) << 16;
-                    break;
-                }
-                slot = (slot + 1u) & (kTileSlots - 1u);
-            }
-        }
+        if (opens && index[r] >= 0) found = (unsigned)index[r] | atomicAdd(&slot_count[index[r]], length) << 16;
         const int opener = 63 - __builtin_clzll(opening & (~0ull >> (63 - lane)));
         found = (unsigned)__shfl((int)found, opener);
         place[r] = index[r] >= 0 && found != kNoPlace ? found + ((unsigned)(lane - opener) << 16) : kNoPlace;
     }
     __syncthreads();   // the slots are counted
 
-    // the count of a slot becomes the place of its first pair, its index the vertex (a thread takes
-    // one slot in use)
-    const int own = (unsigned)tid < n_occupied ? (int)occupied[tid] : -1;
-    const unsigned own_count = own >= 0 ? slot_count[own] : 0u;
-    int own_vertex = own >= 0 ? slot_index[own] : 0;
-    if (cell_vertex && own >= 0) own_vertex = cell_vertex[own_vertex];
+    // the count of a slot becomes the place of its first pair (a thread takes one slot)
+    const unsigned own_count = slot_count[tid];
     unsigned inclusive = own_count;
 #pragma unroll
     for (int d = 1; d < 64; d <<= 1) {
@@ -155,10 +127,8 @@ __global__ __launch_bounds__(kThreads) void k_splat_tile(int d1, int vd, PointMa
         if (w < wave) before += wave_pairs[w];
         pairs += wave_pairs[w];
     }
-    if (own >= 0) {
-        slot_count[own] = before;
-        slot_index[own] = own_vertex;
-    }
+    slot_count[tid] = before;
+    slot_index[tid] = tid < used ? own_vertex : -1;
     __syncthreads();
 
 #pragma unroll
@@ -167,7 +137,6 @@ __global__ __launch_bounds__(kThreads) void k_splat_tile(int d1, int vd, PointMa
         const unsigned slot = place[r] & 0xffffu;
         sorted[slot_count[slot] + (place[r] >> 16)] =
             make_uint2(__float_as_uint(weight[r]), (unsigned)point | slot << 8);
-        if (cell_vertex) replay[(size_t)((int)kSides * r + side) * T + t].index = slot_index[slot];
     }
     __syncthreads();   // the pairs are in the order of their slots
 
@@ -181,10 +150,11 @@ __global__ __launch_bounds__(kThreads) void k_splat_tile(int d1, int vd, PointMa
 #pragma unroll
     for (int k = 0; k < K; ++k) acc[k] = 0.0f;
     auto add_row = [&](unsigned slot) {
-        float *row = values + (unsigned)slot_index[slot] * (unsigned)vd;
+        const int vertex = slot_index[slot];
+        float *row = values + (unsigned)vertex * (unsigned)vd;
 #pragma unroll
         for (int k = 0; k < K; ++k) {
-            if (c0 + 16 * k < vd) atomicAdd(row + c0 + 16 * k, acc[k]);
+            if (vertex >= 0 && c0 + 16 * k < vd) atomicAdd(row + c0 + 16 * k, acc[k]);
             acc[k] = 0.0f;
         }
     };
@@ -223,15 +193,15 @@ __global__ __launch_bounds__(kThreads) void k_splat_tile(int d1, int vd, PointMa
 }  // namespace
 
 hipError_t splat_tile(int pd, int vd, const PointMap &map, const float *input, int in_channels, ReplayEntry *replay,
-                      const int *cell_vertex, float *values, int xcd_aware, hipStream_t s) {
+                      const int *, float *values, int xcd_aware, hipStream_t s) {
     if (map.n_blocks == 0) return hipSuccess;
-    if (!splat_tile_takes(vd) || pd < 1 || pd > kMaxPd || in_channels < 1 || in_channels > vd)
+    if (!map.tile_vertices.table || !splat_tile_takes(vd) || pd < 1 || pd > kMaxPd || in_channels < 1 || in_channels > vd)
         return hipErrorInvalidValue;
     const int d1 = pd + 1;
     const size_t lds = kBlock * ((size_t)d1 * sizeof(uint2) + (size_t)in_channels * sizeof(float));
     const auto kernel = vd <= 16 ? k_splat_tile<1> : k_splat_tile<2>;
     hipLaunchKernelGGL(kernel, dim3(map.n_blocks), dim3(kThreads), lds, s, d1, vd, map, input, in_channels, replay,
-                       cell_vertex, values, xcd_aware);
+                       values, xcd_aware);
     return hipGetLastError();
 }
 

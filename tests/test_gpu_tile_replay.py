@@ -1,0 +1,125 @@
+"""What a merging build leaves of its points (places in their workgroup's table of vertices) and the passes
+that read it, against the oracle: at the edges of the channel blocks, with tiles whose vertices fit the rows
+in LDS and tiles whose do not, in floats and doubles, and where only one of two joint lattices has such
+tiles."""
+import numpy as np
+import pytest
+import torch
+
+from conftest import MAX_ABS_TOL, REL_L2_TOL, rel_l2
+from permutohedral_lattice_amd import synth
+from permutohedral_lattice_amd.crf import MeanField
+
+import oracle
+import permutohedral_lattice_amd as pla
+
+pytestmark = pytest.mark.gpu
+
+
+def dev(a):
+    return torch.from_numpy(np.ascontiguousarray(a)).cuda()
+
+
+def positions(h, w, features, noise, seed):
+    """A grid's coordinates and smooth features with `noise` of a width of noise on them."""
+    rng = np.random.default_rng(seed)
+    yx = np.stack(np.meshgrid(np.arange(h), np.arange(w), indexing="ij"), -1).reshape(-1, 2) / 6.0
+    img = synth.blob_image(h, w, seed=seed).reshape(-1, 3)
+    extra = np.concatenate((img, img[:, ::-1]), axis=1)[:, :features] / 0.2
+    extra = extra + noise * rng.uniform(-1, 1, extra.shape)
+    return np.ascontiguousarray(np.concatenate((yx, extra), axis=1), dtype=np.float32)
+
+
+def vertices_of_tiles(pos, h, w):
+    """Distinct vertices of the workgroups' 16x16 points."""
+    pd = pos.shape[1]
+    keys = oracle.dump_simplex(pos)["keys"].reshape(h, w, pd + 1, pd)
+    return [len(np.unique(keys[y:y + 16, x:x + 16].reshape(-1, pd), axis=0))
+            for y in range(0, h, 16) for x in range(0, w, 16)]
+
+
+def check(got, want):
+    got = got.cpu().numpy()
+    assert np.isfinite(got).all()
+    assert np.abs(got - want).max() <= MAX_ABS_TOL and rel_l2(got, want) <= REL_L2_TOL
+
+
+@pytest.mark.parametrize("vd", [2, 3, 4, 5, 8, 9, 22, 32, 33, 34, 64, 65, 66, 67])
+@pytest.mark.parametrize("h,w,features,noise", [(33, 47, 3, 0.0), (32, 48, 3, 1.1), (20, 30, 5, 0.5), (17, 40, 6, 0.2)])
+def test_filter_and_applies(h, w, features, noise, vd):
+    pos = positions(h, w, features, noise, 7 * h + features)
+    n, pd = pos.shape
+    val = np.random.default_rng(vd).uniform(0.1, 1, (n, vd - 1)).astype(np.float32)
+    want = {reverse: oracle.Lattice(pd, vd, n).filter(val, pos, reverse) for reverse in (False, True)}
+    lat = pla.PermutohedralLattice(pd, vd, n)
+    lat.set_point_grid((h, w))
+    out = torch.empty((n, vd - 1), device="cuda")
+    for reverse in (False, True):
+        lat.filter(out.fill_(float("nan")), dev(val), dev(pos), reverse)
+        check(out, want[reverse])
+    assert lat.info(pla.PL_INFO_BUILD_MERGED) == 1
+    for lists in (0, 1):
+        lat.set_option(pla.PL_OPT_VERTEX_LISTS, lists)
+        lat.build(dev(pos))
+        for reverse in (True, False):
+            lat.apply(out.fill_(float("nan")), dev(val), reverse)
+            check(out, want[reverse])
+    vertex, weight = lat.debug_replay()
+    keys = lat.debug_keys().cpu().numpy()[vertex.cpu().numpy()]
+    simplex = oracle.dump_simplex(pos)
+    assert (keys.transpose(1, 0, 2) == simplex["keys"]).all()
+    assert (weight.cpu().numpy().T == simplex["barycentric"]).all()
+    lat.close()
+
+
+def test_the_noise_crowds_the_tiles():
+    """The inputs above have tiles below and above the rows that fit into LDS (247 of 21 channels, 198 of 32)
+    and none that the merging build cannot take (512)."""
+    smooth = vertices_of_tiles(positions(33, 47, 3, 0.0, 7 * 33 + 3), 33, 47)
+    noisy = vertices_of_tiles(positions(32, 48, 3, 1.1, 7 * 32 + 3), 32, 48)
+    assert max(smooth) < 198 and max(noisy) > 260 and max(noisy) <= 512
+
+
+@pytest.mark.parametrize("vd", [2, 3, 4, 5, 8, 9])
+@pytest.mark.parametrize("h,w,features,noise", [(33, 47, 3, 0.0), (32, 48, 3, 1.1), (17, 40, 6, 0.2)])
+def test_doubles(h, w, features, noise, vd):
+    pos = positions(h, w, features, noise, 7 * h + features).astype(np.float64)
+    n, pd = pos.shape
+    val = np.random.default_rng(vd).uniform(0.1, 1, (n, vd - 1))
+    lat = pla.PermutohedralLattice(pd, vd, n, dtype=torch.float64)
+    lat.set_point_grid((h, w))
+    out = torch.empty((n, vd - 1), device="cuda", dtype=torch.float64)
+    for reverse in (False, True):
+        want = oracle.Lattice(pd, vd, n, dtype=np.float64).filter(val, pos, reverse)
+        lat.filter(out.fill_(float("nan")), dev(val), dev(pos), reverse)
+        assert np.abs(out.cpu().numpy() - want).max() <= 1e-12
+        lat.build(dev(pos))
+        lat.apply(out.fill_(float("nan")), dev(val), reverse)
+        assert np.abs(out.cpu().numpy() - want).max() <= 1e-12
+    lat.close()
+
+
+# (0.02: every tile's vertices fit into LDS; 25: of the two lattices 160 to 400, of one at most 350; 300: the
+# bilateral lattice is built without merging, the spatial one is not)
+@pytest.mark.parametrize("noise,merged", [(0.02, 1), (25.0, 1), (300.0, 0)])
+@pytest.mark.parametrize("classes", [4, 5, 21, 31])
+def test_joint_messages(noise, merged, classes):
+    batch, h, w = 2, 40, 56
+    rng = np.random.default_rng(classes)
+    guide = np.stack([synth.blob_image(h, w, seed=b) * 255.0 for b in range(batch)])
+    guide = (guide + noise * rng.uniform(-1, 1, guide.shape)).astype(np.float32)
+    logits = synth.normal_image((batch, h, w, classes), 10)
+    upstream = synth.normal_image((batch, h, w, classes), 11)
+    mf = MeanField(dev(guide), classes, theta_alpha=80.0, theta_beta=13.0)
+    for lat in mf.bilateral:
+        assert lat.info(pla.PL_INFO_BUILD_MERGED) == merged
+    for lat in mf.spatial:
+        assert lat.info(pla.PL_INFO_BUILD_MERGED) == 1
+    q = mf.infer(dev(logits), iterations=2).cpu().numpy()
+    rev = mf.reverse(dev(upstream)).cpu().numpy()
+    want_q, want_rev = oracle.mean_field(logits, guide, 2, upstream=upstream)
+    assert np.isfinite(q).all() and np.abs(q.sum(axis=-1) - 1.0).max() <= 1e-5
+    assert np.abs(q - want_q).max() <= MAX_ABS_TOL and rel_l2(q, want_q) <= REL_L2_TOL
+    assert np.abs(rev - want_rev).max() <= MAX_ABS_TOL * max(1.0, float(np.abs(want_rev).max()))
+    assert rel_l2(rev, want_rev) <= REL_L2_TOL
+    mf.close()
