@@ -16,7 +16,7 @@ LIB_PATH = os.path.join(_HERE, "libpermutohedral_hip.so")
 
 SOURCES = [os.path.join(_HERE, "csrc", name)
            for name in ("pl_kernels.hip", "pl_kernels_f64.hip", "pl_order.hip", "pl_gather.hip", "pl_mean_field.hip",
-                      "pl_splat_tile.hip", "pl_many.hip", "pl_api.cpp")]
+                      "pl_splat_tile.hip", "pl_many.hip", "pl_tile_lists.hip", "pl_api.cpp")]
 
 # -ffp-contract=off: the lattice's integer results need unfused IEEE float operations.
 # -munsafe-fp-atomics: float atomicAdd becomes the hardware global_atomic_add_f32.

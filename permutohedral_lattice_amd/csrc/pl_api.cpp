@@ -131,6 +131,7 @@ struct pl_lattice {
     size_t lists_for_vertices = 0;         // max_vertices the arrays were allocated for
     bool lists_valid = false;              // they describe the last build
     unsigned list_chunks = 0, long_lists = 0;   // of the last build: chunks in all, lists of several
+    size_t partial_floats = 0;             // lists_of_vertices.chunks.partial_rows has room for
 
     plk::Counters *d_counters = nullptr;   // two sets, used by alternate builds
     int counter_set = 0;                   // the set of the last build
@@ -366,6 +367,7 @@ int ensure_vertex_lists(pl_lattice *h) {
     l.chunks.max_chunks = (unsigned)max_chunks;
     l.chunks.max_long = (unsigned)max_long;
     l.chunks.rows = plk::list_chunk_rows(h->vd);
+    h->partial_floats = max_chunks * (size_t)h->vd;
     h->lists_for_vertices = mv;
     l.capacity = h->replay_capacity;
     return PL_OK;
@@ -1214,6 +1216,9 @@ int enqueue_build_only(pl_lattice *h, const plk::PointFeatures &features, const 
         // vertices densely).  Enqueued before the host waits for the build's report.
         rc = ensure_vertex_lists(h);
         if (rc != PL_OK) return rc;
+        h->lists_of_vertices.map = h->map;
+        if (!plk::lists_of_tiles(h->vd, h->N)) h->lists_of_vertices.map.tile_vertices = plk::TileVertices{};
+        h->lists_of_vertices.pd = h->pd;
         PL_HIP(plk::build_vertex_lists(h->pd, h->map, h->replay,
                                        h->replay_holds_cells ? h->cell_vertex : nullptr,
                                        h->max_vertices(), h->lists_of_vertices,
@@ -1267,8 +1272,27 @@ int build_end(pl_lattice *h) {
         const volatile unsigned *info = reinterpret_cast<const volatile unsigned *>(h->h_status + 1);
         const int rc = wait_for_report(h, info + 2);
         if (rc != PL_OK) return rc;
-        const plk::ListChunks &c = h->lists_of_vertices.chunks;
-        h->long_lists = info[0] < c.max_long ? info[0] : c.max_long;
+        plk::ListChunks &c = h->lists_of_vertices.chunks;
+        if (h->lists_of_vertices.map.tile_vertices.table) {
+            // (of a merging build: the rows of sums an apply makes.  More than there is room for only
+            // where workgroups share their vertices with several others each.)
+            const size_t floats = (size_t)info[0] * plk::tile_row_floats(h->vd);
+            if (floats > h->partial_floats) {
+                const hipError_t waited = hipStreamSynchronize(h->stream);
+                h->dfree(c.partial_rows);
+                h->partial_floats = 0;
+                if (!hip_failed(waited)) c.partial_rows = (float *)h->dmalloc(sizeof(float) * (floats + floats / 8));
+                if (!c.partial_rows) {
+                    h->dfree(h->lists_of_vertices.start);   // (the next build allocates the lists anew)
+                    h->built = false;
+                    return hip_failed(waited) ? PL_EHIP : PL_ENOMEM;
+                }
+                h->partial_floats = floats + floats / 8;
+            }
+            h->long_lists = 0;
+        } else {
+            h->long_lists = info[0] < c.max_long ? info[0] : c.max_long;
+        }
         h->list_chunks = info[1] < c.max_chunks ? info[1] : c.max_chunks;
         h->lists_valid = true;
     }
@@ -1505,7 +1529,7 @@ int pl_get_info(pl_handle h, int what, long *value) {
                 b += sizeof(unsigned) * (3 * h->lists_for_vertices + 5 +
                                          2 * (plk::vertex_list_scan_blocks((int)h->lists_for_vertices) + 1)) +
                      sizeof(plk::LongList) * h->lists_of_vertices.chunks.max_long +
-                     (size_t)h->lists_of_vertices.chunks.max_chunks * (sizeof(plk::ListChunk) + sizeof(float) * h->vd) +
+                     (size_t)h->lists_of_vertices.chunks.max_chunks * sizeof(plk::ListChunk) + h->partial_floats * sizeof(float) +
                      h->lists_of_vertices.capacity * (sizeof(plk::ListEntry) + sizeof(unsigned));
             if (h->point_order) {
                 const unsigned max_bins = plk::locality_bins_for(h->order_capacity);
@@ -1751,7 +1775,7 @@ int enqueue_pairs(int n, const pl_handle *bilateral, const pl_handle *spatial, f
             pl_lattice *h = lattice[i] = i < pairs ? bilateral[first + i] : spatial[first + i - pairs];
             const plk::VertexLists &l = h->lists_of_vertices;
             gather[i] = plk::GatherWork{l.chunks, l.entries, input + (size_t)(first + i % pairs) * item, h->values[0],
-                                        h->list_chunks, h->long_lists};
+                                        h->list_chunks, h->long_lists, &l};
             h->values_zeroed = false;
             h->current_values = 0;
         }

@@ -187,7 +187,8 @@ __global__ __launch_bounds__(kBlock) void k_scan_block_sums(const unsigned *__re
 // zero, as the next build's k_list_places must find them.
 __global__ __launch_bounds__(kBlock) void k_scan_starts(unsigned *count, unsigned n,
                                                          const uint2 *__restrict__ block_sums,
-                                                         unsigned *start, ListChunks chunks) {
+                                                         unsigned *start, ListChunks chunks, unsigned *host_info,
+                                                         unsigned sequence) {
     const size_t first = (size_t)blockIdx.x * kScanItems + (size_t)threadIdx.x * kScanPerThread;
     unsigned c[kScanPerThread];
     load_counts(count, first, n, c);
@@ -245,6 +246,13 @@ __global__ __launch_bounds__(kBlock) void k_scan_starts(unsigned *count, unsigne
         start[n] = all.x;
         chunks.chunk_start[n] = all.y;
         chunks.info[1] = all.y < chunks.max_chunks ? all.y : chunks.max_chunks;
+        // (lists of a merging build; see k_list_fill)
+        if (host_info) {
+            host_info[0] = all.x;
+            host_info[1] = all.y;
+            __threadfence_system();
+            __hip_atomic_store(&host_info[2], sequence, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM);
+        }
     }
 }
 
@@ -536,6 +544,20 @@ hipError_t build_vertex_lists(int pd, const PointMap &map, ReplayEntry *replay, 
     if (max_vertices <= 0 || map.n_blocks == 0) return hipSuccess;
     // (lists.count is all zeros: filled so when it was allocated, left so by every k_scan_starts)
     const dim3 block(kBlock), grid(map.n_blocks);
+    if (lists.map.tile_vertices.table) {
+        // (one chunk a vertex, however many rows)
+        ListChunks chunks = lists.chunks;
+        chunks.rows = 1u << 30;
+        const hipError_t e = sort_tiles(pd, map, replay, max_vertices, lists, s);
+        if (e != hipSuccess) return e;
+        const unsigned n = (unsigned)max_vertices, scan_blocks = (unsigned)vertex_list_scan_blocks(max_vertices);
+        uint2 *block_sums = reinterpret_cast<uint2 *>(lists.block_sums);
+        hipLaunchKernelGGL(k_scan_block_sums, dim3(scan_blocks), block, 0, s, lists.count, n, block_sums, chunks.info,
+                           chunks.rows);
+        hipLaunchKernelGGL(k_scan_starts, dim3(scan_blocks), block, 0, s, lists.count, n, block_sums, lists.start, chunks,
+                           host_info, sequence);
+        return place_rows(map, lists, s);
+    }
     PLK_DISPATCH_PD(pd, hipLaunchKernelGGL((k_list_places<PD + 1>), grid, block, 0, s, map, replay,
                                            cell_vertex, lists.count, lists.places, max_vertices));
     const unsigned n = (unsigned)max_vertices;
@@ -544,7 +566,7 @@ hipError_t build_vertex_lists(int pd, const PointMap &map, ReplayEntry *replay, 
     hipLaunchKernelGGL(k_scan_block_sums, dim3(scan_blocks), block, 0, s, lists.count, n, block_sums,
                        lists.chunks.info, lists.chunks.rows);
     hipLaunchKernelGGL(k_scan_starts, dim3(scan_blocks), block, 0, s, lists.count, n, block_sums,
-                       lists.start, lists.chunks);
+                       lists.start, lists.chunks, (unsigned *)nullptr, 0u);
     PLK_DISPATCH_PD(pd, hipLaunchKernelGGL((k_list_fill<PD + 1>), grid, block, 0, s, map, replay,
                                            lists.places, lists.start, lists.entries, max_vertices,
                                            lists.capacity, lists.chunks, host_info, sequence));
@@ -584,13 +606,30 @@ static hipError_t splat_gather_channels(int vd, int in_channels, int n, const Ga
 
 hipError_t splat_gather_many(int vd, int in_channels, int n, const GatherWork *work, hipStream_t s) {
     if (n < 1 || n > kManyItems || vd < kManyChannels) return hipErrorInvalidValue;
-    return splat_gather_channels<kManyItems>(vd, in_channels, n, work, s);
+    GatherWork rows[kManyItems];   // the lattices whose builds did not merge
+    int n_rows = 0;
+    bool pairs = n % 2 == 0 && splat_tile_pairs_take(work[0].lists->pd, work[n / 2].lists->pd, vd);
+    for (int i = 0; i < n; ++i) {
+        if (!work[i].lists->map.tile_vertices.table) rows[n_rows++] = work[i];
+        if (i < n / 2)
+            pairs = pairs && work[i].input == work[n / 2 + i].input && work[i].lists->pd == work[0].lists->pd &&
+                    work[n / 2 + i].lists->pd == work[n / 2].lists->pd;
+    }
+    if (n_rows == 0 && pairs) return splat_tile_pairs(vd, in_channels, n, work, s);
+    for (int i = 0; i < n; ++i) {
+        if (!work[i].lists->map.tile_vertices.table) continue;
+        const hipError_t e = splat_tile_lists(vd, *work[i].lists, work[i].n_chunks, work[i].input, in_channels,
+                                              work[i].values, s);
+        if (e != hipSuccess) return e;
+    }
+    return n_rows ? splat_gather_channels<kManyItems>(vd, in_channels, n_rows, rows, s) : hipSuccess;
 }
 
 hipError_t splat_gather(int vd, const VertexLists &lists, unsigned n_chunks, unsigned n_long,
                         const float *input, int in_channels, float *values, hipStream_t s) {
     if (n_chunks == 0) return hipSuccess;
-    const GatherWork work{lists.chunks, lists.entries, input, values, n_chunks, n_long};
+    if (lists.map.tile_vertices.table) return splat_tile_lists(vd, lists, n_chunks, input, in_channels, values, s);
+    const GatherWork work{lists.chunks, lists.entries, input, values, n_chunks, n_long, &lists};
     const dim3 block(kBlock);
 #define PLK_GATHER(VD)                                                                               \
     case VD:                                                                                        \

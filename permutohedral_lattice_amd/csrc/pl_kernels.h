@@ -416,6 +416,12 @@ struct VertexLists {
     unsigned *block_sums;  // [2 * (vertex_list_scan_blocks(max_vertices) + 1)] scratch, 8-byte aligned
     size_t capacity;
     ListChunks chunks;
+    // Of which build.  After a merging one, where lists_of_tiles (map.tile_vertices), the lists are of the rows of sums that its
+    // workgroups make, one per vertex of a workgroup's table (pl_tile_lists.hip): start and chunk (a chunk a
+    // vertex) count those rows, partial_rows holds them in this order; entries are the workgroups' corners
+    // in the order of their places, and places the rows [workgroup * kTileSlots + place].
+    PointMap map;
+    int pd;
 };
 size_t vertex_list_scan_blocks(int max_vertices);
 size_t vertex_list_max_chunks(int max_vertices, size_t rows);
@@ -423,7 +429,9 @@ size_t vertex_list_max_long(size_t rows);
 // cell_vertex != nullptr: the replay rows still hold hash cells; they are translated and written
 // back.  When the stream has run this, lists.chunks.info holds the numbers splat_gather wants,
 // and so do the first two of the three words at host_info (pinned memory the host reads); the
-// third is `sequence`, written last by the pass's last launch as that launch starts.
+// third is `sequence`, written last by the pass's last launch as that launch starts.  (Lists of a merging
+// build: info[0] is the number of rows, which chunks.partial_rows must have room for in an apply,
+// tile_row_floats(vd) each.)
 hipError_t build_vertex_lists(int pd, const PointMap &map, ReplayEntry *replay, const int *cell_vertex,
                               int max_vertices, const VertexLists &lists, unsigned *host_info,
                               unsigned sequence, hipStream_t s);
@@ -441,7 +449,25 @@ struct GatherWork {
     const float *input;
     float *values;
     unsigned n_chunks, n_long;
+    const VertexLists *lists;
 };
+// Which lattices whose build merged get lists of its workgroups' rows of sums, not of its points' corners.  Up
+// to four channels an apply takes a launch more for them, and where the launches count that is what it
+// takes longer; us an apply, lists of corners and of rows, pd 5, vd 4: 256x256 points 18.4 and 21.5, 512x512
+// 24.2 and 25.8, 700x700 32.4 and 32.4, 1024x1024 49.0 and 44.9 (under noise 62.0 and 54.8).  With more channels
+// rows are ahead at every size: vd 22 64x64 26.5 and 25.2, 512x512 62.2 and 48.0; vd 9 47.4 and 34.8; vd 40
+// 95.2 and 88.9.
+inline bool lists_of_tiles(int vd, int N) { return vd > 4 || N >= (1 << 19); }
+// The lists of a merging build (pl_tile_lists.hip).  Floats from one of their rows of sums to the next:
+constexpr int tile_row_floats(int vd) { return vd <= 4 ? vd : (vd + 7) / 8 * 8; }
+hipError_t sort_tiles(int pd, const PointMap &map, const ReplayEntry *replay, int max_vertices, const VertexLists &lists,
+                      hipStream_t s);
+hipError_t place_rows(const PointMap &map, const VertexLists &lists, hipStream_t s);
+hipError_t splat_tile_lists(int vd, const VertexLists &lists, unsigned n_vertices, const float *input, int in_channels,
+                            float *values, hipStream_t s);
+// n / 2 pairs of lattices over the same points and input, the first of all pairs first.
+bool splat_tile_pairs_take(int pd_a, int pd_b, int vd);
+hipError_t splat_tile_pairs(int vd, int in_channels, int n, const GatherWork *work, hipStream_t s);
 hipError_t splat_gather_many(int vd, int in_channels, int n, const GatherWork *work, hipStream_t s);
 // Stage 4 of several lattices: one axis each, or two (nbr_second), in one launch.
 struct BlurWork {

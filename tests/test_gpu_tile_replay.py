@@ -123,3 +123,49 @@ def test_joint_messages(noise, merged, classes):
     assert np.abs(rev - want_rev).max() <= MAX_ABS_TOL * max(1.0, float(np.abs(want_rev).max()))
     assert rel_l2(rev, want_rev) <= REL_L2_TOL
     mf.close()
+
+
+# Up to four channels a workgroup's rows of sums are listed from 2^19 points on.  flat: most of a tile's corners
+# name a few vertices (runs over several wavefronts); wild: values that sums of products by 0 and 1 cannot take.
+@pytest.mark.parametrize("vd", [2, 3, 4])
+@pytest.mark.parametrize("kind", ["image", "flat", "coordinates", "list", "wild"])
+def test_rows_of_few_channels(kind, vd):
+    gen = torch.Generator(device="cuda").manual_seed(vd)
+    h, w = 725, 724
+    n = h * w
+    assert n >= 1 << 19
+    y, x = torch.meshgrid(torch.arange(h, device="cuda"), torch.arange(w, device="cuda"), indexing="ij")
+    guide = torch.stack([torch.sin(x / 50.0), torch.cos(y / 40.0), torch.sin((x + y) / 70.0)], -1)
+    guide = guide + 0.1 * torch.rand(guide.shape, generator=gen, device="cuda")
+    if kind == "flat":
+        pos = pla.compute_positions((0.01 * guide).contiguous(), (h, w), 40.0, 1.0)
+    elif kind == "coordinates":
+        pos = pla.compute_positions(None, (h, w), 8.0)
+    else:
+        pos = pla.compute_positions(guide.contiguous(), (h, w), 8.0, 0.5)
+    if kind == "list":
+        pos = pos[:, :3][torch.randperm(n, generator=gen, device="cuda")].contiguous()
+    for normalize in (1, 0):
+        channels = vd - 1 if normalize else vd
+        val = torch.rand((n, channels), generator=gen, device="cuda") + 0.1
+        if kind == "wild":
+            val[::1000] *= 1e31
+        lat = pla.PermutohedralLattice(pos.shape[1], vd, n)
+        if kind != "list":
+            lat.set_point_grid((h, w))
+        lat.set_option(pla.PL_OPT_NORMALIZE, normalize)
+        filtered, applied = torch.empty_like(val), torch.empty_like(val)
+        want = {reverse: lat.filter(filtered, val, pos, reverse).clone() for reverse in (False, True)}
+        lat.build(pos)
+        assert lat.info(pla.PL_INFO_BUILD_MERGED) == 1
+        for reverse in (False, True):
+            lat.apply(applied.fill_(float("nan")), val, reverse)
+            # (the same terms in another order: sums of some 10^4 positive floats, 2^-24 an addition on
+            # either side and far less on average)
+            assert torch.isfinite(applied).all()
+            assert float(((applied - want[reverse]).abs() / want[reverse].abs()).max()) <= 1e-4
+            assert float((applied - want[reverse]).double().norm() / want[reverse].double().norm()) <= 2e-6
+            first = applied.clone()
+            lat.apply(applied, val, reverse)
+            assert (applied == first).all()     # (one order on every call)
+        lat.close()
