@@ -266,6 +266,20 @@ int pl_build_image(pl_handle h, const float *reference, int n_reference_channels
                    float feature_std);
 
 /*
+ * pl_filter_image for n images of one shape, each on a lattice of its own: output, input and reference
+ * hold the images' arrays one behind the other (reference: [n][N][n_reference_channels]).  Lattices of
+ * the same pd, vd and N and of floats, no one twice (PL_EINVAL).  Where all of them work on one stream their
+ * passes are enqueued together, one launch for all lattices; where that cannot be, one lattice after the other.
+ * The same results either way.
+ * pl_apply_many: pl_apply for n such lattices; like pl_apply it only launches kernels on the lattices' streams.
+ * Stand in for the op's loop over the batch (src/LatticeFilterKernel.cpp:152-179) and the gradient's.
+ */
+int pl_filter_images(int n, const pl_handle *lattices, float *output, const float *input, const float *reference,
+                     int n_reference_channels, int n_spatial_dims, const int *spatial_dims, float spatial_std,
+                     float feature_std, int reverse);
+int pl_apply_many(int n, const pl_handle *lattices, float *output, const float *input, int reverse);
+
+/*
  * pl_filter / pl_filter_image in two halves, for callers that keep several lattices (each on a
  * stream of its own) in flight: *_begin enqueues the whole call on the lattice's stream and
  * returns at once; pl_filter_end waits for the build's report and, should the hash table have

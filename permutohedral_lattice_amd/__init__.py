@@ -42,7 +42,7 @@ REPLAY_ROW_BYTES = 8
 EXPORTS = (
     "pl_supported", "pl_strerror", "pl_last_hip_error", "pl_library_info", "pl_create", "pl_destroy", "pl_filter",
     "pl_filter_static", "pl_build", "pl_apply", "pl_set_point_grid", "pl_get_point_grid", "pl_num_vertices", "pl_set_option", "pl_get_info", "pl_stage_ms", "pl_debug_simplex",
-    "pl_debug_keys", "pl_debug_values", "pl_debug_replay", "pl_compute_positions", "pl_filter_image", "pl_build_image",
+    "pl_debug_keys", "pl_debug_values", "pl_debug_replay", "pl_compute_positions", "pl_filter_image", "pl_build_image", "pl_filter_images", "pl_apply_many",
     "pl_filter_begin", "pl_filter_image_begin", "pl_filter_end",
     "pl_build_begin", "pl_build_image_begin", "pl_build_end", "pl_lattice_filter_op",
     "pl_set_op_concurrency", "pl_mean_field_update", "pl_mean_field_messages", "pl_mean_field_infer",
@@ -107,6 +107,8 @@ def _load(path=LIB_PATH):
     lib.pl_debug_replay.argtypes = [vp, vp, vp]
     lib.pl_compute_positions.argtypes = [vp, vp, ci, ci, ci, C.POINTER(ci), cf, cf, vp]
     lib.pl_filter_image.argtypes = [vp, vp, vp, vp, ci, ci, C.POINTER(ci), cf, cf, ci]
+    lib.pl_filter_images.argtypes = [ci, C.POINTER(vp), vp, vp, vp, ci, ci, C.POINTER(ci), cf, cf, ci]
+    lib.pl_apply_many.argtypes = [ci, C.POINTER(vp), vp, vp, ci]
     lib.pl_build_image.argtypes = [vp, vp, ci, ci, C.POINTER(ci), cf, cf]
     lib.pl_filter_begin.argtypes = [vp, vp, vp, vp, ci]
     lib.pl_filter_image_begin.argtypes = [vp, vp, vp, vp, ci, ci, C.POINTER(ci), cf, cf, ci]
@@ -484,6 +486,33 @@ def _lattice_filter_raw(input_image, reference_image, bilateral, theta_alpha, th
     return out
 
 
+def _handles(lattices):
+    return (C.c_void_p * len(lattices))(*(lat._h for lat in lattices))
+
+
+def _filter_images(lattices, output, input, reference, spatial_dims, spatial_std, feature_std, reverse):
+    """``filter_image`` of every item of a batch on a lattice of its own, the lattices' passes together."""
+    lat = lattices[0]
+    if len(lattices) == 1:      # (the same call, a launch's arguments less)
+        shape = (lat.N, lat.vd - 1)
+        lat.filter_image(output.view(shape), input.view(shape), None if reference is None else reference[0],
+                         spatial_dims, spatial_std, feature_std, reverse)
+        return
+    n = len(lattices) * lat.N
+    rc = lat.pd - len(spatial_dims)
+    dims = (C.c_int * len(spatial_dims))(*spatial_dims)
+    _check(_lib.pl_filter_images(len(lattices), _handles(lattices), _dev_f32(output, "output", n * (lat.vd - 1)),
+                                 _dev_f32(input, "input", n * (lat.vd - 1)),
+                                 _dev_f32(reference, "reference", n * rc) if rc else None, rc, len(spatial_dims), dims,
+                                 float(spatial_std), float(feature_std), int(bool(reverse))), "pl_filter_images")
+
+
+def _apply_many(lattices, output, input, reverse):
+    n = len(lattices) * lattices[0].N * (lattices[0].vd - 1)
+    _check(_lib.pl_apply_many(len(lattices), _handles(lattices), _dev_f32(output, "output", n),
+                              _dev_f32(input, "input", n), int(bool(reverse))), "pl_apply_many")
+
+
 class _LatticePool:
     """Lattices kept between calls, so that the forward and the backward pass of one op call can
     share what the forward pass built: the positions are the same, only the blur order differs
@@ -572,10 +601,7 @@ class _LatticeFilterFunction(torch.autograd.Function):
         ref = reference_image.contiguous() if rc else None
         out = torch.empty_like(inp)
         spatial_std = theta_alpha if bilateral else theta_gamma
-        for b, lat in enumerate(lent.lattices):
-            lat.filter_image(out[b].view(n, vd - 1), inp[b].view(n, vd - 1),
-                             ref[b].view(n, rc) if rc else None, sd, spatial_std,
-                             theta_beta if bilateral else 1.0, reverse)
+        _filter_images(lent.lattices, out, inp, ref, sd, spatial_std, theta_beta if bilateral else 1.0, reverse)
         ctx.lent = lent
         return out
 
@@ -590,8 +616,7 @@ class _LatticeFilterFunction(torch.autograd.Function):
                 lent.key[-1] == torch.cuda.current_stream().cuda_stream:
             g = grad.contiguous()
             grad_vals = torch.empty_like(g)
-            for b, lat in enumerate(lent.lattices):
-                lat.apply(grad_vals[b].view(lat.N, lat.vd - 1), g[b].view(lat.N, lat.vd - 1), True)
+            _apply_many(lent.lattices, grad_vals, g, True)
         else:
             grad_vals = _lattice_filter_raw(grad, reference_image, bilateral, theta_alpha,
                                             theta_beta, theta_gamma, True)

@@ -443,12 +443,27 @@ bool is_captured(hipStream_t stream) {
     return true;
 }
 
-// Enqueue one build with a table of `cells` cells.  Nothing here waits for the device.
+// A build about to be enqueued: what its kernels are given
+struct BuildPlan {
+    plk::PointFeatures features;
+    const double *positions64;
+    uint32_t cells;
+    const void *splat_input;
+    bool wide, merge, fused, numbers_in_build;
+    int previous_set;
+    plk::HostReport report_to;
+    plk::VertexTables vertices;
+    plk::CreatedLists lists;
+    plk::InBuildNumbering numbering;
+    plk::RegionSource regions;
+};
+
+// Makes the lattice's arrays ready for a build with a table of `cells` cells.  Nothing here waits for the device.
 // splat_input != nullptr: the build kernel also splats these values (when it can for this vd),
 // and the value table holds them when the build is done.
 // A lattice for double values takes its positions from positions64 and never splats in the build.
-int enqueue_build(pl_lattice *h, const plk::PointFeatures &features, const double *positions64,
-                  uint32_t cells, const void *splat_input) {
+int prepare_build(pl_lattice *h, const plk::PointFeatures &features, const double *positions64,
+                  uint32_t cells, const void *splat_input, BuildPlan *plan) {
     // keys of two words while a build that needed them is recent (the plain build only)
     const bool wide = h->wide_for > 0;
     h->own_stream_used = true;
@@ -540,6 +555,8 @@ int enqueue_build(pl_lattice *h, const plk::PointFeatures &features, const doubl
         !numbers_in_build ? 0 : (h->one_segment_for > 0 ? 1 : plk::segments_for((uint32_t)h->max_vertices(),
                                                                               h->forced_segments == 64 ? 1u << 20 : h->forced_segments == 8 ? 1u : h->working_blocks()))};
     if (numbers_in_build && h->one_segment_for > 0) h->one_segment_for -= 1;
+    // (from here on the lattice's arrays are those of a build that has not run)
+    h->built = false;
     // keys go to the part of the table that belongs to their band of rows when the points are
     // known to be a grid (and feature 0 then runs with its slowest extent)
     plk::RegionSource regions{};
@@ -564,51 +581,71 @@ int enqueue_build(pl_lattice *h, const plk::PointFeatures &features, const doubl
         regions.last = (float)((double)((h->map.mode == 3 ? h->map.dims[0] : h->image64.n_spatial_dims == 3 ? 1 : h->map.dims[1]) - 1) /
                                h->image64.spatial_std);
     }
+    *plan = BuildPlan{features, positions64, cells, splat_input, wide, merge, fused, numbers_in_build, previous_set,
+                      report_to, vertices, lists, numbering, regions};
+    return PL_OK;
+}
+
+// What is known of the lattice when its build's kernels are enqueued
+void build_enqueued(pl_lattice *h, const BuildPlan &plan) {
+    h->replay_holds_cells = !plan.merge;
+    h->values_zeroed = !plan.fused;
+    h->values_splatted = plan.fused;
+    h->built = true;
+    h->verified = false;
+    h->lists_valid = false;
+}
+
+int launch_build(pl_lattice *h, const BuildPlan &plan) {
+    const bool fused = plan.fused;
     if (h->f64) {
         plk::Points64 points = h->image64;
-        points.positions = positions64;
+        points.positions = plan.positions64;
         points.weights = h->weights64;
         points.scale = h->scale64;
-        PL_HIP(plk::build_f64(h->pd, points, h->map, h->cell_keys, cells, h->counters(), h->replay,
-                              h->xcd_aware ? 1 : 0, lists, regions, merge ? &numbering : nullptr,
+        PL_HIP(plk::build_f64(h->pd, points, h->map, h->cell_keys, plan.cells, h->counters(), h->replay,
+                              h->xcd_aware ? 1 : 0, plan.lists, plan.regions, plan.merge ? &plan.numbering : nullptr,
                               fused ? h->vd : 0,
-                              static_cast<const double *>(splat_input),
+                              static_cast<const double *>(plan.splat_input),
                               h->normalize ? h->vd - 1 : h->vd,
-                              reinterpret_cast<double *>(h->cell_values), wide, h->stream));
+                              reinterpret_cast<double *>(h->cell_values), plan.wide, h->stream));
     } else {
-        PL_HIP(plk::build(h->pd, features, h->map, h->scale, h->cell_keys, cells, h->counters(),
+        PL_HIP(plk::build(h->pd, plan.features, h->map, h->scale, h->cell_keys, plan.cells, h->counters(),
                           h->replay, h->xcd_aware ? 1 : 0, fused ? h->vd : 0,
-                          static_cast<const float *>(splat_input),
-                          h->normalize ? h->vd - 1 : h->vd, h->cell_values, lists,
-                          regions, merge ? &numbering : nullptr, wide, h->stream));
+                          static_cast<const float *>(plan.splat_input),
+                          h->normalize ? h->vd - 1 : h->vd, h->cell_values, plan.lists,
+                          plan.regions, plan.merge ? &plan.numbering : nullptr, plan.wide, h->stream));
     }
     h->mark(EV_BUILD);
-    if (!numbers_in_build) {
+    if (!plan.numbers_in_build) {
         // the numbering pass zeroes the vertices' value rows: a row of vd doubles is 2*vd zero floats
-        PL_HIP(plk::number_vertices(h->pd, h->map, lists,
-                                    h->chunk_count + (size_t)previous_set * h->n_chunks,
-                                    (unsigned)h->n_chunks, vertices,
+        PL_HIP(plk::number_vertices(h->pd, h->map, plan.lists,
+                                    h->chunk_count + (size_t)plan.previous_set * h->n_chunks,
+                                    (unsigned)h->n_chunks, plan.vertices,
                                     h->values[0], h->f64 ? 2 * h->vd : h->vd,
                                     fused ? h->cell_values : nullptr, h->counters(),
-                                    h->d_counters + previous_set, report_to, wide, h->stream));
+                                    h->d_counters + plan.previous_set, plan.report_to, plan.wide, h->stream));
     }
     h->mark(EV_IDS);
     // (the vertices that a merging build's workgroups did not number get their numbers in the workgroups'
     // tables here; the rows a build that numbered its vertices listed for them join the value
     // table, and its counts reach the host from here)
-    PL_HIP(plk::neighbours(h->pd, vertices, h->counters(), h->cell_keys, cells,
-                           h->launch_vertices(), merge ? &lists : nullptr,
+    PL_HIP(plk::neighbours(h->pd, plan.vertices, h->counters(), h->cell_keys, plan.cells,
+                           h->launch_vertices(), plan.merge ? &plan.lists : nullptr,
                            h->map.n_blocks, h->values[0], h->vd, h->f64,
-                           numbers_in_build ? h->counters() : nullptr,
-                           h->d_counters + previous_set, report_to, wide, h->stream));
+                           plan.numbers_in_build ? h->counters() : nullptr,
+                           h->d_counters + plan.previous_set, plan.report_to, plan.wide, h->stream));
     h->mark(EV_NBR);
-    h->replay_holds_cells = !merge;
-    h->values_zeroed = !fused;
-    h->values_splatted = fused;
-    h->built = true;
-    h->verified = false;
-    h->lists_valid = false;
+    build_enqueued(h, plan);
     return PL_OK;
+}
+
+// Enqueue one build (prepare_build).
+int enqueue_build(pl_lattice *h, const plk::PointFeatures &features, const double *positions64,
+                  uint32_t cells, const void *splat_input) {
+    BuildPlan plan;
+    const int rc = prepare_build(h, features, positions64, cells, splat_input, &plan);
+    return rc == PL_OK ? launch_build(h, plan) : rc;
 }
 
 // The value passes for a lattice of doubles: plain splat, one blur launch per axis, slice.
@@ -1363,6 +1400,233 @@ int filter_lattice(pl_lattice *h, void *output, const void *input,
 }
 
 }  // namespace
+
+// ------------------------------------------------------------------------------------------------
+// Several lattices of floats of one shape on one stream: the passes of all in one launch each.
+// ------------------------------------------------------------------------------------------------
+namespace {
+
+// Whether these lattices' passes can be enqueued together (else one lattice after the other)
+bool can_join(int n, const pl_handle *lattices) {
+    const pl_lattice *first = lattices[0];
+    if (n < 2 || !plk::joint_takes(first->pd, first->vd) || first->profile || first->stop_after != 0 || !first->pair_blur)
+        return false;
+    for (int i = 1; i < n; ++i) {
+        const pl_lattice *h = lattices[i];
+        if (h->pd != first->pd || h->vd != first->vd || h->N != first->N || h->stream != first->stream ||
+            h->device != first->device || h->normalize != first->normalize || h->xcd_aware != first->xcd_aware ||
+            h->profile || h->stop_after != 0 || !h->pair_blur)
+            return false;
+    }
+    return true;
+}
+
+int enqueue_joint_apply(int n, pl_lattice *const *lattice, float *const *output, const float *const *input, int reverse) {
+    const pl_lattice *first = lattice[0];
+    const int pd = first->pd, vd = first->vd;
+    const hipStream_t stream = first->stream;
+    plk::PointsWork points[plk::kJointItems];
+    for (int i = 0; i < n; ++i) {
+        pl_lattice *h = lattice[i];
+        h->own_stream_used = true;
+        if (vd >= plk::kManyChannels && !h->captured) h->captured = is_captured(stream);
+        points[i] = plk::PointsWork{h->map, h->replay, input[i], h->values[0], output[i]};
+    }
+    if (!first->values_splatted) {
+        static_assert(plk::kJointItems <= plk::kFillRanges, "a range a lattice");
+        plk::FillRanges fill{};
+        for (int i = 0; i < n; ++i) {
+            pl_lattice *h = lattice[i];
+            const size_t filled = h->verified && h->n_segments == 0 ? (size_t)h->M : (size_t)h->max_vertices();
+            if (h->values_zeroed) continue;
+            // (a caller's allocator may align to less than the ranges want)
+            if (reinterpret_cast<uintptr_t>(h->values[0]) % 16u == 0u)
+                fill.range[i] = {reinterpret_cast<uint32_t *>(h->values[0]), filled * vd, 0u, 0u};
+            else
+                PL_HIP(plk::fill_zero(h->values[0], filled * vd, stream));
+        }
+        PL_HIP(plk::fill_ranges(fill, stream));
+        PL_HIP(plk::splat_joint(pd, vd, n, points, first->normalize ? vd - 1 : vd, first->xcd_aware ? 1 : 0, stream));
+    }
+    for (int i = 0; i < n; ++i) {
+        lattice[i]->values_zeroed = lattice[i]->values_splatted = false;
+        lattice[i]->current_values = 0;
+    }
+    for (int step = 0; step <= pd;) {
+        // (as many axes a launch as enqueue_apply takes)
+        const int left = pd + 1 - step;
+        const int axes = plk::blur_can_take_three_axes(vd) && left == 3 && step == 0 ? 3 : left >= 2 ? 2 : 1;
+        const int axis = reverse ? pd - step : step, d = reverse ? -1 : 1;
+        plk::BlurWork blur[plk::kJointItems];
+        for (int i = 0; i < n; ++i) {
+            pl_lattice *h = lattice[i];
+            const int mv = h->max_vertices(), cur = h->current_values;
+            const bool reset = !h->table_clean && step == 0 && !h->wide_keys;
+            blur[i] = plk::BlurWork{h->counters(), h->values[cur], h->values[1 - cur],
+                                    h->neighbours + (size_t)axis * mv,
+                                    axes >= 2 ? h->neighbours + (size_t)(axis + d) * mv : nullptr,
+                                    reset ? h->cell_keys : nullptr, h->vertex_cell, mv, h->launch_vertices(),
+                                    axes == 3 ? h->neighbours + (size_t)(axis + 2 * d) * mv : nullptr};
+        }
+        PL_HIP(plk::blur_joint(vd, n, blur, stream));
+        for (int i = 0; i < n; ++i) {
+            if (blur[i].reset_cell_keys) lattice[i]->table_clean = true;
+            lattice[i]->current_values = 1 - lattice[i]->current_values;
+        }
+        step += axes;
+    }
+    for (int i = 0; i < n; ++i) points[i].values = lattice[i]->values[lattice[i]->current_values];
+    PL_HIP(plk::slice_joint(pd, vd, n, points, first->normalize ? 1 : 0, stream));
+    return PL_OK;
+}
+
+// The builds and applies of lattices that can_join (their features made from images), enqueued.
+int enqueue_joint_filter(int n, pl_lattice *const *lattice, const plk::PointFeatures *features, float *const *output,
+                         const float *const *input, int reverse) {
+    BuildPlan plan[plk::kJointItems];
+    bool together = true;
+    for (int i = 0; i < n; ++i) {
+        const int rc = prepare_build(lattice[i], features[i], nullptr, initial_cells(lattice[i]), input[i], &plan[i]);
+        if (rc != PL_OK) return rc;
+        together = together && plan[i].merge && plan[i].fused == plan[0].fused && lattice[i]->map.mode >= 2;
+    }
+    if (!together) {
+        for (int i = 0; i < n; ++i) {
+            int rc = launch_build(lattice[i], plan[i]);
+            if (rc == PL_OK) rc = enqueue_apply(lattice[i], output[i], input[i], reverse);
+            if (rc != PL_OK) return rc;
+        }
+        return PL_OK;
+    }
+    const pl_lattice *first = lattice[0];
+    const hipStream_t stream = first->stream;
+    plk::BuildWork work[plk::kJointItems], to_number[plk::kJointItems];
+    int n_to_number = 0;
+    for (int i = 0; i < n; ++i) {
+        pl_lattice *h = lattice[i];
+        const BuildPlan &p = plan[i];
+        work[i] = plk::BuildWork{p.features, h->map, h->cell_keys, p.cells - 1u, h->counters(),
+                                 h->d_counters + p.previous_set, h->replay, p.fused ? input[i] : nullptr,
+                                 p.fused ? h->cell_values : nullptr, p.lists, p.regions, p.numbering,
+                                 h->chunk_count + (size_t)p.previous_set * h->n_chunks, (unsigned)h->n_chunks, p.vertices,
+                                 h->values[0], p.report_to, h->launch_vertices()};
+        if (!p.numbers_in_build) to_number[n_to_number++] = work[i];
+    }
+    PL_HIP(plk::build_joint(first->pd, n, work, first->scale, first->xcd_aware ? 1 : 0, plan[0].fused ? first->vd : 0,
+                            first->normalize ? first->vd - 1 : first->vd, stream));
+    if (n_to_number) PL_HIP(plk::number_vertices_joint(first->pd, n_to_number, to_number, first->vd, stream));
+    PL_HIP(plk::neighbours_joint(first->pd, n, work, first->vd, stream));
+    for (int i = 0; i < n; ++i) build_enqueued(lattice[i], plan[i]);
+    return enqueue_joint_apply(n, lattice, output, input, reverse);
+}
+
+}  // namespace
+
+int pl_filter_images(int n, const pl_handle *lattices, float *output, const float *input, const float *reference,
+                     int n_reference_channels, int n_spatial_dims, const int *spatial_dims, float spatial_std,
+                     float feature_std, int reverse) {
+    if (n < 1 || !lattices) return PL_EINVAL;
+    for (int i = 0; i < n; ++i) {
+        const pl_lattice *h = lattices[i];
+        if (!h || h->f64 || h->N != lattices[0]->N || h->vd != lattices[0]->vd || h->pd != lattices[0]->pd ||
+            h->normalize != lattices[0]->normalize)
+            return PL_EINVAL;
+        if (h->pending.active) return PL_ESTATE;
+        for (int j = 0; j < i; ++j)
+            if (lattices[j] == lattices[i]) return PL_EINVAL;
+    }
+    const size_t N = (size_t)lattices[0]->N, channels = (size_t)lattices[0]->vd - (lattices[0]->normalize ? 1 : 0);
+    if (N > 0 && (!output || !input)) return PL_EINVAL;
+    auto reference_of = [&](int i) { return reference ? reference + (size_t)i * N * (size_t)n_reference_channels : nullptr; };
+    const bool join = N > 0 && can_join(n, lattices);
+    for (int from = 0; from < n; from += plk::kJointItems) {
+        const int count = n - from < plk::kJointItems ? n - from : plk::kJointItems;
+        if (!join || count == 1) {
+            for (int i = from; i < from + count; ++i) {
+                const int rc = pl_filter_image(lattices[i], output + (size_t)i * N * channels, input + (size_t)i * N * channels,
+                                               reference_of(i), n_reference_channels, n_spatial_dims, spatial_dims,
+                                               spatial_std, feature_std, reverse);
+                if (rc != PL_OK) return rc;
+            }
+            continue;
+        }
+        pl_lattice *lattice[plk::kJointItems];
+        plk::PointFeatures features[plk::kJointItems];
+        float *out[plk::kJointItems];
+        const float *in[plk::kJointItems];
+        for (int k = 0; k < count; ++k) {
+            pl_lattice *h = lattice[k] = lattices[from + k];
+            out[k] = output + (size_t)(from + k) * N * channels;
+            in[k] = input + (size_t)(from + k) * N * channels;
+            const int rc = features_from_image(h, reference_of(from + k), n_reference_channels, n_spatial_dims, spatial_dims,
+                                               spatial_std, feature_std, &features[k]);
+            if (rc != PL_OK) return rc;
+            h->built = false;
+            h->M = 0;
+        }
+        int rc = enqueue_joint_filter(count, lattice, features, out, in, reverse);
+        if (rc != PL_OK) {
+            // (some of the builds may be under way, on arrays that the lattices' next calls use again)
+            for (int k = 0; k < count; ++k) lattice[k]->built = lattice[k]->table_clean = lattice[k]->cell_values_clean = false;
+            (void)hipStreamSynchronize(lattice[0]->stream);
+            return rc;
+        }
+        for (int k = 0; k < count; ++k) {
+            pl_lattice::Pending &pending = lattice[k]->pending;
+            pending.active = true;
+            pending.build_only = false;
+            pending.features = features[k];
+            pending.positions64 = nullptr;
+            pending.output = out[k];
+            pending.input = in[k];
+            pending.reverse = reverse;
+        }
+        // (every lattice's build is looked at, also behind one that failed)
+        for (int k = 0; k < count; ++k) {
+            const int ended = filter_end(lattice[k]);
+            if (rc == PL_OK) rc = ended;
+        }
+        if (rc != PL_OK) return rc;
+    }
+    return PL_OK;
+}
+
+int pl_apply_many(int n, const pl_handle *lattices, float *output, const float *input, int reverse) {
+    if (n < 1 || !lattices) return PL_EINVAL;
+    for (int i = 0; i < n; ++i) {
+        const pl_lattice *h = lattices[i];
+        if (!h || h->f64 || h->N != lattices[0]->N || h->vd != lattices[0]->vd || h->normalize != lattices[0]->normalize)
+            return PL_EINVAL;
+        if (!h->built || !h->verified || h->pending.active) return PL_ESTATE;
+        for (int j = 0; j < i; ++j)
+            if (lattices[j] == lattices[i]) return PL_EINVAL;
+    }
+    const size_t N = (size_t)lattices[0]->N, channels = (size_t)lattices[0]->vd - (lattices[0]->normalize ? 1 : 0);
+    if (N == 0) return PL_OK;
+    if (!output || !input) return PL_EINVAL;
+    bool join = can_join(n, lattices);
+    for (int i = 0; i < n && join; ++i)
+        join = lattices[i]->last_build_merged && !lattices[i]->lists_valid && !lattices[i]->values_splatted &&
+               lattices[i]->map.mode >= 2;
+    for (int from = 0; from < n; from += plk::kJointItems) {
+        const int count = n - from < plk::kJointItems ? n - from : plk::kJointItems;
+        pl_lattice *lattice[plk::kJointItems];
+        float *out[plk::kJointItems];
+        const float *in[plk::kJointItems];
+        for (int k = 0; k < count; ++k) {
+            lattice[k] = lattices[from + k];
+            out[k] = output + (size_t)(from + k) * N * channels;
+            in[k] = input + (size_t)(from + k) * N * channels;
+        }
+        int rc = PL_OK;
+        if (join && count > 1)
+            rc = enqueue_joint_apply(count, lattice, out, in, reverse);
+        else
+            for (int k = 0; k < count && rc == PL_OK; ++k) rc = enqueue_apply(lattice[k], out[k], in[k], reverse);
+        if (rc != PL_OK) return rc;
+    }
+    return PL_OK;
+}
 
 int pl_build(pl_handle h, const float *positions) {
     if (!h || (!positions && h->N > 0)) return PL_EINVAL;

@@ -494,18 +494,22 @@ __device__ __forceinline__ int point_of_thread(const PointMap &m, unsigned vbloc
 // xcd_aware), false when it has none: the workgroups behind the last that holds points of an
 // ordered list.  Those keep their own number as vblock, so that every workgroup of the grid has
 // one of its own.
-__device__ __forceinline__ bool block_of_points(const PointMap &m, int xcd_aware, unsigned &vblock) {
-    unsigned nb = gridDim.x;
+__device__ __forceinline__ bool block_of_points(const PointMap &m, int xcd_aware, unsigned block, unsigned blocks,
+                                                unsigned &vblock) {
+    unsigned nb = blocks;
     if (m.mode == 1) {
         const unsigned tiles = *m.n_tiles;
         nb = tiles < nb ? tiles : nb;
-        if (blockIdx.x >= nb) {
-            vblock = blockIdx.x;
+        if (block >= nb) {
+            vblock = block;
             return false;
         }
     }
-    vblock = xcd_contiguous_block(blockIdx.x, nb, xcd_aware);
+    vblock = xcd_contiguous_block(block, nb, xcd_aware);
     return true;
+}
+__device__ __forceinline__ bool block_of_points(const PointMap &m, int xcd_aware, unsigned &vblock) {
+    return block_of_points(m, xcd_aware, blockIdx.x, gridDim.x, vblock);
 }
 
 // The words and the weights of a workgroup's points in the replay of a merging build (TileVertices).

@@ -478,6 +478,7 @@ struct BlurWork {
     uint64_t *reset_cell_keys;
     const int *vertex_cell;
     int max_vertices, launch_vertices;
+    const int2 *nbr_third;     // blur_joint, rows of up to four channels
 };
 hipError_t blur_many(int vd, int n, const BlurWork *work, hipStream_t s);
 // Stage 5 of pairs of lattices over the same points (same point map, normalising): output := the sum of
@@ -526,6 +527,51 @@ hipError_t slice(int pd, int vd, const PointMap &map, const ReplayEntry *replay,
 // Five to sixty-four channels of a lattice whose build merged (pl_many.hip).
 hipError_t slice_tile_channels(int pd, int vd, const PointMap &map, const ReplayEntry *replay, const float *values,
                             float *output, int normalize, hipStream_t s);
+
+// The passes of several lattices of floats on grids in one launch each, as build, number_vertices, neighbours,
+// splat_merge or splat_tile, blur_* and slice take one: the images of a batch.  A pass over the vertices of one
+// image is a launch of 5 us that fills a part of the GPU for three round trips to memory, and an image of a
+// tenth of a million points fills it in no pass.  An op and its gradient, one image after the other and
+// together, us: 4 x 1024x1024 points, pd 5, vd 2, 631 and 483; 2 x 321x481 points, vd 22, 270 and 209.
+// (joint_takes: what the kernels are compiled for: the guides of one to three channels of images, volumes
+// under their own intensities, coordinates alone.)
+constexpr int kJointItems = 4;
+struct BuildWork {
+    PointFeatures features;
+    PointMap map;
+    uint64_t *cell_keys;
+    uint32_t mask;             // cells - 1
+    Counters *counters, *next_counters;
+    ReplayEntry *replay;
+    const float *input;        // splatted in the build (splat_vd)
+    float *cell_values;        // (nullptr: not splatted)
+    CreatedLists lists;
+    RegionSource regions;
+    InBuildNumbering numbering;
+    // number_vertices and neighbours
+    int *next_chunk_count;
+    unsigned n_chunks;
+    VertexTables vertices;
+    float *values;
+    HostReport report_to;
+    int launch_vertices;
+};
+struct PointsWork {
+    PointMap map;
+    const ReplayEntry *replay;
+    const float *input;
+    float *values, *output;
+};
+inline bool joint_takes(int pd, int vd) { return pd >= 2 && pd <= 5 && vd <= 32; }
+hipError_t build_joint(int pd, int n, const BuildWork *work, const ScaleFactor &scale, int xcd_aware, int splat_vd,
+                       int in_channels, hipStream_t s);
+hipError_t number_vertices_joint(int pd, int n, const BuildWork *work, int vd, hipStream_t s);
+hipError_t neighbours_joint(int pd, int n, const BuildWork *work, int vd, hipStream_t s);
+hipError_t splat_joint(int pd, int vd, int n, const PointsWork *work, int in_channels, int xcd_aware, hipStream_t s);
+hipError_t splat_tile_joint(int pd, int vd, int n, const PointsWork *work, int in_channels, int xcd_aware, hipStream_t s);
+hipError_t blur_joint(int vd, int n, const BlurWork *work, hipStream_t s);
+hipError_t slice_joint(int pd, int vd, int n, const PointsWork *work, int normalize, hipStream_t s);
+hipError_t slice_tile_channels_joint(int pd, int vd, int n, const PointsWork *work, int normalize, hipStream_t s);
 
 hipError_t debug_simplex(int pd, const float *positions, int N, const ScaleFactor &scale,
                          short *rem0, short *rank, short *keys, float *barycentric, hipStream_t s);

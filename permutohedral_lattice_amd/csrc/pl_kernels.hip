@@ -679,24 +679,22 @@ __device__ __forceinline__ void add_to_slots(T *slot_sum, const unsigned (&group
 static_assert(kTileSlots == 2 * kBlock, "a thread places at most two slots in the table");
 constexpr int kTileProbeLimit = 48;
 
-// (at most 102 scalar registers: with more a SIMD holds seven wavefronts, not eight)
-template <int PD, int SPLAT_VD, typename T = float>
-__global__ __launch_bounds__(kBlock) __attribute__((amdgpu_num_sgpr(102))) void k_build_tile(PointFeatures features, PointMap map,
-                                                        ScaleFactor scale, uint64_t *cell_keys,
-                                                        uint32_t mask, Counters *counters,
-                                                        ReplayEntry *__restrict__ replay,
-                                                        int xcd_aware, const void *__restrict__ input_any,
-                                                        int in_channels, void *cell_values_any,
-                                                        CreatedLists created_lists,
-                                                        Points64 points64, RegionSource region_source,
-                                                        InBuildNumbering numbering) {
+// (workgroup `block` of the `blocks` of a lattice)
+template <int PD, int SPLAT_VD, typename T>
+__device__ __forceinline__ void build_tile(const PointFeatures &features, const PointMap &map, const ScaleFactor &scale,
+                                           uint64_t *cell_keys, uint32_t mask, Counters *counters,
+                                           ReplayEntry *__restrict__ replay, int xcd_aware,
+                                           const void *__restrict__ input_any, int in_channels, void *cell_values_any,
+                                           const CreatedLists &created_lists, const Points64 &points64,
+                                           const RegionSource &region_source, const InBuildNumbering &numbering,
+                                           unsigned block, unsigned blocks) {
     constexpr bool kDouble = sizeof(T) == sizeof(double);
     constexpr int D1 = PD + 1;
     constexpr int VD = SPLAT_VD ? SPLAT_VD : 2;
     constexpr int P = (VD == 2 && !kDouble) ? 2 : 4;      // values per LDS row of sums
     const T *__restrict__ input = static_cast<const T *>(input_any);
     unsigned vblock;
-    if (!block_of_points(map, xcd_aware, vblock)) {
+    if (!block_of_points(map, xcd_aware, block, blocks, vblock)) {
         // (no points: nothing created, no rows of sums for the passes that walk the lists)
         if (threadIdx.x == 0) created_lists.block_count[vblock] = created_lists.tiles.used[vblock] = 0;
         return;
@@ -782,7 +780,7 @@ __global__ __launch_bounds__(kBlock) __attribute__((amdgpu_num_sgpr(102))) void 
     // (i + kBlock)-th when a tile has that many, in rounds over both as in k_build).  A tile of an
     // image has about a hundred, so two of the four wavefronts have nothing to do here.
     const KeyRegions regions = key_regions(region_source);
-    if (blockIdx.x == 0 && tid == 0) {
+    if (block == 0 && tid == 0) {
         counters->region_lo = regions.lo;
         counters->region_per_unit = regions.per_unit;
     }
@@ -958,20 +956,20 @@ __global__ __launch_bounds__(kBlock) __attribute__((amdgpu_num_sgpr(102))) void 
         // eighth of that (vblock runs through an XCD's share of the workgroups in order)
         const unsigned parts = (unsigned)numbering.n_segments / kXcds;
         if (xcd_aware) {
-            const unsigned nb = map.mode == 1 && *map.n_tiles < gridDim.x ? *map.n_tiles : gridDim.x;
-            const unsigned xcd = blockIdx.x % kXcds;
+            const unsigned nb = map.mode == 1 && *map.n_tiles < blocks ? *map.n_tiles : blocks;
+            const unsigned xcd = block % kXcds;
             const unsigned share = nb / kXcds + (xcd < nb % kXcds ? 1u : 0u);
-            const unsigned index = blockIdx.x / kXcds;
+            const unsigned index = block / kXcds;
             segment = xcd * parts + (share ? (unsigned)(((size_t)index * parts) / share) : 0u);
         } else {
-            segment = (unsigned)(((size_t)vblock * (size_t)numbering.n_segments) / gridDim.x);
+            segment = (unsigned)(((size_t)vblock * (size_t)numbering.n_segments) / blocks);
         }
     }
     const unsigned count = (unsigned)group_created;
     unsigned first = 0;
     if (tid == 0 && count) first = atomicAdd(&counters->segment_count[segment].n, count);
     write_replay();
-    if (blockIdx.x == 0 && tid < kMaxSegments) {
+    if (block == 0 && tid < kMaxSegments) {
         counters->n_segments = numbering.n_segments;
         counters->segment_count[tid].n_segments = numbering.n_segments;
     }
@@ -1049,9 +1047,31 @@ __global__ __launch_bounds__(kBlock) __attribute__((amdgpu_num_sgpr(102))) void 
         created_lists.block_count[vblock] = n_foreign;
         created_lists.tiles.used[vblock] = n_in_use;
         // (how many such rows there are in all tells the host whether numbering here pays)
-        if ((blockIdx.x / kXcds) % kForeignSampling == 0 && n_foreign)
+        if ((block / kXcds) % kForeignSampling == 0 && n_foreign)
             atomicAdd(&counters->foreign_rows_sampled.n, (unsigned)n_foreign);
     }
+}
+
+// (at most 102 scalar registers: with more a SIMD holds seven wavefronts, not eight)
+template <int PD, int SPLAT_VD, typename T = float>
+__global__ __launch_bounds__(kBlock) __attribute__((amdgpu_num_sgpr(102))) void k_build_tile(
+    PointFeatures features, PointMap map, ScaleFactor scale, uint64_t *cell_keys, uint32_t mask, Counters *counters,
+    ReplayEntry *__restrict__ replay, int xcd_aware, const void *__restrict__ input_any, int in_channels,
+    void *cell_values_any, CreatedLists created_lists, Points64 points64, RegionSource region_source,
+    InBuildNumbering numbering) {
+    build_tile<PD, SPLAT_VD, T>(features, map, scale, cell_keys, mask, counters, replay, xcd_aware, input_any, in_channels,
+                                cell_values_any, created_lists, points64, region_source, numbering, blockIdx.x, gridDim.x);
+}
+// The same for several lattices of floats.
+template <int PD, int SPLAT_VD>
+__global__ __launch_bounds__(kBlock) __attribute__((amdgpu_num_sgpr(102))) void k_build_tiles(
+    Items<BuildWork, kJointItems> items, ScaleFactor scale, int xcd_aware, int in_channels) {
+    unsigned block, blocks;
+    const BuildWork &work = item_of(items, block, blocks);
+    if (block >= work.map.n_blocks) return;
+    build_tile<PD, SPLAT_VD, float>(work.features, work.map, scale, work.cell_keys, work.mask, work.counters, work.replay,
+                                    xcd_aware, work.input, in_channels, work.cell_values, work.lists, Points64{},
+                                    work.regions, work.numbering, block, work.map.n_blocks);
 }
 
 // The flags a report carries: the build's, and what was seen of the list it ordered.
@@ -1070,17 +1090,15 @@ __device__ __forceinline__ int reported_flags(const Counters *counters) {
 // and to host-visible memory and clears what the next build will count in.
 // WIDE: the build had keys of two words: two entries per vertex (key, then cell), and
 // vertex_keys holds two words per vertex.
-template <int D1, bool WIDE = false>
-__global__ __launch_bounds__(64) void k_number_vertices(CreatedLists lists, int *next_chunk_count,
-                                                        unsigned n_chunks,
-                                                        VertexTables vertices, float *values, int vd,
-                                                        float *cell_values, Counters *counters,
-                                                        Counters *next_counters,
-                                                        HostReport host_report) {
+template <int D1, bool WIDE>
+__device__ __forceinline__ void number_list(const CreatedLists &lists, int *next_chunk_count, unsigned n_chunks,
+                                            const VertexTables &vertices, float *values, int vd, float *cell_values,
+                                            Counters *counters, Counters *next_counters, const HostReport &host_report,
+                                            unsigned block, unsigned blocks) {
     HostStatus *host_status = host_report.status;
     // (an XCD takes the lists of one contiguous range of tiles: their cells are in its part of the
     // table and their vertex numbers in one range)
-    const unsigned b = xcd_contiguous_block(blockIdx.x, gridDim.x, 1);
+    const unsigned b = xcd_contiguous_block(block, blocks, 1);
     const int lane = threadIdx.x;
     const unsigned chunk = b / kBlocksPerChunk;
     const size_t list = (size_t)b * (size_t)lists.stride;
@@ -1117,7 +1135,7 @@ __global__ __launch_bounds__(64) void k_number_vertices(CreatedLists lists, int 
     for (int off = 32; off >= 1; off >>= 1) before += __shfl_xor(before, off);
     const int max_vertices = vertices.max_vertices;
 
-    if (b == gridDim.x - 1) {
+    if (b == blocks - 1) {
         if (lane == 0) {
             const uint32_t m = (uint32_t)(before + count);
             const int flags = reported_flags(counters);
@@ -1183,6 +1201,23 @@ __global__ __launch_bounds__(64) void k_number_vertices(CreatedLists lists, int 
     }
 }
 
+template <int D1, bool WIDE = false>
+__global__ __launch_bounds__(64) void k_number_vertices(CreatedLists lists, int *next_chunk_count, unsigned n_chunks,
+                                                        VertexTables vertices, float *values, int vd,
+                                                        float *cell_values, Counters *counters, Counters *next_counters,
+                                                        HostReport host_report) {
+    number_list<D1, WIDE>(lists, next_chunk_count, n_chunks, vertices, values, vd, cell_values, counters, next_counters,
+                          host_report, blockIdx.x, gridDim.x);
+}
+template <int D1>
+__global__ __launch_bounds__(64) void k_number_vertices_of(Items<BuildWork, kJointItems> items, int vd) {
+    unsigned block, blocks;
+    const BuildWork &work = item_of(items, block, blocks);
+    if (block >= work.map.n_blocks) return;
+    number_list<D1, false>(work.lists, work.next_chunk_count, work.n_chunks, work.vertices, work.values, vd,
+                           work.cell_values, work.counters, work.next_counters, work.report_to, block, work.map.n_blocks);
+}
+
 // ------------------------------------------------------------------------------------------------
 // Neighbour table: along axis a the neighbours of key k are k + (1,..,1) - (pd+1) e_a and its
 // mirror image (reference: src/PermutohedralLatticeCPU.h:381-388).  In (r, q) form the first is
@@ -1217,23 +1252,24 @@ __device__ __forceinline__ void add_foreign_rows(const CreatedLists &lists, unsi
     }
 }
 
+__host__ __device__ inline unsigned tile_blocks_for(unsigned n_lists) {
+    return (n_lists + kBlock / 64 * kXcds - 1u) / (kBlock / 64 * kXcds) * kXcds;
+}
 // WIDE: keys and cells of two words (see k_build), one cell per probe step, plain hashing.
-template <int PD, bool WIDE = false>
-__global__ __launch_bounds__(kBlock) void k_neighbours(VertexTables vertices,
-                                                        const Counters *counters,
-                                                        const uint64_t *__restrict__ cell_keys,
-                                                        uint32_t mask, unsigned tile_blocks,
-                                                        CreatedLists lists, unsigned n_lists,
-                                                        void *values, int vd, int values_are_double,
-                                                        Counters *report, Counters *next_counters,
-                                                        HostReport host_report) {
+template <int PD, bool WIDE>
+__device__ __forceinline__ void find_neighbours(const VertexTables &vertices, const Counters *counters,
+                                                const uint64_t *__restrict__ cell_keys, uint32_t mask,
+                                                unsigned tile_blocks, const CreatedLists &lists, unsigned n_lists,
+                                                void *values, int vd, int values_are_double, Counters *report,
+                                                Counters *next_counters, const HostReport &host_report, unsigned block,
+                                                unsigned blocks) {
     constexpr int D1 = PD + 1;
     HostStatus *host_status = host_report.status;
     // After a merging build nothing has told the host yet how the build went: the segments' counts
     // are summed here, and what the next build will count in is cleared.
     // (by the first wavefront of the first workgroup that looks up neighbours, which starts with
     // the launch: a lane per segment)
-    if (report && blockIdx.x == tile_blocks && threadIdx.x < 64) {
+    if (report && block == tile_blocks && threadIdx.x < 64) {
         static_assert(kMaxSegments <= 64, "a lane per segment");
         const int n_segments = report->n_segments;
         const unsigned c = (int)threadIdx.x < n_segments ? report->segment_count[threadIdx.x].n : 0u;
@@ -1260,8 +1296,8 @@ __global__ __launch_bounds__(kBlock) void k_neighbours(VertexTables vertices,
             reset_counters(next_counters);
         }
     }
-    if (blockIdx.x < tile_blocks) {
-        const unsigned list = xcd_contiguous_block(blockIdx.x, tile_blocks, 1) * (kBlock / 64) + (threadIdx.x >> 6);
+    if (block < tile_blocks) {
+        const unsigned list = xcd_contiguous_block(block, tile_blocks, 1) * (kBlock / 64) + (threadIdx.x >> 6);
         if (list >= n_lists) return;
         if (!lists.foreign_rows) {
             int *const table = lists.tiles.of(list);
@@ -1279,7 +1315,7 @@ __global__ __launch_bounds__(kBlock) void k_neighbours(VertexTables vertices,
     }
     const KeyRegions regions{counters->region_lo, counters->region_per_unit};
     const int max_vertices = vertices.max_vertices;
-    SegmentWalk walk(counters, max_vertices, blockIdx.x - tile_blocks, gridDim.x - tile_blocks);
+    SegmentWalk walk(counters, max_vertices, block - tile_blocks, blocks - tile_blocks);
     unsigned ib;
     while (walk.next(1u, D1, ib)) {
     const int a = (int)(ib % D1);
@@ -1332,6 +1368,25 @@ __global__ __launch_bounds__(kBlock) void k_neighbours(VertexTables vertices,
         entries[2 * ((size_t)a * max_vertices + u) + 1] = v;      // out[a][u].y
     }
     }
+}
+
+template <int PD, bool WIDE = false>
+__global__ __launch_bounds__(kBlock) void k_neighbours(VertexTables vertices, const Counters *counters,
+                                                        const uint64_t *__restrict__ cell_keys, uint32_t mask,
+                                                        unsigned tile_blocks, CreatedLists lists, unsigned n_lists,
+                                                        void *values, int vd, int values_are_double, Counters *report,
+                                                        Counters *next_counters, HostReport host_report) {
+    find_neighbours<PD, WIDE>(vertices, counters, cell_keys, mask, tile_blocks, lists, n_lists, values, vd,
+                              values_are_double, report, next_counters, host_report, blockIdx.x, gridDim.x);
+}
+template <int PD>
+__global__ __launch_bounds__(kBlock) void k_neighbours_of(Items<BuildWork, kJointItems> items, int vd) {
+    unsigned block, blocks;
+    const BuildWork &work = item_of(items, block, blocks);
+    find_neighbours<PD, false>(work.vertices, work.counters, work.cell_keys, work.mask, tile_blocks_for(work.map.n_blocks),
+                               work.lists, work.map.n_blocks, work.values, vd, 0,
+                               work.numbering.n_segments ? work.counters : nullptr, work.next_counters, work.report_to,
+                               block, blocks);
 }
 
 // Several ranges of words at once, each to a word of its own: a workgroup takes 1024 words of one.
@@ -1435,13 +1490,13 @@ __global__ __launch_bounds__(kBlock) void k_splat_dpp(PointMap map,
 // its instructions and the requests to the L2 atomic unit; 1024x1024 points, pd 5, vd 2: 21.5 us a launch, 30.8
 // when it looked its vertices up in a table of hashes first.
 template <int VD, int D1>
-__global__ __launch_bounds__(kBlock) void k_splat_merge(PointMap map, const float *__restrict__ input,
-                                                         int in_channels, const ReplayEntry *__restrict__ replay,
-                                                         float *values, int xcd_aware) {
+__device__ __forceinline__ void splat_merged(const PointMap &map, const float *__restrict__ input, int in_channels,
+                                             const ReplayEntry *__restrict__ replay, float *values, int xcd_aware,
+                                             unsigned block, unsigned blocks) {
     static_assert(VD >= 2 && VD <= 4, "register splat handles 2..4 channels");
     constexpr int P = VD == 2 ? 2 : 4;   // values per LDS row of sums
     unsigned vblock;
-    if (!block_of_points(map, xcd_aware, vblock)) return;
+    if (!block_of_points(map, xcd_aware, block, blocks, vblock)) return;
     __shared__ float place_sum[kTileSlots * P];
     const int tid = threadIdx.x, lane = tid & 63;
     for (int i = tid; i < kTileSlots * P; i += kBlock) place_sum[i] = 0.0f;
@@ -1478,6 +1533,21 @@ __global__ __launch_bounds__(kBlock) void k_splat_merge(PointMap map, const floa
         const int v = table[i];
         if (v >= 0 && channel < VD) atomicAdd(values + (size_t)v * VD + channel, place_sum[i * P + channel]);
     }
+}
+
+template <int VD, int D1>
+__global__ __launch_bounds__(kBlock) void k_splat_merge(PointMap map, const float *__restrict__ input,
+                                                         int in_channels, const ReplayEntry *__restrict__ replay,
+                                                         float *values, int xcd_aware) {
+    splat_merged<VD, D1>(map, input, in_channels, replay, values, xcd_aware, blockIdx.x, gridDim.x);
+}
+template <int VD, int D1>
+__global__ __launch_bounds__(kBlock) void k_splat_merge_of(Items<PointsWork, kJointItems> items, int in_channels,
+                                                            int xcd_aware) {
+    unsigned block, blocks;
+    const PointsWork &work = item_of(items, block, blocks);
+    if (block >= work.map.n_blocks) return;
+    splat_merged<VD, D1>(work.map, work.input, in_channels, work.replay, work.values, xcd_aware, block, work.map.n_blocks);
 }
 
 // Any vd: the same, four channels at a time.  The deduplication loop runs once per block of four
@@ -1892,6 +1962,47 @@ __global__ __launch_bounds__(kBlock) void k_blur3_row(const Counters *counters, 
     }
 }
 
+// One, two or three axes (nbr_third: rows of up to four channels where three are all there are) of several lattices.
+template <int VD>
+__global__ __launch_bounds__(kBlock) void k_blur_rows_of(Items<BlurWork, kJointItems> items) {
+    unsigned block, blocks;
+    const BlurWork &work = item_of(items, block, blocks);
+    const ValueRow<VD> *__restrict__ src = reinterpret_cast<const ValueRow<VD> *>(work.src);
+    ValueRow<VD> *__restrict__ dst = reinterpret_cast<ValueRow<VD> *>(work.dst);
+    SegmentWalk walk(work.counters, work.max_vertices, block, blocks);
+    unsigned vb;
+    while (walk.next(1u, 1u, vb)) {
+        const unsigned i = vb * kBlock + threadIdx.x;
+        if (i >= walk.count) continue;
+        const int v = (int)(walk.first + i);
+        if (work.nbr_third) {
+            int u[27];
+            three_axis_sources(work.nbr_first, work.nbr_second, work.nbr_third, v, u);
+            ValueRow<VD> row[27], after_a[9];
+            gather_rows<VD, float, 27>(src, u, row);
+#pragma unroll
+            for (int k = 0; k < 9; ++k) after_a[k] = blur_rows<VD>(row[3 * k], row[3 * k + 1], row[3 * k + 2]);
+            dst[v] = blur_rows<VD>(blur_rows<VD>(after_a[0], after_a[1], after_a[2]),
+                                   blur_rows<VD>(after_a[3], after_a[4], after_a[5]),
+                                   blur_rows<VD>(after_a[6], after_a[7], after_a[8]));
+        } else if (work.nbr_second) {
+            int u[9];
+            two_axis_sources(work.nbr_first, work.nbr_second, v, u);
+            ValueRow<VD> row[9];
+            gather_rows<VD, float, 9>(src, u, row);
+            dst[v] = blur_rows<VD>(blur_rows<VD>(row[0], row[1], row[2]), blur_rows<VD>(row[3], row[4], row[5]),
+                                   blur_rows<VD>(row[6], row[7], row[8]));
+        } else {
+            const int2 nb = work.nbr_first[v];
+            const int u[3] = {nb.x, v, nb.y};
+            ValueRow<VD> row[3];
+            gather_rows<VD, float, 3>(src, u, row);
+            dst[v] = blur_rows<VD>(row[0], row[1], row[2]);
+        }
+        if (work.reset_cell_keys) work.reset_cell_keys[work.vertex_cell[v]] = kEmptyCell;
+    }
+}
+
 // ------------------------------------------------------------------------------------------------
 // Stage 5: slice (reference: src/PermutohedralLatticeCPU.h:333-352)
 // ------------------------------------------------------------------------------------------------
@@ -2017,10 +2128,9 @@ __global__ __launch_bounds__(kBlock) void k_slice_rows_f64(PointMap map,
 // this, us: 1024x1024 points pd 5 vd 4 15.1 and 10.1, vd 2 12.2 and 8.5; 128x256x256 voxels pd 4 vd 2 103.8
 // and 57.3; 601x803 points in doubles 14.3 and 8.8.
 template <int VD, int D1, typename S>
-__global__ __launch_bounds__(kBlock) void k_slice_tile(PointMap map, const ReplayEntry *__restrict__ replay,
-                                                        const double *__restrict__ weights64,
-                                                        const S *__restrict__ values, S *__restrict__ output,
-                                                        int normalize) {
+__device__ __forceinline__ void slice_of_tile(const PointMap &map, const ReplayEntry *__restrict__ replay,
+                                              const double *__restrict__ weights64, const S *__restrict__ values,
+                                              S *__restrict__ output, int normalize, unsigned block, unsigned blocks) {
     constexpr bool kDouble = sizeof(S) == sizeof(double);
     constexpr int P = VD == 2 ? 2 : 4;   // values per row in LDS
     struct alignas(16) Row {
@@ -2030,7 +2140,7 @@ __global__ __launch_bounds__(kBlock) void k_slice_tile(PointMap map, const Repla
     static_assert(sizeof(Packed) == P * sizeof(S), "rows without gaps");
     __shared__ Packed rows[kTileSlots];
     unsigned vblock;
-    if (!block_of_points(map, 1, vblock)) return;
+    if (!block_of_points(map, 1, block, blocks, vblock)) return;
     const int tid = threadIdx.x;
     const uint32_t *words = words_of_tile<kDouble>(replay, vblock, D1);
     const int *table = map.tile_vertices.of(vblock);
@@ -2077,6 +2187,22 @@ __global__ __launch_bounds__(kBlock) void k_slice_tile(PointMap map, const Repla
 #pragma unroll
         for (int j = 0; j < VD; ++j) output[(size_t)n * VD + j] = acc[j];
     }
+}
+
+template <int VD, int D1, typename S>
+__global__ __launch_bounds__(kBlock) void k_slice_tile(PointMap map, const ReplayEntry *__restrict__ replay,
+                                                        const double *__restrict__ weights64,
+                                                        const S *__restrict__ values, S *__restrict__ output,
+                                                        int normalize) {
+    slice_of_tile<VD, D1, S>(map, replay, weights64, values, output, normalize, blockIdx.x, gridDim.x);
+}
+template <int VD, int D1>
+__global__ __launch_bounds__(kBlock) void k_slice_tile_of(Items<PointsWork, kJointItems> items, int normalize) {
+    unsigned block, blocks;
+    const PointsWork &work = item_of(items, block, blocks);
+    if (block >= work.map.n_blocks) return;
+    slice_of_tile<VD, D1, float>(work.map, work.replay, nullptr, work.values, work.output, normalize, block,
+                                 work.map.n_blocks);
 }
 
 // Any vd: one thread per point and run of four channels.  The pd+1 replay rows, then the value
@@ -2520,7 +2646,7 @@ hipError_t neighbours(int pd, const VertexTables &vertices, const Counters *coun
                       HostReport host_report, bool wide_keys, hipStream_t s) {
     if (vertices.max_vertices <= 0) return hipErrorInvalidValue;
     const size_t items = (size_t)(pd + 1) * (size_t)launch_vertices;
-    const unsigned tile_blocks = tiles ? (blocks_for(n_lists, kBlock / 64) + kXcds - 1u) / kXcds * kXcds : 0u;
+    const unsigned tile_blocks = tiles ? tile_blocks_for(n_lists) : 0u;
 #define PLK_NEIGHBOURS(WIDE, DISPATCH)                                                             \
     DISPATCH(pd, hipLaunchKernelGGL((k_neighbours<PD, WIDE>),                                      \
                                            dim3(tile_blocks + vertex_blocks(items)),            \
@@ -2822,6 +2948,122 @@ hipError_t slice_rows_f64(int pd, int vd, const PointMap &map, const ReplayEntry
         default: return hipErrorInvalidValue;
     }
 #undef PLK_SLICE_ROWS
+    return hipGetLastError();
+}
+
+// ------------------------------------------------------------------------------------------------
+// The passes of several lattices
+// ------------------------------------------------------------------------------------------------
+#define PLK_DISPATCH_JOINT_PD(pd, CALL)               \
+    switch (pd) {                                     \
+        case 2: { constexpr int PD = 2; CALL; } break; \
+        case 3: { constexpr int PD = 3; CALL; } break; \
+        case 4: { constexpr int PD = 4; CALL; } break; \
+        case 5: { constexpr int PD = 5; CALL; } break; \
+        default: return hipErrorInvalidValue;         \
+    }
+
+static Items<BuildWork, kJointItems> build_items(int n, const BuildWork *work) {
+    Items<BuildWork, kJointItems> items{};
+    items.n = n;
+    for (int i = 0; i < n; ++i) {
+        items.item[i] = work[i];
+        items.blocks[i] = multiple_of_xcds(work[i].map.n_blocks);
+    }
+    return items;
+}
+
+hipError_t build_joint(int pd, int n, const BuildWork *work, const ScaleFactor &scale, int xcd_aware, int splat_vd,
+                       int in_channels, hipStream_t s) {
+    if (n < 1 || n > kJointItems) return hipErrorInvalidValue;
+    const Items<BuildWork, kJointItems> items = build_items(n, work);
+#define PLK_BUILD_JOINT(SPLAT_VD)                                                                                    \
+    case SPLAT_VD:                                                                                                   \
+        PLK_DISPATCH_JOINT_PD(pd, hipLaunchKernelGGL((k_build_tiles<PD, SPLAT_VD>), dim3(all_blocks(items)), dim3(kBlock), \
+                                                     0, s, items, scale, xcd_aware, in_channels))                    \
+        break;
+    switch (splat_vd) {
+        PLK_BUILD_JOINT(0) PLK_BUILD_JOINT(2) PLK_BUILD_JOINT(3) PLK_BUILD_JOINT(4)
+        default: return hipErrorInvalidValue;
+    }
+#undef PLK_BUILD_JOINT
+    return hipGetLastError();
+}
+
+hipError_t number_vertices_joint(int pd, int n, const BuildWork *work, int vd, hipStream_t s) {
+    if (n < 1 || n > kJointItems) return hipErrorInvalidValue;
+    const Items<BuildWork, kJointItems> items = build_items(n, work);
+    PLK_DISPATCH_JOINT_PD(pd, hipLaunchKernelGGL((k_number_vertices_of<PD + 1>), dim3(all_blocks(items)), dim3(64), 0, s,
+                                                 items, vd));
+    return hipGetLastError();
+}
+
+hipError_t neighbours_joint(int pd, int n, const BuildWork *work, int vd, hipStream_t s) {
+    if (n < 1 || n > kJointItems) return hipErrorInvalidValue;
+    Items<BuildWork, kJointItems> items = build_items(n, work);
+    for (int i = 0; i < n; ++i)
+        items.blocks[i] = tile_blocks_for(work[i].map.n_blocks) +
+                          vertex_blocks((size_t)(pd + 1) * (size_t)work[i].launch_vertices);
+    PLK_DISPATCH_JOINT_PD(pd, hipLaunchKernelGGL((k_neighbours_of<PD>), dim3(all_blocks(items)), dim3(kBlock), 0, s, items,
+                                                 vd));
+    return hipGetLastError();
+}
+
+static Items<PointsWork, kJointItems> points_items(int n, const PointsWork *work) {
+    Items<PointsWork, kJointItems> items{};
+    items.n = n;
+    for (int i = 0; i < n; ++i) {
+        items.item[i] = work[i];
+        items.blocks[i] = multiple_of_xcds(work[i].map.n_blocks);
+    }
+    return items;
+}
+
+hipError_t splat_joint(int pd, int vd, int n, const PointsWork *work, int in_channels, int xcd_aware, hipStream_t s) {
+    if (n < 1 || n > kJointItems) return hipErrorInvalidValue;
+    if (vd > 4) return splat_tile_joint(pd, vd, n, work, in_channels, xcd_aware, s);
+    const Items<PointsWork, kJointItems> items = points_items(n, work);
+#define PLK_SPLAT_JOINT(VD)                                                                                              \
+    case VD:                                                                                                             \
+        PLK_DISPATCH_JOINT_PD(pd, hipLaunchKernelGGL((k_splat_merge_of<VD, PD + 1>), dim3(all_blocks(items)), dim3(kBlock), \
+                                                     0, s, items, in_channels, xcd_aware))                               \
+        break;
+    switch (vd) {
+        PLK_SPLAT_JOINT(2) PLK_SPLAT_JOINT(3) PLK_SPLAT_JOINT(4)
+        default: return hipErrorInvalidValue;
+    }
+#undef PLK_SPLAT_JOINT
+    return hipGetLastError();
+}
+
+hipError_t blur_joint(int vd, int n, const BlurWork *work, hipStream_t s) {
+    if (n < 1 || n > kJointItems) return hipErrorInvalidValue;
+    if (vd > 4) return blur_many(vd, n, work, s);
+    Items<BlurWork, kJointItems> items{};
+    items.n = n;
+    for (int i = 0; i < n; ++i) {
+        items.item[i] = work[i];
+        items.blocks[i] = vertex_blocks((size_t)work[i].launch_vertices);
+    }
+    const auto kernel = vd == 2 ? k_blur_rows_of<2> : vd == 3 ? k_blur_rows_of<3> : k_blur_rows_of<4>;
+    hipLaunchKernelGGL(kernel, dim3(all_blocks(items)), dim3(kBlock), 0, s, items);
+    return hipGetLastError();
+}
+
+hipError_t slice_joint(int pd, int vd, int n, const PointsWork *work, int normalize, hipStream_t s) {
+    if (n < 1 || n > kJointItems) return hipErrorInvalidValue;
+    if (vd > 4) return slice_tile_channels_joint(pd, vd, n, work, normalize, s);
+    const Items<PointsWork, kJointItems> items = points_items(n, work);
+#define PLK_SLICE_JOINT(VD)                                                                                              \
+    case VD:                                                                                                             \
+        PLK_DISPATCH_JOINT_PD(pd, hipLaunchKernelGGL((k_slice_tile_of<VD, PD + 1>), dim3(all_blocks(items)), dim3(kBlock), \
+                                                     0, s, items, normalize))                                            \
+        break;
+    switch (vd) {
+        PLK_SLICE_JOINT(2) PLK_SLICE_JOINT(3) PLK_SLICE_JOINT(4)
+        default: return hipErrorInvalidValue;
+    }
+#undef PLK_SLICE_JOINT
     return hipGetLastError();
 }
 

@@ -433,16 +433,14 @@ __device__ __forceinline__ void points_to_lds(float *lds, const PointRows &rows,
 
 // workgroup (x, y): channels 32 y .. of the points of block x.  Q: pieces of four channels of a workgroup's.
 template <int D1, int Q>
-__global__ __launch_bounds__(kTileThreads) void k_slice_tile_channels(int vd, PointMap map,
-                                                                      const ReplayEntry *__restrict__ replay,
-                                                                      const float *__restrict__ values,
-                                                                      float *__restrict__ output, int normalize,
-                                                                      int n_rows, PointRows rows) {
-    extern __shared__ float4 lds4[];
+__device__ __forceinline__ void slice_channels_of_tile(float *lds, int vd, const PointMap &map,
+                                                       const ReplayEntry *__restrict__ replay,
+                                                       const float *__restrict__ values, float *__restrict__ output,
+                                                       int normalize, int n_rows, PointRows rows, unsigned block,
+                                                       unsigned blocks) {
     __shared__ int n_of[kBlock + 1];
-    float *lds = reinterpret_cast<float *>(lds4);
     unsigned vblock;
-    if (!block_of_points(map, 1, vblock)) return;
+    if (!block_of_points(map, 1, block, blocks, vblock)) return;
     const int tid = threadIdx.x, sub = tid % kTileLanes, point = tid / kTileLanes;
     rows.from = kTileChannels * (int)blockIdx.y;
     if (rows.stride - rows.from < rows.channels) {   // (the last of several workgroups of a tile)
@@ -484,6 +482,27 @@ __global__ __launch_bounds__(kTileThreads) void k_slice_tile_channels(int vd, Po
     }
     __syncthreads();
     store_points(lds, output, rows, n_of);
+}
+template <int D1, int Q>
+__global__ __launch_bounds__(kTileThreads) void k_slice_tile_channels(int vd, PointMap map,
+                                                                      const ReplayEntry *__restrict__ replay,
+                                                                      const float *__restrict__ values,
+                                                                      float *__restrict__ output, int normalize,
+                                                                      int n_rows, PointRows rows) {
+    extern __shared__ float4 lds[];
+    slice_channels_of_tile<D1, Q>(reinterpret_cast<float *>(lds), vd, map, replay, values, output, normalize, n_rows, rows,
+                                  blockIdx.x, gridDim.x);
+}
+// The same for several lattices.
+template <int D1, int Q>
+__global__ __launch_bounds__(kTileThreads) void k_slice_tile_channels_of(Items<PointsWork, kJointItems> items, int vd,
+                                                                         int normalize, int n_rows, PointRows rows) {
+    extern __shared__ float4 lds[];
+    unsigned block, blocks;
+    const PointsWork &work = item_of(items, block, blocks);
+    if (block >= work.map.n_blocks) return;
+    slice_channels_of_tile<D1, Q>(reinterpret_cast<float *>(lds), vd, work.map, work.replay, work.values, work.output,
+                                  normalize, n_rows, rows, block, work.map.n_blocks);
 }
 
 // Q: pieces of four classes
@@ -613,6 +632,39 @@ hipError_t slice_tile_channels(int pd, int vd, const PointMap &map, const Replay
         default: return hipErrorInvalidValue;
     }
 #undef PLK_SLICE_TILE
+    return hipGetLastError();
+}
+
+hipError_t slice_tile_channels_joint(int pd, int vd, int n, const PointsWork *work, int normalize, hipStream_t s) {
+    const int out_ch = normalize ? vd - 1 : vd;
+    if (n < 1 || n > kJointItems || vd < kManyChannels || out_ch > kTileChannels) return hipErrorInvalidValue;
+    Items<PointsWork, kJointItems> items{};
+    items.n = n;
+    for (int i = 0; i < n; ++i) {
+        items.item[i] = work[i];
+        items.blocks[i] = multiple_of_xcds(work[i].map.n_blocks);
+    }
+    const int Q = (out_ch + 3) / 4;
+    const unsigned n_rows = tile_rows(Q);
+    const dim3 grid(all_blocks(items)), block(kTileThreads);
+#define PLK_SLICE_TILE_OF(PD, Q)                                                                                     \
+    case Q:                                                                                                          \
+        hipLaunchKernelGGL((k_slice_tile_channels_of<PD + 1, Q>), grid, block, tile_lds(Q, n_rows), s, items, vd,    \
+                           normalize, (int)n_rows, point_rows(out_ch, out_ch));                                      \
+        break;
+#define PLK_SLICE_TILES(PD)                                                                                          \
+    case PD:                                                                                                         \
+        switch (Q) {                                                                                                 \
+            PLK_SLICE_TILE_OF(PD, 1) PLK_SLICE_TILE_OF(PD, 2) PLK_SLICE_TILE_OF(PD, 3) PLK_SLICE_TILE_OF(PD, 4)      \
+            PLK_SLICE_TILE_OF(PD, 5) PLK_SLICE_TILE_OF(PD, 6) PLK_SLICE_TILE_OF(PD, 7) PLK_SLICE_TILE_OF(PD, 8)      \
+        }                                                                                                            \
+        break;
+    switch (pd) {
+        PLK_SLICE_TILES(2) PLK_SLICE_TILES(3) PLK_SLICE_TILES(4) PLK_SLICE_TILES(5)
+        default: return hipErrorInvalidValue;
+    }
+#undef PLK_SLICE_TILES
+#undef PLK_SLICE_TILE_OF
     return hipGetLastError();
 }
 

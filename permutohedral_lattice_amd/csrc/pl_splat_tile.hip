@@ -29,15 +29,16 @@ constexpr unsigned kSides = 2, kThreads = kSides * kBlock;
 constexpr unsigned kMaxCorners = (kMaxPd + 1 + kSides - 1) / kSides;   // of a thread
 
 template <int K>
-__global__ __launch_bounds__(kThreads) void k_splat_tile(int d1, int vd, PointMap map, const float *__restrict__ input,
-                                                        int in_channels, const ReplayEntry *__restrict__ replay,
-                                                        float *values, int xcd_aware) {
-    extern __shared__ uint2 sorted[];   // [kBlock * d1]: weight, point | slot << 8; then the points' rows
+__device__ __forceinline__ void splat_tile_of(uint2 *sorted, int d1, int vd, const PointMap &map,
+                                              const float *__restrict__ input, int in_channels,
+                                              const ReplayEntry *__restrict__ replay, float *values, int xcd_aware,
+                                              unsigned block, unsigned blocks) {
+    // sorted: [kBlock * d1]: weight, point | slot << 8; then the points' rows
     __shared__ int slot_index[kTileSlots];
     __shared__ unsigned slot_count[kTileSlots];
     __shared__ unsigned wave_pairs[kThreads / 64];
     unsigned vblock;
-    if (!block_of_points(map, xcd_aware, vblock)) return;
+    if (!block_of_points(map, xcd_aware, block, blocks, vblock)) return;
     float *rows = reinterpret_cast<float *>(sorted + (size_t)kBlock * d1);   // [kBlock][in_channels]
     const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
     const int point = tid % kBlock, side = tid / kBlock;   // (its corners: side, side + 2, ...)
@@ -189,6 +190,24 @@ __global__ __launch_bounds__(kThreads) void k_splat_tile(int d1, int vd, PointMa
     }
     add_row(current);
 }
+template <int K>
+__global__ __launch_bounds__(kThreads) void k_splat_tile(int d1, int vd, PointMap map, const float *__restrict__ input,
+                                                        int in_channels, const ReplayEntry *__restrict__ replay,
+                                                        float *values, int xcd_aware) {
+    extern __shared__ uint2 sorted[];
+    splat_tile_of<K>(sorted, d1, vd, map, input, in_channels, replay, values, xcd_aware, blockIdx.x, gridDim.x);
+}
+// The same for several lattices.
+template <int K>
+__global__ __launch_bounds__(kThreads) void k_splat_tiles(Items<PointsWork, kJointItems> items, int d1, int vd,
+                                                         int in_channels, int xcd_aware) {
+    extern __shared__ uint2 sorted[];
+    unsigned block, blocks;
+    const PointsWork &work = item_of(items, block, blocks);
+    if (block >= work.map.n_blocks) return;
+    splat_tile_of<K>(sorted, d1, vd, work.map, work.input, in_channels, work.replay, work.values, xcd_aware, block,
+                     work.map.n_blocks);
+}
 
 }  // namespace
 
@@ -202,6 +221,22 @@ hipError_t splat_tile(int pd, int vd, const PointMap &map, const float *input, i
     const auto kernel = vd <= 16 ? k_splat_tile<1> : k_splat_tile<2>;
     hipLaunchKernelGGL(kernel, dim3(map.n_blocks), dim3(kThreads), lds, s, d1, vd, map, input, in_channels, replay,
                        values, xcd_aware);
+    return hipGetLastError();
+}
+
+hipError_t splat_tile_joint(int pd, int vd, int n, const PointsWork *work, int in_channels, int xcd_aware, hipStream_t s) {
+    if (!splat_tile_takes(vd) || pd < 1 || pd > kMaxPd || in_channels < 1 || in_channels > vd || n < 1 || n > kJointItems)
+        return hipErrorInvalidValue;
+    Items<PointsWork, kJointItems> items{};
+    items.n = n;
+    for (int i = 0; i < n; ++i) {
+        items.item[i] = work[i];
+        items.blocks[i] = multiple_of_xcds(work[i].map.n_blocks);
+    }
+    const int d1 = pd + 1;
+    const size_t lds = kBlock * ((size_t)d1 * sizeof(uint2) + (size_t)in_channels * sizeof(float));
+    const auto kernel = vd <= 16 ? k_splat_tiles<1> : k_splat_tiles<2>;
+    hipLaunchKernelGGL(kernel, dim3(all_blocks(items)), dim3(kThreads), lds, s, items, d1, vd, in_channels, xcd_aware);
     return hipGetLastError();
 }
 
