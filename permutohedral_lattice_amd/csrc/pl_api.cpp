@@ -258,7 +258,8 @@ struct pl_lattice {
     int list_stride() const { return plk::created_list_stride(pd, f64) * (lists_wide ? 2 : 1); }
     plk::CreatedLists lists(int set) const {
         return plk::CreatedLists{created_entries, block_count, chunk_count + (size_t)set * n_chunks,
-                                 list_stride(), map.tile_vertices, false};
+                                 list_stride(), map.tile_vertices, false,
+                                 n_cells >= max_cells ? ~0u : plk::kProbeLimit};
     }
 };
 

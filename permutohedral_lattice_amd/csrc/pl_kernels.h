@@ -172,7 +172,13 @@ struct CreatedLists {
     int stride;
     TileVertices tiles;   // of a merging build
     bool foreign_rows;    // it numbered its vertices and lists such rows
+    // Probes of a key before the build gives up and is repeated with a larger table, where there is one.  In
+    // a table less than three quarters full the chance of a run of a thousand cells is about e^-38; in a
+    // full one every key that does not fit probed all its cells (256x256 points of noise, the first call on
+    // a new lattice: 256 ms, this 4.6).
+    uint32_t probe_limit;
 };
+constexpr uint32_t kProbeLimit = 1024;
 // uint4 a workgroup's part must hold: its 256 * (pd+1) possible vertices, or kTileSlots rows of
 // four values, as many pairs of a cell and a place, and, at tile_table_from, the workgroup's table (which is
 // kept with the replay: no other allocation of megabytes for a new handle)

@@ -396,7 +396,8 @@ __global__ __launch_bounds__(kBlock) void k_build(PointFeatures features, PointM
     if constexpr (!WIDE) {
 #pragma unroll
     for (int r = 0; r < D1; ++r) cell[r] = cell_of_key<PD>(key[r], mask, regions);
-    for (uint32_t probe = 0; any_open && probe <= mask + 2u; ++probe) {
+    const uint32_t limit = created_lists.probe_limit < mask + 2u ? created_lists.probe_limit : mask + 2u;
+    for (uint32_t probe = 0; any_open && probe <= limit; ++probe) {
 #pragma unroll
         for (int r = 0; r < D1; ++r)
             seen[r] = (open >> r) & 1u ? *cell_at(cell_keys, cell[r]) : key[r];
@@ -807,7 +808,8 @@ __device__ __forceinline__ void build_tile(const PointFeatures &features, const 
             pair_index[h] = 0;
         }
         bool any_open = open != 0;
-        for (uint32_t turn = 0; any_open && turn <= 2u * mask + 8u; ++turn) {
+        const uint32_t limit = created_lists.probe_limit < 2u * mask + 8u ? created_lists.probe_limit : 2u * mask + 8u;
+        for (uint32_t turn = 0; any_open && turn <= limit; ++turn) {
 #pragma unroll
             for (int h = 0; h < H; ++h)
                 if ((open >> h) & 1u)
@@ -1243,12 +1245,21 @@ __device__ __forceinline__ void add_foreign_rows(const CreatedLists &lists, unsi
     int *const table = lists.tiles.of(list);
     const int channel = lane & 3;
     // (what bounds this is the atomic unit, a request per row: asking for all rows of the four
-    // lists at once instead of sixteen rows at a time per list made it slower)
-    for (int e = lane >> 2; e < n; e += 16) {
-        const int2 cell = cells[e];   // (and its place in the workgroup's table)
-        const int v = cell_vertex[cell.x];
-        if (channel == 0) table[cell.y] = v;
-        if (channel < vd) atomicAdd(values + (size_t)v * vd + channel, rows[(size_t)e * 4 + channel]);
+    // lists at once instead of sixteen rows at a time per list made it slower.  On a small image it is the
+    // chain, of which the next sixteen's cells and rows are asked for early: 64x64 points 6.9 and 6.4 us.)
+    int e = lane >> 2;
+    int2 cell = cells[e < n ? e : 0];   // (and its place in the workgroup's table)
+    S x = rows[(size_t)(e < n ? e : 0) * 4 + channel];
+    while (e < n) {
+        const int v = cell_vertex[cell.x], place = cell.y;
+        const S sum = x;
+        e += 16;
+        if (e < n) {
+            cell = cells[e];
+            x = rows[(size_t)e * 4 + channel];
+        }
+        if (channel == 0) table[place] = v;
+        if (channel < vd) atomicAdd(values + (size_t)v * vd + channel, sum);
     }
 }
 
@@ -1313,6 +1324,10 @@ __device__ __forceinline__ void find_neighbours(const VertexTables &vertices, co
         }
         return;
     }
+    // (a build that is repeated: in a full table a key that is not there is looked for in every cell.  Eight
+    // images of 256x256 points of noise, whose first tables are a sixth of what they need: minutes.  Asked here,
+    // looked at behind the first keys: a return here waits for it, 1.5 us a launch.)
+    const int given_up = counters->flags & (kFlagTableFull | kFlagTileFull | kFlagKeyRange);
     const KeyRegions regions{counters->region_lo, counters->region_per_unit};
     const int max_vertices = vertices.max_vertices;
     SegmentWalk walk(counters, max_vertices, block - tile_blocks, blocks - tile_blocks);
@@ -1341,7 +1356,7 @@ __device__ __forceinline__ void find_neighbours(const VertexTables &vertices, co
     if constexpr (WIDE) {
         const Key128 want = WideCodec<PD>::pack(qp, wrap_up ? 0 : r + 1);
         uint32_t h = hash_key(want) & mask;
-        for (uint32_t index = 0; index <= mask; ++index) {
+        for (uint32_t index = 0; !given_up && index <= mask; ++index) {
             const ulonglong2 cur = reinterpret_cast<const ulonglong2 *>(cell_keys)[h];
             if (cur.x == want.a && cur.y == want.b) {
                 u = vertices.cell_vertex[h];
@@ -1353,6 +1368,7 @@ __device__ __forceinline__ void find_neighbours(const VertexTables &vertices, co
     }
     const uint64_t want = WIDE ? 0ull : KeyCodec<PD>::pack(qp, wrap_up ? 0 : r + 1);
     uint32_t h = WIDE ? 0u : cell_of_key<PD>(want, mask, regions);
+    if (given_up) return;
     for (uint32_t index = 0; !WIDE && index <= (mask >> 1) + 1u; ++index) {
         const ulonglong2 cur = *reinterpret_cast<const ulonglong2 *>(cell_keys + h);
         if (cur.x == want || (cur.x != kEmptyCell && cur.y == want)) {

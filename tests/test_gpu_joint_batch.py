@@ -106,3 +106,20 @@ def test_what_is_refused():
     torch.cuda.synchronize()
     for lat in (a, b, other):
         lat.close()
+
+
+def test_noise_meets_a_table_that_is_far_too_small():
+    """A build gives up on its table long before every key has seen all of its cells, and the results are
+    those of the largest table."""
+    h = w = 96
+    gen = torch.Generator(device="cuda").manual_seed(1)
+    pos = torch.rand((h * w, 5), generator=gen, device="cuda") * 200.0 - 100.0
+    val = torch.rand((h * w, 3), generator=gen, device="cuda")
+    out, want = torch.empty_like(val), torch.empty_like(val)
+    for cells, into in ((4096, out), (131072, want)):
+        lat = pla.PermutohedralLattice(5, 4, h * w)
+        lat.set_option(pla.PL_OPT_TABLE_CELLS, cells)
+        lat.filter(into, val, pos)
+        assert lat.num_vertices > 50000
+        lat.close()
+    close(out, want)
