@@ -2121,10 +2121,13 @@ extern "C" int pl_mean_field_infer(int n, const pl_handle *bilateral, const pl_h
 namespace {
 
 // With the default allocator the op keeps its lattices between calls (per device, shape and
-// stream), because hipMalloc/hipFree per call would serialise the device.  A batch is spread
-// over up to g_op_lanes lattices, the first on the caller's stream, the others on streams of
-// their own: the items are independent lattices (LatticeFilterKernel.cpp:152-179), and the
-// kernels over the few hundred thousand vertices of one item leave most of the GPU idle.
+// stream), because hipMalloc/hipFree per call would serialise the device.  The items of a batch are independent
+// lattices (LatticeFilterKernel.cpp:152-179), and the kernels over the few hundred thousand vertices of one item
+// leave most of the GPU idle, so up to g_op_lanes items are in flight at a time: their passes enqueued together
+// on the caller's stream (pl_filter_images) where there are kernels for it, else on lattices with streams of
+// their own, the first on the caller's.  us a call, on streams and together, RGB under itself: 2 x 64x64
+// points 101 and 39, 2 x 512x512 101 and 70, 8 x 256x256 228 and 118, 2 x 1024x1024 221 and 179; 2 x 321x481,
+// 21 channels, 128 and 122.
 // With a caller-supplied allocator everything is taken from it and returned before the call
 // ends, as the reference does with TensorFlow temporaries (src/DeviceMemoryAllocator.h:52-71),
 // and the items run one after the other.
@@ -2139,6 +2142,9 @@ struct OpCacheEntry {
     hipStream_t stream;
     bool f64;                       // lattices of doubles
     std::vector<OpLane> lanes;
+    std::vector<pl_handle> joint;   // behind lanes[0], on the caller's stream: items whose passes go together
+    // calls that go on streams after one whose builds could not all be merged (as pl_lattice::tiles_off_for)
+    int joint_off_for = 0;
     hipEvent_t fork = nullptr;
     double *positions64 = nullptr;  // [N*pd], the positions of the item being filtered (doubles only)
 };
@@ -2154,6 +2160,8 @@ void destroy_entry(OpCacheEntry &e) {
         if (lane.done) (void)hipEventDestroy(lane.done);
         if (lane.owns_stream && lane.stream) (void)hipStreamDestroy(lane.stream);
     }
+    for (pl_handle h : e.joint) pl_destroy(h);
+    e.joint.clear();
     if (e.fork) (void)hipEventDestroy(e.fork);
     if (e.positions64) (void)hipFree(e.positions64);
     e.positions64 = nullptr;
@@ -2170,7 +2178,7 @@ OpCacheEntry *op_cache_entry(int device, int pd, int vd, int N, hipStream_t stre
         destroy_entry(g_op_cache.front());
         g_op_cache.erase(g_op_cache.begin());
     }
-    g_op_cache.push_back(OpCacheEntry{device, pd, vd, N, stream, f64, {}, nullptr, nullptr});
+    g_op_cache.push_back(OpCacheEntry{device, pd, vd, N, stream, f64, {}, {}, 0, nullptr, nullptr});
     return &g_op_cache.back();
 }
 
@@ -2196,6 +2204,36 @@ int ensure_lanes(OpCacheEntry &e, int want) {
         e.lanes.push_back(lane);
     }
     if (want > 1 && !e.fork) PL_HIP(hipEventCreateWithFlags(&e.fork, hipEventDisableTiming));
+    return PL_OK;
+}
+
+// The items of a batch, n_lanes at a time, their passes together on the entry's stream.
+int filter_items_together(OpCacheEntry &e, int n_lanes, const float *input, const float *reference, float *output,
+                          int batch, int n_spatial_dims, const int *spatial_dims, int channels, int ref_ch,
+                          float spatial_std, float feature_std, int reverse) {
+    int rc = ensure_lanes(e, 1);
+    if (rc != PL_OK) return rc;
+    while ((int)e.joint.size() < n_lanes - 1) {
+        pl_handle h = nullptr;
+        rc = pl_create(e.pd, e.vd, e.N, (pl_stream)e.stream, nullptr, &h);
+        if (rc != PL_OK) return rc;
+        e.joint.push_back(h);
+    }
+    pl_handle lattices[kOpLanesMax] = {e.lanes[0].lattice};
+    for (int i = 1; i < n_lanes; ++i) lattices[i] = e.joint[i - 1];
+    const size_t N = (size_t)e.N;
+    for (int b = 0; b < batch; b += n_lanes) {
+        const int count = batch - b < n_lanes ? batch - b : n_lanes;
+        rc = pl_filter_images(count, lattices, output + (size_t)b * N * channels, input + (size_t)b * N * channels,
+                              ref_ch ? reference + (size_t)b * N * ref_ch : nullptr, ref_ch, n_spatial_dims, spatial_dims,
+                              spatial_std, feature_std, reverse);
+        if (rc != PL_OK) return rc;
+    }
+    for (int i = 0; i < n_lanes; ++i) {
+        const int off = lattices[i]->last_build_merged ? 0
+                        : lattices[i]->tiles_off_for > lattices[i]->wide_for ? lattices[i]->tiles_off_for : lattices[i]->wide_for;
+        if (off > e.joint_off_for) e.joint_off_for = off;
+    }
     return PL_OK;
 }
 
@@ -2254,6 +2292,13 @@ extern "C" int pl_lattice_filter_op(const float *input, const float *reference, 
     // 1.32 ms for one / two / four at a time).
     int n_lanes = batch < g_op_lanes ? batch : g_op_lanes;
     if (N > (1 << 19) && n_lanes > 2) n_lanes = 2;
+    if (n_lanes > 1 && plk::joint_takes(pd, vd) && plk::make_point_map(N, n_spatial_dims, spatial_dims).mode >= 2) {
+        if (entry->joint_off_for == 0)
+            return filter_items_together(*entry, n_lanes, input, reference, output, batch, n_spatial_dims, spatial_dims,
+                                         n_input_channels, ref_ch, spatial_std, feature_std, reverse);
+        if (--entry->joint_off_for == 0)
+            for (pl_handle h : entry->joint) h->tiles_off_for = h->wide_for = 0;
+    }
     int rc = ensure_lanes(*entry, n_lanes);
     if (rc != PL_OK) return rc;
 

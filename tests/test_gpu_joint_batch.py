@@ -108,6 +108,22 @@ def test_what_is_refused():
         lat.close()
 
 
+@pytest.mark.parametrize("batch,channels,guide", [(2, 3, 3), (5, 1, 3), (3, 21, 3), (9, 3, 0)])
+def test_the_op_on_batches(batch, channels, guide):
+    """Together, on streams after an image that a merging build cannot take, and together again (32 calls on)."""
+    gen = torch.Generator(device="cuda").manual_seed(batch)
+    sides = (29, 52)
+    thetas = dict(bilateral=guide > 0, theta_alpha=6.0, theta_beta=0.4, theta_gamma=5.0)
+    for call in range(37):
+        kinds = ["wild" if call == 1 and b == batch - 1 else "noisy" if b % 3 == 1 else "smooth" for b in range(batch)]
+        ref = torch.stack([guide_of(sides, guide, kind, gen) for kind in kinds]) if guide else None
+        x = torch.rand((batch,) + sides + (channels,), generator=gen, device="cuda")
+        out = pla.lattice_filter(x, ref, **thetas)
+        if call in (0, 1, 2, 3, 33, 34, 35, 36):
+            for b in range(batch):
+                close(out[b:b + 1], pla.lattice_filter(x[b:b + 1], None if ref is None else ref[b:b + 1], **thetas))
+
+
 def test_noise_meets_a_table_that_is_far_too_small():
     """A build gives up on its table long before every key has seen all of its cells, and the results are
     those of the largest table."""
