@@ -1978,8 +1978,10 @@ __global__ __launch_bounds__(kBlock) void k_blur3_row(const Counters *counters, 
     }
 }
 
-// One, two or three axes (nbr_third: rows of up to four channels where three are all there are) of several lattices.
-template <int VD>
+// One or two axes, or (THREE) three where they are all there are, of several lattices.  (The three axes' 27 rows
+// need registers for three wavefronts a SIMD; as a branch beside the others, two axes of 4 x 182 000 vertices of
+// two channels 12.5 us, this 11.7; an op on 4 x 1024x1024 points, RGB, 381 and 370.)
+template <int VD, bool THREE>
 __global__ __launch_bounds__(kBlock) void k_blur_rows_of(Items<BlurWork, kJointItems> items) {
     unsigned block, blocks;
     const BlurWork &work = item_of(items, block, blocks);
@@ -1991,7 +1993,7 @@ __global__ __launch_bounds__(kBlock) void k_blur_rows_of(Items<BlurWork, kJointI
         const unsigned i = vb * kBlock + threadIdx.x;
         if (i >= walk.count) continue;
         const int v = (int)(walk.first + i);
-        if (work.nbr_third) {
+        if constexpr (THREE) {
             int u[27];
             three_axis_sources(work.nbr_first, work.nbr_second, work.nbr_third, v, u);
             ValueRow<VD> row[27], after_a[9];
@@ -3061,7 +3063,10 @@ hipError_t blur_joint(int vd, int n, const BlurWork *work, hipStream_t s) {
         items.item[i] = work[i];
         items.blocks[i] = vertex_blocks((size_t)work[i].launch_vertices);
     }
-    const auto kernel = vd == 2 ? k_blur_rows_of<2> : vd == 3 ? k_blur_rows_of<3> : k_blur_rows_of<4>;
+    const auto kernel = work[0].nbr_third ? (vd == 2   ? k_blur_rows_of<2, true>
+                                             : vd == 3 ? k_blur_rows_of<3, true> : k_blur_rows_of<4, true>)
+                                          : (vd == 2   ? k_blur_rows_of<2, false>
+                                             : vd == 3 ? k_blur_rows_of<3, false> : k_blur_rows_of<4, false>);
     hipLaunchKernelGGL(kernel, dim3(all_blocks(items)), dim3(kBlock), 0, s, items);
     return hipGetLastError();
 }
