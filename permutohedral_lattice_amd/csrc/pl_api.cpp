@@ -135,6 +135,9 @@ struct pl_lattice {
 
     plk::Counters *d_counters = nullptr;   // two sets, used by alternate builds
     int counter_set = 0;                   // the set of the last build
+    // The kernels of a build leave the other set of counters zero, and the other set of chunk sums as
+    // chunk_count_clean says.  false: a build was prepared of which not every kernel has been enqueued.
+    bool counts_clean = true;
     plk::HostStatus *h_status = nullptr;   // pinned, written by the device
     unsigned status_sequence = 0;          // the number of the last build enqueued: what its report carries
     // a lattice in the library's static scratch (pl_filter_static) owns no pinned memory and no
@@ -460,6 +463,7 @@ struct BuildPlan {
 };
 
 // Makes the lattice's arrays ready for a build with a table of `cells` cells.  Nothing here waits for the device.
+// (Of lattices built together the memory of a later one may be refused: then this build is not enqueued.)
 // splat_input != nullptr: the build kernel also splats these values (when it can for this vd),
 // and the value table holds them when the build is done.
 // A lattice for double values takes its positions from positions64 and never splats in the build.
@@ -519,8 +523,14 @@ int prepare_build(pl_lattice *h, const plk::PointFeatures &features, const doubl
     h->stage_ran[1] = true;
     h->stage_ran[2] = !numbers_in_build;
     h->stage_ran[3] = true;
-    // the previous vertex-numbering kernel (or pl_create) left the other counter set zeroed
+    // the last build's kernels (or pl_create) left the other counter set zeroed, if they were enqueued
     const int previous_set = h->counter_set;
+    if (!h->counts_clean) {
+        PL_HIP(plk::fill_zero(reinterpret_cast<float *>(h->d_counters), 2 * sizeof(plk::Counters) / sizeof(float), h->stream));
+        PL_HIP(plk::fill_zero(reinterpret_cast<float *>(h->chunk_count), 2 * h->n_chunks, h->stream));
+        h->chunk_count_clean[0] = h->chunk_count_clean[1] = true;
+    }
+    h->counts_clean = false;   // (until build_enqueued)
     h->list_counted = -1;
     if (h->map.mode == 1) {
         const plk::LocalityTable counting{h->bin_table, &h->d_counters[1 - previous_set].order_tally,
@@ -589,6 +599,7 @@ int prepare_build(pl_lattice *h, const plk::PointFeatures &features, const doubl
 
 // What is known of the lattice when its build's kernels are enqueued
 void build_enqueued(pl_lattice *h, const BuildPlan &plan) {
+    h->counts_clean = true;
     h->replay_holds_cells = !plan.merge;
     h->values_zeroed = !plan.fused;
     h->values_splatted = plan.fused;

@@ -96,6 +96,16 @@ bool launched(const char *name) {
 plk::Points64 g_points64;             // of the last build of doubles
 const float *g_values[2];             // value tables of the lattice blurred last in a joint pass
 
+// What a build counts in must be zero when it starts (it and the passes behind it then zero the other set)
+void count_in(plk::Counters *counters, const plk::CreatedLists &lists) {
+    static const plk::Counters zero{};
+    expect(std::memcmp(counters, &zero, sizeof(zero)) == 0, "a build counts in counters that are not zero");
+    counters->vertices = counters->segment_count[0].n = 100;
+    if (lists.foreign_rows) return;
+    expect(lists.chunk_count[0] == 0, "a build counts in chunk sums that are not zero");
+    lists.chunk_count[0] = 100;
+}
+
 void report(plk::HostReport to) {
     to.status->num_vertices = 100;
     to.status->flags = 0;
@@ -178,11 +188,30 @@ size_t vertex_list_max_long(size_t rows) { return rows; }
 bool slice_pairs_take(int, int, int) { return true; }
 
 hipError_t clear_table(uint64_t *keys, uint32_t, hipStream_t s) { return launch("clear_table", s, {}, {keys}); }
-hipError_t fill_zero(float *p, size_t, hipStream_t s) { return launch("fill_zero", s, {}, {p}); }
+hipError_t fill_zero(float *p, size_t n, hipStream_t s) {
+    const hipError_t e = launch("fill_zero", s, {}, {p});
+    if (e == hipSuccess) std::memset(p, 0, n * sizeof(float));
+    return e;
+}
+hipError_t fill_ranges(FillRanges ranges, hipStream_t s) {
+    std::vector<const void *> written;
+    for (const auto &r : ranges.range) written.push_back(r.words_at);
+    return launch("fill_ranges", s, {}, written);
+}
 hipError_t build(int, const PointFeatures &, const PointMap &, const ScaleFactor &, uint64_t *keys, uint32_t,
-                 Counters *, ReplayEntry *replay, int, int, const float *, int, float *, const CreatedLists &,
+                 Counters *counters, ReplayEntry *replay, int, int, const float *, int, float *, const CreatedLists &lists,
                  const RegionSource &, const InBuildNumbering *, bool, hipStream_t s) {
-    return launch("build", s, {}, {keys, replay});
+    const hipError_t e = launch("build", s, {}, {keys, replay});
+    if (e == hipSuccess) count_in(counters, lists);
+    return e;
+}
+hipError_t build_joint(int, int n, const BuildWork *work, const ScaleFactor &, int, int, int, hipStream_t s) {
+    hipError_t e = hipSuccess;
+    for (int i = 0; i < n && e == hipSuccess; ++i) {
+        e = launch("build_joint", s, {}, {work[i].cell_keys, work[i].replay});
+        if (e == hipSuccess) count_in(work[i].counters, work[i].lists);
+    }
+    return e;
 }
 hipError_t build_f64(int, const Points64 &points, const PointMap &, uint64_t *keys, uint32_t, Counters *,
                      ReplayEntry *replay, int, const CreatedLists &, const RegionSource &, const InBuildNumbering *,
@@ -190,16 +219,37 @@ hipError_t build_f64(int, const Points64 &points, const PointMap &, uint64_t *ke
     g_points64 = points;
     return launch("build_f64", s, {}, {keys, replay});
 }
-hipError_t number_vertices(int, const PointMap &, const CreatedLists &, int *, unsigned, const VertexTables &,
-                           float *values, int, float *, Counters *, Counters *, HostReport to, bool, hipStream_t s) {
+hipError_t number_vertices(int, const PointMap &, const CreatedLists &, int *next_chunk_count, unsigned n_chunks,
+                           const VertexTables &, float *values, int, float *, Counters *, Counters *next_counters,
+                           HostReport to, bool, hipStream_t s) {
     report(to);
+    *next_counters = Counters{};
+    std::memset(next_chunk_count, 0, n_chunks * sizeof(int));
     return launch("number_vertices", s, {}, {values});
 }
+hipError_t number_vertices_joint(int pd, int n, const BuildWork *work, int vd, hipStream_t s) {
+    hipError_t e = hipSuccess;
+    for (int i = 0; i < n && e == hipSuccess; ++i)
+        e = number_vertices(pd, work[i].map, work[i].lists, work[i].next_chunk_count, work[i].n_chunks, work[i].vertices,
+                            work[i].values, vd, nullptr, work[i].counters, work[i].next_counters, work[i].report_to, false, s);
+    return e;
+}
 hipError_t neighbours(int, const VertexTables &vertices, const Counters *, const uint64_t *keys, uint32_t, int,
-                      const CreatedLists *, unsigned, void *values, int, bool, Counters *to_report, Counters *,
-                      HostReport to, bool, hipStream_t s) {
-    if (to_report) report(to);
+                      const CreatedLists *, unsigned, void *values, int, bool, Counters *to_report,
+                      Counters *next_counters, HostReport to, bool, hipStream_t s) {
+    if (to_report) {
+        report(to);
+        *next_counters = Counters{};
+    }
     return launch("neighbours", s, {keys}, {vertices.neighbours, values});
+}
+hipError_t neighbours_joint(int pd, int n, const BuildWork *work, int vd, hipStream_t s) {
+    hipError_t e = hipSuccess;
+    for (int i = 0; i < n && e == hipSuccess; ++i)
+        e = neighbours(pd, work[i].vertices, work[i].counters, work[i].cell_keys, 0, 0, nullptr, 0, work[i].values, vd, false,
+                       work[i].numbering.n_segments ? work[i].counters : nullptr, work[i].next_counters, work[i].report_to,
+                       false, s);
+    return e;
 }
 hipError_t build_vertex_lists(int, const PointMap &, ReplayEntry *replay, const int *, int, const VertexLists &lists,
                               unsigned *info, unsigned sequence, hipStream_t s) {
@@ -216,6 +266,23 @@ hipError_t splat_gather_many(int, int, int n, const GatherWork *work, hipStream_
     hipError_t e = hipSuccess;
     for (int i = 0; i < n && e == hipSuccess; ++i)
         e = launch("splat_gather_many", s, {work[i].entries, work[i].input}, {work[i].values});
+    return e;
+}
+hipError_t splat_tile(int, int, const PointMap &, const float *input, int, ReplayEntry *replay, const int *, float *values,
+                      int, hipStream_t s) {
+    return launch("splat_tile", s, {input, replay}, {values});
+}
+hipError_t splat_joint(int, int, int n, const PointsWork *work, int, int, hipStream_t s) {
+    hipError_t e = hipSuccess;
+    for (int i = 0; i < n && e == hipSuccess; ++i)
+        e = launch("splat_joint", s, {work[i].input, work[i].replay}, {work[i].values});
+    return e;
+}
+hipError_t blur_joint(int vd, int n, const BlurWork *work, hipStream_t s) { return blur_many(vd, n, work, s); }
+hipError_t slice_joint(int, int, int n, const PointsWork *work, int, hipStream_t s) {
+    hipError_t e = hipSuccess;
+    for (int i = 0; i < n && e == hipSuccess; ++i)
+        e = launch("slice_joint", s, {work[i].replay, work[i].values}, {work[i].output});
     return e;
 }
 hipError_t splat_f64(int, int, const PointMap &, const double *input, int, ReplayEntry *replay, const double *,
@@ -449,6 +516,47 @@ void no_pointer_kept() {
     expect(g_points64.positions && !g_points64.reference, "the reference image of a call that has returned");
 }
 
+// a batch that cannot be enqueued whole -- the memory of one of its lattices is refused, or a launch fails --
+// leaves lattices whose next builds are like any other
+bool g_refuse = false;
+void *alloc_if_allowed(void *, size_t bytes) { return g_refuse ? nullptr : std::calloc(1, bytes); }
+void free_any(void *, void *p) { std::free(p); }
+void failed_batch() {
+    const hipStream_t s = named_stream(1);
+    const int dims[2] = {kH, kW};
+    const pl_alloc alloc{alloc_if_allowed, free_any, nullptr};
+    for (const int channels : {3, kClasses}) {
+        const size_t bytes = sizeof(float) * 2 * kH * kW * kClasses;
+        float *in = nullptr, *out = nullptr, *guide = nullptr;
+        for (float **p : {&in, &out, &guide}) (void)hipMalloc((void **)p, bytes);
+        pl_handle h[2];
+        expect(pl_create(5, channels + 1, kH * kW, s, nullptr, &h[0]) == PL_OK, "pl_create");
+        expect(pl_create(5, channels + 1, kH * kW, s, &alloc, &h[1]) == PL_OK, "pl_create");
+        auto alone = [&](int i) { return pl_filter_image(h[i], out, in, guide, 3, 2, dims, 8.0f, 0.1f, 0); };
+        auto together = [&]() { return pl_filter_images(2, h, out, in, guide, 3, 2, dims, 8.0f, 0.1f, 0); };
+        expect(alone(0) == PL_OK && alone(0) == PL_OK, "the first");
+        g_refuse = true;
+        for (int turn = 0; turn < 3; ++turn) {
+            expect(together() == PL_ENOMEM, "a batch without the memory for its second lattice");
+            if (turn != 1) expect(alone(0) == PL_OK, "the first after it");
+        }
+        g_refuse = false;
+        expect(together() == PL_OK && together() == PL_OK, "the batch with memory");
+        for (const char *launch : {"build_joint", "neighbours", "blur_many", "slice_joint"}) {
+            g_fail_next = launch;
+            expect(together() == PL_EHIP, std::string(launch) + " failed");
+            expect(alone(1) == PL_OK && together() == PL_OK && alone(0) == PL_OK, std::string("after ") + launch);
+        }
+        for (const char *launch : {"build", "neighbours", "blur_two_axes"}) {
+            g_fail_next = launch;
+            expect(alone(0) == PL_EHIP, std::string(launch) + " failed");
+            expect(alone(0) == PL_OK && together() == PL_OK, std::string("after ") + launch);
+        }
+        for (const pl_handle l : h) (void)pl_destroy(l);
+        g_arrays.clear();
+    }
+}
+
 }  // namespace
 
 int main(int argc, char **argv) {
@@ -462,6 +570,7 @@ int main(int argc, char **argv) {
         {"own_stream_captured", own_stream_captured},
         {"failed_blur", failed_blur},
         {"no_pointer_kept", no_pointer_kept},
+        {"failed_batch", failed_batch},
     };
     const auto found = scenarios.find(argc > 1 ? argv[1] : "");
     if (found == scenarios.end()) {

@@ -183,3 +183,53 @@ def test_double_op_with_caller_scratch_returns_everything_before_it_returns():
         assert rc in (pla.PL_ENOMEM, pla.PL_OK)
         assert not short.live and short.n_free == short.n_alloc
     assert rc == pla.PL_ENOMEM      # eleven allocations are not enough for a lattice
+
+
+@pytest.mark.parametrize("channels", [3, 6])
+def test_a_batch_that_one_lattice_has_no_memory_for(channels):
+    """Its other lattice, and both together once there is memory again, filter as if it had not been tried."""
+    h, w = 72, 64
+    n, vd, lib = h * w, channels + 1, pla._lib
+    guides = np.stack([synth.blob_image(h, w, seed=95 + i) for i in range(2)])
+    values = synth.uniform_image((2, n, channels), 97)
+    lattices = [oracle.Lattice(5, vd, n) for _ in range(2)]
+    want = np.stack([lat.filter(x, synth.bilateral_positions(g, 8.0, 0.125), False)
+                     for lat, x, g in zip(lattices, values, guides)])
+    scratch, handles = TorchScratch(), (C.c_void_p * 2)()
+    for i, alloc in enumerate((None, C.byref(scratch.struct))):
+        handle = C.c_void_p()
+        assert lib.pl_create(5, vd, n, None, alloc, C.byref(handle)) == pla.PL_OK
+        handles[i] = handle.value
+    d_ref, d_val = dev(guides), dev(values)
+    out, dims = torch.empty_like(d_val), (C.c_int * 2)(h, w)
+
+    def call(images, *args):
+        out.fill_(float("nan"))
+        torch.cuda.synchronize()
+        return images(*args, out.data_ptr(), d_val.data_ptr(), d_ref.data_ptr(), 3, 2, dims, 8.0, 0.125, 0)
+
+    def check(count):
+        torch.cuda.synchronize()
+        got = out.cpu().numpy()
+        for i in range(count):
+            assert np.abs(got[i] - want[i]).max() <= MAX_ABS_TOL and rel_l2(got[i], want[i]) <= REL_L2_TOL
+            vertices = C.c_int()
+            assert lib.pl_num_vertices(handles[i], C.byref(vertices)) == pla.PL_OK
+            assert vertices.value == lattices[i].num_vertices
+
+    assert call(lib.pl_filter_image, handles[0]) == pla.PL_OK
+    check(1)
+    scratch.fail_after = scratch.n_alloc
+    for alone_behind in (True, False, True):
+        assert call(lib.pl_filter_images, 2, handles) == pla.PL_ENOMEM
+        if alone_behind:
+            assert call(lib.pl_filter_image, handles[0]) == pla.PL_OK
+            check(1)
+    assert call(lib.pl_filter_images, 2, handles) == pla.PL_ENOMEM
+    scratch.fail_after = None
+    for _ in range(2):
+        assert call(lib.pl_filter_images, 2, handles) == pla.PL_OK
+        check(2)
+    for handle in handles:
+        assert lib.pl_destroy(handle) == pla.PL_OK
+    assert not scratch.live
