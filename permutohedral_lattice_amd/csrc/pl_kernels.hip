@@ -1054,9 +1054,12 @@ __device__ __forceinline__ void build_tile(const PointFeatures &features, const 
     }
 }
 
-// (at most 102 scalar registers: with more a SIMD holds seven wavefronts, not eight)
+// At most 96 scalar registers, those the compiler adds for itself among them: they are given out sixteen at a time,
+// and of wavefronts with 112 a SIMD holds seven, not eight.  us a launch with a limit of 102 (99 and 100 used) and
+// with this one: 557x811 points pd 2 vd 2 16.9 and 14.8, 1024x1024 27.1 and 25.7, RGB under itself 53.0 and 50.3;
+// 64x64, where it only costs a few moves of registers, 17.1 and 17.2.
 template <int PD, int SPLAT_VD, typename T = float>
-__global__ __launch_bounds__(kBlock) __attribute__((amdgpu_num_sgpr(102))) void k_build_tile(
+__global__ __launch_bounds__(kBlock) __attribute__((amdgpu_num_sgpr(96))) void k_build_tile(
     PointFeatures features, PointMap map, ScaleFactor scale, uint64_t *cell_keys, uint32_t mask, Counters *counters,
     ReplayEntry *__restrict__ replay, int xcd_aware, const void *__restrict__ input_any, int in_channels,
     void *cell_values_any, CreatedLists created_lists, Points64 points64, RegionSource region_source,
@@ -1066,7 +1069,7 @@ __global__ __launch_bounds__(kBlock) __attribute__((amdgpu_num_sgpr(102))) void 
 }
 // The same for several lattices of floats.
 template <int PD, int SPLAT_VD>
-__global__ __launch_bounds__(kBlock) __attribute__((amdgpu_num_sgpr(102))) void k_build_tiles(
+__global__ __launch_bounds__(kBlock) __attribute__((amdgpu_num_sgpr(96))) void k_build_tiles(
     Items<BuildWork, kJointItems> items, ScaleFactor scale, int xcd_aware, int in_channels) {
     unsigned block, blocks;
     const BuildWork &work = item_of(items, block, blocks);
