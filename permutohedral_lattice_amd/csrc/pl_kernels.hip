@@ -1237,32 +1237,33 @@ __global__ __launch_bounds__(64) void k_number_vertices_of(Items<BuildWork, kJoi
 // 8, or 0) take four workgroups' tables each, one per wavefront, and put vertices in the place of hash
 // cells; where the build numbered its vertices and splatted, they add the rows of sums that it holds for
 // vertices of other workgroups to the value table, a row per group of four lanes.  S: the value type.
+// What bounds it is the chain and, on a large image, the atomic unit (a request per row).  A wavefront's loads wait
+// for the stores and atomics before them, so a round looks up 64 rows' vertices, a lane a row, and only then
+// adds the rows, sixteen at a time.  us a launch, rounds of 16 rows and of 64: RGB under itself 64x64 points 6.6 and
+// 5.3, 181x181 7.9 and 6.5, 700x700 12.6 and 11.3, 1000x900 17.3 and 17.8, 1024x1024 19.4 and 19.9; an op's batch of
+// 4 x 512x512 23.4 and 21.5, 4 x 1024x1024 76.2 and 73.8.
 template <typename S>
 __device__ __forceinline__ void add_foreign_rows(const CreatedLists &lists, unsigned list, int vd,
                                                  const int *__restrict__ cell_vertex, S *values) {
-    const int lane = threadIdx.x & 63;
+    const int lane = threadIdx.x & 63, channel = lane & 3;
     const int n = lists.block_count[list];
     const uint4 *part = lists.entries + (size_t)list * (size_t)lists.stride;
     const S *rows = reinterpret_cast<const S *>(part);
     const int2 *cells = reinterpret_cast<const int2 *>(part + kTileSlots * (sizeof(S) / sizeof(float)));
     int *const table = lists.tiles.of(list);
-    const int channel = lane & 3;
-    // (what bounds this is the atomic unit, a request per row: asking for all rows of the four
-    // lists at once instead of sixteen rows at a time per list made it slower.  On a small image it is the
-    // chain, of which the next sixteen's cells and rows are asked for early: 64x64 points 6.9 and 6.4 us.)
-    int e = lane >> 2;
-    int2 cell = cells[e < n ? e : 0];   // (and its place in the workgroup's table)
-    S x = rows[(size_t)(e < n ? e : 0) * 4 + channel];
-    while (e < n) {
-        const int v = cell_vertex[cell.x], place = cell.y;
-        const S sum = x;
-        e += 16;
-        if (e < n) {
-            cell = cells[e];
-            x = rows[(size_t)e * 4 + channel];
+    int2 cell = cells[lane < n ? lane : 0];   // (and its place in the workgroup's table)
+    for (int i0 = 0; i0 < n; i0 += 64) {
+        const int i = i0 + lane, place = cell.y, vertex = cell_vertex[cell.x];
+        int e = i0 + (lane >> 2);
+        S x = rows[(size_t)(e < n ? e : i0) * 4 + channel];
+        if (i0 + 64 < n) cell = cells[i + 64 < n ? i + 64 : i0];
+        for (int k = 0; k < 64 && i0 + k < n; k += 16, e += 16) {
+            const int v = __shfl(vertex, k + (lane >> 2));
+            const S sum = x;
+            if (k + 16 < 64 && e + 16 < n) x = rows[(size_t)(e + 16) * 4 + channel];
+            if (e < n && channel < vd) atomicAdd(values + (size_t)v * vd + channel, sum);
         }
-        if (channel == 0) table[place] = v;
-        if (channel < vd) atomicAdd(values + (size_t)v * vd + channel, sum);
+        if (i < n) table[place] = vertex;
     }
 }
 
