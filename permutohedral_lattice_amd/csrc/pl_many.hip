@@ -238,9 +238,15 @@ struct Tile {
     float *rows, *last;   // in LDS: Q pieces of four channels, row_stride(Q) floats apart; the homogeneous channels
 };
 __host__ __device__ constexpr int row_stride(int Q) { return 4 * (Q | 1); }
-// Rows in LDS: with 28 KB a CU holds four workgroups, 32 wavefronts, and of 21 channels a workgroup 247 rows
-inline unsigned tile_rows(int Q) {
-    const unsigned rows = (28u << 10) / (sizeof(float) * (unsigned)(row_stride(Q) + 1));
+// Rows in LDS.  A CU holds four workgroups of these kernels, three of pairs (`per_cu`), whatever LDS each takes up to
+// its share of the CU's, and a launch of fewer workgroups leaves more to each: at 21 channels 335 rows (453 of
+// pairs) and up to all 512, where 28 KB a workgroup were 247.  us an apply, 28 KB and this, crowded tiles (pd 5,
+// 8 corners a vertex): vd 22 64x64 22.1 and 20.8, 321x481 71.4 and 67.6; vd 32 64x64 23.2 and 20.2, 1024x1024 473 and 440;
+// pairs of 2 x 512x512 points, 21 classes, a slice 47.2 and 42.6.  (64 KB at most: what a launch may ask for anywhere.)
+inline unsigned tile_rows(int Q, unsigned workgroups, unsigned per_cu) {
+    const unsigned a_cu = (workgroups + 255u) / 256u, at_once = a_cu < per_cu ? a_cu : per_cu;
+    const unsigned share = (160u << 10) / (at_once ? at_once : 1u), lds = (share < 64u << 10 ? share : 64u << 10) - 2048u;
+    const unsigned rows = lds / (sizeof(float) * (unsigned)(row_stride(Q) + 1));
     return rows < (unsigned)kTileSlots ? rows : (unsigned)kTileSlots;
 }
 // (what the rows leave takes the 256 points' channels later)
@@ -442,7 +448,7 @@ __device__ __forceinline__ void slice_channels_of_tile(float *lds, int vd, const
     unsigned vblock;
     if (!block_of_points(map, 1, block, blocks, vblock)) return;
     const int tid = threadIdx.x, sub = tid % kTileLanes, point = tid / kTileLanes;
-    rows.from = kTileChannels * (int)blockIdx.y;
+    rows.from = rows.channels * (int)blockIdx.y;
     if (rows.stride - rows.from < rows.channels) {   // (the last of several workgroups of a tile)
         rows.channels = rows.stride - rows.from;
         rows.per_channel = ((1u << 20) + (unsigned)rows.channels - 1u) / (unsigned)rows.channels;
@@ -616,10 +622,11 @@ hipError_t slice_tile_channels(int pd, int vd, const PointMap &map, const Replay
                                float *output, int normalize, hipStream_t s) {
     if (map.n_blocks == 0) return hipSuccess;
     if (!map.tile_vertices.table || vd < kManyChannels) return hipErrorInvalidValue;
-    const int out_ch = normalize ? vd - 1 : vd, channels = out_ch < kTileChannels ? out_ch : kTileChannels;
+    const int out_ch = normalize ? vd - 1 : vd, groups = (out_ch + kTileChannels - 1) / kTileChannels;
+    const int channels = groups == 1 ? out_ch : ((out_ch + groups - 1) / groups + 3) / 4 * 4;
     const int Q = (channels + 3) / 4;
-    const unsigned n_rows = tile_rows(Q);
-    const dim3 grid(map.n_blocks, (unsigned)((out_ch + kTileChannels - 1) / kTileChannels)), block(kTileThreads);
+    const dim3 grid(map.n_blocks, (unsigned)groups), block(kTileThreads);
+    const unsigned n_rows = tile_rows(Q, grid.x * grid.y, 4);
 #define PLK_SLICE_TILE(Q)                                                                                     \
     case Q:                                                                                                   \
         PLK_DISPATCH_PD(pd, hipLaunchKernelGGL((k_slice_tile_channels<PD + 1, Q>), grid, block,               \
@@ -645,8 +652,8 @@ hipError_t slice_tile_channels_joint(int pd, int vd, int n, const PointsWork *wo
         items.blocks[i] = multiple_of_xcds(work[i].map.n_blocks);
     }
     const int Q = (out_ch + 3) / 4;
-    const unsigned n_rows = tile_rows(Q);
     const dim3 grid(all_blocks(items)), block(kTileThreads);
+    const unsigned n_rows = tile_rows(Q, grid.x, 4);
 #define PLK_SLICE_TILE_OF(PD, Q)                                                                                     \
     case Q:                                                                                                          \
         hipLaunchKernelGGL((k_slice_tile_channels_of<PD + 1, Q>), grid, block, tile_lds(Q, n_rows), s, items, vd,    \
@@ -710,7 +717,7 @@ hipError_t slice_pairs(int pd_a, int pd_b, int vd, int n, const SlicePair *work,
     bool tiles = true;
     for (int i = 0; i < n; ++i) tiles = tiles && work[i].map.tile_vertices.table && work[i].tiles_b.table;
     const int Q = (vd - 1 + 3) / 4;
-    const unsigned n_rows = tile_rows(Q);
+    const unsigned n_rows = tile_rows(Q, blocks, 3);
     const dim3 grid(blocks, tiles ? 1u : (unsigned)(lanes / kPairPoints)), block(tiles ? kTileThreads : kBlock);
 #define PLK_PAIR_TILES(A, B, Q)                                                                            \
     case Q:                                                                                                \

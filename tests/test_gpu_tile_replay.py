@@ -73,11 +73,40 @@ def test_filter_and_applies(h, w, features, noise, vd):
 
 
 def test_the_noise_crowds_the_tiles():
-    """The inputs above have tiles below and above the rows that fit into LDS (247 of 21 channels, 198 of 32)
-    and none that the merging build cannot take (512)."""
+    """The inputs above have tiles below and above the rows that fit into the least LDS a slice takes (335 of 21
+    channels, 262 of 32: test_crowded_tiles_of_large_images) and none that the merging build cannot take (512)."""
     smooth = vertices_of_tiles(positions(33, 47, 3, 0.0, 7 * 33 + 3), 33, 47)
     noisy = vertices_of_tiles(positions(32, 48, 3, 1.1, 7 * 32 + 3), 32, 48)
-    assert max(smooth) < 198 and max(noisy) > 260 and max(noisy) <= 512
+    assert max(smooth) < 198 and max(noisy) > 262 and max(noisy) <= 512
+
+
+@pytest.mark.parametrize("vd", [22, 33, 40])
+def test_crowded_tiles_of_large_images(vd):
+    """Where the launch fills the GPU a slice has the least rows in LDS: 335 of 21 channels, 262 of 32.  Tiles of
+    more gather from memory; against the same lattice built without merging."""
+    h, w = 512, 530
+    rng = np.random.default_rng(1)
+    y, x = np.meshgrid(np.arange(h), np.arange(w), indexing="ij")
+    smooth = np.stack([np.sin(x / 50.0), np.cos(y / 40.0), np.sin((x + y) / 70.0)], -1) / 0.42
+    # (a few tiles of the most: at 350 of 512 places one in some hundreds looks for its keys too long to be merged)
+    crowd = np.where((x < 48) & (y < 48), 1.0, np.where(x < w // 2, 0.85, 0.1))
+    noise = crowd[..., None] * rng.uniform(-1, 1, (h, w, 3))
+    pos = np.concatenate([np.stack([y, x], -1) / 6.0, smooth + noise], -1).reshape(-1, 5).astype(np.float32)
+    used = vertices_of_tiles(pos, h, w)
+    assert min(used) < 262 and 335 < max(used) <= 512
+    pos, val = dev(pos), dev(rng.uniform(0.1, 1.1, (h * w, vd - 1)).astype(np.float32))
+    outs = {}
+    for merge in (0, 1):
+        lat = pla.PermutohedralLattice(5, vd, h * w)
+        lat.set_point_grid((h, w))
+        lat.set_option(pla.PL_OPT_MERGE_TILES, merge)
+        lat.build(pos)
+        assert lat.info(pla.PL_INFO_BUILD_MERGED) == merge
+        outs[merge] = [lat.apply(torch.full_like(val, float("nan")), val, reverse) for reverse in (False, True)]
+        lat.close()
+    for got, want in zip(outs[1], outs[0]):
+        # (the same terms in another order)
+        assert torch.isfinite(got).all() and float((got - want).abs().max()) <= 2e-5
 
 
 @pytest.mark.parametrize("vd", [2, 3, 4, 5, 8, 9])
