@@ -75,7 +75,9 @@ typedef enum pl_option {
     PL_OPT_VERTEX_LISTS = 10, /* 1 (default): pl_build also writes, per vertex, the list of the (point,
                                weight) rows that name it, and every pl_apply on that lattice splats
                                by gathering along those lists (no atomics, the same order of
-                               additions on every call); 0: pl_apply splats as pl_filter does, point
+                               additions on every call); 2: the same, and which of two kinds of lists
+                               suits pl_mean_field_* on pairs of lattices, which is what this one is
+                               for; 0: pl_apply splats as pl_filter does, point
                                by point with sums per wavefront (same results up to the order of
                                float additions; for measuring the difference).  Float lattices. */
     PL_OPT_NUMBER_SEGMENTS = 11, /* 0 (default): a build that numbers its vertices itself draws the numbers
@@ -394,7 +396,7 @@ int pl_mean_field_update(float *q, const float *logits, const float *message_a,
  * the arrays are read and written in the order of `stream`.  output and q are arrays of their own.  PL_EUNSUPPORTED (nothing is enqueued) where the
  * lattices must be applied one by one: no vertex lists, options that change an apply, 4 classes to 31 only,
  * two or three spatial dimensions with a guide of one or three channels, `stream` or a lattice's own being
- * captured.
+ * captured.  (PL_OPT_VERTEX_LISTS = 2 on the lattices before they are built: lists that suit these calls.)
  * ---------------------------------------------------------------------------------------- */
 int pl_mean_field_messages(int n, const pl_handle *bilateral, const pl_handle *spatial, float *output,
                            const float *input, int reverse, pl_stream stream);

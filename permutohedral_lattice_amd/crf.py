@@ -23,7 +23,7 @@ HIP library's.
 """
 import torch
 
-from . import (PermutohedralLattice, mean_field_infer, mean_field_messages, mean_field_update,
+from . import (PL_OPT_VERTEX_LISTS, PermutohedralLattice, mean_field_infer, mean_field_messages, mean_field_update,
                mean_field_update_supported)
 
 
@@ -51,6 +51,8 @@ class MeanField:
         self.spatial = [PermutohedralLattice(k, self.n_classes + 1, self.n,
                                              stream=self._streams[2 * b + 1])
                         for b in range(self.batch)]
+        for lat in self.bilateral + self.spatial:
+            lat.set_option(PL_OPT_VERTEX_LISTS, 2)      # lists for applies in pairs
         shape = (self.batch, self.n, self.n_classes)
         self._msg_bi = torch.empty(shape, dtype=torch.float32, device=guide.device)
         self._msg_sp = torch.empty(shape, dtype=torch.float32, device=guide.device)

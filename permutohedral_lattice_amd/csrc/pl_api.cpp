@@ -127,6 +127,7 @@ struct pl_lattice {
     // A lattice that is built to be applied (pl_build) also gets, per vertex, the list of the
     // (point, weight) that touch it; pl_apply then splats by gathering (plk::VertexLists)
     bool vertex_lists = true;              // option
+    bool lists_for_pairs = false;          // option: pl_mean_field_* apply this lattice
     plk::VertexLists lists_of_vertices{};
     size_t lists_for_vertices = 0;         // max_vertices the arrays were allocated for
     bool lists_valid = false;              // they describe the last build
@@ -1116,6 +1117,7 @@ int pl_set_option(pl_handle h, int option, long value) {
             return PL_OK;
         case PL_OPT_VERTEX_LISTS:
             h->vertex_lists = value != 0;
+            h->lists_for_pairs = value == 2;
             if (!h->vertex_lists) h->lists_valid = false;
             return PL_OK;
         case PL_OPT_STOP_AFTER:
@@ -1266,7 +1268,17 @@ int enqueue_build_only(pl_lattice *h, const plk::PointFeatures &features, const 
         rc = ensure_vertex_lists(h);
         if (rc != PL_OK) return rc;
         h->lists_of_vertices.map = h->map;
-        if (!plk::lists_of_tiles(h->vd, h->N)) h->lists_of_vertices.map.tile_vertices = plk::TileVertices{};
+        if (h->last_build_merged) {
+            // (a lattice's first lists have just been allocated, and the stream been waited for; a build that
+            // does not fit is repeated, with its lists)
+            if (h->last_M <= 0) {
+                rc = wait_for_report(h, &h->h_status->sequence);
+                if (rc != PL_OK) return rc;
+            }
+            if (!plk::lists_of_tiles(h->pd, h->vd, h->N, h->last_M > 0 ? h->last_M : h->h_status->num_vertices,
+                                     h->lists_for_pairs))
+                h->lists_of_vertices.map.tile_vertices = plk::TileVertices{};
+        }
         h->lists_of_vertices.pd = h->pd;
         PL_HIP(plk::build_vertex_lists(h->pd, h->map, h->replay,
                                        h->replay_holds_cells ? h->cell_vertex : nullptr,

@@ -457,13 +457,24 @@ struct GatherWork {
     unsigned n_chunks, n_long;
     const VertexLists *lists;
 };
-// Which lattices whose build merged get lists of its workgroups' rows of sums, not of its points' corners.  Up
-// to four channels an apply takes a launch more for them, and where the launches count that is what it
-// takes longer; us an apply, lists of corners and of rows, pd 5, vd 4: 256x256 points 18.4 and 21.5, 512x512
-// 24.2 and 25.8, 700x700 32.4 and 32.4, 1024x1024 49.0 and 44.9 (under noise 62.0 and 54.8).  With more channels
-// rows are ahead at every size: vd 22 64x64 26.5 and 25.2, 512x512 62.2 and 48.0; vd 9 47.4 and 34.8; vd 40
-// 95.2 and 88.9.
-inline bool lists_of_tiles(int vd, int N) { return vd > 4 || N >= (1 << 19); }
+// Which lattices whose build merged get lists of its workgroups' rows of sums, not of its points' corners.  Rows
+// take two launches an apply; corners one, and a second where lists are long, which on images they are from a mean
+// of about 320 / pd^2 corners a vertex on.  Where launches count that decides; beyond, rows read less the more
+// corners a point has, and corners the more channels the rows of sums have to be stored and read again.  us an apply,
+// corners and rows: pd 2 vd 22 64x64 14.6 and 17.9 (21 corners a vertex), 20.7 and 19.2 (118), 512x512 32.5 and 32.9;
+// vd 9 321x481 18.1 and 20.3 (23), 23.3 and 21.3 (157); vd 33 512x512 43 and 58; pd 3 vd 16 512x512 34.5 and 28.0, vd 32
+// 38 and 41; pd 4 vd 22 64x96x96 88 and 81; pd 5 vd 6 64x64 25.9 and 21.0, vd 22 512x512 63 and 51, vd 40 1024x1024 718 and 820
+// (8 corners a vertex), 387 and 380 (31).  Up to four channels: pd 2 vd 4 1024x1024 22.3 and 26.1; pd 3 1024x1024 30.1 and 31.7, 2048x2048 104 and 97; pd 5
+// 512x512 23.5 and 24.5, 725x725 35.1 and 35.1, 1024x1024 52.3 and 48.4.
+// pairs: the lattice is applied together with another over the same points (splat_tile_pairs), which rows are for.
+inline bool lists_of_tiles(int pd, int vd, int N, int vertices, bool pairs) {
+    if (vd <= 4) return pd >= 3 && N >= (pd == 3 ? 1 << 21 : 1 << 19);
+    if (pairs && vd <= 32) return true;
+    const double corners = (double)N * (pd + 1) / (vertices > 0 ? vertices : 1);
+    if (N <= 1 << 15) return corners * pd * pd >= 320.0;
+    if (pd >= 4) return vd <= 32;
+    return pd == 3 ? vd <= 24 : vd <= 16 && N <= 1 << 18 && corners >= 100.0;
+}
 // The lists of a merging build (pl_tile_lists.hip).  Floats from one of their rows of sums to the next:
 constexpr int tile_row_floats(int vd) { return vd <= 4 ? vd : (vd + 7) / 8 * 8; }
 hipError_t sort_tiles(int pd, const PointMap &map, const ReplayEntry *replay, int max_vertices, const VertexLists &lists,

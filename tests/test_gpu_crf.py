@@ -188,6 +188,23 @@ def test_what_cannot_be_applied_together_is_applied_one_by_one():
         mf.close()
 
 
+def test_lattices_with_different_kinds_of_lists_are_applied_together():
+    """Built as for applies of their own, a spatial lattice of few corners a vertex lists its corners."""
+    import permutohedral_lattice_amd as pla
+    gen = torch.Generator("cuda").manual_seed(4)
+    guide = torch.rand((2, 60, 76, 3), device="cuda", generator=gen) * 64.0
+    x = torch.randn((2, 60, 76, 21), device="cuda", generator=gen)
+    mf = MeanField(guide, 21)
+    want = mf.messages(x)
+    for lat in mf.bilateral + mf.spatial:
+        lat.set_option(pla.PL_OPT_VERTEX_LISTS, 1)
+    mf.rebuild(guide)
+    out = torch.full((2, 60 * 76, 21), float("nan"), device="cuda")
+    assert pla.mean_field_messages(mf.bilateral, mf.spatial, out, x.view(out.shape))
+    assert float((out.view(want.shape) - want).abs().max()) <= 1e-4
+    mf.close()
+
+
 def test_lattices_applied_together_from_two_streams():
     """The lattices' own streams, and applies of single lattices on them, stay in order with it."""
     gen = torch.Generator("cuda").manual_seed(5)

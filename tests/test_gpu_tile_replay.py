@@ -154,7 +154,7 @@ def test_joint_messages(noise, merged, classes):
     mf.close()
 
 
-# Up to four channels a workgroup's rows of sums are listed from 2^19 points on.  flat: most of a tile's corners
+# Up to four channels a workgroup's rows of sums are listed from 2^19 points on (from four features on).  flat: most of a tile's corners
 # name a few vertices (runs over several wavefronts); wild: values that sums of products by 0 and 1 cannot take.
 @pytest.mark.parametrize("vd", [2, 3, 4])
 @pytest.mark.parametrize("kind", ["image", "flat", "coordinates", "list", "wild"])
@@ -173,7 +173,7 @@ def test_rows_of_few_channels(kind, vd):
     else:
         pos = pla.compute_positions(guide.contiguous(), (h, w), 8.0, 0.5)
     if kind == "list":
-        pos = pos[:, :3][torch.randperm(n, generator=gen, device="cuda")].contiguous()
+        pos = pos[:, :4][torch.randperm(n, generator=gen, device="cuda")].contiguous()
     for normalize in (1, 0):
         channels = vd - 1 if normalize else vd
         val = torch.rand((n, channels), generator=gen, device="cuda") + 0.1

@@ -180,3 +180,35 @@ def test_rebuilding_a_lattice_renews_its_lists():
     torch.cuda.synchronize()
     want = oracle.Lattice(5, 4, n).filter(val1, pos2, True)
     assert np.abs(out.cpu().numpy() - want).max() <= MAX_ABS_TOL
+
+
+@pytest.mark.parametrize("pd,vd,shape,alpha", [
+    # few and many corners a vertex on a small image, whichever lists follow from it; a larger one; the widths
+    # between which it changes
+    (2, 9, (64, 64), 2.0), (2, 9, (64, 64), 12.0), (2, 16, (190, 200), 12.0), (2, 17, (190, 200), 12.0),
+    (3, 24, (190, 200), 6.0), (3, 25, (190, 200), 6.0), (5, 22, (64, 64), 3.0), (5, 40, (190, 200), 8.0),
+    (2, 4, (1024, 1024), 8.0), (3, 2, (1024, 2048), 8.0), (5, 2, (720, 730), 8.0),
+])
+def test_every_kind_of_lists_gives_the_same_applies(pd, vd, shape, alpha):
+    """Lists chosen by the build before (its first, its second) and lists for pairs, against none."""
+    gen = torch.Generator("cuda").manual_seed(vd)
+    h, w = shape
+    ref = None
+    if pd > 2:
+        y, x = torch.meshgrid(torch.arange(h, device="cuda") / 40.0, torch.arange(w, device="cuda") / 30.0, indexing="ij")
+        ref = torch.stack([torch.sin(x * (1 + c)) * torch.cos(y) for c in range(pd - 2)], -1)
+        ref = (ref + 0.1 * torch.rand(ref.shape, device="cuda", generator=gen)).contiguous()
+    val = torch.rand((h * w, vd - 1), device="cuda", generator=gen)
+    outs = []
+    for lists in (0, 1, 2):
+        lat = pla.PermutohedralLattice(pd, vd, h * w)
+        lat.set_option(pla.PL_OPT_VERTEX_LISTS, lists)
+        for _ in range(2 if lists == 1 else 1):
+            lat.build_image(ref, shape, alpha, 0.4)
+            for reverse in (False, True):
+                outs.append(lat.apply(torch.full_like(val, float("nan")), val, reverse))
+        lat.close()
+    for k, out in enumerate(outs[2:]):
+        want = outs[k % 2]
+        # (the same terms in another order: 32-bit sums of up to a few hundred of them)
+        assert float((out - want).abs().max()) <= 2e-5 and torch.isfinite(out).all()
