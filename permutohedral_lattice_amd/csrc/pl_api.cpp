@@ -2155,9 +2155,8 @@ namespace {
 // ends, as the reference does with TensorFlow temporaries (src/DeviceMemoryAllocator.h:52-71),
 // and the items run one after the other.
 struct OpLane {
-    pl_handle lattice = nullptr;
-    hipStream_t stream = nullptr;   // owned unless it is the caller's (lane 0)
-    bool owns_stream = false;
+    pl_handle lattice = nullptr;    // works on the caller's stream or on the lane's, as the call needs it
+    hipStream_t stream = nullptr;   // owned; none before it is needed, and none of lane 0
     hipEvent_t done = nullptr;
 };
 struct OpCacheEntry {
@@ -2165,7 +2164,6 @@ struct OpCacheEntry {
     hipStream_t stream;
     bool f64;                       // lattices of doubles
     std::vector<OpLane> lanes;
-    std::vector<pl_handle> joint;   // behind lanes[0], on the caller's stream: items whose passes go together
     // calls that go on streams after one whose builds could not all be merged (as pl_lattice::tiles_off_for)
     int joint_off_for = 0;
     hipEvent_t fork = nullptr;
@@ -2179,12 +2177,10 @@ int g_op_lanes = 4;
 
 void destroy_entry(OpCacheEntry &e) {
     for (auto &lane : e.lanes) {
-        pl_destroy(lane.lattice);   // waits for the lane's stream
+        pl_destroy(lane.lattice);   // waits for the stream it worked on last
         if (lane.done) (void)hipEventDestroy(lane.done);
-        if (lane.owns_stream && lane.stream) (void)hipStreamDestroy(lane.stream);
+        if (lane.stream) (void)hipStreamDestroy(lane.stream);
     }
-    for (pl_handle h : e.joint) pl_destroy(h);
-    e.joint.clear();
     if (e.fork) (void)hipEventDestroy(e.fork);
     if (e.positions64) (void)hipFree(e.positions64);
     e.positions64 = nullptr;
@@ -2201,32 +2197,29 @@ OpCacheEntry *op_cache_entry(int device, int pd, int vd, int N, hipStream_t stre
         destroy_entry(g_op_cache.front());
         g_op_cache.erase(g_op_cache.begin());
     }
-    g_op_cache.push_back(OpCacheEntry{device, pd, vd, N, stream, f64, {}, {}, 0, nullptr, nullptr});
+    g_op_cache.push_back(OpCacheEntry{device, pd, vd, N, stream, f64, {}, 0, nullptr, nullptr});
     return &g_op_cache.back();
 }
 
-// Lattices and streams for `want` concurrent items.
-int ensure_lanes(OpCacheEntry &e, int want) {
+// Lattices for `want` items in flight, all on the entry's stream or, with `streams`, the lanes behind the first on
+// their own.  (What a lattice did on the other stream is behind it: the entry's stream waits for every lane at the
+// end of a call, and the lanes wait for the entry's stream, `fork`, at its start.)
+int ensure_lanes(OpCacheEntry &e, int want, bool streams) {
     while ((int)e.lanes.size() < want) {
         OpLane lane;
-        if (e.lanes.empty()) {
-            lane.stream = e.stream;
-        } else {
-            PL_HIP(hipStreamCreateWithFlags(&lane.stream, hipStreamNonBlocking));
-            lane.owns_stream = true;
-        }
-        int rc = e.f64 ? pl_create_f64(e.pd, e.vd, e.N, (pl_stream)lane.stream, nullptr, &lane.lattice)
-                       : pl_create(e.pd, e.vd, e.N, (pl_stream)lane.stream, nullptr, &lane.lattice);
-        if (rc == PL_OK && hipEventCreateWithFlags(&lane.done, hipEventDisableTiming) != hipSuccess)
-            rc = PL_EHIP;
-        if (rc != PL_OK) {
-            pl_destroy(lane.lattice);
-            if (lane.owns_stream) (void)hipStreamDestroy(lane.stream);
-            return rc;
-        }
+        const int rc = e.f64 ? pl_create_f64(e.pd, e.vd, e.N, (pl_stream)e.stream, nullptr, &lane.lattice)
+                             : pl_create(e.pd, e.vd, e.N, (pl_stream)e.stream, nullptr, &lane.lattice);
+        if (rc != PL_OK) return rc;
         e.lanes.push_back(lane);
     }
-    if (want > 1 && !e.fork) PL_HIP(hipEventCreateWithFlags(&e.fork, hipEventDisableTiming));
+    if (streams && want > 1 && !e.fork) PL_HIP(hipEventCreateWithFlags(&e.fork, hipEventDisableTiming));
+    for (int l = 0; l < want; ++l) {
+        OpLane &lane = e.lanes[l];
+        const bool own = streams && l > 0;
+        if (own && !lane.stream) PL_HIP(hipStreamCreateWithFlags(&lane.stream, hipStreamNonBlocking));
+        if (own && !lane.done) PL_HIP(hipEventCreateWithFlags(&lane.done, hipEventDisableTiming));
+        lane.lattice->stream = own ? lane.stream : e.stream;
+    }
     return PL_OK;
 }
 
@@ -2234,16 +2227,10 @@ int ensure_lanes(OpCacheEntry &e, int want) {
 int filter_items_together(OpCacheEntry &e, int n_lanes, const float *input, const float *reference, float *output,
                           int batch, int n_spatial_dims, const int *spatial_dims, int channels, int ref_ch,
                           float spatial_std, float feature_std, int reverse) {
-    int rc = ensure_lanes(e, 1);
+    int rc = ensure_lanes(e, n_lanes, false);
     if (rc != PL_OK) return rc;
-    while ((int)e.joint.size() < n_lanes - 1) {
-        pl_handle h = nullptr;
-        rc = pl_create(e.pd, e.vd, e.N, (pl_stream)e.stream, nullptr, &h);
-        if (rc != PL_OK) return rc;
-        e.joint.push_back(h);
-    }
-    pl_handle lattices[kOpLanesMax] = {e.lanes[0].lattice};
-    for (int i = 1; i < n_lanes; ++i) lattices[i] = e.joint[i - 1];
+    pl_handle lattices[kOpLanesMax];
+    for (int i = 0; i < n_lanes; ++i) lattices[i] = e.lanes[i].lattice;
     const size_t N = (size_t)e.N;
     for (int b = 0; b < batch; b += n_lanes) {
         const int count = batch - b < n_lanes ? batch - b : n_lanes;
@@ -2320,9 +2307,9 @@ extern "C" int pl_lattice_filter_op(const float *input, const float *reference, 
             return filter_items_together(*entry, n_lanes, input, reference, output, batch, n_spatial_dims, spatial_dims,
                                          n_input_channels, ref_ch, spatial_std, feature_std, reverse);
         if (--entry->joint_off_for == 0)
-            for (pl_handle h : entry->joint) h->tiles_off_for = h->wide_for = 0;
+            for (OpLane &lane : entry->lanes) lane.lattice->tiles_off_for = lane.lattice->wide_for = 0;
     }
-    int rc = ensure_lanes(*entry, n_lanes);
+    int rc = ensure_lanes(*entry, n_lanes, true);
     if (rc != PL_OK) return rc;
 
     // the other lanes start after whatever the caller's stream holds so far
@@ -2445,7 +2432,7 @@ extern "C" int pl_lattice_filter_op_f64(const double *input, const double *refer
     PL_HIP(hipGetDevice(&device));
     std::lock_guard<std::mutex> lock(g_op_cache_mutex);
     OpCacheEntry *entry = op_cache_entry(device, pd, vd, N, (hipStream_t)stream, true);
-    int rc = ensure_lanes(*entry, 1);
+    int rc = ensure_lanes(*entry, 1, false);
     if (rc != PL_OK) return rc;
     if (!on_grid && !entry->positions64 &&
         hip_failed(hipMalloc((void **)&entry->positions64, position_bytes))) {

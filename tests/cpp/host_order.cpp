@@ -65,6 +65,7 @@ struct Array {
 std::map<const void *, Array> g_arrays;
 std::vector<std::string> g_launches;
 std::string g_fail_next;   // the launch of this name fails, once
+long g_allocated = 0;      // device arrays in existence
 
 hipError_t launch(const char *name, hipStream_t s, const std::vector<const void *> &reads,
                   const std::vector<const void *> &writes) {
@@ -126,14 +127,17 @@ void __hipUnregisterFatBinary(void **) {}
 void __hipRegisterVar(void **, void *, char *, char *, int, size_t, int, int) {}
 hipError_t hipGetDevice(int *d) { return *d = 0, hipSuccess; }
 hipError_t hipGetLastError() { return hipSuccess; }
-hipError_t hipMalloc(void **p, size_t n) { return (*p = std::calloc(1, n)) ? hipSuccess : hipErrorOutOfMemory; }
-hipError_t hipFree(void *p) { return std::free(p), hipSuccess; }
-hipError_t hipHostMalloc(void **p, size_t n, unsigned) { return hipMalloc(p, n); }
-hipError_t hipHostFree(void *p) { return hipFree(p); }
+hipError_t hipHostMalloc(void **p, size_t n, unsigned) { return (*p = std::calloc(1, n)) ? hipSuccess : hipErrorOutOfMemory; }
+hipError_t hipHostFree(void *p) { return std::free(p), hipSuccess; }
+hipError_t hipMalloc(void **p, size_t n) { return g_allocated += 1, hipHostMalloc(p, n, 0); }
+hipError_t hipFree(void *p) { return g_allocated -= p != nullptr, hipHostFree(p); }
 hipError_t hipMemcpyAsync(void *to, const void *from, size_t n, hipMemcpyKind, hipStream_t) {
     return std::memcpy(to, from, n), hipSuccess;
 }
-hipError_t hipStreamCreateWithFlags(hipStream_t *, unsigned) { return hipErrorInvalidValue; }
+hipError_t hipStreamCreateWithFlags(hipStream_t *s, unsigned) {
+    static long made = 1000;
+    return *s = named_stream(++made), hipSuccess;
+}
 hipError_t hipStreamDestroy(hipStream_t s) { return g_streams.erase((void *)s), hipSuccess; }
 hipError_t hipStreamSynchronize(hipStream_t s) { return join(g_host, stream_of(s).clock), hipSuccess; }
 hipError_t hipStreamIsCapturing(hipStream_t s, hipStreamCaptureStatus *status) {
@@ -557,6 +561,25 @@ void failed_batch() {
     }
 }
 
+// batches of one shape whose passes can be enqueued together and whose cannot, in turn: the same lattices
+void batches_either_way() {
+    const int dims[2] = {kH, kW}, flat[1] = {kH * kW};
+    const hipStream_t s = named_stream(1);
+    float *in = nullptr, *out = nullptr, *reference = nullptr;
+    for (float **p : {&in, &out, &reference}) (void)hipMalloc((void **)p, sizeof(float) * 4 * kH * kW * 4);
+    long first = 0;
+    for (const char *turn = "jjssjsjj"; *turn; ++turn) {
+        g_launches.clear();
+        const int rc = *turn == 'j' ? pl_lattice_filter_op(in, reference, out, 3, 2, dims, 3, 3, 1, 8.0f, 0.1f, 1.0f, 0, s, nullptr)
+                                    : pl_lattice_filter_op(in, reference, out, 3, 1, flat, 3, 4, 1, 8.0f, 0.1f, 1.0f, 0, s, nullptr);
+        expect(rc == PL_OK, "the op");
+        expect(launched("build_joint") == (*turn == 'j') && launched("build") == (*turn == 's'), "how it was enqueued");
+        (void)launch("the caller's", s, {out}, {in, reference});
+        if (!first) first = g_allocated;
+        expect(g_allocated == first, "more lattices than items in flight");
+    }
+}
+
 }  // namespace
 
 int main(int argc, char **argv) {
@@ -571,6 +594,7 @@ int main(int argc, char **argv) {
         {"failed_blur", failed_blur},
         {"no_pointer_kept", no_pointer_kept},
         {"failed_batch", failed_batch},
+        {"batches_either_way", batches_either_way},
     };
     const auto found = scenarios.find(argc > 1 ? argv[1] : "");
     if (found == scenarios.end()) {
