@@ -760,12 +760,16 @@ int enqueue_apply(pl_lattice *h, void *output_any, const void *input_any, int re
         const size_t filled = h->verified && h->n_segments == 0 ? (size_t)h->M : (size_t)mv;
         if (!h->values_zeroed) PL_HIP(plk::fill_zero(h->values[0], filled * vd, h->stream));
         h->mark(EV_FILL);
-        const auto splat = !h->last_build_merged ? plk::splat
-                           : vd <= 4             ? plk::splat_merge
-                           : plk::splat_tile_takes(vd) ? plk::splat_tile : plk::splat;
-        PL_HIP(splat(pd, vd, h->map, input, in_channels, h->replay,
-                     h->replay_holds_cells ? h->cell_vertex : nullptr, h->values[0],
-                     h->xcd_aware ? 1 : 0, h->stream));
+        if (h->last_build_merged && vd <= 4)
+            PL_HIP(plk::splat_merge(pd, vd, h->map, input, in_channels, h->replay, h->values[0], h->xcd_aware ? 1 : 0,
+                                    h->stream));
+        else if (h->last_build_merged && plk::splat_tile_takes(vd))
+            PL_HIP(plk::splat_tile(pd, vd, h->map, input, in_channels, h->replay, h->values[0], h->xcd_aware ? 1 : 0,
+                                   h->stream));
+        else
+            PL_HIP(plk::splat(pd, vd, h->map, input, in_channels, h->replay,
+                              h->replay_holds_cells ? h->cell_vertex : nullptr, h->values[0],
+                              h->xcd_aware ? 1 : 0, h->stream));
         h->replay_holds_cells = false;
     } else {
         h->mark(EV_FILL);

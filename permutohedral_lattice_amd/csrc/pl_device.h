@@ -962,6 +962,14 @@ __device__ __forceinline__ double wave_sums_to_quads_f64(bool member, const doub
     return x;
 }
 
+// Four channels of a row, which is only aligned to its floats
+struct alignas(4) FourFloats {
+    float c[4];
+};
+__device__ __forceinline__ float one_of(int i, float a, float b, float c, float d) {
+    return i == 0 ? a : i == 1 ? b : i == 2 ? c : d;
+}
+
 // Which item of a launch a workgroup works for: the items' workgroups follow each other, every item's a
 // multiple of eight, so that workgroup b of an item runs on XCD b % 8 as in a launch of its own.
 template <typename Item, int N = kManyItems>
@@ -986,6 +994,17 @@ unsigned all_blocks(const Items<Item, N> &items) {
     return b;
 }
 inline unsigned multiple_of_xcds(unsigned b) { return (b + kXcds - 1u) / kXcds * kXcds; }
+// (items with the workgroups of their points)
+template <int N, typename Item>
+Items<Item, N> items_of_points(int n, const Item *work) {
+    Items<Item, N> items{};
+    items.n = n;
+    for (int i = 0; i < n; ++i) {
+        items.item[i] = work[i];
+        items.blocks[i] = multiple_of_xcds(work[i].map.n_blocks);
+    }
+    return items;
+}
 
 // (keys of two words exist for the dimensions whose packed key has fields of less than 16 bits)
 #define PLK_DISPATCH_WIDE_PD(pd, CALL)            \

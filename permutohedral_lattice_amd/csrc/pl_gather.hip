@@ -408,10 +408,6 @@ __global__ __launch_bounds__(kBlock) void k_splat_gather(ListChunks chunks, unsi
 // Channels past the input are the homogeneous one: the sum of the bare weights.
 constexpr int kChannelChunk = (int)kListChunkManyChannels;   // rows of a chunk at most (vd > 4)
 
-
-struct alignas(4) FourFloats {
-    float c[4];
-};
 __device__ __forceinline__ float pick(const float (&x)[4], int i) {
     return i == 0 ? x[0] : i == 1 ? x[1] : i == 2 ? x[2] : x[3];
 }

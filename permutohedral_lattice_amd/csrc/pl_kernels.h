@@ -368,7 +368,7 @@ hipError_t splat(int pd, int vd, const PointMap &map, const float *input, int in
 
 // The same for rows of 2 to 4 channels after a merging build: sums merged per workgroup in LDS.
 hipError_t splat_merge(int pd, int vd, const PointMap &map, const float *input, int in_channels,
-                       ReplayEntry *replay, const int *cell_vertex, float *values, int xcd_aware, hipStream_t s);
+                       const ReplayEntry *replay, float *values, int xcd_aware, hipStream_t s);
 
 // The same for rows of 5 to 32 channels after a merging build, whose workgroups' points have at most
 // kTileSlots vertices: pairs sorted by vertex in LDS, see pl_splat_tile.hip.
@@ -377,8 +377,8 @@ hipError_t splat_merge(int pd, int vd, const PointMap &map, const float *input, 
 // 56.9 and 53.0; 120x160 pd 3 vd 17 41.0 and 37.5; 321x481 pd 2 vd 22 54.9 and 53.5, pd 5 vd 5 84.8 and 65.1;
 // 800x1000 pd 2 vd 32 150 and 131, pd 3 vd 8 133 and 97, pd 5 vd 16 278 and 194; in none of 60 shapes slower.)
 inline bool splat_tile_takes(int vd) { return vd >= 5 && vd <= 32; }
-hipError_t splat_tile(int pd, int vd, const PointMap &map, const float *input, int in_channels, ReplayEntry *replay,
-                      const int *cell_vertex, float *values, int xcd_aware, hipStream_t s);
+hipError_t splat_tile(int pd, int vd, const PointMap &map, const float *input, int in_channels,
+                      const ReplayEntry *replay, float *values, int xcd_aware, hipStream_t s);
 
 // The transpose of the replay matrix, for lattices that are applied many times (pl_gather.hip):
 // the rows that name vertex v are entries[start[v] .. start[v+1]), each the point and its weight.

@@ -559,6 +559,8 @@ __global__ __launch_bounds__(kBlock) void k_build(PointFeatures features, PointM
 // What the kernels that merge a workgroup's rows in LDS share.
 static_assert(kTileSlots == 1 << (32 - kTileSlotShift), "the slot is the hash's high bits");
 
+constexpr int kTileProbeLimit = 48;
+
 // A slot of the workgroup's table for every group of the wavefront (wave_groups_in_order of each corner,
 // numbered through): slot[r] := that of the lane's group of corner r, -1 where it has none (bit r of
 // `present` clear) or no slot was found; new slots join the list `occupied`, at place_of_slot.  True: every key
@@ -567,13 +569,11 @@ static_assert(kTileSlots == 1 << (32 - kTileSlotShift), "the slot is the hash's 
 // pixels have about forty), and every lane places one, where a lane with a leader for each of its
 // corners would place up to D1, one behind the other; the slots come back the same way.  (More than 64
 // groups: 64 at a time.)  wave_keys: 64 keys of the wavefront's own, in LDS.
-template <int PROBES, int D1, typename Key, typename Hash>
-__device__ __forceinline__ bool place_groups(const Key (&key)[D1], const unsigned (&group)[D1], unsigned present,
-                                             unsigned n_groups, int lane, Key *wave_keys, Key *table, Key empty,
-                                             Hash hash, unsigned short *occupied, unsigned short *place_of_slot,
-                                             int *n_occupied, int (&slot)[D1]) {
-    using Word = std::conditional_t<sizeof(Key) == 8, unsigned long long, int>;
-    constexpr int kStride = sizeof(Key) / sizeof(int);
+template <int D1>
+__device__ __forceinline__ bool place_groups(const uint64_t (&key)[D1], const unsigned (&group)[D1], unsigned present,
+                                             unsigned n_groups, int lane, uint64_t *wave_keys, uint64_t *table,
+                                             unsigned short *occupied, unsigned short *place_of_slot, int *n_occupied,
+                                             int (&slot)[D1]) {
     int *wave_slots = reinterpret_cast<int *>(wave_keys);
     bool placed = true;
 #pragma unroll
@@ -585,15 +585,16 @@ __device__ __forceinline__ bool place_groups(const Key (&key)[D1], const unsigne
             if (((present >> r) & 1u) && rank_of(group[r]) == 0 && to < 64u) wave_keys[to] = key[r];
         }
         wave_exchange_in_lds();
-        const Key mine = wave_keys[lane];
-        int at_slot = (int)(hash(mine) >> kTileSlotShift);
+        const uint64_t mine = wave_keys[lane];
+        int at_slot = (int)(hash_key(mine) >> kTileSlotShift);
         bool open = from + (unsigned)lane < n_groups, was_empty = false;
         if (!open) at_slot = -1;
-        for (int probe = 0; open && probe < PROBES; ++probe) {
-            const Key seen = (Key)atomicCAS((Word *)&table[at_slot], (Word)empty, (Word)mine);
-            if (seen == empty || seen == mine) {
+        for (int probe = 0; open && probe < kTileProbeLimit; ++probe) {
+            const uint64_t seen = atomicCAS((unsigned long long *)&table[at_slot], (unsigned long long)kEmptyCell,
+                                            (unsigned long long)mine);
+            if (seen == kEmptyCell || seen == mine) {
                 open = false;
-                was_empty = seen == empty;
+                was_empty = seen == kEmptyCell;
             } else {
                 at_slot = (at_slot + 1) & (kTileSlots - 1);
             }
@@ -603,12 +604,12 @@ __device__ __forceinline__ bool place_groups(const Key (&key)[D1], const unsigne
             at_slot = -1;
         }
         wave_exchange_in_lds();
-        wave_slots[kStride * lane] = at_slot;
+        wave_slots[2 * lane] = at_slot;
         wave_exchange_in_lds();
 #pragma unroll
         for (int r = 0; r < D1; ++r) {
             const unsigned to = number_of(group[r]) - from;
-            if (((present >> r) & 1u) && to < 64u) slot[r] = wave_slots[kStride * to];
+            if (((present >> r) & 1u) && to < 64u) slot[r] = wave_slots[2 * to];
         }
         // the slots that were empty join the list of slots in use
         if (was_empty) {
@@ -678,7 +679,6 @@ __device__ __forceinline__ void add_to_slots(T *slot_sum, const unsigned (&group
 // the barriers.  What bounds the kernel is the number of instructions of its wavefronts (800x1200 points,
 // pd 5, vd 4: 64.7 us with 1620 vector and 1226 scalar ones, 54 with 1288 and 750).
 static_assert(kTileSlots == 2 * kBlock, "a thread places at most two slots in the table");
-constexpr int kTileProbeLimit = 48;
 
 // (workgroup `block` of the `blocks` of a lattice)
 template <int PD, int SPLAT_VD, typename T>
@@ -758,9 +758,8 @@ __device__ __forceinline__ void build_tile(const PointFeatures &features, const 
         vertex_keys_of<PD>(s, key);
 #pragma unroll
         for (int r = 0; r < D1; ++r) group[r] = wave_groups_in_order(key[r], among, &n_groups);
-        const bool all_placed = place_groups<kTileProbeLimit>(
-            key, group, active ? (1u << D1) - 1u : 0u, n_groups, lane, group_keys[tid >> 6], slot_key, kEmptyCell,
-            [](uint64_t k) { return hash_key(k); }, occupied, place_of_slot, &n_occupied, slot);
+        const bool all_placed = place_groups(key, group, active ? (1u << D1) - 1u : 0u, n_groups, lane, group_keys[tid >> 6],
+                                             slot_key, occupied, place_of_slot, &n_occupied, slot);
         if (!all_placed) atomicOr(&counters->flags, kFlagTileFull);
     }
 
@@ -2295,9 +2294,6 @@ __global__ __launch_bounds__(kBlock) void k_slice_channels(int vd, PointMap map,
 // handed round.  The lane on the row's last channels reads the row's last four instead, so that
 // no load leaves the row, and its sums are shifted back before they are stored.  Same sums in the
 // same order as k_slice_channels.
-struct alignas(4) FourFloats {
-    float c[4];
-};
 constexpr int kSlicePoints = 2;   // points per group of L lanes (1: 2 % slower, 4: 4 %)
 template <int D1, int L>
 __global__ __launch_bounds__(kBlock) void k_slice_quads(int vd, PointMap map,
@@ -2705,7 +2701,7 @@ hipError_t fill_zero(float *p, size_t n, hipStream_t s) {
 }
 
 hipError_t splat_merge(int pd, int vd, const PointMap &map, const float *input, int in_channels,
-                       ReplayEntry *replay, const int *, float *values, int xcd_aware, hipStream_t s) {
+                       const ReplayEntry *replay, float *values, int xcd_aware, hipStream_t s) {
     if (map.n_blocks == 0) return hipSuccess;
     if (!map.tile_vertices.table) return hipErrorInvalidValue;
     const dim3 grid(map.n_blocks), block(kBlock);
@@ -2985,20 +2981,10 @@ hipError_t slice_rows_f64(int pd, int vd, const PointMap &map, const ReplayEntry
         default: return hipErrorInvalidValue;         \
     }
 
-static Items<BuildWork, kJointItems> build_items(int n, const BuildWork *work) {
-    Items<BuildWork, kJointItems> items{};
-    items.n = n;
-    for (int i = 0; i < n; ++i) {
-        items.item[i] = work[i];
-        items.blocks[i] = multiple_of_xcds(work[i].map.n_blocks);
-    }
-    return items;
-}
-
 hipError_t build_joint(int pd, int n, const BuildWork *work, const ScaleFactor &scale, int xcd_aware, int splat_vd,
                        int in_channels, hipStream_t s) {
     if (n < 1 || n > kJointItems) return hipErrorInvalidValue;
-    const Items<BuildWork, kJointItems> items = build_items(n, work);
+    const Items<BuildWork, kJointItems> items = items_of_points<kJointItems>(n, work);
 #define PLK_BUILD_JOINT(SPLAT_VD)                                                                                    \
     case SPLAT_VD:                                                                                                   \
         PLK_DISPATCH_JOINT_PD(pd, hipLaunchKernelGGL((k_build_tiles<PD, SPLAT_VD>), dim3(all_blocks(items)), dim3(kBlock), \
@@ -3014,7 +3000,7 @@ hipError_t build_joint(int pd, int n, const BuildWork *work, const ScaleFactor &
 
 hipError_t number_vertices_joint(int pd, int n, const BuildWork *work, int vd, hipStream_t s) {
     if (n < 1 || n > kJointItems) return hipErrorInvalidValue;
-    const Items<BuildWork, kJointItems> items = build_items(n, work);
+    const Items<BuildWork, kJointItems> items = items_of_points<kJointItems>(n, work);
     PLK_DISPATCH_JOINT_PD(pd, hipLaunchKernelGGL((k_number_vertices_of<PD + 1>), dim3(all_blocks(items)), dim3(64), 0, s,
                                                  items, vd));
     return hipGetLastError();
@@ -3022,7 +3008,7 @@ hipError_t number_vertices_joint(int pd, int n, const BuildWork *work, int vd, h
 
 hipError_t neighbours_joint(int pd, int n, const BuildWork *work, int vd, hipStream_t s) {
     if (n < 1 || n > kJointItems) return hipErrorInvalidValue;
-    Items<BuildWork, kJointItems> items = build_items(n, work);
+    Items<BuildWork, kJointItems> items = items_of_points<kJointItems>(n, work);
     for (int i = 0; i < n; ++i)
         items.blocks[i] = tile_blocks_for(work[i].map.n_blocks) +
                           vertex_blocks((size_t)(pd + 1) * (size_t)work[i].launch_vertices);
@@ -3031,20 +3017,10 @@ hipError_t neighbours_joint(int pd, int n, const BuildWork *work, int vd, hipStr
     return hipGetLastError();
 }
 
-static Items<PointsWork, kJointItems> points_items(int n, const PointsWork *work) {
-    Items<PointsWork, kJointItems> items{};
-    items.n = n;
-    for (int i = 0; i < n; ++i) {
-        items.item[i] = work[i];
-        items.blocks[i] = multiple_of_xcds(work[i].map.n_blocks);
-    }
-    return items;
-}
-
 hipError_t splat_joint(int pd, int vd, int n, const PointsWork *work, int in_channels, int xcd_aware, hipStream_t s) {
     if (n < 1 || n > kJointItems) return hipErrorInvalidValue;
     if (vd > 4) return splat_tile_joint(pd, vd, n, work, in_channels, xcd_aware, s);
-    const Items<PointsWork, kJointItems> items = points_items(n, work);
+    const Items<PointsWork, kJointItems> items = items_of_points<kJointItems>(n, work);
 #define PLK_SPLAT_JOINT(VD)                                                                                              \
     case VD:                                                                                                             \
         PLK_DISPATCH_JOINT_PD(pd, hipLaunchKernelGGL((k_splat_merge_of<VD, PD + 1>), dim3(all_blocks(items)), dim3(kBlock), \
@@ -3078,7 +3054,7 @@ hipError_t blur_joint(int vd, int n, const BlurWork *work, hipStream_t s) {
 hipError_t slice_joint(int pd, int vd, int n, const PointsWork *work, int normalize, hipStream_t s) {
     if (n < 1 || n > kJointItems) return hipErrorInvalidValue;
     if (vd > 4) return slice_tile_channels_joint(pd, vd, n, work, normalize, s);
-    const Items<PointsWork, kJointItems> items = points_items(n, work);
+    const Items<PointsWork, kJointItems> items = items_of_points<kJointItems>(n, work);
 #define PLK_SLICE_JOINT(VD)                                                                                              \
     case VD:                                                                                                             \
         PLK_DISPATCH_JOINT_PD(pd, hipLaunchKernelGGL((k_slice_tile_of<VD, PD + 1>), dim3(all_blocks(items)), dim3(kBlock), \

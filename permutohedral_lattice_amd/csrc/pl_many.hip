@@ -18,9 +18,6 @@ namespace {
 
 using namespace device;
 
-struct alignas(4) FourFloats {
-    float c[4];
-};
 
 // ------------------------------------------------------------------------------------------------
 // Blur of rows of five and more channels: a thread per vertex and run of four of its channels (the
@@ -253,9 +250,6 @@ inline unsigned tile_rows(int Q, unsigned workgroups, unsigned per_cu) {
 inline size_t tile_lds(int Q, unsigned rows) {
     const size_t in = (size_t)rows * (row_stride(Q) + 1), out = (size_t)kBlock * 4 * Q;
     return sizeof(float) * (in > out ? in : out);
-}
-__device__ __forceinline__ float one_of(int i, float a, float b, float c, float d) {
-    return i == 0 ? a : i == 1 ? b : i == 2 ? c : d;
 }
 // The four channels from c on of a row in memory (what is past vd: anything)
 __device__ __forceinline__ FourFloats piece_of_row(const float *row, int vd, int c) {
@@ -645,12 +639,7 @@ hipError_t slice_tile_channels(int pd, int vd, const PointMap &map, const Replay
 hipError_t slice_tile_channels_joint(int pd, int vd, int n, const PointsWork *work, int normalize, hipStream_t s) {
     const int out_ch = normalize ? vd - 1 : vd;
     if (n < 1 || n > kJointItems || vd < kManyChannels || out_ch > kTileChannels) return hipErrorInvalidValue;
-    Items<PointsWork, kJointItems> items{};
-    items.n = n;
-    for (int i = 0; i < n; ++i) {
-        items.item[i] = work[i];
-        items.blocks[i] = multiple_of_xcds(work[i].map.n_blocks);
-    }
+    const Items<PointsWork, kJointItems> items = items_of_points<kJointItems>(n, work);
     const int Q = (out_ch + 3) / 4;
     const dim3 grid(all_blocks(items)), block(kTileThreads);
     const unsigned n_rows = tile_rows(Q, grid.x, 4);
@@ -705,12 +694,7 @@ bool slice_pairs_take(int pd_a, int pd_b, int vd) {
 
 hipError_t slice_pairs(int pd_a, int pd_b, int vd, int n, const SlicePair *work, hipStream_t s) {
     if (n < 1 || n > kManyItems || !slice_pairs_take(pd_a, pd_b, vd)) return hipErrorInvalidValue;
-    Items<SlicePair> items{};
-    items.n = n;
-    for (int i = 0; i < n; ++i) {
-        items.item[i] = work[i];
-        items.blocks[i] = multiple_of_xcds(work[i].map.n_blocks);
-    }
+    const Items<SlicePair> items = items_of_points<kManyItems>(n, work);
     const unsigned blocks = all_blocks(items);
     if (!blocks) return hipSuccess;
     const int lanes = vd <= 16 ? 4 : 8;

@@ -96,7 +96,7 @@ __device__ __forceinline__ void splat_tile_of(uint2 *sorted, int d1, int vd, con
     // the slot's.  The first lane of a run of lanes with one vertex counts for the run (8x8
     // pixels: 29 runs; LDS atomics on one address take turns).
     unsigned place[kMaxCorners];
-    constexpr unsigned kNoPlace = 0xffffffffu;
+    constexpr unsigned kNoPair = 0xffffffffu;
 #pragma unroll
     for (int r = 0; r < (int)kMaxCorners; ++r) {
         const int before = __shfl_up(index[r], 1);
@@ -104,11 +104,11 @@ __device__ __forceinline__ void splat_tile_of(uint2 *sorted, int d1, int vd, con
         const uint64_t opening = wave_ballot(opens);
         const uint64_t behind = lane == 63 ? 0ull : opening >> (lane + 1);
         const unsigned length = behind ? (unsigned)__builtin_ctzll(behind) + 1u : 64u - (unsigned)lane;
-        unsigned found = kNoPlace;
+        unsigned found = kNoPair;
         if (opens && index[r] >= 0) found = (unsigned)index[r] | atomicAdd(&slot_count[index[r]], length) << 16;
         const int opener = 63 - __builtin_clzll(opening & (~0ull >> (63 - lane)));
         found = (unsigned)__shfl((int)found, opener);
-        place[r] = index[r] >= 0 && found != kNoPlace ? found + ((unsigned)(lane - opener) << 16) : kNoPlace;
+        place[r] = index[r] >= 0 && found != kNoPair ? found + ((unsigned)(lane - opener) << 16) : kNoPair;
     }
     __syncthreads();   // the slots are counted
 
@@ -134,7 +134,7 @@ __device__ __forceinline__ void splat_tile_of(uint2 *sorted, int d1, int vd, con
 
 #pragma unroll
     for (int r = 0; r < (int)kMaxCorners; ++r) {
-        if (place[r] == kNoPlace) continue;
+        if (place[r] == kNoPair) continue;
         const unsigned slot = place[r] & 0xffffu;
         sorted[slot_count[slot] + (place[r] >> 16)] =
             make_uint2(__float_as_uint(weight[r]), (unsigned)point | slot << 8);
@@ -211,8 +211,8 @@ __global__ __launch_bounds__(kThreads) void k_splat_tiles(Items<PointsWork, kJoi
 
 }  // namespace
 
-hipError_t splat_tile(int pd, int vd, const PointMap &map, const float *input, int in_channels, ReplayEntry *replay,
-                      const int *, float *values, int xcd_aware, hipStream_t s) {
+hipError_t splat_tile(int pd, int vd, const PointMap &map, const float *input, int in_channels, const ReplayEntry *replay,
+                      float *values, int xcd_aware, hipStream_t s) {
     if (map.n_blocks == 0) return hipSuccess;
     if (!map.tile_vertices.table || !splat_tile_takes(vd) || pd < 1 || pd > kMaxPd || in_channels < 1 || in_channels > vd)
         return hipErrorInvalidValue;
@@ -227,12 +227,7 @@ hipError_t splat_tile(int pd, int vd, const PointMap &map, const float *input, i
 hipError_t splat_tile_joint(int pd, int vd, int n, const PointsWork *work, int in_channels, int xcd_aware, hipStream_t s) {
     if (!splat_tile_takes(vd) || pd < 1 || pd > kMaxPd || in_channels < 1 || in_channels > vd || n < 1 || n > kJointItems)
         return hipErrorInvalidValue;
-    Items<PointsWork, kJointItems> items{};
-    items.n = n;
-    for (int i = 0; i < n; ++i) {
-        items.item[i] = work[i];
-        items.blocks[i] = multiple_of_xcds(work[i].map.n_blocks);
-    }
+    const Items<PointsWork, kJointItems> items = items_of_points<kJointItems>(n, work);
     const int d1 = pd + 1;
     const size_t lds = kBlock * ((size_t)d1 * sizeof(uint2) + (size_t)in_channels * sizeof(float));
     const auto kernel = vd <= 16 ? k_splat_tiles<1> : k_splat_tiles<2>;

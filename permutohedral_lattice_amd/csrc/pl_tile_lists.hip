@@ -19,12 +19,6 @@ namespace {
 
 using namespace device;
 
-struct alignas(4) FourFloats {
-    float c[4];
-};
-__device__ __forceinline__ float one_of(int i, float a, float b, float c, float d) {
-    return i == 0 ? a : i == 1 ? b : i == 2 ? c : d;
-}
 
 // ------------------------------------------------------------------------------------------------
 // When the lattice is built: every workgroup's corners sorted by their places in its table, 64 * 4 * D1 of

@@ -272,8 +272,8 @@ hipError_t splat_gather_many(int, int, int n, const GatherWork *work, hipStream_
         e = launch("splat_gather_many", s, {work[i].entries, work[i].input}, {work[i].values});
     return e;
 }
-hipError_t splat_tile(int, int, const PointMap &, const float *input, int, ReplayEntry *replay, const int *, float *values,
-                      int, hipStream_t s) {
+hipError_t splat_tile(int, int, const PointMap &, const float *input, int, const ReplayEntry *replay, float *values, int,
+                      hipStream_t s) {
     return launch("splat_tile", s, {input, replay}, {values});
 }
 hipError_t splat_joint(int, int, int n, const PointsWork *work, int, int, hipStream_t s) {
