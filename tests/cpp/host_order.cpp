@@ -66,6 +66,8 @@ std::map<const void *, Array> g_arrays;
 std::vector<std::string> g_launches;
 std::string g_fail_next;   // the launch of this name fails, once
 long g_allocated = 0;      // device arrays in existence
+unsigned g_rows_of_sums = 0;                // what the lists of a merging build report
+std::map<const void *, size_t> g_sizes;     // of arrays from alloc_if_allowed
 
 hipError_t launch(const char *name, hipStream_t s, const std::vector<const void *> &reads,
                   const std::vector<const void *> &writes) {
@@ -257,13 +259,16 @@ hipError_t neighbours_joint(int pd, int n, const BuildWork *work, int vd, hipStr
 }
 hipError_t build_vertex_lists(int, const PointMap &, ReplayEntry *replay, const int *, int, const VertexLists &lists,
                               unsigned *info, unsigned sequence, hipStream_t s) {
-    info[0] = 0;
+    info[0] = lists.map.tile_vertices.table ? g_rows_of_sums : 0u;
     info[1] = 1;
     info[2] = sequence;
     return launch("build_vertex_lists", s, {replay}, {lists.entries});
 }
-hipError_t splat_gather(int, const VertexLists &lists, unsigned, unsigned, const float *input, int, float *values,
+hipError_t splat_gather(int vd, const VertexLists &lists, unsigned, unsigned, const float *input, int, float *values,
                         hipStream_t s) {
+    if (g_rows_of_sums && lists.map.tile_vertices.table)
+        expect(g_sizes[lists.chunks.partial_rows] >= sizeof(float) * g_rows_of_sums * tile_row_floats(vd),
+               "the rows of sums have no room");
     return launch("splat_gather", s, {lists.entries, input}, {values});
 }
 hipError_t splat_gather_many(int, int, int n, const GatherWork *work, hipStream_t s) {
@@ -523,8 +528,16 @@ void no_pointer_kept() {
 // a batch that cannot be enqueued whole -- the memory of one of its lattices is refused, or a launch fails --
 // leaves lattices whose next builds are like any other
 bool g_refuse = false;
-void *alloc_if_allowed(void *, size_t bytes) { return g_refuse ? nullptr : std::calloc(1, bytes); }
-void free_any(void *, void *p) { std::free(p); }
+void *alloc_if_allowed(void *, size_t bytes) {
+    if (g_refuse) return nullptr;
+    void *p = std::calloc(1, bytes);
+    g_sizes[p] = bytes;
+    return p;
+}
+void free_any(void *, void *p) {
+    g_sizes.erase(p);
+    std::free(p);
+}
 void failed_batch() {
     const hipStream_t s = named_stream(1);
     const int dims[2] = {kH, kW};
@@ -580,6 +593,31 @@ void batches_either_way() {
     }
 }
 
+// the rows of sums that a build's lists turn out to have are given room when the build ends; where there is
+// none, the lattice has to be built again
+void more_rows_of_sums() {
+    const hipStream_t s = named_stream(1);
+    const int dims[2] = {kH, kW};
+    const pl_alloc alloc{alloc_if_allowed, free_any, nullptr};
+    const size_t bytes = sizeof(float) * kH * kW * kClasses;
+    float *in = nullptr, *out = nullptr, *guide = nullptr;
+    for (float **p : {&in, &out, &guide}) (void)hipMalloc((void **)p, bytes);
+    pl_handle h = nullptr;
+    expect(pl_create(5, kClasses + 1, kH * kW, s, &alloc, &h) == PL_OK, "pl_create");
+    auto build = [&]() { return pl_build_image(h, guide, 3, 2, dims, 8.0f, 0.1f); };
+    for (unsigned rows : {1u, 5000u, 40000u, 70u, 50000u}) {
+        g_rows_of_sums = rows;
+        expect(build() == PL_OK && pl_apply(h, out, in, 0) == PL_OK, "a build and an apply");
+    }
+    g_rows_of_sums = 90000u;
+    g_refuse = true;
+    expect(build() == PL_ENOMEM && pl_apply(h, out, in, 0) == PL_ESTATE, "no memory for the rows");
+    g_refuse = false;
+    expect(build() == PL_OK && pl_apply(h, out, in, 0) == PL_OK, "with memory again");
+    (void)pl_destroy(h);
+    expect(g_sizes.empty(), "memory is left");
+}
+
 }  // namespace
 
 int main(int argc, char **argv) {
@@ -595,6 +633,7 @@ int main(int argc, char **argv) {
         {"no_pointer_kept", no_pointer_kept},
         {"failed_batch", failed_batch},
         {"batches_either_way", batches_either_way},
+        {"more_rows_of_sums", more_rows_of_sums},
     };
     const auto found = scenarios.find(argc > 1 ? argv[1] : "");
     if (found == scenarios.end()) {

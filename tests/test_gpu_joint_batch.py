@@ -55,6 +55,31 @@ def test_batches(sides, guide, kinds, channels):
             ref = ref.flip(0).contiguous()
 
 
+def test_vertices_numbered_by_the_build_and_by_the_pass_in_one_launch():
+    """Of two volumes one has so many rows of sums for vertices of other workgroups that its lattice leaves the
+    numbering to the pass in its next build; the other's numbers its vertices."""
+    gen = torch.Generator(device="cuda").manual_seed(2)
+    sides = (48, 96, 96)
+    n = 48 * 96 * 96
+    ref = torch.stack([torch.rand((n, 1), generator=gen, device="cuda"),
+                       torch.linspace(0.0, 1.0, n, device="cuda").view(n, 1)]).view((2,) + sides + (1,))
+    thetas = dict(bilateral=True, theta_alpha=6.0, theta_beta=0.2, theta_gamma=1.0)
+    for call in range(4):
+        x = torch.rand((2,) + sides + (2,), generator=gen, device="cuda").requires_grad_(True)
+        up = torch.randn(x.shape, generator=gen, device="cuda")
+        out = pla.lattice_filter(x, ref, **thetas)
+        listed = [lat.info(pla.PL_INFO_FOREIGN_ROWS) >= 0 for lat in out.grad_fn.lent.lattices]
+        assert all(lat.info(pla.PL_INFO_BUILD_MERGED) == 1 for lat in out.grad_fn.lent.lattices)
+        if call:
+            assert sorted(listed) == [False, True]
+        (grad,) = torch.autograd.grad(out, x, up)
+        for b in range(2):
+            with torch.no_grad():
+                close(out[b:b + 1], pla.lattice_filter(x[b:b + 1], ref[b:b + 1], **thetas))
+                close(grad[b:b + 1], pla.lattice_filter(up[b:b + 1], ref[b:b + 1], reverse=True, **thetas))
+        del out, grad
+
+
 def test_applies_behind_one_build_each():
     """Lattices that were built one by one, with and without lists, applied together."""
     gen = torch.Generator(device="cuda").manual_seed(5)

@@ -12,7 +12,7 @@ from permutohedral_lattice_amd import build as hip_build
 
 SCENARIOS = ["read_on_the_own_stream", "replay_on_the_own_stream", "one_stream_for_all", "handle_given_out_again",
              "two_callers_and_builds", "changing_company", "own_stream_captured", "failed_blur", "no_pointer_kept",
-             "failed_batch", "batches_either_way"]
+             "failed_batch", "batches_either_way", "more_rows_of_sums"]
 
 
 @pytest.fixture(scope="module")
