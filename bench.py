@@ -64,34 +64,48 @@ def measured_traffic(kernel_name, grid_threads, stem="bench_bilateral_1024_pd5_v
     return int(sum(table[key])), stamp
 
 
-def kernel_names(pd, vd, in_channels=None, gathered=False):
-    """The kernels a filter() call of a grid of points runs for these dimensions, by stage
-    (gathered: an apply of a lattice that pl_build gave per-vertex lists)."""
+def kernel_names(pd, vd, in_channels=None, gathered=False, n=0, vertices=0, pairs=False):
+    """The kernels a filter() call of a grid of points whose build merges runs for these dimensions, by
+    stage (gathered: an apply of a lattice that pl_build gave lists; which lists depends on the points n,
+    the vertices and whether they are for pairs: lists_of_tiles in pl_kernels.h)."""
     fused = vd <= 4
     d1 = pd + 1
-    lanes = 4 if vd <= 16 else (8 if vd <= 32 else 16)
+    in_channels = in_channels if in_channels else vd - 1
+    groups = -(-(vd - 1) // 32)
+    channels = vd - 1 if groups == 1 else -(-(-(-(vd - 1) // groups)) // 4) * 4
     if fused:
         blur = "k_blur3_row<%d, float>" % vd if pd == 2 else "k_blur2_row<%d, float>" % vd
-        slice_k = "k_slice_point<%d, %d>" % (vd, d1)
+        slice_k = "k_slice_tile<%d, %d, float>" % (vd, d1)
     else:
-        blur = "k_blur2_element<float>"
-        if vd <= 8:
-            slice_k = "k_slice_point<%d, 0>" % vd
-        elif vd <= 64:
-            slice_k = "k_slice_quads<%d, %d>" % (d1, lanes)
-        else:
-            slice_k = "k_slice_channels<%d>" % d1
-    width = 16 if vd <= 16 else (32 if vd <= 32 else 64)
+        blur = "k_blur_runs<1>"
+        slice_k = "k_slice_tile_channels<%d, %d>" % (d1, -(-channels // 4)) if vd <= 64 else "k_slice_channels<%d>" % d1
     if gathered:
-        splat = ("k_splat_gather<%d, %d>" % (vd, in_channels if in_channels else vd - 1) if fused
-                 else "k_splat_gather_channels<%d>" % lanes)
+        lanes = 4 if vd <= 16 else (8 if vd <= 32 else 16)
+        corners = n * d1 / max(vertices, 1)
+        if fused:
+            rows = pd >= 3 and n >= (1 << 21 if pd == 3 else 1 << 19)
+        elif pairs and vd <= 32:
+            rows = True
+        elif n <= 1 << 15:
+            rows = corners * pd * pd >= 320
+        else:
+            rows = vd <= (32 if pd >= 4 else 24) if pd >= 3 else vd <= 16 and n <= 1 << 18 and corners >= 100
+        if rows:
+            width = 8 * min(4, -(-vd // 8))
+            splat = ("k_splat_rows<%d, %d, %d>" % (vd, in_channels, d1) if fused
+                     else "k_splat_rows_channels<%d, 0, %d, 1>" % (d1, width))
+        else:
+            splat = ("k_splat_gather<%d, %d>" % (vd, in_channels) if fused
+                     else "k_splat_gather_channels<%d, 1>" % lanes)
+    elif fused:
+        splat = "k_splat_merge<%d, %d>" % (vd, d1)
     else:
-        splat = "k_splat_dpp<%d, %d>" % (vd, d1) if fused else "k_splat_channels<%d>" % width
+        splat = "k_splat_tile<%d>" % (1 if vd <= 16 else 2) if vd <= 32 else "k_splat_channels<64>"
     return {"build": "k_build_tile<%d, %d, float>" % (pd, vd if fused else 0),
             "splat": splat, "blur_axis": blur, "slice": slice_k}
 
 
-def stage_report(lat, call, n, pd, vd, samples=5, fused_splat=True, gathered=False):
+def stage_report(lat, call, n, pd, vd, samples=5, fused_splat=True, gathered=False, pairs=False):
     """Per-stage milliseconds of `call()` (one filter or apply on `lat`) from HIP events on the
     lattice's stream, and the stage that takes longest with its share of the HBM roofline."""
     import permutohedral_lattice_amd as pla
@@ -107,7 +121,7 @@ def stage_report(lat, call, n, pd, vd, samples=5, fused_splat=True, gathered=Fal
     alg = algorithmic_bytes(n, m, pd, vd)
     if vd <= 4 and fused_splat:
         alg["build"] += alg["splat"]      # filter() splats inside the build kernel
-    names = kernel_names(pd, vd, gathered=gathered)
+    names = kernel_names(pd, vd, gathered=gathered, n=n, vertices=m, pairs=pairs)
     candidates = [k for k in ("build", "splat", "slice") if stages[k] > 0.0]
     dominant = max(candidates, key=lambda k: stages[k])
     if stages["blur"] > stages[dominant]:
@@ -190,9 +204,9 @@ def run_configs(args, pla, synth, with_cpu):
     msg = torch.empty_like(q0)
     torch.cuda.synchronize()      # (the lattices work on streams of their own)
     st_bi, dom_bi = stage_report(mf.bilateral[0], lambda: mf.bilateral[0].apply(msg, q0, False), n5, 5,
-                                 classes + 1, fused_splat=False, gathered=True)
+                                 classes + 1, fused_splat=False, gathered=True, pairs=True)
     st_sp, dom_sp = stage_report(mf.spatial[0], lambda: mf.spatial[0].apply(msg, q0, False), n5, 2,
-                                 classes + 1, fused_splat=False, gathered=True)
+                                 classes + 1, fused_splat=False, gathered=True, pairs=True)
     # an apply moves what a filter moves less the positions and the keys (the lattice is there)
     def apply_bytes(m, pd, vd):
         return 4 * n5 * 2 * (vd - 1) + m * 4 * vd * (2 * (pd + 1) + 2)
@@ -659,8 +673,7 @@ def main():
     if stages["blur"] > stages[dominant]:
         dominant = "blur_axis"
     achieved = alg[dominant] / (per_launch_ms[dominant] * 1e-3) / 1e9
-    kernel_name = {"build": "k_build_tile<5, 4, float>" if fused else "k_build_tile<5, 0, float>", "splat": "k_splat_dpp<4, 6>",
-                   "blur_axis": "k_blur2_row<4, float>", "slice": "k_slice_point<4, 6>"}[dominant]
+    kernel_name = kernel_names(pd, vd)[dominant]
     traffic, traffic_stamp = measured_traffic(kernel_name, n)
     roofline = {"bound": "hbm", "kernel": kernel_name, "achieved": round(achieved, 2),
                 "peak": HBM_PEAK_GBS, "unit": "GB/s", "frac": round(achieved / HBM_PEAK_GBS, 5),
