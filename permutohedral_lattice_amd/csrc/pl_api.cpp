@@ -2151,8 +2151,8 @@ namespace {
 // stream), because hipMalloc/hipFree per call would serialise the device.  The items of a batch are independent
 // lattices (LatticeFilterKernel.cpp:152-179), and the kernels over the few hundred thousand vertices of one item
 // leave most of the GPU idle, so up to g_op_lanes items are in flight at a time: their passes enqueued together
-// on the caller's stream (pl_filter_images) where there are kernels for it, else on lattices with streams of
-// their own, the first on the caller's.  us a call, on streams and together, RGB under itself: 2 x 64x64
+// on the caller's stream (pl_filter_images) where there are kernels for it, else on streams of their own,
+// the first on the caller's.  us a call, on streams and together, RGB under itself: 2 x 64x64
 // points 101 and 39, 2 x 512x512 101 and 70, 8 x 256x256 228 and 118, 2 x 1024x1024 221 and 179; 2 x 321x481,
 // 21 channels, 128 and 122.
 // With a caller-supplied allocator everything is taken from it and returned before the call
